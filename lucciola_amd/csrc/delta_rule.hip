@@ -267,7 +267,7 @@ struct TokenRows {
 template <int ROWS, int CHUNK, bool DEEP, int COLS, bool REMOVE>
 __global__ __launch_bounds__(COLS * SCAN_LANES) void delta_scan_kernel(
     const float* __restrict__ coef, const float* __restrict__ v, float* __restrict__ state, float* __restrict__ out,
-    const int* __restrict__ q_offsets, const int* __restrict__ slot_ids, int T, int heads, int dk, int dv) {
+    const int* __restrict__ q_offsets, const int* __restrict__ slot_ids, int T, int heads, int dk, int dv, int below) {
     constexpr int SCAN_COLUMNS = COLS, SCAN_THREADS = COLS * SCAN_LANES;
     constexpr int DKP = ROWS * SCAN_LANES;                 // key rows with padding
     constexpr int NP = REMOVE ? 5 : 3;                     // vectors a token
@@ -286,6 +286,7 @@ __global__ __launch_bounds__(COLS * SCAN_LANES) void delta_scan_kernel(
     const int head = blockIdx.y, req = blockIdx.z;
     const int j = blockIdx.x * SCAN_COLUMNS + col;         // the value channel
     const int first = q_offsets[req], last = q_offsets[req + 1];
+    if (last - first >= below) return;                     // another kernel's (scan_chunks.hip)
     float* S_home = state + (((size_t)slot_ids[req] * heads + head) * dv + (j < dv ? j : 0)) * dk + lane * ROWS;
     const bool whole = (dk % 4 == 0) && (ROWS % 4 == 0) && (lane + 1) * ROWS <= dk && j < dv;
     float S[ROWS];
@@ -532,21 +533,21 @@ LC_API int lc_conv_tail_update(const float* proj, int cols, int T, float* tails,
 }
 
 // coef [planes, T, heads dk]: five planes (decay, probe, removal, write, read) or three (decay, write,
-// read: no removal term)
+// read: no removal term).  Requests of fewer than `below` tokens; the others' states and rows of out are left alone.
 LC_API int lc_delta_scan(const float* coef, int planes, const float* v, float* state, int slots, float* out,
-                         const int* q_offsets, const int* slot_ids, int R, int T, int heads, int dk, int dv,
+                         const int* q_offsets, const int* slot_ids, int R, int T, int heads, int dk, int dv, int below,
                          hipStream_t stream) {
-    LC_CHECK(R >= 0 && T >= 0 && heads > 0 && dk > 0 && dv > 0 && slots >= 0, "delta_scan: bad sizes");
+    LC_CHECK(R >= 0 && T >= 0 && heads > 0 && dk > 0 && dv > 0 && slots >= 0 && below > 0, "delta_scan: bad sizes");
     LC_CHECK(planes == 5 || planes == 3, "delta_scan: %d vectors a token are neither 5 nor 3", planes);
     LC_CHECK(dk <= DELTA_MAX_KEY, "delta_scan: heads of %d key channels are above %d", dk, DELTA_MAX_KEY);
     if (R == 0 || T == 0) return 0;
     LC_CHECK(coef && v && state && out && q_offsets && slot_ids, "delta_scan: null pointer");
     LC_CHECK(R <= 65535 && heads <= 65535, "delta_scan: too many requests or heads for the grid");
-    const bool deep = T >= 16 * R;       // portions of prompts, mostly
+    const bool deep = T >= 16 * R && below > T;       // portions of prompts, mostly
     const dim3 grid((dv + 15) / 16, heads, R);
 #define LC_SCAN_AS(ROWS, CHUNK, DEEP, COLS, REMOVE)                                                        \
     delta_scan_kernel<ROWS, CHUNK, DEEP, COLS, REMOVE><<<grid, COLS * SCAN_LANES, 0, stream>>>(              \
-        coef, v, state, out, q_offsets, slot_ids, T, heads, dk, dv)
+        coef, v, state, out, q_offsets, slot_ids, T, heads, dk, dv, below)
 #define LC_SCAN(ROWS, CHUNK)                                            \
     do {                                                                \
         if (planes == 5) {                                              \

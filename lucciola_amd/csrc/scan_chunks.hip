@@ -1,0 +1,595 @@
+// The recurrence of delta_rule.hip,
+//     S <- diag(decay) S - removal (probe^T S) + write v^T,    o = S^T read,
+// for portions of prompts, a chunk of SC = 32 tokens at a time on the float32 matrix instruction.  Token by token a step
+// is a chain of dependent vector instructions, 0.21 us a token without and 0.29 us with the removal term, on a wave that
+// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 105 and 180).
+//
+// Inside a chunk, from the state S that the chunk before left, with a_i the product of the decays of tokens 0..i (key
+// channel by key channel), r_ij that of the tokens j+1..i, and y_i = probe_i^T S_(i-1) what token i takes out:
+//     y_i = (probe_i a_(i-1))^T S + sum_(j<i) [M_ij v_j - L_ij y_j]    L_ij = probe_i . (r_(i-1)j removal_j), M_ij with write_j
+//     o_i = (read_i a_i)^T S + sum_(j<=i) [W_ij v_j - R_ij y_j]        W_ij = read_i . (r_ij write_j),        R_ij with removal_j
+// With T = (1 + L)^-1 (unit lower triangular: forward substitution in blocks of 16), Y = T probe~ S + T M V, and put in:
+//     O  = (read~ - R T probe~) S + (W - R T M) V
+//     S' = diag(a_last) S + (write~^T - removal~^T T M) V - removal~^T (T probe~ S)
+// All that does not hold S or V is made first, chunks and heads side by side (scan_chunk_prepare_kernel); then a workgroup
+// per 16 value channels and head walks a request's chunks in order (scan_chunk_walk_kernel), with S in the accumulators.
+// Everything is float32: operands, products and sums.  No decay is ever divided by: products between tokens of one block
+// of 16 are made pair by pair, those between blocks are split at the border, so a decay of any size (0 too) is exact.
+// A token's sums are taken in another order than token by token and depend on where its chunk begins, so callers that
+// promise the same bits for every cut of a prompt (float32 models) and steps of few tokens keep the other kernel.
+// A chunk's products meet every value of the chunk: a NaN or an infinity in a token's vectors or values reaches the
+// chunk's earlier tokens too (never another request).
+#include "common.h"
+
+namespace lc {
+
+constexpr int SC = 32;                  // tokens of a chunk: two blocks of 16
+constexpr int SCP = SC + 4;             // floats of a row of a [SC x SC] matrix in LDS: b128 reads of 16 rows meet no bank twice
+
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+
+__device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0); }
+
+// What the first kernel leaves of a chunk and head, in floats: read^ [SC][DK], Z [DK][SC], the chunk's decay [2][DK] (the
+// number in 32 bits and what that leaves out: a model's constant decay would be off by the same last bit in every chunk),
+// W^ [SC][SC], and with a removal term T probe~ [SC][DK] and -removal~^T [DK][SC].  The matrices lie as the operands that the
+// second kernel loads, 1 KB a [16 x 16] tile: lane (row, quad) has entries 4 quad .. + 3 of a row (in rows
+// the walk, whose loads then touch sixteen half lines each, took 109 us where it takes 95 and, removing, 199 us where 145).
+template <int DK, bool REMOVE>
+struct ChunkRecord {
+    static constexpr int READ = 0, Z = SC * DK, DECAY = 2 * SC * DK, MIX = DECAY + 2 * DK, PROBE = MIX + SC * SC,
+                         REMOVAL = PROBE + SC * DK, SIZE = REMOVE ? REMOVAL + SC * DK : PROBE;
+};
+
+// The records of request r's chunks begin at q_offsets[r] / SC + r: no two requests share one, whatever their lengths.
+__device__ __forceinline__ int first_record(const int* __restrict__ q_offsets, int r) { return q_offsets[r] / SC + r; }
+
+// The [16 x 16] tile A B over 16 KT k, k = 16 t + 4 (lane / 16) + i: a(t) holds four neighbouring k of the lane's row of A, b(t)
+// of its column of B, so that rows are read 16 bytes at a time.  A lane gets rows 4 (lane / 16) .. + 3 of column lane % 16,
+// which is in the same order what it holds of a B operand of 16 k.  Every t has a sum of its own, added pairwise: the
+// matrix instruction adds one product after the other, and the long sums were what set a chunk's error (16 heads of
+// 128, float64 beside it: 2.3e-7 of the result with one sum, 1.5e-7 so; token by token 1.4e-7).
+template <int KT, class A, class B>
+__device__ __forceinline__ f32x4 tile_product(A a, B b) {
+    f32x4 c[KT];
+#pragma unroll
+    for (int t = 0; t < KT; ++t) {
+        const f32x4 x = a(t), y = b(t);
+        c[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < 4; ++i) c[t] = mfma4(x[i], y[i], c[t]);
+    }
+#pragma unroll
+    for (int n = KT / 2; n >= 1; n /= 2)
+#pragma unroll
+        for (int t = 0; t < n; ++t) c[t] += c[t + n];
+    return c[0];
+}
+
+// grid (records, heads).  coef [5 or 3][T, heads DK] as delta_rule.hip has it.  2,048 tokens, 16 heads of 128: 26 us, and with
+// a removal term, where a workgroup fills its CU's LDS and its steps follow each other, 62 us.
+template <int DK, bool REMOVE, int THREADS>
+__global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float* __restrict__ coef,
+                                                                     const int* __restrict__ q_offsets, int R, int T,
+                                                                     int heads, int least, float* __restrict__ records) {
+    typedef ChunkRecord<DK, REMOVE> Rec;
+    constexpr int DKP = DK + 4, WAVES = THREADS / kWave, NP = REMOVE ? 5 : 3;
+    constexpr int DECAY = 0, PROBE = 1, REMOVAL = 2, WRITE = REMOVE ? 3 : 1, READ = REMOVE ? 4 : 2;
+    constexpr int MATS = REMOVE ? 4 : 1;                    // W = read x write, R = read x removal, M = probe x write, L = probe x removal
+    __shared__ __attribute__((aligned(16))) float plane[NP][SC][DKP];
+    __shared__ __attribute__((aligned(16))) float mat[MATS][SC][SCP];
+    __shared__ __attribute__((aligned(16))) float inverse[REMOVE ? SC : 1][SCP], scratch[REMOVE ? 16 : 1][20];
+    __shared__ __attribute__((aligned(16))) float total[2][DK];     // a block's decay
+    __shared__ double whole[2][DK];
+    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, row = lane & 15, quad = lane >> 4;
+    const int record = blockIdx.x, head = blockIdx.y;
+    int low = 0, high = R - 1;                              // the request whose records hold this one
+    while (low < high) {
+        const int mid = (low + high + 1) / 2;
+        if (first_record(q_offsets, mid) <= record) low = mid;
+        else high = mid - 1;
+    }
+    const int last = q_offsets[low + 1], t0 = q_offsets[low] + (record - first_record(q_offsets, low)) * SC;
+    if (t0 >= last || last - q_offsets[low] < least) return;
+    const int count = min(SC, last - t0);
+    float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
+
+    // the chunk's vectors; a place behind the request's end keeps the state and adds nothing
+    for (int idx = tid; idx < NP * SC * (DK / 4); idx += THREADS) {
+        const int i = idx % (DK / 4), t = idx / (DK / 4) % SC, p = idx / (DK / 4 * SC);
+        const float pad = p == DECAY ? 1.f : 0.f;
+        f32x4 x = {pad, pad, pad, pad};
+        if (t < count) x = *reinterpret_cast<const f32x4*>(coef + ((size_t)p * T + t0 + t) * heads * DK + (size_t)head * DK + 4 * i);
+        *reinterpret_cast<f32x4*>(&plane[p][t][4 * i]) = x;
+    }
+    __syncthreads();
+
+    // every vector at its block's border.  A thread is a key channel of a block, and of the reading (read, probe) or the
+    // writing side (write, removal); the products of the decays are made in 64 bits and rounded once.
+    constexpr int SIDES = THREADS / (2 * DK);
+    static_assert(SIDES >= 1, "a thread a channel of a block");
+    const int block = tid / DK % 2, channel = tid % DK, side = tid / (2 * DK);
+    float decay[16];
+#pragma unroll
+    for (int i = 0; i < 16; ++i) decay[i] = plane[DECAY][16 * block + i][channel];
+    double through = 1.0;
+#pragma unroll
+    for (int i = 0; i < 16; ++i) through *= (double)decay[i];
+    if (side == 0) {
+        whole[block][channel] = through;
+        total[block][channel] = (float)through;
+    }
+    // Where no channel forgets more than 2^-60 of itself in 16 tokens, the pairs of a block are products of the vectors times
+    // and over the decays from the block's first token on, on the matrix instruction: a division by what is far from the
+    // smallest number loses nothing.  Else the pairs are made one by one, by vector instructions, several times as long.
+    const bool far = __syncthreads_or(!(through >= 0x1p-60 && through <= 0x1p60));
+    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+    auto put = [&](float (*to)[SCP], int r0, int c0, f32x4 v) {
+#pragma unroll
+        for (int i = 0; i < 4; ++i) to[r0 + 4 * quad + i][c0 + row] = v[i];
+    };
+    auto keep_tile = [&](int matrix, int tile, f32x4 v) { *reinterpret_cast<f32x4*>(out + matrix + tile * 256 + lane * 4) = v; };
+    // four neighbouring entries of the lane's row of a matrix or plane, and of its column
+    auto along = [&](const float* m, int pitch, int r0, int c0) { return *reinterpret_cast<const f32x4*>(m + (r0 + row) * pitch + c0 + 4 * quad); };
+    auto down = [&](const float* m, int pitch, int r0, int c0) {
+        f32x4 v;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) v[i] = m[(r0 + 4 * quad + i) * pitch + c0 + row];
+        return v;
+    };
+    if (far) {
+        // lane (j, quad) carries write_j and removal_j through the decays of the tokens behind j, for every fourth group of
+        // four key channels, and meets read_i or probe_i (which does not see token i's decay) on the way
+        constexpr int ROLES = REMOVE ? 4 : 2;               // (block, read or probe)
+        constexpr int G = DK / 16;
+        static_assert(WAVES >= ROLES, "a wave a role");
+        if (wave < ROLES) {
+            const int base = 16 * (wave & 1);
+            const bool by_probe = wave >= 2;
+            f32x4 w[G], x[REMOVE ? G : 1];
+#pragma unroll
+            for (int m = 0; m < G; ++m) {
+                w[m] = *reinterpret_cast<const f32x4*>(&plane[WRITE][base + row][16 * m + 4 * quad]);
+                if constexpr (REMOVE) x[m] = *reinterpret_cast<const f32x4*>(&plane[REMOVAL][base + row][16 * m + 4 * quad]);
+            }
+            for (int i = 0; i < 16; ++i) {
+                const int from = by_probe ? i - 1 : i;      // the last decay that the reader sees
+                float with_w = 0.f, with_x = 0.f;
+                const float* by = &plane[REMOVE && by_probe ? PROBE : READ][base + i][4 * quad];
+                const float* keep = &plane[DECAY][base + max(from, 0)][4 * quad];
+#pragma unroll
+                for (int m = 0; m < G; ++m) {
+                    const f32x4 d = *reinterpret_cast<const f32x4*>(keep + 16 * m), q = *reinterpret_cast<const f32x4*>(by + 16 * m);
+#pragma unroll
+                    for (int e = 0; e < 4; ++e) {
+                        const float f = from > row ? d[e] : 1.f;
+                        w[m][e] *= f;
+                        with_w = fmaf(q[e], w[m][e], with_w);
+                        if constexpr (REMOVE) {
+                            x[m][e] *= f;
+                            with_x = fmaf(q[e], x[m][e], with_x);
+                        }
+                    }
+                }
+                with_w += __shfl_xor(with_w, 16, kWave);
+                with_w += __shfl_xor(with_w, 32, kWave);
+                const bool seen = by_probe ? row < i : row <= i;
+                if (quad == 0) mat[REMOVE && by_probe ? 2 : 0][base + i][base + row] = seen ? with_w : 0.f;
+                if constexpr (REMOVE) {
+                    with_x += __shfl_xor(with_x, 16, kWave);
+                    with_x += __shfl_xor(with_x, 32, kWave);
+                    if (quad == 0) mat[by_probe ? 3 : 1][base + i][base + row] = seen ? with_x : 0.f;
+                }
+            }
+        }
+        __syncthreads();
+    }
+    // far: read and probe from the block's first token on, write and removal to its last; else those over the decays
+    auto scale_reading = [&]() {
+        double a = 1.0;
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            if constexpr (REMOVE) plane[PROBE][16 * block + i][channel] *= (float)a;
+            a *= (double)decay[i];
+            plane[READ][16 * block + i][channel] *= (float)a;
+        }
+    };
+    auto scale_writing = [&]() {
+        double a = far ? 1.0 : 1.0 / through;
+#pragma unroll
+        for (int i = 15; i >= 0; --i) {
+            plane[WRITE][16 * block + i][channel] *= (float)a;
+            if constexpr (REMOVE) plane[REMOVAL][16 * block + i][channel] *= (float)a;
+            a *= (double)decay[i];
+        }
+    };
+    if (side == 0) scale_reading();
+    if (side == SIDES - 1) scale_writing();
+    __syncthreads();
+
+    // pairs between the two blocks (nothing of the second reaches the first), and, unless they are there, inside them
+    auto rows_of = [&](int p, int first) { return [&, p, first](int t) { return along(&plane[p][0][0], DKP, first, 16 * t); }; };
+    for (int role = wave; role < MATS * 3; role += WAVES) {
+        const int m = role % MATS, tile = role / MATS;      // tile 0: between; 1, 2: inside
+        const bool probes = REMOVE && m >= 2;
+        const int by = probes ? PROBE : READ, with = REMOVE && (m & 1) ? REMOVAL : WRITE;
+        if (tile == 0) {
+            auto lasting = [&](int t) {
+                f32x4 v = rows_of(with, 0)(t);
+                if (!far) v *= *reinterpret_cast<const f32x4*>(&total[0][16 * t + 4 * quad]);
+                return v;
+            };
+            put(mat[m], 16, 0, tile_product<DK / 16>(rows_of(by, 16), lasting));
+            put(mat[m], 0, 16, zero);
+        } else if (!far) {
+            const int base = 16 * (tile - 1);
+            f32x4 v = tile_product<DK / 16>(rows_of(by, base), rows_of(with, base));
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                const int reader = 4 * quad + i;
+                v[i] = (probes ? row < reader : row <= reader) ? v[i] : 0.f;
+            }
+            put(mat[m], base, base, v);
+        }
+    }
+    __syncthreads();
+
+    // from the chunk's first token on, and to its last
+    for (int idx = tid; idx < 16 * DK; idx += THREADS) {
+        const int i = idx / DK, k = idx % DK;
+        const float to_border = far ? 1.f : total[0][k], rest = far ? 1.f : total[1][k];
+        plane[READ][16 + i][k] *= total[0][k];
+        plane[WRITE][i][k] *= to_border * total[1][k];
+        plane[WRITE][16 + i][k] *= rest;
+        if constexpr (REMOVE) {
+            plane[PROBE][16 + i][k] *= total[0][k];
+            plane[REMOVAL][i][k] *= to_border * total[1][k];
+            plane[REMOVAL][16 + i][k] *= rest;
+        }
+    }
+    for (int k = tid; k < DK; k += THREADS) {
+        const double d = whole[0][k] * whole[1][k];
+        const float near = (float)d;
+        out[Rec::DECAY + k] = near;
+        out[Rec::DECAY + DK + k] = (float)(d - (double)near);
+    }
+
+    __syncthreads();
+    constexpr int KEYS = DK / 16, TILES = 2 * KEYS;
+    if constexpr (REMOVE) {
+        const float *W = mat[0][0], *Rm = mat[1][0], *M = mat[2][0], *L = mat[3][0];
+        float* inv = inverse[0];
+        // T's diagonal blocks: lane (column, block) by forward substitution
+        if (wave == 0 && lane < 32) {
+            const int base = lane & 16, c = lane & 15;
+            float x[16];
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                float s = i == c ? 1.f : 0.f;
+#pragma unroll
+                for (int j = 0; j < i; ++j) s = fmaf(-L[(base + i) * SCP + base + j], x[j], s);
+                x[i] = s;
+            }
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                inverse[base + i][base + c] = x[i];
+                if (base) inverse[i][16 + c] = 0.f;
+            }
+        }
+        __syncthreads();
+        // T10 = -T11 L10 T00
+        if (wave == 0) {
+            const f32x4 lt = tile_product<1>([&](int) { return along(L, SCP, 16, 0); }, [&](int) { return down(inv, SCP, 0, 0); });
+#pragma unroll
+            for (int i = 0; i < 4; ++i) scratch[4 * quad + i][row] = -lt[i];
+        }
+        __syncthreads();
+        if (wave == 0)
+            put(inverse, 16, 0, tile_product<1>([&](int) { return along(inv, SCP, 16, 16); },
+                                                [&](int) { return down(scratch[0], 20, 0, 0); }));
+        __syncthreads();
+        // T M over M's place (kept in registers until everybody has read M); T probe~, transposed, over the decays
+        f32x4 tm = zero;
+        if (wave < 4)
+            tm = tile_product<2>([&](int t) { return along(inv, SCP, 16 * (wave >> 1), 16 * t); },
+                                 [&](int t) { return down(M, SCP, 16 * t, 16 * (wave & 1)); });
+        for (int tile = wave; tile < TILES; tile += WAVES) {
+            const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
+            const f32x4 v = tile_product<2>([&](int t) { return down(plane[PROBE][0], DKP, 16 * t, k0); },
+                                            [&](int t) { return along(inv, SCP, t0, 16 * t); });
+            *reinterpret_cast<f32x4*>(&plane[DECAY][t0 + row][k0 + 4 * quad]) = v;
+            keep_tile(Rec::PROBE, tile, v);
+        }
+        __syncthreads();
+        if (wave < 4) put(mat[2], 16 * (wave >> 1), 16 * (wave & 1), tm);
+        __syncthreads();
+        // read^ = read~ - R (T probe~);  Z = write~^T - removal~^T (T M);  W^ = W - R (T M): each transposed, as a lane's entries lie
+        for (int tile = wave; tile < TILES; tile += WAVES) {
+            const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
+            const f32x4 v = tile_product<2>([&](int t) { return down(plane[DECAY][0], DKP, 16 * t, k0); },
+                                            [&](int t) { return along(Rm, SCP, t0, 16 * t); });
+            keep_tile(Rec::READ, tile, along(plane[READ][0], DKP, t0, k0) - v);
+        }
+        for (int tile = wave; tile < TILES; tile += WAVES) {
+            const int k0 = 16 * (tile / 2), t0 = 16 * (tile % 2);
+            const f32x4 z = tile_product<2>([&](int t) { return down(M, SCP, 16 * t, t0); },
+                                            [&](int t) { return down(plane[REMOVAL][0], DKP, 16 * t, k0); });
+            keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, t0, k0) - z);
+            keep_tile(Rec::REMOVAL, tile, -down(plane[REMOVAL][0], DKP, t0, k0));
+        }
+        if (wave < 4) {
+            const int r0 = 16 * (wave >> 1), c0 = 16 * (wave & 1);
+            const f32x4 v = tile_product<2>([&](int t) { return down(M, SCP, 16 * t, c0); },
+                                            [&](int t) { return along(Rm, SCP, r0, 16 * t); });
+            keep_tile(Rec::MIX, wave, along(W, SCP, r0, c0) - v);
+        }
+    } else {
+        for (int tile = wave; tile < TILES; tile += WAVES) {
+            keep_tile(Rec::READ, tile, along(plane[READ][0], DKP, 16 * (tile / KEYS), 16 * (tile % KEYS)));
+            keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, 16 * (tile % 2), 16 * (tile / 2)));
+        }
+        for (int tile = wave; tile < 4; tile += WAVES) keep_tile(Rec::MIX, tile, along(mat[0][0], SCP, 16 * (tile >> 1), 16 * (tile & 1)));
+    }
+}
+
+// One workgroup per (16 value channels, head, request).  Four waves keep S, a quarter of the key rows each, as accumulators
+// (KT tiles of 16), which are B operands of the next products as they are, and take it from chunk to chunk; four others make
+// the chunks' read-outs from copies of S that the first leave in LDS, a chunk behind.  So a SIMD has two waves, and one's loads,
+// LDS trips and address arithmetic pass beside the other's products (with the read-outs made by the waves that keep S, one wave a
+// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 79 and 119).  What the
+// waves make of their key rows meets in LDS, two buffers in turn, one barrier a chunk.  A chunk's record is asked for two chunks
+// ahead.  Workgroups are numbered so that the blocks of one head, which read the same records, run on one XCD (workgroup
+// i on XCD i % 8) where the heads are a multiple of 8.
+template <int DK, bool REMOVE>
+__global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __restrict__ records, const float* __restrict__ v,
+                                                              float* __restrict__ state, float* __restrict__ out,
+                                                              const int* __restrict__ q_offsets,
+                                                              const int* __restrict__ slot_ids, int heads, int dv, int least) {
+    typedef ChunkRecord<DK, REMOVE> Rec;
+    constexpr int KT = DK / 64, TT = SC / 16, KEYS = DK / 16;
+    __shared__ f32x4 states[2][4][KT][kWave], reads[2][4][TT][kWave], taken[REMOVE ? 2 : 1][4][TT][kWave];
+    const int lane = threadIdx.x % kWave, row = lane & 15, quad = lane >> 4;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) & 3;
+    const bool keeps = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) < 4;
+    const int head = blockIdx.x % heads, block = blockIdx.x / heads, req = blockIdx.y;
+    const int first = q_offsets[req], last = q_offsets[req + 1];
+    if (last - first < least) return;
+    const int chunks = (last - first + SC - 1) / SC;
+    const int j = block * 16 + row;                         // the value channel
+    const bool mine = j < dv;                               // a channel behind dv works through the head's first one's values
+    const int column = mine ? j : 0;
+    const unsigned line = heads * dv;                       // floats from a token's values to the next one's, below 2^23
+    const float* values = v + (size_t)first * line + (size_t)head * dv;
+    const float* record = records + ((size_t)first_record(q_offsets, req) * heads + head) * Rec::SIZE;
+    // a chunk's record and values; behind the last chunk the last one's once more.  Entries that lie behind the request's
+    // end are zero in the records, so such a token's value (the last token's) only has to be a number.
+    auto record_of = [&](int c) { return record + (size_t)min(c, chunks - 1) * heads * Rec::SIZE; };
+    auto tile = [&](const float* rec, int matrix, int n) { return *reinterpret_cast<const f32x4*>(rec + (matrix + n * 256) + lane * 4); };
+    auto value_of = [&](int c, int t, int i) {
+        const int base = min(c, chunks - 1) * SC;
+        const unsigned token = min(16 * t + 4 * quad + i, last - first - 1 - base);
+        return (values + (size_t)base * line)[__umul24(token, line) + column];
+    };
+    // only LDS has to be in order between the waves: loads from memory stay in flight
+    auto meet = []() {
+        asm volatile("" ::: "memory");
+        wait_lgkmcnt<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    if (keeps) {
+        float* home = state + (((size_t)slot_ids[req] * heads + head) * dv + column) * DK + wave * 16 * KT + 4 * quad;
+        f32x4 S[KT];
+#pragma unroll
+        for (int k = 0; k < KT; ++k) S[k] = *reinterpret_cast<const f32x4*>(home + 16 * k);
+        struct Loaded {
+            f32x4 z[KT][TT], probe[REMOVE ? TT : 1][KT], removal[KT][REMOVE ? TT : 1], decay[KT], rest[KT];
+            float value[TT][4];
+        };
+        auto fetch = [&](Loaded& l, int c) {
+            const float* rec = record_of(c);
+            if constexpr (REMOVE) {
+#pragma unroll
+                for (int t = 0; t < TT; ++t)
+#pragma unroll
+                    for (int k = 0; k < KT; ++k) l.probe[t][k] = tile(rec, Rec::PROBE, t * KEYS + wave * KT + k);
+            }
+#pragma unroll
+            for (int k = 0; k < KT; ++k) {
+                const float* decay = rec + (Rec::DECAY + 16 * (wave * KT + k)) + 4 * quad;
+                l.decay[k] = *reinterpret_cast<const f32x4*>(decay);
+                l.rest[k] = *reinterpret_cast<const f32x4*>(decay + DK);
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) l.value[t][i] = value_of(c, t, i);
+#pragma unroll
+                for (int k = 0; k < KT; ++k) l.z[k][t] = tile(rec, Rec::Z, (wave * KT + k) * TT + t);
+            }
+            if constexpr (REMOVE) {
+#pragma unroll
+                for (int t = 0; t < TT; ++t)
+#pragma unroll
+                    for (int k = 0; k < KT; ++k) l.removal[k][t] = tile(rec, Rec::REMOVAL, (wave * KT + k) * TT + t);
+            }
+        };
+        auto work = [&](const Loaded& l, int c) {
+            const int turn = c & 1;
+#pragma unroll
+            for (int k = 0; k < KT; ++k) states[turn][wave][k][lane] = S[k];
+            if constexpr (REMOVE) {
+                f32x4 y[TT];
+#pragma unroll
+                for (int t = 0; t < TT; ++t) y[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int k = 0; k < KT; ++k)
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int t = 0; t < TT; ++t) y[t] = mfma4(l.probe[t][k][i], S[k][i], y[t]);
+#pragma unroll
+                for (int t = 0; t < TT; ++t) taken[turn][wave][t][lane] = y[t];
+            }
+#pragma unroll
+            for (int k = 0; k < KT; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i) S[k][i] = fmaf(S[k][i], l.rest[k][i], S[k][i] * l.decay[k][i]);
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int k = 0; k < KT; ++k) S[k] = mfma4(l.z[k][t][i], l.value[t][i], S[k]);
+            meet();
+            if constexpr (REMOVE) {
+#pragma unroll
+                for (int t = 0; t < TT; ++t) {
+                    const f32x4 y = (taken[turn][0][t][lane] + taken[turn][1][t][lane]) +
+                                    (taken[turn][2][t][lane] + taken[turn][3][t][lane]);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i)
+#pragma unroll
+                        for (int k = 0; k < KT; ++k) S[k] = mfma4(l.removal[k][t][i], y[i], S[k]);
+                }
+            }
+        };
+        Loaded sets[3];
+        fetch(sets[0], 0);
+        fetch(sets[1], 1);
+        for (int c = 0;;) {
+            fetch(sets[2], c + 2);
+            work(sets[0], c);
+            if (++c == chunks) break;
+            fetch(sets[0], c + 2);
+            work(sets[1], c);
+            if (++c == chunks) break;
+            fetch(sets[1], c + 2);
+            work(sets[2], c);
+            if (++c == chunks) break;
+        }
+        meet();                                             // the last chunk's read-outs
+        if (mine) {
+#pragma unroll
+            for (int k = 0; k < KT; ++k) *reinterpret_cast<f32x4*>(home + 16 * k) = S[k];
+        }
+    } else {
+        struct Loaded {
+            f32x4 read[TT][KT], mix;
+            float value[4];
+        };
+        auto fetch = [&](Loaded& l, int c) {
+            const float* rec = record_of(c);
+#pragma unroll
+            for (int t = 0; t < TT; ++t)
+#pragma unroll
+                for (int k = 0; k < KT; ++k) l.read[t][k] = tile(rec, Rec::READ, t * KEYS + wave * KT + k);
+            l.mix = tile(rec, Rec::MIX, wave);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) l.value[i] = value_of(c, wave & 1, i);
+        };
+        auto work = [&](const Loaded& l, int c) {
+            const int turn = c & 1;
+            meet();                                         // the state before chunk c is there
+            f32x4 o[TT], mixed = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int t = 0; t < TT; ++t) o[t] = mixed;
+            // a wave takes one of the four blocks of W^ (the one above the diagonal is zero)
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mixed = mfma4(l.mix[i], l.value[i], mixed);
+#pragma unroll
+            for (int k = 0; k < KT; ++k) {
+                const f32x4 S = states[turn][wave][k][lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int t = 0; t < TT; ++t) o[t] = mfma4(l.read[t][k][i], S[i], o[t]);
+            }
+#pragma unroll
+            for (int t = 0; t < TT; ++t) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) o[t][i] += wave >> 1 == t ? mixed[i] : 0.f;
+                reads[turn][wave][t][lane] = o[t];
+            }
+        };
+        // chunk c's read-outs, two of a tile's rows a wave, once every wave has left its part
+        float* to = out + (size_t)first * line + (size_t)head * dv;
+        const int t = wave & 1, half = wave >> 1;
+        auto write = [&](int c) {
+            const float2* part = reinterpret_cast<const float2*>(&reads[c & 1][0][t][lane]) + half;
+            constexpr int NEXT = TT * kWave * 2;            // float2s from a wave's part to the next one's
+            const float2 p = part[0], q = part[NEXT], r = part[2 * NEXT], s = part[3 * NEXT];
+            const int token = 16 * t + 4 * quad + 2 * half, count = last - first - c * SC;
+            float* at = to + (size_t)(c * SC) * line;
+            if (mine && token < count) at[__umul24(token, line) + j] = (p.x + q.x) + (r.x + s.x);
+            if (mine && token + 1 < count) at[__umul24(token + 1, line) + j] = (p.y + q.y) + (r.y + s.y);
+        };
+        Loaded sets[3];
+        fetch(sets[0], 0);
+        fetch(sets[1], 1);
+        for (int c = 0;;) {
+            fetch(sets[2], c + 2);
+            work(sets[0], c);
+            if (c > 0) write(c - 1);
+            if (++c == chunks) break;
+            fetch(sets[0], c + 2);
+            work(sets[1], c);
+            write(c - 1);
+            if (++c == chunks) break;
+            fetch(sets[1], c + 2);
+            work(sets[2], c);
+            write(c - 1);
+            if (++c == chunks) break;
+        }
+        meet();
+        write(chunks - 1);
+    }
+}
+
+template <int DK, bool REMOVE>
+static void scan_chunks(const float* coef, const float* v, float* state, float* out, float* records, const int* q_offsets,
+                        const int* slot_ids, int R, int T, int heads, int dv, int least, hipStream_t stream) {
+    constexpr int THREADS = REMOVE ? 4 * DK : 2 * DK;
+    scan_chunk_prepare_kernel<DK, REMOVE, THREADS>
+        <<<dim3(T / SC + R, heads), THREADS, 0, stream>>>(coef, q_offsets, R, T, heads, least, records);
+    scan_chunk_walk_kernel<DK, REMOVE><<<dim3(heads * ((dv + 15) / 16), R), 512, 0, stream>>>(
+        records, v, state, out, q_offsets, slot_ids, heads, dv, least);
+}
+
+}  // namespace lc
+
+using namespace lc;
+
+// Floats that lc_scan_chunks wants as `records` for T tokens of R requests, or 0 where it does not take these sizes.
+LC_API long long lc_scan_chunks_records(int planes, int R, int T, int heads, int dk, int dv) {
+    if (R <= 0 || T <= 0 || heads <= 0 || dv <= 0 || (long long)heads * dv >= (1 << 23) || (planes != 3 && planes != 5) || (dk != 64 && dk != 128)) return 0;
+    const long long size = dk == 64 ? (planes == 5 ? ChunkRecord<64, true>::SIZE : ChunkRecord<64, false>::SIZE)
+                                    : (planes == 5 ? ChunkRecord<128, true>::SIZE : ChunkRecord<128, false>::SIZE);
+    return size * heads * (T / SC + R);
+}
+
+// The recurrence for the requests of at least `least` tokens; the others' states and rows of out are left alone.
+// coef, v, state, out as for lc_delta_scan, all 16-byte aligned.
+LC_API int lc_scan_chunks(const float* coef, int planes, const float* v, float* state, int slots, float* out, float* records,
+                          const int* q_offsets, const int* slot_ids, int R, int T, int heads, int dk, int dv, int least,
+                          hipStream_t stream) {
+    LC_CHECK(R >= 0 && T >= 0 && heads > 0 && dk > 0 && dv > 0 && slots >= 0 && least >= 1, "scan_chunks: bad sizes");
+    if (R == 0 || T == 0) return 0;
+    LC_CHECK(lc_scan_chunks_records(planes, R, T, heads, dk, dv) > 0, "scan_chunks: sizes it does not take");
+    LC_CHECK(coef && v && state && out && records && q_offsets && slot_ids, "scan_chunks: null pointer");
+    LC_CHECK(((uintptr_t)coef | (uintptr_t)state | (uintptr_t)records) % 16 == 0, "scan_chunks: not aligned to 16 bytes");
+    LC_CHECK(R <= 65535 && heads <= 65535, "scan_chunks: too many requests or heads for the grid");
+    LC_CHECK((long long)heads * dv < (1 << 23), "scan_chunks: a token's values are too many");
+#define LC_CHUNKS(DK)                                                                                                      \
+    do {                                                                                                                   \
+        if (planes == 5)                                                                                                   \
+            scan_chunks<DK, true>(coef, v, state, out, records, q_offsets, slot_ids, R, T, heads, dv, least, stream);       \
+        else                                                                                                               \
+            scan_chunks<DK, false>(coef, v, state, out, records, q_offsets, slot_ids, R, T, heads, dv, least, stream);      \
+    } while (0)
+    if (dk == 128) LC_CHUNKS(128);
+    else LC_CHUNKS(64);
+#undef LC_CHUNKS
+    LC_LAUNCH_CHECK("scan_chunks");
+    return 0;
+}

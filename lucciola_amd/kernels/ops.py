@@ -99,7 +99,8 @@ _SIGNATURES = {
     "lc_general_delta_prepare": "piiiipppffppp",
     "lc_gated_delta_prepare": "piiiiiippippfpppppp",
     "lc_conv_tail_update": "piipiiippip",
-    "lc_delta_scan": "pippipppiiiiip",
+    "lc_delta_scan": "pippipppiiiiiip",
+    "lc_scan_chunks": "pippippppiiiiiip",
     "lc_head_gate_norm": "ppiipifiiiipip",
     "lc_moe_route_logits": "pipiiippp",
     "lc_moe_combine_shared": "pppiiipipiipip",
@@ -178,6 +179,8 @@ def library():
         lib.lc_gemm_generic_workspace.argtypes = [ctypes.c_int] * 3
         lib.lc_attention_generic_workspace.restype = ctypes.c_longlong
         lib.lc_attention_generic_workspace.argtypes = [ctypes.c_int] * 5
+        lib.lc_scan_chunks_records.restype = ctypes.c_longlong
+        lib.lc_scan_chunks_records.argtypes = [ctypes.c_int] * 6
         for name, sig in _SIGNATURES.items():
             _declare(lib, name, sig)
         if lib.lc_attn_page_granule() != ATTENTION_PAGE_GRANULE:
@@ -1866,8 +1869,54 @@ def delta_scan(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, q_offse
     out = torch.empty((T, heads * value_dim), dtype=torch.float32, device=v.device)
     if T:
         _call("lc_delta_scan", _ptr(coef), coef.shape[0], _ptr(v), _ptr(state), state.shape[0], _ptr(out), _ptr(q_offsets),
-              _ptr(slot_ids), num_requests, T, heads, key_dim, value_dim, _stream())
+              _ptr(slot_ids), num_requests, T, heads, key_dim, value_dim, 0x7FFFFFFF, _stream())
     return out
+
+
+# From this many tokens on a request's portion goes a chunk at a time (``delta_scan_step``).
+SCAN_CHUNKS_FROM = 64
+
+
+def delta_scan_chunks(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, q_offsets: torch.Tensor, slot_ids: torch.Tensor,
+                      num_requests: int, heads: int, key_dim: int, value_dim: int, some_short: bool) -> torch.Tensor:
+    """As ``delta_scan``, the requests of SCAN_CHUNKS_FROM tokens and more a chunk at a time: float32 throughout, but a token's
+    sums are taken in an order that depends on where its request's portion begins.  ``some_short``: there are requests of
+    fewer tokens, which go token by token."""
+    T = v.shape[0]
+    need = library().lc_scan_chunks_records(coef.shape[0], num_requests, T, heads, key_dim, value_dim)
+    if need <= 0:
+        raise KernelError(f"delta_scan_chunks: heads of {key_dim} key channels are not 64 or 128")
+    if tuple(coef.shape[1:]) != (T, heads * key_dim) or v.shape[1] != heads * value_dim or \
+            tuple(state.shape[1:]) != (heads, value_dim, key_dim):
+        raise KernelError("delta_scan_chunks: coef, v or the state do not fit the heads")
+    for t, what in ((coef, "coef"), (v, "v"), (state, "state")):
+        _need(t, f"delta_scan_chunks {what}", torch.float32, t.dim())
+    if q_offsets.shape[0] != num_requests + 1 or slot_ids.shape[0] != num_requests:
+        raise KernelError("delta_scan_chunks: the request lists do not fit")
+    _need(q_offsets, "q_offsets", torch.int32, 1)
+    _need(slot_ids, "slot_ids", torch.int32, 1)
+    out = torch.empty((T, heads * value_dim), dtype=torch.float32, device=v.device)
+    records = torch.empty(need, dtype=torch.float32, device=v.device)
+    lists = (_ptr(q_offsets), _ptr(slot_ids), num_requests, T, heads, key_dim, value_dim, SCAN_CHUNKS_FROM, _stream())
+    _call("lc_scan_chunks", _ptr(coef), coef.shape[0], _ptr(v), _ptr(state), state.shape[0], _ptr(out), _ptr(records), *lists)
+    if some_short:
+        _call("lc_delta_scan", _ptr(coef), coef.shape[0], _ptr(v), _ptr(state), state.shape[0], _ptr(out), *lists)
+    return out
+
+
+def delta_scan_step(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, batch, heads: int, key_dim: int,
+                    value_dim: int, dtype: torch.dtype) -> torch.Tensor:
+    """The recurrence for a step's batch in a model of ``dtype``.  A float32 model's logits have the same bits for every cut
+    of a prompt, so its tokens go one by one; a bfloat16 model's long portions go a chunk at a time, where the head's sizes
+    are ones that the chunks' kernels take and the tensors begin at a whole 16 bytes.  16 heads of 128 x 128, one portion, us
+    token by token and in chunks: 48 tokens 12 and 15, 64 tokens 15 and 15, 96 tokens 21 and 15, 2,048 tokens 439 and 105; with
+    the removal term 15 and 19, 19 and 20, 30 and 23, 590 and 180."""
+    lists = (batch.q_offsets, batch.slot_ids, batch.num_requests, heads, key_dim, value_dim)
+    if dtype != torch.float32 and key_dim in (64, 128) and v.is_cuda and batch.num_tokens >= SCAN_CHUNKS_FROM:
+        lengths = [b - a for a, b in zip(batch.q_start, batch.q_start[1:])]
+        if max(lengths) >= SCAN_CHUNKS_FROM and not (coef.data_ptr() | state.data_ptr()) % 16:
+            return delta_scan_chunks(coef, v, state, *lists, some_short=min(lengths) < SCAN_CHUNKS_FROM)
+    return delta_scan(coef, v, state, *lists)
 
 
 HEAD_GATES = {"sigmoid": 0, "silu": 1}

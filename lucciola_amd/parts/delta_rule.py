@@ -89,8 +89,7 @@ class GeneralDelta(Part):
         proj = ops.gemm(x, self.proj, torch.float32)
         coef, v = ops.general_delta_prepare(proj, self.nh, self.d, self.inner, self.decay_out, self.decay_bias,
                                             self.removal_bias, self.unit_eps, self.decay_scale)
-        o = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, batch.num_requests,
-                           self.nh, self.d, self.d)
+        o = ops.delta_scan_step(coef, v, state, batch, self.nh, self.d, self.d, self.dtype)
         n = self.nh * self.d
         y = ops.head_gate_norm(o, proj, 3 * n, self.norm, True, self.norm_eps, "sigmoid", self.nh, self.d,
                                self.dtype)
@@ -142,8 +141,7 @@ class GatedDelta(Part):
                                           batch.q_offsets, batch.slot_ids)
         ops.conv_tail_update(proj, tail, self.channels, self.taps, batch.q_offsets, batch.slot_ids,
                              batch.num_requests)
-        o = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, batch.num_requests,
-                           self.nh, self.dk, self.dv)
+        o = ops.delta_scan_step(coef, v, state, batch, self.nh, self.dk, self.dv, self.dtype)
         y = ops.head_gate_norm(o, proj, self.channels, self.norm, False, self.norm_eps, "silu", self.nh, self.dv,
                                self.dtype)
         return ops.gemm(y, self.o, self.dtype, defer=True)
@@ -206,8 +204,7 @@ class ChannelDelta(Part):
                                             self.unit_eps, batch.tok_req, batch.q_offsets, batch.slot_ids)
         ops.conv_tail_update(proj, tail, self.channels, self.taps, batch.q_offsets, batch.slot_ids,
                              batch.num_requests)
-        o = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, batch.num_requests,
-                           self.nh, self.dk, self.dv)
+        o = ops.delta_scan_step(coef, v, state, batch, self.nh, self.dk, self.dv, self.dtype)
         y = ops.head_gate_norm(o, gates, self.nh * self.dk, self.norm, False, self.norm_eps, "sigmoid", self.nh,
                                self.dv, self.dtype)
         return ops.gemm(y, self.o, self.dtype, defer=True)

@@ -68,7 +68,6 @@ class GatedLinear(Part):
         rates = ops.gemm(inner, self.outer, torch.float32)
         coef, v = ops.gated_linear_prepare(proj, rates, 0, self.rate_bias, 1.0 / self.tau, self.dk ** -0.5, self.nh,
                                            self.dk, self.dv)
-        o = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, batch.num_requests, self.nh, self.dk,
-                           self.dv)
+        o = ops.delta_scan_step(coef, v, state, batch, self.nh, self.dk, self.dv, self.dtype)
         y = ops.head_gate_norm(o, proj, self.gate_column, self.norm, False, self.norm_eps, "silu", self.nh, self.dv, self.dtype)
         return ops.gemm(y, self.o, self.dtype, defer=True)

@@ -61,8 +61,7 @@ class Lightning(Part):
         (state,) = site.cache
         proj = ops.gemm(x, self.proj, torch.float32)
         coef, v = ops.lightning_prepare(proj, self.nh, self.dk, self.dv, self.decay)
-        o = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, batch.num_requests,
-                           self.nh, self.dk, self.dv)
+        o = ops.delta_scan_step(coef, v, state, batch, self.nh, self.dk, self.dv, self.dtype)
         # one norm over all heads together, the weight and the gate in the same kernel
         y = ops.lightning_readout(o, proj, 2 * self.nh * self.dk + self.nh * self.dv, self.norm, self.norm_eps,
                                   self.dtype)

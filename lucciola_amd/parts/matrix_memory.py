@@ -69,8 +69,7 @@ class MatrixMemory(Part):
         coef, v, bottoms = ops.mlstm_prepare(proj, self.nh, self.dk, self.dv, self.i_column, self.i_column + self.nh,
                                              self.i_bias, self.f_bias, self.cap, self.dk ** -0.5, reference,
                                              batch.q_offsets, batch.slot_ids, batch.num_requests)
-        o = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, batch.num_requests, self.nh, self.dk,
-                           self.dv + 1)
+        o = ops.delta_scan_step(coef, v, state, batch, self.nh, self.dk, self.dv + 1, self.dtype)
         y = ops.mlstm_readout(o, bottoms, self.floor, proj, self.gate_column, self.norm, self.norm_eps, self.nh,
                               self.dv, self.dtype)
         return ops.gemm(y, self.o, self.dtype, defer=True)

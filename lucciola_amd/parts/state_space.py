@@ -86,8 +86,7 @@ class StateSpace(Part):
         if self.taps > 1:
             ops.conv_tail_update(proj, tail, self.channels, self.taps, batch.q_offsets, batch.slot_ids,
                                  batch.num_requests)
-        o = ops.delta_scan(coef, xs, state, batch.q_offsets, batch.slot_ids, batch.num_requests, self.nh, self.N,
-                           self.dv)
+        o = ops.delta_scan_step(coef, xs, state, batch, self.nh, self.N, self.dv, self.dtype)
         y = ops.state_space_readout(o, xs, proj, self.channels, self.skip, self.nh, self.dv, self.norm, self.parts,
                                     self.norm_eps, self.dtype)
         return ops.gemm(y, self.o, self.dtype, defer=True)

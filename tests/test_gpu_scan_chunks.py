@@ -1,0 +1,85 @@
+"""The recurrence a chunk at a time (``ops.delta_scan_chunks``) against its definition in float64 and beside the
+token-by-token kernel, and the rule that chooses between the two."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+import reference_ops
+from lucciola_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+# Both kernels round a sum of some 130 float32 terms a token, and what a state holds is the sum of the tokens it remembers:
+# a few units of 2^-24 of the result's root mean square.  The token-by-token kernel is measured beside and the chunks may
+# be off by twice as much (another order of the same sums), or by eight units where both are that small.
+UNIT = 2.0 ** -24
+
+
+def vectors(kind, T, heads, dk, g):
+    def unit(x):
+        return x / torch.sqrt((x * x).sum(-1, keepdim=True) + 1e-6)
+    q, k = torch.randn(T, heads, dk, generator=g), unit(torch.randn(T, heads, dk, generator=g))
+    beta = torch.rand(T, heads, 1, generator=g)
+    if kind == "steady":            # one decay a head, close to 1
+        d = (1 - 2.0 ** -torch.arange(5, 5 + heads).float())[None, :, None].expand(T, heads, dk)
+    elif kind == "by channel":
+        d = torch.rand(T, heads, dk, generator=g) * 0.4 + 0.6
+    else:                           # decays of every size, 0 and 1 among them: pairs are made one by one
+        d = torch.rand(T, heads, dk, generator=g) ** 8
+        d[torch.rand(T, heads, dk, generator=g) < 0.1] = 0.0
+        d[torch.rand(T, heads, dk, generator=g) < 0.1] = 1.0
+    removing = [d, d * k, beta * k, beta * k, q]
+    return torch.stack(removing).reshape(5, T, heads * dk), torch.stack([d, k, q]).reshape(3, T, heads * dk)
+
+
+@pytest.mark.parametrize("planes", [5, 3])
+@pytest.mark.parametrize("kind", ["steady", "by channel", "any"])
+@pytest.mark.parametrize("heads,dk,dv,lengths", [(2, 128, 128, [64]), (3, 128, 48, [65, 95, 96, 97]), (1, 64, 17, [1, 127, 63, 64]),
+                                                 (8, 64, 1, [161, 5]), (2, 128, 129, [3, 200, 1, 1, 80])])
+def test_chunks(planes, kind, heads, dk, dv, lengths):
+    g = torch.Generator().manual_seed(7 * dk + dv + planes)
+    T, R = sum(lengths), len(lengths)
+    coef = vectors(kind, T, heads, dk, g)[0 if planes == 5 else 1]
+    v = torch.randn(T, heads * dv, generator=g)
+    state = torch.randn(R + 2, heads, dv, dk, generator=g) * 0.2
+    starts = [0] + torch.tensor(lengths).cumsum(0).tolist()
+    lists = torch.tensor(starts, dtype=torch.int32), torch.randperm(R + 2, generator=g)[:R].to(torch.int32)
+    states = [state.to(DEV), state.to(DEV)]
+    on_gpu = (coef.to(DEV), v.to(DEV)), tuple(x.to(DEV) for x in lists)
+    want_state = state.double()
+    want = reference_ops.delta_scan(coef, v, want_state, *lists, R, heads, dk, dv).double()
+    plain = ops.delta_scan(*on_gpu[0], states[0], *on_gpu[1], R, heads, dk, dv).cpu().double()
+    got = ops.delta_scan_chunks(*on_gpu[0], states[1], *on_gpu[1], R, heads, dk, dv,
+                                some_short=min(lengths) < ops.SCAN_CHUNKS_FROM).cpu().double()
+
+    def off(x, y):
+        return float((x - y).norm() / y.norm())
+    assert off(got, want) <= max(2 * off(plain, want), 8 * UNIT), "read-outs"
+    plain_state, got_state = (s.cpu().double() for s in states)
+    assert off(got_state, want_state) <= max(2 * off(plain_state, want_state), 8 * UNIT), "states"
+    idle = [s for s in range(R + 2) if s not in lists[1].tolist()]
+    assert torch.equal(got_state[idle], state.double()[idle]), "another request's state"
+    for r, n in enumerate(lengths):     # the short ones go token by token: the same bits
+        if n < ops.SCAN_CHUNKS_FROM:
+            assert torch.equal(got[starts[r]:starts[r + 1]], plain[starts[r]:starts[r + 1]])
+
+
+@pytest.mark.parametrize("dtype,dk,lengths,chunked", [(torch.bfloat16, 128, [64, 2], True), (torch.float32, 128, [64, 2], False),
+                                                      (torch.bfloat16, 128, [63, 2], False), (torch.bfloat16, 32, [90], False),
+                                                      (torch.bfloat16, 64, [1, 70], True)])
+def test_which_steps_go_in_chunks(monkeypatch, dtype, dk, lengths, chunked):
+    g = torch.Generator().manual_seed(dk)
+    T, heads, dv = sum(lengths), 2, 16
+    starts = [0] + torch.tensor(lengths).cumsum(0).tolist()
+    batch = SimpleNamespace(q_offsets=torch.tensor(starts, dtype=torch.int32, device=DEV), q_start=starts, num_tokens=T,
+                            slot_ids=torch.arange(len(lengths), dtype=torch.int32, device=DEV), num_requests=len(lengths))
+    coef = vectors("by channel", T, heads, dk, g)[1].to(DEV)
+    v, state = torch.randn(T, heads * dv, generator=g).to(DEV), torch.zeros(len(lengths), heads, dv, dk, device=DEV)
+    called, real = [], ops.delta_scan_chunks
+    monkeypatch.setattr(ops, "delta_scan_chunks", lambda *a, **k: called.append(1) or real(*a, **k))
+    got = ops.delta_scan_step(coef, v, state.clone(), batch, heads, dk, dv, dtype)
+    plain = ops.delta_scan(coef, v, state, batch.q_offsets, batch.slot_ids, len(lengths), heads, dk, dv)
+    assert bool(called) == chunked
+    assert torch.equal(got, plain) or chunked
+    assert float((got - plain).norm() / plain.norm()) < 1e-6
