@@ -16,53 +16,10 @@
 // and no matrix instruction (src/kernels/linear.cu:7-56).
 #include "common.h"
 
+#include "gemm_tile.h"
+
 namespace lc {
 
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float floatx4 __attribute__((ext_vector_type(4)));
-typedef float floatx16 __attribute__((ext_vector_type(16)));
-
-template <typename TO> __device__ __forceinline__ void store_out(TO* p, float v);
-template <> __device__ __forceinline__ void store_out<float>(float* p, float v) { *p = v; }
-template <> __device__ __forceinline__ void store_out<bf16>(bf16* p, float v) { *p = static_cast<bf16>(v); }
-
-// two adjacent elements in one store; p is aligned to the pair
-template <typename TO> __device__ __forceinline__ void store_pair(TO* p, float a, float b);
-template <> __device__ __forceinline__ void store_pair<float>(float* p, float a, float b) {
-    *reinterpret_cast<float2*>(p) = make_float2(a, b);
-}
-template <> __device__ __forceinline__ void store_pair<bf16>(bf16* p, float a, float b) {
-    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
-    bf16x2 v;
-    v[0] = static_cast<bf16>(a);
-    v[1] = static_cast<bf16>(b);
-    *reinterpret_cast<bf16x2*>(p) = v;
-}
-
-// the value of another lane of the same row of 16 lanes, by a DPP move: CTRL 0xB1 swaps
-// neighbours (lane ^ 1), 0x128 rotates the row by 8 (lane ^ 8).  All lanes must be active.
-template <int CTRL> __device__ __forceinline__ float lane_swap(float v) {
-    return __builtin_bit_cast(float, __builtin_amdgcn_mov_dpp(__builtin_bit_cast(int, v), CTRL, 0xF, 0xF, true));
-}
-
-// What the gated epilogue makes of a gate and an up entry: with g' = min(g, limit) and u' = u held inside
-// -limit .. limit, g' sigmoid(slope g') (u' + shift).  No limit, slope 1 and shift 0 is silu(g) u (reference:
-// src/kernels/swiglu.cu:8,31-35), to the bit.
-struct GateForm {
-    float limit, slope, shift;
-};
-static constexpr GateForm kSilu{INFINITY, 1.f, 0.f};
-
-// exp and the reciprocal are the hardware's single instructions (about one unit in the last
-// place each); the results of these products are rounded to bfloat16 afterwards.
-__device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
-    g = fminf(g, form.limit);
-    u = fminf(fmaxf(u, -form.limit), form.limit);
-    return g * __builtin_amdgcn_rcpf(1.f + __expf(-form.slope * g)) * (u + form.shift);
-}
-
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-typedef __attribute__((address_space(1))) const void* glb_ptr_t;
 
 // ------------------------------------------------------------------------------- skinny
 constexpr int SK_KBLOCK = 128; // k elements per wave iteration
@@ -590,25 +547,7 @@ __global__ __launch_bounds__(1024) void gemm_runs_kernel(const bf16* __restrict_
 }
 
 // ------------------------------------------------------------------------------- tiled
-// Workgroup tile BM x BN x 64, four waves in a 2 x 2 grid, each owning (BM/64) x (BN/64) tiles
-// of 32 x 32.
-//
-// Operand tiles go from global memory straight into LDS (global_load_lds_dwordx4: lane l's 16
-// bytes land at the instruction's LDS base + 16 l, no registers in between) into a ring of
-// TL_STAGES stages.  Inside a stage a row's eight 16-byte chunks are stored at column
-// (chunk ^ ((row >> 1) & 7)): the 16 lanes that the LDS serves per cycle for a 128-bit read
-// (16 consecutive rows, one chunk) then cover all 64 banks.
-//
-// The loop is scheduled by hand, because a SIMD holds a single wave of this kernel and nothing
-// else hides a stall.  Per k-step of 16 the wave issues its (BM/64)*(BN/64) products; between
-// them, one at a time, go the LDS reads of the NEXT k-step's operands (ds_read_b128 in inline
-// assembly with explicit waits: the compiler cannot tell the stages apart and would make every
-// load in flight land before any read) and, in a block's first k-step, the global loads of the
-// block TL_STAGES-1 ahead.  In a block's last k-step the wave waits for its own loads of the
-// next block, meets the others at a bare barrier (all waves' loads are then visible, and all
-// have finished reading the stage that the next loads overwrite) and reads the next block's
-// first operands while the rest of its products run.  sched_barrier pins that order.
-constexpr int TL_K = 64;
+// Workgroup tiles of the loop in gemm_tile.h.
 
 // The grid's workgroups take the tiles [tile_base, tile_base + tile_count) of the tiles_m x
 // tiles_n tiles of the product.
@@ -623,19 +562,9 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
                                                          int M, int N, int K, int tiles_m, int tile_base,
                                                          int tile_count, int compact, int skew_step,
                                                          GateForm form) {
-    // WM x WN waves, each owning (BM / WM) x (BN / WN) of the tile as TM x TN products of 32 x 32
-    constexpr int S = TL_STAGES;
-    constexpr int NW = WM * WN;
-    constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN);
-    constexpr int KS = TL_K / 16;                             // k-steps per block
-    constexpr int LPA = BM * 8 / (64 * NW), LPB = BN * 8 / (64 * NW), LP = LPA + LPB;   // load instructions per thread and stage
-    static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0, "whole products per wave");
-    static_assert((BM * 8) % (64 * NW) == 0 && (BN * 8) % (64 * NW) == 0, "whole load instructions per wave");
-    constexpr int NM = TM * TN, NR = TM + TN;                 // products and operand reads per k-step
-    constexpr int A_STAGE = BM * TL_K * 2, B_STAGE = BN * TL_K * 2;          // bytes
-    static_assert(S >= 2 && (S == 2 ? 2 : S - 1) * LP <= 63, "the load counter holds 63");
-    static_assert(S * (A_STAGE + B_STAGE) <= 160 * 1024, "LDS");
-    __shared__ __attribute__((aligned(1024))) char lds[S * (A_STAGE + B_STAGE)];   // A stages, then B stages
+    typedef TileLoop<BM, BN, TL_STAGES, WM, WN> Loop;
+    constexpr int TM = Loop::TM, TN = Loop::TN, LPA = Loop::LPA, LPB = Loop::LPB;
+    __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
 
     // renumber: workgroups go round-robin over 8 XCDs; give each XCD a contiguous run of
     // tiles, m fastest, so that one XCD's L2 keeps the w tile that its workgroups share
@@ -654,26 +583,20 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
-    const int lr = lane & 31, kg = lane >> 5;
-    auto swz = [](int row) { return (row >> 1) & 7; };
+    const int lr = lane & 31;
 
     const int nk_all = K / TL_K;
     const int kb0 = SPLIT ? (int)((long long)blockIdx.y * nk_all / gridDim.y) : 0;
     const int nk = (SPLIT ? (int)((long long)(blockIdx.y + 1) * nk_all / gridDim.y) : nk_all) - kb0;
 
-    // chunk p = (i * NW + wave) * 64 + lane of a stage holds row p / 8, global chunk (p % 8) ^ swz(row)
     const bf16* xg[LPA];
     const bf16* wg[LPB];
 #pragma unroll
-    for (int i = 0; i < LPA; ++i) {
-        const int p = (i * NW + wave) * 64 + lane, row = p >> 3, kc = (p & 7) ^ swz(row);
-        xg[i] = x + (size_t)min(m0 + row, M - 1) * K + (size_t)kb0 * TL_K + kc * 8;
-    }
+    for (int i = 0; i < LPA; ++i)
+        xg[i] = x + (size_t)min(m0 + Loop::row_of(i, wave, lane), M - 1) * K + (size_t)kb0 * TL_K + Loop::chunk_of(i, wave, lane) * 8;
 #pragma unroll
-    for (int i = 0; i < LPB; ++i) {
-        const int p = (i * NW + wave) * 64 + lane, row = p >> 3, kc = (p & 7) ^ swz(row);
-        wg[i] = w + (size_t)min(n0 + row, N - 1) * K + (size_t)kb0 * TL_K + kc * 8;
-    }
+    for (int i = 0; i < LPB; ++i)
+        wg[i] = w + (size_t)min(n0 + Loop::row_of(i, wave, lane), N - 1) * K + (size_t)kb0 * TL_K + Loop::chunk_of(i, wave, lane) * 8;
     // With a single row of tiles (M <= BM: decode steps of 17 to 64 tokens) every workgroup
     // streams rows of w that nobody else reads, all rows 2 K bytes apart, and all workgroups
     // would walk k in step: at any moment the whole GPU would ask for the same few columns, which
@@ -682,157 +605,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
     // (tile number times skew_step, modulo the number of k-blocks) and wraps around: 37.2 us.  (With several rows of tiles the workgroups that share a tile of w
     // should read it at the same time, and do.)
     const int skew = (!SPLIT && tiles_m == 1 && skew_step) ? (int)(((unsigned)id * (unsigned)skew_step) % (unsigned)nk) : 0;
-    // load instruction idx (x first, then w) of block kb into a stage
-    auto issue_one = [&](int idx, int kb, int stage) {
-        kb += skew;
-        kb -= kb >= nk ? nk : 0;
-        if (idx < LPA)
-            __builtin_amdgcn_global_load_lds((glb_ptr_t)(xg[idx] + kb * TL_K),
-                (lds_ptr_t)(lds + stage * A_STAGE + (idx * NW + wave) * 1024), 16, 0, 0);
-        else
-            __builtin_amdgcn_global_load_lds((glb_ptr_t)(wg[idx - LPA] + kb * TL_K),
-                (lds_ptr_t)(lds + S * A_STAGE + stage * B_STAGE + ((idx - LPA) * NW + wave) * 1024), 16, 0, 0);
-    };
-    // With two stages, a block's loads are issued a block early: in the last k-step of block it,
-    // once every wave has read the last of the stage, block it + 2 goes into it, behind block
-    // it + 1 that is still arriving.  (Issued only after block it + 1 has landed, the loads
-    // would start with nothing in flight: their first data would be a whole latency away, and
-    // the way from L2 into the CU, which bounds these kernels, would stand idle meanwhile.)
-    constexpr bool EARLY = S == 2;
-    constexpr int AHEAD = EARLY ? 2 : S - 1;                  // blocks in flight at the start
-#pragma unroll
-    for (int s = 0; s < AHEAD; ++s)
-        if (s < nk) {
-#pragma unroll
-            for (int i = 0; i < LP; ++i) issue_one(i, s, s);
-        }
-
     floatx16 acc[TM][TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i)
-#pragma unroll
-        for (int j = 0; j < TN; ++j)
-#pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
-
-    // LDS address of this lane's operand rows in stage 0, with the lane's part of the swizzle;
-    // k-step ks flips chunk bits: ((2 ks + kg) ^ swz) * 16 = ((kg ^ swz) * 16) ^ (ks * 32)
-    const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)lds;
-    unsigned pa[TM], pb[TN];
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-        const int row = wm + i * 32 + lr;
-        pa[i] = lds0 + row * 128 + ((kg ^ swz(row)) * 16);
-    }
-#pragma unroll
-    for (int j = 0; j < TN; ++j) {
-        const int row = wn + j * 32 + lr;
-        pb[j] = lds0 + S * A_STAGE + row * 128 + ((kg ^ swz(row)) * 16);
-    }
-
-    bf16x8 a[2][TM], b[2][TN];
-    auto read_one = [&](int r, int stage, int ks, int buf) {
-        if (r < TM) {
-            const unsigned addr = (pa[r] ^ (ks * 32)) + stage * A_STAGE;
-            asm volatile("ds_read_b128 %0, %1" : "=v"(a[buf][r]) : "v"(addr));
-        } else {
-            const unsigned addr = (pb[r - TM] ^ (ks * 32)) + stage * B_STAGE;
-            asm volatile("ds_read_b128 %0, %1" : "=v"(b[buf][r - TM]) : "v"(addr));
-        }
-    };
-    // the products that follow a wait must not be moved above it: tie their operands to that point
-    auto tie = [&](int buf) {
-#pragma unroll
-        for (int i = 0; i < TM; ++i) asm volatile("" : "+v"(a[buf][i]));
-#pragma unroll
-        for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(b[buf][j]));
-    };
-    auto product = [&](int k, int buf) {
-        const int i = k / TN, j = k % TN;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0);
-    };
-
-    // where the reads and loads sit among the NM products of a k-step
-    constexpr int QR = (2 * NR + NM - 1) / NM;                 // reads after each product, from the first on
-    constexpr int RS = (NR + QR - 1) / QR;                     // products that the reads take
-    constexpr int QL = NM > RS ? (LP + (NM - RS) - 1) / (NM - RS) : LP;   // loads after each later product
-    constexpr int BAR = NM / 4;                                // the product after which a block's last k-step syncs
-    constexpr int QT = NM - BAR - 1 > 0 ? (NR + (NM - BAR - 1) - 1) / (NM - BAR - 1) : NR;
-
-    // block 0 has landed when at most the younger blocks are still in flight
-    if (nk >= AHEAD) wait_vmcnt<(AHEAD - 1) * LP>(); else wait_vmcnt<0>();
-    __builtin_amdgcn_s_barrier();
-#pragma unroll
-    for (int r = 0; r < NR; ++r) read_one(r, 0, 0, 0);
-
-    int stage = 0, lstage = S - 1;   // the stage of block `it`; the stage that block it+S-1 goes to
-    auto block = [&](int it, auto load_tag) {
-        constexpr bool LOAD = decltype(load_tag)::value;       // block it+S-1 exists and is loaded here
-        const int nstage = stage + 1 == S ? 0 : stage + 1;
-#pragma unroll
-        for (int ks = 0; ks < KS; ++ks) {
-            const int cur = ks & 1, nxt = cur ^ 1;
-            wait_lgkmcnt<0>();
-            tie(cur);
-            __builtin_amdgcn_sched_barrier(0);
-            if (ks < KS - 1) {
-#pragma unroll
-                for (int k = 0; k < NM; ++k) {
-                    product(k, cur);
-                    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-                    for (int r = k * QR; r < (k + 1) * QR; ++r)
-                        if (r < NR) read_one(r, stage, ks + 1, nxt);
-                    if (LOAD && !EARLY && ks == 0 && (k >= RS || NM == RS)) {
-                        const int first = NM == RS ? k * QL : (k - RS) * QL;
-#pragma unroll
-                        for (int l = first; l < first + QL; ++l)
-                            if (l < LP) issue_one(l, it + S - 1, lstage);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            } else {
-#pragma unroll
-                for (int k = 0; k < NM; ++k) {
-                    product(k, cur);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (LOAD) {
-                        if (k == BAR && EARLY) {
-                            __builtin_amdgcn_s_barrier();          // nobody reads this stage any more
-#pragma unroll
-                            for (int l = 0; l < LP; ++l) issue_one(l, it + 2, stage);
-                            wait_vmcnt<LP>();                      // block it + 1 has landed
-                            __builtin_amdgcn_s_barrier();
-                        } else if (k == BAR) {
-                            wait_vmcnt<(S - 2) * LP>();
-                            __builtin_amdgcn_s_barrier();
-                        }
-                        if (NM - BAR - 1 > 0) {
-#pragma unroll
-                            for (int r = (k - BAR - 1) * QT; r < (k - BAR) * QT; ++r)
-                                if (k > BAR && r < NR) read_one(r, nstage, 0, nxt);
-                        } else if (k == BAR) {
-#pragma unroll
-                            for (int r = 0; r < NR; ++r) read_one(r, nstage, 0, nxt);
-                        }
-                    } else if (k == BAR) {
-                        if (it + 1 < nk) {
-                            wait_vmcnt<0>();
-                            __builtin_amdgcn_s_barrier();
-#pragma unroll
-                            for (int r = 0; r < NR; ++r) read_one(r, nstage, 0, nxt);
-                        }
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
-                }
-            }
-        }
-        stage = nstage;
-        lstage = lstage + 1 == S ? 0 : lstage + 1;
-    };
-    int it = 0;
-    for (; it + AHEAD < nk; ++it) block(it, std::true_type{});
-    for (; it < nk; ++it) block(it, std::false_type{});
+    Loop::run(lds, xg, wg, nk, skew, wave, lane, acc);
 
     // acc[i][j][v]: row m = (v/4)*8 + (lane/32)*4 + v%4, column n = lane%32 of the 32x32 tile.
     const int mrow = m0 + wm + (lane >> 5) * 4;     // + i * 32 + (v / 4) * 8 + v % 4

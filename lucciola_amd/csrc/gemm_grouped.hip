@@ -18,23 +18,14 @@
 #include "common.h"
 
 #include "activations.h"
+#include "gemm_grouped.h"
 
 namespace lc {
 
 constexpr int GG_N = 64, GG_K = 16, GG_CHUNK = 256, GG_PAD = 16;
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-static thread_local int g_grouped_fast = 1;
-
-struct GroupedArgs {
-    const void* x; long long ldx, x_group;
-    const void* w;
-    void* out; long long ldo, out_group;
-    int M, N, K, G;
-    const int* gather; const int* row_start; const int* tile_start;
-    int epilogue;
-    const void* gate; long long ldg, gate_group;
-};
+static thread_local int g_grouped_fast = 1, g_grouped_tiled = 1;
 
 template <typename TX, typename TW, typename TO, int BM, int WM, int WN>
 __global__ __launch_bounds__(256, 2) void gemm_grouped_kernel(GroupedArgs a) {
@@ -352,6 +343,13 @@ LC_API int lc_gemm_grouped_fast(int on) {
     return before;
 }
 
+// Tests and tuning: whether those products may take the kernels of gemm_grouped_tiled.hip, likewise.
+LC_API int lc_gemm_grouped_tiled(int on) {
+    const int before = g_grouped_tiled;
+    if (on >= 0) g_grouped_tiled = on ? 1 : 0;
+    return before;
+}
+
 // Whether tiles of `tile_rows` rows exist for these operand types (16 and 64: always; 128: the
 // bfloat16 kernel only).  The lists' tile_start must have been made for the size that is asked for.
 LC_API int lc_gemm_grouped_takes_tile(int tile_rows, int x_dt, int w_dt) {
@@ -377,10 +375,13 @@ LC_API int lc_gemm_grouped(const void* x, int x_dt, long long ldx, long long x_g
     LC_CHECK(tile_rows == 16 || tile_rows == 64 || tile_rows == 128, "grouped product: tiles of %d rows", tile_rows);
     LC_CHECK(G <= 65535 && (row_start ? max_tiles : (M + 15) / 16) <= 65535, "grouped product: too many tiles");
     GroupedArgs a{x, ldx, x_group, w, out, ldo, out_group, M, N, K, G, gather, row_start, tile_start,
-                  epilogue, gate, ldg, gate_group};
+                  epilogue, gate, ldg, gate_group,
+                  N % 2 == 0 && ldo % 2 == 0 && out_group % 2 == 0 && (uintptr_t)out % (out_dt == DT_BF16 ? 4 : 8) == 0};
     // bfloat16 operands whose pieces of 8 are whole and aligned: the bfloat16 matrix instruction
     if (x_dt == DT_BF16 && w_dt == DT_BF16 && K % 8 == 0 && ldx % 8 == 0 && x_group % 8 == 0 &&
         (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && g_grouped_fast) {
+        if (g_grouped_tiled && (out_dt == DT_BF16 || out_dt == DT_F32) && grouped_tiled_takes(a, tile_rows))
+            return launch_grouped_tiled(a, max_tiles, tile_rows, out_dt == DT_BF16, stream);
         if (out_dt == DT_BF16) return launch_grouped_bf16<bf16>(a, max_tiles, tile_rows, stream);
         if (out_dt == DT_F32) return launch_grouped_bf16<float>(a, max_tiles, tile_rows, stream);
     }

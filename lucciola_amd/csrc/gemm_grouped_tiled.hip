@@ -1,0 +1,194 @@
+// The grouped products of gemm_grouped.hip for bfloat16 operands, in two shapes of their own:
+//
+//   tiles    many rows a group (prompts): tiles of 64 or 128 rows by 128 columns through the loop of the dense products
+//            (gemm_tile.h): direct loads to LDS, v_mfma_f32_32x32x16_bf16, scheduled by hand.  Bound by the CUs' way from L2,
+//            18 to 23 bytes a clock each.  Two or three workgroups a CU, because a group's K is short (32 blocks) and
+//            a tile's first loads and its stores pass beside another's products: 8,192 rows over 32 matrices of 2,048 x 2,048
+//            take 125 us (through registers in tiles of 128 x 128, as in gemm_grouped.hip: 175), where the tiles of 128 x 256,
+//            which ask L2 for a third less and have a CU to themselves, take 172; 4,096 x 2,048: 278 -> 221 us.
+//   stream   few rows a group (decoding: 16 rows a tile): bound by reading every group's matrix once, so what counts is
+//            how much of it is on its way.  256 rows over 32 matrices of 2,048 x 2,048 (268 MB): 68 -> 51 us (5.3 TB/s); 32 rows,
+//            21 matrices: 51 -> 31; 512 rows, 32 matrices of 4,096 x 2,048: 156 -> 98.
+//
+// Which rows are whose, the gather list and the epilogues are as described there.
+#include "common.h"
+
+#include "activations.h"
+#include "gemm_grouped.h"
+#include "gemm_tile.h"
+
+namespace lc {
+
+// One element's epilogue.
+__device__ __forceinline__ float grouped_finish(const GroupedArgs& a, const bf16* gate, int m, int n, float v) {
+    if (a.epilogue == ACT_SIGMOID_GATE) return v * sigmoid(to_f32(gate[(size_t)m * a.ldg + n]));
+    if (a.epilogue == ACT_SIGMOID_GROUP_GATE) return v * sigmoid(to_f32(gate[(size_t)m * a.ldg]));
+    return activate(v, a.epilogue);
+}
+
+// grid (column tiles, row tiles, groups or 1): neighbouring workgroups, which go to different XCDs, take different columns
+// of w, and the row tiles of a group that share columns of w run on one XCD where the column tiles are a multiple of 8.
+template <typename TO, int BM, int BN, int STAGES, int WM, int WN>
+__global__ __launch_bounds__(64 * WM * WN) void gemm_grouped_tiled_kernel(GroupedArgs a) {
+    typedef TileLoop<BM, BN, STAGES, WM, WN> Loop;
+    constexpr int TM = Loop::TM, TN = Loop::TN;
+    __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
+    GroupedTile tile;
+    if (!find_tile(a, BM, tile)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int n0 = blockIdx.x * BN, N = a.N, K = a.K;
+    const bf16* x = reinterpret_cast<const bf16*>(a.x) + (size_t)tile.group * a.x_group;
+    const bf16* w = reinterpret_cast<const bf16*>(a.w) + (size_t)tile.group * N * K;
+    const bf16* xg[Loop::LPA];
+    const bf16* wg[Loop::LPB];
+#pragma unroll
+    for (int i = 0; i < Loop::LPA; ++i) {
+        const int m = min(tile.first + Loop::row_of(i, wave, lane), tile.end - 1);      // a row behind the group's end is its last one
+        xg[i] = x + (size_t)(a.gather ? a.gather[m] : m) * a.ldx + Loop::chunk_of(i, wave, lane) * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < Loop::LPB; ++i)
+        wg[i] = w + (size_t)min(n0 + Loop::row_of(i, wave, lane), N - 1) * K + Loop::chunk_of(i, wave, lane) * 8;
+    floatx16 acc[TM][TN];
+    Loop::run(lds, xg, wg, K / TL_K, 0, wave, lane, acc);
+
+    // acc[i][j][v]: row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32 of the 32 x 32 tile
+    TO* out = reinterpret_cast<TO*>(a.out) + (size_t)tile.group * a.out_group;
+    const bf16* gate = a.gate ? reinterpret_cast<const bf16*>(a.gate) + (size_t)tile.group * a.gate_group : nullptr;
+    const int m0 = tile.first + (wave / WN) * (BM / WM) + (lane >> 5) * 4, c0 = n0 + (wave % WN) * (BN / WN) + (lane & 31);
+    if (a.pairs) {
+        // neighbouring lanes swap every other value and store two columns of a row together: even lanes the even v
+        const bool odd = lane & 1;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; v += 2) {
+                    const int m = m0 + i * 32 + (v >> 2) * 8 + (v & 3), n = c0 + j * 32, pair = n & ~1;
+                    float first = acc[i][j][v], second = acc[i][j][v + 1];
+                    asm volatile("" : "+v"(first), "+v"(second));   // two values, not one indexed by `odd`
+                    const float got = lane_swap<0xB1>(odd ? first : second);    // lane ^ 1
+                    const int row = m + (odd ? 1 : 0);
+                    if (row < tile.end && pair < N)
+                        store_pair<TO>(out + (size_t)row * a.ldo + pair, grouped_finish(a, gate, row, pair, odd ? got : first),
+                                       grouped_finish(a, gate, row, pair + 1, odd ? second : got));
+                }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int m = m0 + i * 32 + (v >> 2) * 8 + (v & 3), n = c0 + j * 32;
+                    if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish(a, gate, m, n, acc[i][j][v]));
+                }
+    }
+}
+
+// Tiles of 16 rows by 64 columns, K in blocks of 128: a row of w comes 256 bytes at a time, and a ring of STREAM_STAGES blocks
+// keeps all but one of them on their way, two workgroups a CU: 120 KB a CU, where the CU's share of the memory's rate
+// needs some 64.  A row's 16-byte chunk c lies at place c ^ (row % 16): the 16 rows that LDS serves together meet no bank twice.
+// A wave multiplies 16 of the columns by itself.  Every column tile starts at a block of its own and wraps around, so that the
+// workgroups, whose rows lie a multiple of 2 K bytes apart, do not all ask the same memory channels at once; the order of
+// an element's sum depends on its group and column alone.
+constexpr int STREAM_K = 128, STREAM_STAGES = 4, STREAM_N = 64;
+
+template <typename TO>
+__global__ __launch_bounds__(256) void gemm_grouped_stream_kernel(GroupedArgs a) {
+    constexpr int XB = 16 * STREAM_K * 2, WB = STREAM_N * STREAM_K * 2, LOADS = 5;
+    __shared__ __attribute__((aligned(1024))) char lds[STREAM_STAGES * (XB + WB)];
+    GroupedTile tile;
+    if (!find_tile(a, 16, tile)) return;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int col = lane & 15, quad = lane >> 4;
+    const int n0 = blockIdx.x * STREAM_N, N = a.N, K = a.K, blocks = K / STREAM_K;
+    const bf16* x = reinterpret_cast<const bf16*>(a.x) + (size_t)tile.group * a.x_group;
+    const bf16* w = reinterpret_cast<const bf16*>(a.w) + (size_t)tile.group * N * K;
+    // a load instruction brings four rows: lane l the chunk at place l % 16 of row l / 16
+    const bf16* from[LOADS];
+    {
+        const int row = 4 * wave + quad, m = min(tile.first + row, tile.end - 1);
+        from[0] = x + (size_t)(a.gather ? a.gather[m] : m) * a.ldx + (col ^ row) * 8;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const int r = 4 * i + quad;
+            from[1 + i] = w + (size_t)min(n0 + 16 * wave + r, N - 1) * K + (col ^ r) * 8;
+        }
+    }
+    const int skew = (int)(((unsigned)blockIdx.x * 17u + (unsigned)tile.group * 5u) % (unsigned)blocks);
+    auto issue = [&](int b) {
+        char* stage = lds + (b % STREAM_STAGES) * (XB + WB);
+        int k = b + skew;
+        k -= k >= blocks ? blocks : 0;
+        __builtin_amdgcn_global_load_lds((glb_ptr_t)(from[0] + k * STREAM_K), (lds_ptr_t)(stage + wave * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(from[1 + i] + k * STREAM_K),
+                                             (lds_ptr_t)(stage + XB + (4 * wave + i) * 1024), 16, 0, 0);
+    };
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)lds;
+    const unsigned row_x = lds0 + col * 256, row_w = lds0 + XB + (16 * wave + col) * 256;
+    floatx4 acc = {0.f, 0.f, 0.f, 0.f};
+    for (int b = 0; b < min(STREAM_STAGES - 1, blocks); ++b) issue(b);
+    for (int b = 0; b < blocks; ++b) {
+        // this wave's loads of block b have landed when only those of the younger blocks are left
+        const int younger = min(blocks - 1 - b, STREAM_STAGES - 2);
+        if (younger == STREAM_STAGES - 2) wait_vmcnt<(STREAM_STAGES - 2) * LOADS>();
+        else if (younger == 1) wait_vmcnt<LOADS>();
+        else wait_vmcnt<0>();
+        static_assert(STREAM_STAGES == 4, "the waits above");
+        __builtin_amdgcn_s_barrier();                       // everybody's have; nobody reads the block before any more
+        asm volatile("" ::: "memory");
+        if (b + STREAM_STAGES - 1 < blocks) issue(b + STREAM_STAGES - 1);       // into the place of the block before
+        const unsigned stage = (b % STREAM_STAGES) * (XB + WB);
+        bf16x8 xa[4], wb[4];
+        unsigned ax[4], aw[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+            const unsigned place = ((4 * s + quad) ^ col) * 16;
+            ax[s] = row_x + stage + place;
+            aw[s] = row_w + stage + place;
+        }
+        // in inline assembly, because the compiler would wait for every load to LDS in flight before an LDS read
+        asm volatile("ds_read_b128 %0, %8\n\tds_read_b128 %1, %9\n\tds_read_b128 %2, %10\n\tds_read_b128 %3, %11\n\t"
+                     "ds_read_b128 %4, %12\n\tds_read_b128 %5, %13\n\tds_read_b128 %6, %14\n\tds_read_b128 %7, %15\n\t"
+                     "s_waitcnt lgkmcnt(0)"
+                     : "=&v"(xa[0]), "=&v"(wb[0]), "=&v"(xa[1]), "=&v"(wb[1]), "=&v"(xa[2]), "=&v"(wb[2]), "=&v"(xa[3]), "=&v"(wb[3])
+                     : "v"(ax[0]), "v"(aw[0]), "v"(ax[1]), "v"(aw[1]), "v"(ax[2]), "v"(aw[2]), "v"(ax[3]), "v"(aw[3])
+                     : "memory");
+#pragma unroll
+        for (int s = 0; s < 4; ++s) acc = __builtin_amdgcn_mfma_f32_16x16x32_bf16(xa[s], wb[s], acc, 0, 0, 0);
+    }
+    TO* out = reinterpret_cast<TO*>(a.out) + (size_t)tile.group * a.out_group;
+    const bf16* gate = a.gate ? reinterpret_cast<const bf16*>(a.gate) + (size_t)tile.group * a.gate_group : nullptr;
+    const int n = n0 + 16 * wave + col;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int m = tile.first + 4 * quad + i;
+        if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish(a, gate, m, n, acc[i]));
+    }
+}
+
+template <typename TO>
+static int grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, hipStream_t stream) {
+    auto grid = [&](int bm, int bn) {
+        return dim3((a.N + bn - 1) / bn, a.row_start ? max_tiles : (a.M + bm - 1) / bm, a.row_start ? 1 : a.G);
+    };
+    if (tile_rows == 16) gemm_grouped_stream_kernel<TO><<<grid(16, STREAM_N), 256, 0, stream>>>(a);
+    else if (tile_rows == 64) gemm_grouped_tiled_kernel<TO, 64, 128, 2, 2, 2><<<grid(64, 128), 256, 0, stream>>>(a);
+    else gemm_grouped_tiled_kernel<TO, 128, 128, 2, 4, 1><<<grid(128, 128), 256, 0, stream>>>(a);
+    LC_LAUNCH_CHECK("gemm_grouped_tiled");
+    return 0;
+}
+
+bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows) {
+    return tile_rows == 16 ? a.K % STREAM_K == 0 : a.K % TL_K == 0;
+}
+
+int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, hipStream_t stream) {
+    return out_bf16 ? grouped_tiled<bf16>(a, max_tiles, tile_rows, stream) : grouped_tiled<float>(a, max_tiles, tile_rows, stream);
+}
+
+}  // namespace lc

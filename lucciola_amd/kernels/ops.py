@@ -79,6 +79,7 @@ _SIGNATURES = {
     "lc_rms_shift": "ppipffppppppiiip",
     "lc_gemm_grouped": "piqqpipiqqiiiipppiiipqqp",
     "lc_gemm_grouped_fast": "i",
+    "lc_gemm_grouped_tiled": "i",
     "lc_gemm_grouped_takes_tile": "iii",
     "lc_latent_prepare": "pqpiqiiiiipfppiipppp",
     "lc_latent_attention": "piiiiippppiifippp",
@@ -1205,16 +1206,11 @@ def _check_strided(s: Strided, what: str, rows: int, groups: int, width: int, dt
                           f"and {rows} rows do not fit {tuple(s.tensor.shape)}")
 
 
-def _grouped_tile(rows: int, N: int, groups: int, x: torch.Tensor, w: torch.Tensor) -> int:
-    """Rows of a grouped product's tiles, for ``rows`` rows a group: 16 for a step of few tokens, 128
-    (by 128 columns) where the operands take the bfloat16 kernel and there are so many rows and
-    columns that even tiles of that size are several to a CU (measured: 2,048 rows, 16 heads and 128
-    or 512 columns are faster in tiles of 64 x 64, which are four times as many)."""
-    if rows <= 16:
-        return 16
-    if (-(-rows // 128)) * (-(-N // 128)) * groups >= 2048 and library().lc_gemm_grouped_takes_tile(128, _dt(x), _dt(w)):
-        return 128
-    return 64
+def _grouped_tile(rows: int) -> int:
+    """Rows of the tiles of a product per head over ``rows`` rows: 16 for a step of few tokens, else 64 (these products
+    are short, K of 128 or 512 and as many columns, so what counts is many workgroups: 2,048 rows, 32 heads, 512 columns of
+    128 k: 36 us in tiles of 64 x 128 and 80 in 128 x 128; 128 columns of 512 k 22 and 32)."""
+    return 16 if rows <= 16 else 64
 
 
 def grouped_gemm(x: Strided, w: torch.Tensor, out: Strided, rows: int, gate: Optional[Strided] = None,
@@ -1238,7 +1234,7 @@ def grouped_gemm(x: Strided, w: torch.Tensor, out: Strided, rows: int, gate: Opt
         return
     _call("lc_gemm_grouped", x.pointer(), _dt(x.tensor), x.tensor.shape[1], x.group, _ptr(w), _dt(w),
           out.pointer(), _dt(out.tensor), out.tensor.shape[1], out.group, rows, N, K, G, None, None, None, 0,
-          _grouped_tile(rows, N, G, x.tensor, w), epilogue, gate.pointer() if gate is not None else None,
+          _grouped_tile(rows), epilogue, gate.pointer() if gate is not None else None,
           gate.tensor.shape[1] if gate is not None else 0, gate.group if gate is not None else 0, _stream())
 
 
@@ -1409,6 +1405,15 @@ class Routing:
     max_tiles: int
 
 
+def _routed_tile(rows: int, experts: int, large_tiles: bool) -> int:
+    """Rows of the experts' tiles for ``rows`` (token, choice) pairs: 16 where an expert has that many on average, which reads
+    every matrix at the memory's rate (32 experts of 4,096 x 2,048, 16 rows each: 98 us against 119 in tiles of 64, the
+    matrices alone 98); 128 where it has more than one tile of 128 and the caller's products take them, else 64 (2,048 x 2,048
+    matrices, 75, 190 and 256 rows an expert: 75, 104 and 125 us in tiles of 64, 78, 102 and 125 in tiles of 128; 6,144 x 4,096,
+    256 rows: 751 and 644, since the larger tile asks L2 for less)."""
+    return 16 if rows <= 16 * experts else 128 if large_tiles and rows >= 192 * experts else 64
+
+
 def moe_route(logits: torch.Tensor, top: int, renormalise: bool = True, eps: float = 1e-20,
               large_tiles: bool = False) -> Routing:
     """From the router's float32 ``logits`` [T, E]: softmax over all experts, the ``top`` largest scores of
@@ -1422,8 +1427,7 @@ def moe_route(logits: torch.Tensor, top: int, renormalise: bool = True, eps: flo
     weights = torch.empty((T, top), dtype=torch.float32, device=dev)
     _call("lc_moe_route", _ptr(logits), T, E, top, 1 if renormalise else 0, float(eps), _ptr(ids), _ptr(weights),
           _stream())
-    # few rows an expert: tiles of 16 rows; many, and the caller's products take them: of 128; else of 64
-    tile = 16 if T * top <= 16 * E else 128 if (large_tiles and T * top >= 192 * E) else 64
+    tile = _routed_tile(T * top, E, large_tiles)
     lists = torch.empty((2 * (E + 1) + 2 * T * top,), dtype=torch.int32, device=dev)
     row_start, tile_start = lists[:E + 1], lists[E + 1:2 * (E + 1)]
     sorted_token, entry_row = lists[2 * (E + 1):2 * (E + 1) + T * top], lists[2 * (E + 1) + T * top:]
@@ -1449,7 +1453,7 @@ def moe_route_sigmoid(logits: torch.Tensor, top: int, correction: Optional[torch
     weights = torch.empty((T, top), dtype=torch.float32, device=dev)
     _call("lc_moe_route_sigmoid", _ptr(logits), _ptr(correction), T, E, top, int(groups), int(keep), float(scale),
           _ptr(ids), _ptr(weights), _stream())
-    tile = 16 if T * top <= 16 * E else 128 if (large_tiles and T * top >= 192 * E) else 64
+    tile = _routed_tile(T * top, E, large_tiles)
     lists = torch.empty((2 * (E + 1) + 2 * T * top,), dtype=torch.int32, device=dev)
     row_start, tile_start = lists[:E + 1], lists[E + 1:2 * (E + 1)]
     sorted_token, entry_row = lists[2 * (E + 1):2 * (E + 1) + T * top], lists[2 * (E + 1) + T * top:]
@@ -1962,7 +1966,7 @@ def moe_route_logits(logits: torch.Tensor, experts: int, top: int, bias: Optiona
     ids = torch.empty((T, top), dtype=torch.int32, device=dev)
     weights = torch.empty((T, top), dtype=torch.float32, device=dev)
     _call("lc_moe_route_logits", _ptr(logits), cols, _ptr(bias), T, E, top, _ptr(ids), _ptr(weights), _stream())
-    tile = 16 if T * top <= 16 * E else 128 if (large_tiles and T * top >= 192 * E) else 64
+    tile = _routed_tile(T * top, E, large_tiles)
     lists = torch.empty((2 * (E + 1) + 2 * T * top,), dtype=torch.int32, device=dev)
     row_start, tile_start = lists[:E + 1], lists[E + 1:2 * (E + 1)]
     sorted_token, entry_row = lists[2 * (E + 1):2 * (E + 1) + T * top], lists[2 * (E + 1) + T * top:]

@@ -1,0 +1,83 @@
+"""The grouped products' tiled and streaming kernels (``csrc/gemm_grouped_tiled.hip``) against plain products in float32, at the
+edges of their tiles, blocks of K and lists, and beside the general kernels that take what they refuse."""
+import pytest
+import torch
+
+from lucciola_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def off_by(got, want, K):
+    """The largest error in units of what is allowed: float32 sums of K products of bfloat16 numbers (a unit of 2^-24 of the
+    terms' root mean square sum a term, on average far less), and half a unit of bfloat16 where the result is rounded."""
+    want = want.to(DEV)
+    allowed = K * 2.0 ** -24 * want.pow(2).mean().sqrt() + 1e-30
+    if got.dtype == torch.bfloat16:
+        allowed = allowed + want.abs() * 2.0 ** -8
+    return float(((got.float() - want).abs() / allowed).max())
+
+
+def switched(on, f):
+    before = ops.library().lc_gemm_grouped_tiled(on)
+    try:
+        return f()
+    finally:
+        ops.library().lc_gemm_grouped_tiled(before)
+
+
+# rows an expert: some none, one, around 16, 64 and 128; K of one block and more; columns behind a tile, odd ones
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("tile", [16, 64, 128])
+@pytest.mark.parametrize("counts,N,K", [([0, 1, 17], 128, 128), ([16, 0, 63, 64, 65, 1], 130, 256), ([127, 128, 129], 64, 512),
+                                        ([3, 200], 257, 384), ([1, 2, 3, 4], 1, 640)])
+def test_experts(out, tile, counts, N, K):
+    g = torch.Generator().manual_seed(N + K + len(counts))
+    E, rows = len(counts), sum(counts)
+    ids = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(counts)])[torch.randperm(rows, generator=g)]
+    lists = torch.empty(2 * (E + 1) + 2 * rows, dtype=torch.int32, device=DEV)
+    starts, tiles = lists[:E + 1], lists[E + 1:2 * (E + 1)]
+    token, entry = lists[2 * (E + 1):2 * (E + 1) + rows], lists[2 * (E + 1) + rows:]
+    ids = ids.to(DEV)[:, None].contiguous()
+    ops._call("lc_moe_lists", ops._ptr(ids), rows, 1, E, tile, ops._ptr(starts), ops._ptr(tiles), ops._ptr(token), ops._ptr(entry),
+              ops._stream())
+    routing = ops.Routing(ids, torch.ones(rows, 1, device=DEV), starts, tiles, token, entry, E, tile, rows // tile + E)
+    x = torch.randn(rows, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(E, N, K, generator=g).bfloat16().to(DEV)
+    for gather, act in ((True, "relu_squared"), (False, None)):
+        got = switched(1, lambda: ops.moe_experts(x, w, routing, out, activation=act, gather=gather))
+        plain = switched(0, lambda: ops.moe_experts(x, w, routing, out, activation=act, gather=gather))
+        expert = ids[:, 0].long()[entry.argsort()] if gather else None
+        order = token.long()
+        src = x[order] if gather else x
+        expert = ids[:, 0].long()[order]
+        want = torch.empty(rows, N, device=DEV)
+        for e in range(E):
+            want[expert == e] = src[expert == e].float() @ w[e].float().T
+        z = torch.relu(want) ** 2 if act else want
+        scale = 1.0 if not act else 2.0 * float(want.abs().max())       # the square's slope
+        assert off_by(got, z, K) <= max(1.0, scale), (gather, act)
+        assert off_by(plain, z, K) <= max(1.0, scale), (gather, act)
+
+
+@pytest.mark.parametrize("rows,G,N,K,gap", [(1, 3, 128, 128, 0), (16, 2, 65, 256, 8), (17, 4, 512, 128, 64), (64, 3, 128, 512, 0),
+                                            (65, 2, 33, 64, 8), (200, 5, 130, 192, 0)])
+def test_heads(rows, G, N, K, gap):
+    g = torch.Generator().manual_seed(rows + N)
+    x = torch.randn(rows, G * (K + gap), generator=g).bfloat16().to(DEV)
+    w = torch.randn(G, N, K, generator=g).bfloat16().to(DEV)
+    gate = torch.randn(rows, G * N + 2, generator=g).bfloat16().to(DEV)
+    plain = torch.stack([x[:, i * (K + gap):i * (K + gap) + K].float() @ w[i].float().T for i in range(G)], dim=1)
+    for kind in ("none", "entry", "group"):
+        out = torch.zeros(rows, G * N + 3, dtype=torch.bfloat16, device=DEV)
+        gates = None if kind == "none" else ops.Strided(gate, 2, N if kind == "entry" else 1)
+        switched(1, lambda: ops.grouped_gemm(ops.Strided(x, 0, K + gap), w, ops.Strided(out, 3, N), rows, gates,
+                                             gate_per_group=kind == "group"))
+        want = plain
+        if kind == "entry":
+            want = plain * torch.sigmoid(gate[:, 2:].float().view(rows, G, N))
+        elif kind == "group":
+            want = plain * torch.sigmoid(gate[:, 2:2 + G].float())[:, :, None]
+        assert off_by(out[:, 3:], want.reshape(rows, G * N), K) <= 1.0, kind
+        assert float(out[:, :3].abs().max()) == 0.0, "columns before the first group were written"
