@@ -40,7 +40,7 @@ template <int NR, int KS>
 __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     const bf16* __restrict__ qa, int H, int R, int rot, const bf16* __restrict__ cache,
     const int* __restrict__ tiles, const int* __restrict__ block_table, int max_blocks, int page_size,
-    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits,
+    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int by_tile,
     float* __restrict__ part_o, float* __restrict__ part_ml) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int Dk = R + rot, Dp = KS * 32;
@@ -270,23 +270,25 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
                 for (int r = 0; r < 4; ++r) dst[r] = static_cast<bf16>(o[d][r] * inv);
             }
     } else {
-        float* dst = part_o + (qi * splits + blockIdx.z) * R;
+        // a share's place: by token, or, where every tile is a lone token, by tile (the step may hold many other tokens)
+        const size_t place = by_tile ? (size_t)blockIdx.x * H + q_head : qi;
+        float* dst = part_o + (place * splits + blockIdx.z) * R;
 #pragma unroll
         for (int d = 0; d < NH; ++d)
             if ((half * NH + d) * 16 < R)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) dst[(half * NH + d) * 16 + 4 * g + r] = o[d][r];
         if (g == 0 && half == 0) {
-            part_ml[(qi * splits + blockIdx.z) * 2] = m_run;
-            part_ml[(qi * splits + blockIdx.z) * 2 + 1] = l_run;
+            part_ml[(place * splits + blockIdx.z) * 2] = m_run;
+            part_ml[(place * splits + blockIdx.z) * 2 + 1] = l_run;
         }
     }
 }
 
-// One workgroup per (token, head): the shares' sums, taken in from the first.
+// One workgroup per (token, head), or (tiles given) per (tile of one token, head): the shares' sums, taken in from the first.
 __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                              int splits, int R, int H, const float* __restrict__ sink,
-                                             bf16* __restrict__ out) {
+                                             const int* __restrict__ tiles, bf16* __restrict__ out) {
     __shared__ float weight[64];
     __shared__ float total;
     const size_t qi = blockIdx.x;
@@ -303,10 +305,11 @@ __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, c
     }
     __syncthreads();
     const float inv = 1.f / total;
+    const size_t row = tiles ? (size_t)tiles[4 * (qi / H)] * H + qi % H : qi;
     for (int d = threadIdx.x; d < R; d += blockDim.x) {
         float acc = 0.f;
         for (int z = 0; z < splits; ++z) acc = fmaf(part_o[(qi * splits + z) * R + d], weight[z], acc);
-        out[qi * R + d] = static_cast<bf16>(acc * inv);
+        out[row * R + d] = static_cast<bf16>(acc * inv);
     }
 }
 
@@ -343,8 +346,8 @@ LC_API int lc_latent_bf16_splits(int workgroups, int max_keys) {
 
 // qa [T, H, R + rot], cache [slots, R + rot] -> out [T, H, R].  tiles [NT, 4]: first token row, tokens
 // (1 to 16), request, first position.  any_portion: whether a tile has more than one token (the
-// grid then has a workgroup per four heads).  splits > 1: part_o [T H splits R] and part_ml [T H
-// splits 2] float32.
+// grid then has a workgroup per four heads).  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32,
+// n = T or, without a portion, num_tiles.
 LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot, const void* cache, const int* tiles,
                                     int num_tiles, int any_portion, const int* block_table, int max_blocks,
                                     int page_size, float scale, int window, const float* sink, void* out, int splits,
@@ -369,7 +372,7 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
                      "latent attention: %zu bytes of LDS refused", lds);                                           \
         latent_attention_bf16_kernel<NR, KS><<<grid, LM_THREADS, lds, stream>>>(                                    \
             (const bf16*)qa, H, R, rot, (const bf16*)cache, tiles, block_table, max_blocks, page_size, scale, window, \
-            sink, (bf16*)out, splits, part_o, part_ml);                                                               \
+            sink, (bf16*)out, splits, any_portion ? 0 : 1, part_o, part_ml);                                          \
     } while (0)
     if (nr == 4) LC_LM_LAUNCH(4, 4);
     else if (nr == 8) LC_LM_LAUNCH(8, 8);
@@ -378,7 +381,8 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
 #undef LC_LM_LAUNCH
     LC_LAUNCH_CHECK("latent_attention_bf16");
     if (splits > 1) {
-        latent_attention_join_kernel<<<T * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink, (bf16*)out);
+        latent_attention_join_kernel<<<(any_portion ? T : num_tiles) * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink,
+                                                                                          any_portion ? nullptr : tiles, (bf16*)out);
         LC_LAUNCH_CHECK("latent_attention_join");
     }
     return 0;

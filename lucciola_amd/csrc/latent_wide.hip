@@ -1,0 +1,289 @@
+// Latent attention for a prompt's portion, head by head.
+//
+// In the latent's space (latent_bf16.hip) a query meets 512 + 64 entries of a cached row and sums 512 of them, whatever the
+// head's own size: what a step of lone tokens wants, because it reads nothing but the rows.  A portion of many tokens has
+// many queries for every row, so it pays to take the rows out of the latent's space once: k_j = W_uk c_j beside the rotated
+// part, v_j = W_uv c_j, and to attend with 128 + 64 and 128 entries a head (320 multiply-adds a query and key where there were 1,088).
+// Three steps: latent_rows_kernel lays a request's visible rows side by side out of their pages; two dense products make
+// [row][head, entry] keys and, with the operands in the other order, [head, entry][row] values, which is the transposed form
+// that O^T = V^T P^T wants; latent_wide_kernel attends and applies the output gate.
+#include "common.h"
+
+#include "activations.h"
+#include "gemm_tile.h"
+
+namespace lc {
+
+typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
+
+constexpr int LW_KEYS = 64;         // keys of a stage; a request's rows are filled up to whole stages
+constexpr int LW_TOKENS = 128;      // queries of a workgroup, 32 a wave
+constexpr int LW_DIM = 128, LW_ROT = 64, LW_VDIM = 128;
+
+// grid (rows / 4): a wave a row.  Row i of the request's rows (position lo + i, its page's place in table) -> c [i][R], turned [i][rot];
+// zeros behind `count`.
+__global__ __launch_bounds__(256) void latent_rows_kernel(const bf16* __restrict__ cache, const int* __restrict__ table, int page_size,
+                                                          int R, int rot, int lo, int count, int rows, bf16* __restrict__ c,
+                                                          bf16* __restrict__ turned) {
+    const int i = blockIdx.x * 4 + threadIdx.x / kWave, lane = threadIdx.x % kWave;
+    if (i >= rows) return;
+    const int j = lo + i, pieces = (R + rot) / 8;
+    const bool live = i < count;
+    const bf16* row = cache + (size_t)(live ? table[j / page_size] * page_size + j % page_size : 0) * (R + rot);
+    for (int p = lane; p < pieces; p += kWave) {
+        bf16x8 v;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16>(0.f);
+        if (live) v = *reinterpret_cast<const bf16x8*>(row + p * 8);
+        if (p * 8 < R) *reinterpret_cast<bf16x8*>(c + (size_t)i * R + p * 8) = v;
+        else *reinterpret_cast<bf16x8*>(turned + (size_t)i * rot + (p * 8 - R)) = v;
+    }
+}
+
+struct WideArgs {
+    const bf16* q; long long ldq;               // [T][head][128 + 64], the rotated entries as they were
+    const bf16* q_turned; long long q_row, q_head;   // token t, head h: the 64 rotated entries at t q_row + h q_head
+    const bf16* keys; const bf16* turned;       // [row][H 128], [row][64]
+    const bf16* values; long long ldv;          // [H 128][row]
+    int H, first, tokens, position, lo;         // the portion: its first token's row of q and position; the rows' first position
+    float scale_log2; int window;
+    const float* sink;
+    const bf16* gate; long long ldg, gate_head; // token t, head h: at t ldg + h gate_head, 128 entries or (gate_head 1) one
+    bf16* out; long long ldo;
+};
+
+// Four operands of LDS and the wait for them in one piece: the compiler would wait for every load to LDS in flight before
+// an LDS read of its own.
+__device__ __forceinline__ void lds_four(bf16x8 (&r)[4], unsigned a, unsigned b, unsigned c, unsigned d) {
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+                 : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
+                 : "v"(a), "v"(b), "v"(c), "v"(d)
+                 : "memory");
+}
+
+// grid (heads, tiles of 128 tokens, the last first: it sees the most keys).  Head h runs on XCD h % 8, whose L2 keeps its keys and
+// values for all tiles.  A wave owns 32 queries: S^T = K Q^T by v_mfma_f32_32x32x16_bf16, with the rows of K taken in the order
+// that leaves a lane eight neighbouring keys of its query for each 16, which is what P^T needs as an operand; softmax
+// base 2 against a reference point that moves when a score outgrows it by 2^8; O^T += V^T P^T.  A stage of 64 keys (40 KB) comes
+// straight into LDS while the one before is worked through; 16-byte chunks lie at places xor the row, so that no operand's 16
+// rows meet a bank twice.  Two workgroups a CU, whose waves fill each other's waits.
+__global__ __launch_bounds__(256, 2) void latent_wide_kernel(WideArgs a) {
+    constexpr int KB = LW_KEYS * LW_DIM * 2, TB = LW_KEYS * LW_ROT * 2, VB = LW_VDIM * LW_KEYS * 2, STAGE = KB + TB + VB;
+    constexpr int KS = (LW_DIM + LW_ROT) / 16, VT = LW_VDIM / 32;
+    __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 31, half = lane >> 5;
+    const int head = blockIdx.x, tile = gridDim.y - 1 - blockIdx.y;
+    const int row = tile * LW_TOKENS + wave * 32 + col;     // the lane's token of the portion
+    const bool live = row < a.tokens;
+    const int token = a.first + min(row, a.tokens - 1);
+    const int tile_last = min(tile * LW_TOKENS + LW_TOKENS, a.tokens) - 1;
+    // keys are counted from the rows' first position on
+    const int at = a.position - a.lo + min(row, a.tokens - 1);      // the last key that the lane's query sees
+    const int from = a.window > 0 ? at - a.window + 1 : 0;          // and the first
+    const int wave_first = tile * LW_TOKENS + wave * 32;
+    const int wave_lo = a.window > 0 ? a.position - a.lo + wave_first - a.window + 1 : 0;
+    const int wave_hi = a.position - a.lo + min(wave_first + 31, a.tokens - 1);
+    const bool wave_live = wave_first < a.tokens;
+    const int tile_lo = a.window > 0 ? max(0, a.position - a.lo + tile * LW_TOKENS - a.window + 1) : 0;
+    const int s_begin = tile_lo / LW_KEYS, s_end = (a.position - a.lo + tile_last) / LW_KEYS + 1;
+
+    bf16x8 qf[KS];
+    {
+        const bf16* plain = a.q + (size_t)token * a.ldq + (size_t)head * (LW_DIM + LW_ROT) + 8 * half;
+        const bf16* turned = a.q_turned + (size_t)token * a.q_row + (size_t)head * a.q_head + 8 * half;
+#pragma unroll
+        for (int k = 0; k < KS; ++k)
+            qf[k] = *reinterpret_cast<const bf16x8*>(k < LW_DIM / 16 ? plain + 16 * k : turned + 16 * k - LW_DIM);
+    }
+    // load instructions: four rows of 256 bytes of the keys, eight of 128 of their rotated parts and of the values
+    const int r4 = lane >> 4, r8 = lane >> 3;
+    const bf16 *k_from[4], *t_from[2], *v_from[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        const int key = 16 * wave + 4 * i + r4;
+        k_from[i] = a.keys + (size_t)key * a.H * LW_DIM + (size_t)head * LW_DIM + (((lane & 15) ^ (key & 15)) * 8);
+        const int entry = 32 * wave + 8 * i + r8;
+        v_from[i] = a.values + ((size_t)head * LW_VDIM + entry) * a.ldv + (((lane & 7) ^ ((entry >> 1) & 7)) * 8);
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+        const int key = 16 * wave + 8 * i + r8;
+        t_from[i] = a.turned + (size_t)key * LW_ROT + (((lane & 7) ^ ((key >> 1) & 7)) * 8);
+    }
+    auto issue = [&](int s) {
+        char* stage = lds + (s & 1) * STAGE;
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(k_from[i] + (size_t)s * LW_KEYS * a.H * LW_DIM),
+                                             (lds_ptr_t)(stage + (4 * wave + i) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 2; ++i)
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(t_from[i] + (size_t)s * LW_KEYS * LW_ROT),
+                                             (lds_ptr_t)(stage + KB + (2 * wave + i) * 1024), 16, 0, 0);
+#pragma unroll
+        for (int i = 0; i < 4; ++i)
+            __builtin_amdgcn_global_load_lds((glb_ptr_t)(v_from[i] + (size_t)s * LW_KEYS),
+                                             (lds_ptr_t)(stage + KB + TB + (4 * wave + i) * 1024), 16, 0, 0);
+    };
+    // row r of a tile of S^T is key 16 (r / 16) + 8 ((r / 4) % 2) + 4 ((r / 8) % 2) + r % 4 of its 32: the lane's 16 values, rows
+    // 8 (v / 4) + 4 half + v % 4, are then the keys 16 (v / 8) + 8 half + v % 8
+    const int key = 16 * (col >> 4) + 8 * ((col >> 2) & 1) + 4 * ((col >> 3) & 1) + (col & 3);
+    const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)lds;
+    const unsigned k_row = lds0 + key * 256, t_row = lds0 + KB + key * 128, v_row = lds0 + KB + TB + col * 128;
+    const unsigned k_swz = key & 15, t_swz = (key >> 1) & 7, v_swz = (col >> 1) & 7;     // the same for the rows 32 further on
+
+    floatx16 o[VT];
+#pragma unroll
+    for (int i = 0; i < VT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) o[i][v] = 0.f;
+    float m_ref = -INFINITY, l = 0.f;
+    if (s_begin < s_end) issue(s_begin);
+    for (int s = s_begin; s < s_end; ++s) {
+        wait_vmcnt<0>();                                    // this wave's loads of the stage have landed
+        __builtin_amdgcn_s_barrier();                       // everybody's have; nobody reads the other stage any more
+        asm volatile("" ::: "memory");
+        if (s + 1 < s_end) issue(s + 1);
+        const int c0 = s * LW_KEYS;
+        if (!wave_live || c0 > wave_hi || c0 + LW_KEYS <= wave_lo) continue;
+        const unsigned stage = (s & 1) * STAGE;
+        floatx16 sc[2];
+#pragma unroll
+        for (int t = 0; t < 2; ++t) {
+#pragma unroll
+            for (int v = 0; v < 16; ++v) sc[t][v] = 0.f;
+#pragma unroll
+            for (int k = 0; k < KS; k += 4) {
+                bf16x8 ka[4];
+                unsigned where[4];
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int x = k + i;
+                    where[i] = x < LW_DIM / 16 ? k_row + stage + t * 32 * 256 + (((2 * x + half) ^ k_swz) * 16)
+                                               : t_row + stage + t * 32 * 128 + (((2 * (x - LW_DIM / 16) + half) ^ t_swz) * 16);
+                }
+                lds_four(ka, where[0], where[1], where[2], where[3]);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) sc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[i], qf[k + i], sc[t], 0, 0, 0);
+            }
+        }
+        // scores in units of log 2; what the query does not see is -infinity
+        const bool all = c0 + LW_KEYS - 1 <= wave_hi - 31 && c0 >= wave_lo + 31;       // every query of the wave sees every key
+        float mx = -INFINITY;
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                float x = sc[t][v] * a.scale_log2;
+                if (!all) {
+                    const int j = c0 + 32 * t + 16 * (v >> 3) + 8 * half + (v & 7);
+                    x = j <= at && j >= from ? x : -INFINITY;
+                }
+                sc[t][v] = x;
+                mx = fmaxf(mx, x);
+            }
+        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+        if (__builtin_amdgcn_ballot_w64(mx > m_ref + 8.f) != 0) {      // also at a query's first visible key
+            const float m_new = mx > m_ref + 8.f ? mx : m_ref;
+            const float keep = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
+            l *= keep;
+#pragma unroll
+            for (int i = 0; i < VT; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[i][v] *= keep;
+            m_ref = m_new;
+        }
+        const float ref = m_ref == -INFINITY ? 0.f : m_ref;
+        bf16x8 p[4];
+#pragma unroll
+        for (int t = 0; t < 2; ++t)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float w = __builtin_amdgcn_exp2f(sc[t][v] - ref);
+                l += w;
+                p[2 * t + (v >> 3)][v & 7] = static_cast<bf16>(w);
+            }
+#pragma unroll
+        for (int i = 0; i < VT; ++i) {
+            bf16x8 va[4];
+            unsigned where[4];
+#pragma unroll
+            for (int b = 0; b < 4; ++b) where[b] = v_row + stage + i * 32 * 128 + (((2 * b + half) ^ v_swz) * 16);
+            lds_four(va, where[0], where[1], where[2], where[3]);
+#pragma unroll
+            for (int b = 0; b < 4; ++b) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[b], p[b], o[i], 0, 0, 0);
+        }
+    }
+    if (!live) return;
+    l += __shfl_xor(l, 32, kWave);
+    float inv = 1.f / l;
+    if (a.sink) {       // one more term in the denominator, a key with that score and no value
+        const float s2 = a.sink[head] * 1.4426950408889634f, m_all = fmaxf(m_ref, s2);
+        const float keep = __builtin_amdgcn_exp2f(m_ref - m_all);
+        inv = keep / fmaf(l, keep, __builtin_amdgcn_exp2f(s2 - m_all));
+    }
+    const bf16* gate = a.gate ? a.gate + (size_t)token * a.ldg + (size_t)head * a.gate_head : nullptr;
+    if (gate && a.gate_head == 1) inv *= sigmoid(to_f32(gate[0]));
+    bf16* out = a.out + (size_t)token * a.ldo + (size_t)head * LW_VDIM;
+#pragma unroll
+    for (int i = 0; i < VT; ++i)
+#pragma unroll
+        for (int v = 0; v < 16; v += 4) {
+            const int e = 32 * i + 2 * v + 4 * half;        // rows 8 (v / 4) + 4 half ...
+            bf16x4 g, y;
+            if (gate && a.gate_head != 1) g = *reinterpret_cast<const bf16x4*>(gate + e);
+#pragma unroll
+            for (int n = 0; n < 4; ++n) {
+                float x = o[i][v + n] * inv;
+                if (gate && a.gate_head != 1) x *= sigmoid(static_cast<float>(g[n]));
+                y[n] = static_cast<bf16>(x);
+            }
+            *reinterpret_cast<bf16x4*>(out + e) = y;
+        }
+}
+
+}  // namespace lc
+
+using namespace lc;
+
+// Whether these heads have a kernel.
+LC_API int lc_latent_wide_supported(int R, int dim, int rot, int vdim) {
+    return dim == LW_DIM && rot == LW_ROT && vdim == LW_VDIM && R > 0 && R % 64 == 0 ? 1 : 0;
+}
+
+LC_API int lc_latent_rows(const void* cache, const int* table, int page_size, int R, int rot, int lo, int count, int rows, void* c,
+                          void* turned, hipStream_t stream) {
+    LC_CHECK(page_size > 0 && R > 0 && R % 8 == 0 && rot >= 0 && rot % 8 == 0 && lo >= 0 && count >= 0 && rows >= count, "latent_rows: bad sizes");
+    if (rows == 0) return 0;
+    LC_CHECK(cache && table && c && (turned || rot == 0), "latent_rows: null pointer");
+    LC_CHECK(((uintptr_t)cache | (uintptr_t)c | (uintptr_t)turned) % 16 == 0, "latent_rows: not aligned to 16 bytes");
+    latent_rows_kernel<<<(rows + 3) / 4, 256, 0, stream>>>((const bf16*)cache, table, page_size, R, rot, lo, count, rows, (bf16*)c,
+                                                           (bf16*)turned);
+    LC_LAUNCH_CHECK("latent_rows");
+    return 0;
+}
+
+// A portion of `tokens` tokens from row `first` of q on, at `position`, over the request's rows from position lo on: keys and
+// turned filled up to whole stages of 64 rows, values [H 128][ldv] likewise.
+LC_API int lc_latent_wide(const void* q, long long ldq, const void* q_turned, long long q_row, long long q_head, const void* keys,
+                          const void* turned, const void* values, long long ldv, int H, int first, int tokens, int position,
+                          int lo, float scale, int window, const float* sink, const void* gate, long long ldg, long long gate_head,
+                          void* out, long long ldo, hipStream_t stream) {
+    LC_CHECK(H > 0 && first >= 0 && tokens >= 0 && lo >= 0 && position >= lo && window >= 0, "latent_wide: bad sizes");
+    if (tokens == 0) return 0;
+    LC_CHECK(q && q_turned && keys && turned && values && out, "latent_wide: null pointer");
+    LC_CHECK(window == 0 ? lo == 0 : lo <= (position - window + 1 > 0 ? position - window + 1 : 0), "latent_wide: rows are missing");
+    LC_CHECK(((uintptr_t)q | (uintptr_t)q_turned | (uintptr_t)keys | (uintptr_t)turned | (uintptr_t)values) % 16 == 0 &&
+                 (ldq | q_row | q_head | ldv) % 8 == 0, "latent_wide: not aligned to 16 bytes");
+    LC_CHECK(ldv >= (position + tokens - lo + LW_KEYS - 1) / LW_KEYS * LW_KEYS, "latent_wide: the values' rows are too short");
+    LC_CHECK((uintptr_t)out % 8 == 0 && ldo % 4 == 0, "latent_wide: the output is not aligned to 8 bytes");
+    LC_CHECK(!gate || gate_head == 1 || (gate_head == LW_VDIM && (uintptr_t)gate % 8 == 0 && ldg % 4 == 0), "latent_wide: bad gates");
+    const int tiles = (tokens + LW_TOKENS - 1) / LW_TOKENS;
+    LC_CHECK(tiles <= 65535, "latent_wide: too many tokens");
+    WideArgs a{(const bf16*)q, ldq, (const bf16*)q_turned, q_row, q_head, (const bf16*)keys, (const bf16*)turned, (const bf16*)values, ldv,
+               H, first, tokens, position, lo, scale * 1.4426950408889634f, window, sink, (const bf16*)gate, ldg, gate_head,
+               (bf16*)out, ldo};
+    latent_wide_kernel<<<dim3(H, tiles), 256, 0, stream>>>(a);
+    LC_LAUNCH_CHECK("latent_wide");
+    return 0;
+}

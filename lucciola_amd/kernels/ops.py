@@ -11,7 +11,7 @@ import ctypes
 import heapq
 import threading
 from dataclasses import dataclass, replace
-from typing import Optional, Tuple
+from typing import Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -84,6 +84,9 @@ _SIGNATURES = {
     "lc_latent_prepare": "pqpiqiiiiipfppiipppp",
     "lc_latent_attention": "piiiiippppiifippp",
     "lc_latent_bf16_supported": "ii",
+    "lc_latent_wide_supported": "iiii",
+    "lc_latent_rows": "ppiiiiiippp",
+    "lc_latent_wide": "pqpqqpppqiiiiifippqqpqp",
     "lc_latent_bf16_splits": "ii",
     "lc_latent_attention_bf16": "piiiippiipiifippippp",
     "lc_moe_max_experts": "",
@@ -1206,11 +1209,15 @@ def _check_strided(s: Strided, what: str, rows: int, groups: int, width: int, dt
                           f"and {rows} rows do not fit {tuple(s.tensor.shape)}")
 
 
-def _grouped_tile(rows: int) -> int:
-    """Rows of the tiles of a product per head over ``rows`` rows: 16 for a step of few tokens, else 64 (these products
-    are short, K of 128 or 512 and as many columns, so what counts is many workgroups: 2,048 rows, 32 heads, 512 columns of
-    128 k: 36 us in tiles of 64 x 128 and 80 in 128 x 128; 128 columns of 512 k 22 and 32)."""
-    return 16 if rows <= 16 else 64
+def _grouped_tile(rows: int, N: int, groups: int, x: torch.Tensor, w: torch.Tensor) -> int:
+    """Rows of the tiles of a product per head over ``rows`` rows: 16 for a step of few tokens, else 64; bfloat16 operands stay
+    with 16 up to 1,024 workgroups (these products are short, K of 128 or 512 and as many columns, so what counts is many
+    workgroups: 64 rows, 16 heads, 128 columns of 512 k: 4.2 us in tiles of 16 x 64, 8.4 to 8.9 in larger ones; 512 rows 8.0 and
+    8.5; 512 columns of 128 k, 160 rows 6.7 and 6.6, 512 rows 16 and 8)."""
+    if rows <= 16:
+        return 16
+    few = x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and -(-rows // 16) * -(-N // 64) * groups <= 1024
+    return 16 if few else 64
 
 
 def grouped_gemm(x: Strided, w: torch.Tensor, out: Strided, rows: int, gate: Optional[Strided] = None,
@@ -1234,7 +1241,7 @@ def grouped_gemm(x: Strided, w: torch.Tensor, out: Strided, rows: int, gate: Opt
         return
     _call("lc_gemm_grouped", x.pointer(), _dt(x.tensor), x.tensor.shape[1], x.group, _ptr(w), _dt(w),
           out.pointer(), _dt(out.tensor), out.tensor.shape[1], out.group, rows, N, K, G, None, None, None, 0,
-          _grouped_tile(rows), epilogue, gate.pointer() if gate is not None else None,
+          _grouped_tile(rows, N, G, x.tensor, w), epilogue, gate.pointer() if gate is not None else None,
           gate.tensor.shape[1] if gate is not None else 0, gate.group if gate is not None else 0, _stream())
 
 
@@ -1333,6 +1340,78 @@ def plan_latent_attention(layout):
              "num_tiles": len(tiles)})
 
 
+# From this many tokens on a request's portion attends head by head (``latent_wide``) where the heads have the kernel.
+LATENT_WIDE_FROM = 64
+LATENT_SHORT_PLAN = "latent_attention of short portions"
+
+
+def plan_latent_short(layout):
+    """As ``plan_latent_attention``, without the portions that attend head by head."""
+    keep = [r for r in range(layout.num_requests) if layout.q_start[r + 1] - layout.q_start[r] < LATENT_WIDE_FROM]
+    arrays, info = plan_latent_attention(layout)
+    if len(keep) < layout.num_requests:
+        tiles = arrays["tiles"][np.isin(arrays["tiles"][:, 2], keep)]
+        arrays = {"tiles": tiles if len(tiles) else np.zeros((1, 4), np.int32)}     # one that no launch reads
+        info = {"any_portion": bool((tiles[:, 1] > 1).any()), "any_lone": bool((tiles[:, 1] == 1).any()), "num_tiles": len(tiles)}
+    return arrays, info
+
+
+def latent_wide_takes(rank: int, dim: int, rot: int, vdim: int, dtype: torch.dtype, device: torch.device) -> bool:
+    """Whether a prompt's portion can attend head by head: bfloat16, heads of 128 + 64 and values of 128, a latent of whole
+    blocks of 64."""
+    return bool(dtype == torch.bfloat16 and device.type == "cuda" and library().lc_latent_wide_supported(rank, dim, rot, vdim))
+
+
+def latent_wide_requests(batch) -> list:
+    """The requests of a step whose portions attend head by head (none with ``latent_matrix_cores(False)``)."""
+    if not _latent_fast.on or batch.num_tokens < LATENT_WIDE_FROM:
+        return []
+    return [r for r in range(batch.num_requests) if batch.q_start[r + 1] - batch.q_start[r] >= LATENT_WIDE_FROM]
+
+
+def latent_wide(q: torch.Tensor, qa: torch.Tensor, heads: int, rank: int, dim: int, rot: int, vdim: int, uk: torch.Tensor,
+                uv: torch.Tensor, cache: torch.Tensor, block_table: torch.Tensor, page_size: int, requests: Sequence[int],
+                q_start: Sequence[int], first_position: Sequence[int], scale: float, window: int, sink: Optional[torch.Tensor],
+                gate: Optional[Strided], gate_per_head: bool, out: torch.Tensor) -> None:
+    """Latent attention of the portions of ``requests`` head by head: every visible row c of a request becomes a key [W_uk c |
+    rotated part] and a value W_uv c of each head, and the tokens attend over those.  ``q`` [T, heads (dim + rot) (+ more)] with
+    the plain query entries, ``qa`` [T, heads (rank + rot)] with the rotated ones behind each head's ``rank`` entries (which
+    are not read), ``uk`` [heads dim, rank], ``uv`` [heads vdim, rank]; the result times sigmoid(gate) goes to the tokens' rows of
+    ``out`` [T, heads vdim]."""
+    for t, what in ((q, "q"), (qa, "qa"), (uk, "uk"), (uv, "uv"), (cache, "cache"), (out, "out")):
+        _need(t, f"latent_wide {what}", torch.bfloat16, t.dim())
+    _need(block_table, "block table", torch.int32, 2)
+    T = q.shape[0]
+    if qa.shape != (T, heads * (rank + rot)) or q.shape[1] < heads * (dim + rot) or cache.shape[-1] != rank + rot or \
+            uk.shape != (heads * dim, rank) or uv.shape != (heads * vdim, rank) or out.shape != (T, heads * vdim):
+        raise KernelError("latent_wide: the tensors do not fit the heads")
+    if gate is not None:
+        _check_strided(gate, "latent_wide gate", T, heads, 1 if gate_per_head else vdim, torch.bfloat16)
+    spans, total = [], 0
+    for r in requests:
+        position, tokens = int(first_position[r]), q_start[r + 1] - q_start[r]
+        lo = max(0, position - window + 1) if window else 0
+        if (position + tokens - 1) // page_size >= block_table.shape[1]:
+            raise KernelError(f"latent_wide: request {r}'s block table is too short")
+        spans.append((r, position, tokens, lo, total))
+        total += -(-(position + tokens - lo) // 64) * 64
+    c = torch.empty((total, rank), dtype=q.dtype, device=q.device)
+    turned = torch.empty((total, rot), dtype=q.dtype, device=q.device)
+    stream = _stream()
+    for n, (r, position, tokens, lo, at) in enumerate(spans):
+        rows = (spans[n + 1][4] if n + 1 < len(spans) else total) - at
+        _call("lc_latent_rows", _ptr(cache), _ptr(block_table[r]), page_size, rank, rot, lo, position + tokens - lo, rows,
+              _ptr(c[at:]), _ptr(turned[at:]), stream)
+    keys = gemm(c, uk, q.dtype)
+    values = gemm(uv, c, q.dtype)               # [heads vdim, rows]: transposed as the product leaves it
+    for r, position, tokens, lo, at in spans:
+        _call("lc_latent_wide", _ptr(q), q.shape[1], ctypes.c_void_p(qa.data_ptr() + rank * 2), heads * (rank + rot), rank + rot,
+              _ptr(keys[at:]), _ptr(turned[at:]), ctypes.c_void_p(values.data_ptr() + at * 2), total, heads, q_start[r], tokens,
+              position, lo, float(scale), int(window), _ptr(sink), gate.pointer() if gate is not None else None,
+              gate.tensor.shape[1] if gate is not None else 0, (1 if gate_per_head else vdim) if gate is not None else 0,
+              _ptr(out), heads * vdim, stream)
+
+
 def latent_attention(qa: torch.Tensor, heads: int, rank: int, rot: int, tok_req: torch.Tensor,
                      positions: torch.Tensor, block_table: torch.Tensor, cache: torch.Tensor, page_size: int,
                      scale: float, window: int = 0, plan=None, max_ctx: int = 0,
@@ -1369,9 +1448,13 @@ def latent_attention(qa: torch.Tensor, heads: int, rank: int, rot: int, tok_req:
         most = block_table.shape[1] * page_size if max_ctx <= 0 else max_ctx
         splits = lib.lc_latent_bf16_splits(workgroups, min(most, window) if window > 0 else most)
         part_o = part_ml = None
+        # the shares' places: by tile where all are lone tokens, else by token of the step, of which only few may have any
+        places = (T if any_portion else tiles.shape[0]) * heads
+        if any_portion and splits > 1:
+            splits = max(1, min(splits, (128 << 20) // (places * rank * 4)))
         if splits > 1:
-            part_o = torch.empty((T * heads * splits * rank,), dtype=torch.float32, device=qa.device)
-            part_ml = torch.empty((T * heads * splits * 2,), dtype=torch.float32, device=qa.device)
+            part_o = torch.empty((places * splits * rank,), dtype=torch.float32, device=qa.device)
+            part_ml = torch.empty((places * splits * 2,), dtype=torch.float32, device=qa.device)
         _call("lc_latent_attention_bf16", _ptr(qa), T, heads, rank, rot, _ptr(cache), _ptr(tiles), tiles.shape[0],
               1 if any_portion else 0, _ptr(block_table), block_table.shape[1], page_size, float(scale), int(window),
               _ptr(sink), _ptr(out), splits, _ptr(part_o), _ptr(part_ml), _stream())

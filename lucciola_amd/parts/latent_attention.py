@@ -38,6 +38,7 @@ from .feed_forward import stack_rows
 @MIXERS.register("latent_attention")
 class LatentAttention(Part):
     graph_safe = True   # launches only kernels whose arguments stay put between steps
+    wide = False        # until bind: whether long portions attend head by head
 
     def __init__(self, hidden_size: int, num_heads: int, dim: int, rot_dim: int, vdim: int,
                  kv_rank: int, scale: float, eps: float, position: Optional[PartSpec] = None,
@@ -92,6 +93,13 @@ class LatentAttention(Part):
         self.uv = tensors["uv"].view(self.H, self.vdim, self.rank).contiguous()
         self.o = tensors["o"]
         self.dtype = ctx.dtype
+        # the long portions of prompts attend head by head, over keys and values taken out of the latent's space
+        gate_column = self.first_cols + self.rank + self.rot
+        self.wide = ops.latent_wide_takes(self.rank, self.dim, self.rot, self.vdim, ctx.dtype, ctx.device) and \
+            all(t.dtype == torch.bfloat16 for t in (self.qdg, self.uv, tensors["uk"])) and \
+            self.qdg.shape[0] % 8 == 0 and (self.gate_per_head or gate_column % 4 == 0)
+        if self.wide:
+            self.uk, self.uv_rows = tensors["uk"].contiguous(), self.uv.view(self.H * self.vdim, self.rank)
         if self.position is not None:
             self.position.bind({}, ctx)
 
@@ -99,6 +107,8 @@ class LatentAttention(Part):
         return PagedLatent(self.rank + self.rot, self.window)
 
     def batch_planner(self):
+        if self.wide:
+            return ops.LATENT_SHORT_PLAN, ops.plan_latent_short
         return ops.LATENT_PLAN, ops.plan_latent_attention
 
     def tables_epoch(self) -> int:
@@ -126,15 +136,21 @@ class LatentAttention(Part):
         ops.latent_prepare(qdg, H, dim, rot, rank, self.norm_weight, self.eps, batch.positions, table,
                            pairing, site.cache, pages.slots if site.writes_cache else None, qa,
                            q=q, kv_column=self.first_cols)
-        if dim:
-            ops.grouped_gemm(ops.Strided(q, 0, dim + rot), self.uk_t, ops.Strided(qa, 0, rank + rot), T)
-        latent = ops.latent_attention(qa, H, rank, rot, batch.tok_req, batch.positions, pages.block_table,
-                                      site.cache, pages.page_size, self.scale, self.window or 0,
-                                      plan=batch.plans.get(ops.LATENT_PLAN), max_ctx=batch.max_ctx, sink=self.sink)
         heads = torch.empty((T, H * vdim), dtype=self.dtype, device=qdg.device)
         gate = None
         if self.gate:
             gate = ops.Strided(qdg, self.first_cols + rank + rot, 1 if self.gate_per_head else vdim)
-        ops.grouped_gemm(ops.Strided(latent, 0, rank), self.uv, ops.Strided(heads, 0, vdim), T, gate=gate,
-                         gate_per_group=self.gate_per_head)
+        long = ops.latent_wide_requests(batch) if self.wide else []
+        if len(long) < batch.num_requests:
+            if dim:
+                ops.grouped_gemm(ops.Strided(q, 0, dim + rot), self.uk_t, ops.Strided(qa, 0, rank + rot), T)
+            latent = ops.latent_attention(qa, H, rank, rot, batch.tok_req, batch.positions, pages.block_table,
+                                          site.cache, pages.page_size, self.scale, self.window or 0,
+                                          plan=batch.plans.get(self.batch_planner()[0]), max_ctx=batch.max_ctx, sink=self.sink)
+            ops.grouped_gemm(ops.Strided(latent, 0, rank), self.uv, ops.Strided(heads, 0, vdim), T, gate=gate,
+                             gate_per_group=self.gate_per_head)
+        if long:        # over what the products above made of these tokens' rows, which nothing has attended for
+            ops.latent_wide(q, qa, H, rank, dim, rot, vdim, self.uk, self.uv_rows, site.cache, pages.block_table, pages.page_size,
+                            long, batch.q_start, batch.first_position, self.scale, self.window or 0, self.sink, gate,
+                            self.gate_per_head, heads)
         return ops.gemm(heads, self.o, self.dtype, defer=True)

@@ -1,0 +1,98 @@
+"""Latent attention of long portions head by head (``ops.latent_wide``) against the same formulas in float64, in steps of
+several requests, behind histories, windows and pages that were given back; and which steps take it."""
+import pytest
+import torch
+
+from lucciola_amd.engine.batch import HostLayout
+from lucciola_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+DIM, ROT, VDIM = 128, 64, 128
+
+
+def reference(q, turned_q, c, turned, uk, uv, position, scale, window, sink):
+    """One head's tokens in float64 over one request's rows: keys and values rounded as the products leave them."""
+    k = torch.cat([(c @ uk.T).bfloat16().double(), turned], 1)
+    v = (c @ uv.T).bfloat16().double()
+    s = torch.cat([q, turned_q], 1) @ k.T * scale
+    i, j = position + torch.arange(len(q), device=DEV)[:, None], torch.arange(len(c), device=DEV)[None]
+    seen = j <= i
+    if window:
+        seen &= j > i - window
+    s = s.masked_fill(~seen, float("-inf"))
+    top = s.max(1, keepdim=True).values
+    if sink is not None:
+        top = torch.maximum(top, sink)
+    e = torch.exp(s - top)
+    return e @ v / (e.sum(1, keepdim=True) + (torch.exp(sink - top) if sink is not None else 0.0))
+
+
+@pytest.mark.parametrize("heads,rank,page,window,gate,with_sink,requests", [
+    (2, 512, 16, 0, "entry", False, [(0, 64)]), (3, 64, 16, 0, "head", True, [(0, 65), (63, 127), (100, 128)]),
+    (1, 128, 4, 50, "none", True, [(0, 129), (200, 300)]), (2, 192, 32, 64, "entry", False, [(7, 191), (64, 64)]),
+    (1, 512, 16, 0, "none", False, [(1000, 257)])])
+def test_wide(heads, rank, page, window, gate, with_sink, requests):
+    g = torch.Generator().manual_seed(heads * 1000 + rank + window)
+    def made(*shape):
+        return torch.randn(*shape, generator=g)
+    T = sum(n for _, n in requests) + 3                      # three tokens of others in front
+    q_start = [3]
+    for _, n in requests:
+        q_start.append(q_start[-1] + n)
+    first = [p for p, _ in requests]
+    pages_each = [-(-(p + n) // page) for p, n in requests]
+    cache = (made(sum(pages_each) + 1, page, rank + ROT) * 0.7).bfloat16().to(DEV)
+    order = torch.randperm(sum(pages_each), generator=g) + 1
+    table = torch.full((len(requests), max(pages_each) + 1), -1, dtype=torch.int32)
+    at = 0
+    for r, n in enumerate(pages_each):
+        table[r, :n] = order[at:at + n]
+        at += n
+        if window:          # pages behind the window have gone back
+            table[r, :max(0, first[r] - window + 1) // page] = -1
+    ldq = heads * (DIM + ROT) + 8
+    q, qa = made(T, ldq).bfloat16().to(DEV), made(T, heads * (rank + ROT)).bfloat16().to(DEV)
+    uk, uv = (made(heads * n, rank).mul(rank ** -0.5).bfloat16().to(DEV) for n in (DIM, VDIM))
+    gates = made(T, heads * VDIM + 4).bfloat16().to(DEV)
+    sink = made(heads).to(DEV) if with_sink else None
+    out = torch.zeros(T, heads * VDIM, dtype=torch.bfloat16, device=DEV)
+    scale = (DIM + ROT) ** -0.5 * 2.0
+    strided = None if gate == "none" else ops.Strided(gates, 4, VDIM if gate == "entry" else 1)
+    ops.latent_wide(q, qa, heads, rank, DIM, ROT, VDIM, uk, uv, cache, table.to(DEV), page, range(len(requests)), q_start, first,
+                    scale, window, sink, strided, gate == "head", out)
+    assert float(out[:3].abs().max()) == 0.0, "other tokens' rows were written"
+    for r, (p, n) in enumerate(requests):
+        slots = [max(0, int(table[r, j // page])) * page + j % page for j in range(p + n)]
+        rows = cache.view(-1, rank + ROT)[slots].double()
+        mine = slice(q_start[r], q_start[r] + n)
+        for h in range(heads):
+            plain = q[mine, h * (DIM + ROT):h * (DIM + ROT) + DIM].double()
+            turned_q = qa[mine].view(n, heads, rank + ROT)[:, h, rank:].double()
+            want = reference(plain, turned_q, rows[:, :rank], rows[:, rank:], uk[h * DIM:(h + 1) * DIM].double(),
+                             uv[h * VDIM:(h + 1) * VDIM].double(), p, scale, window, sink[h].double() if with_sink else None)
+            if gate == "entry":
+                want = want * torch.sigmoid(gates[mine, 4 + h * VDIM:4 + (h + 1) * VDIM].double())
+            elif gate == "head":
+                want = want * torch.sigmoid(gates[mine, 4 + h:5 + h].double())
+            got = out[mine, h * VDIM:(h + 1) * VDIM].double()
+            # the weights and the result are rounded to bfloat16 (2^-9 each, of numbers up to the largest value), and so are
+            # keys and values, where another order of a sum may round to the neighbour now and then
+            bound = 3 * 2.0 ** -9 * float(rows.abs().max().clamp(min=4.0))
+            assert float((got - want).abs().max()) <= bound, (r, h)
+            assert float((got - want).norm() / want.norm()) <= 2.0 ** -8, (r, h)
+
+
+def test_short_portions_keep_their_tiles():
+    lengths, first = [1, 64, 63, 200, 1], [500, 0, 9, 100, 3]
+    q_start = [0]
+    for n in lengths:
+        q_start.append(q_start[-1] + n)
+    layout = HostLayout(5, q_start[-1], q_start, first, 16, False)
+    arrays, info = ops.plan_latent_short(layout)
+    assert sorted(set(arrays["tiles"][:, 2].tolist())) == [0, 2, 4]
+    assert int(arrays["tiles"][:, 1].sum()) == 65 and info == {"any_portion": True, "any_lone": True, "num_tiles": 6}
+    every, _ = ops.plan_latent_short(HostLayout(1, 90, [0, 90], [0], 16, False))
+    assert every["tiles"].shape == (1, 4)
+    assert torch.equal(torch.tensor(ops.plan_latent_short(HostLayout(1, 60, [0, 60], [5], 16, False))[0]["tiles"]),
+                       torch.tensor(ops.plan_latent_attention(HostLayout(1, 60, [0, 60], [5], 16, False))[0]["tiles"]))
