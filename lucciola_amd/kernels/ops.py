@@ -1340,20 +1340,32 @@ def plan_latent_attention(layout):
              "num_tiles": len(tiles)})
 
 
-# From this many tokens on a request's portion attends head by head (``latent_wide``) where the heads have the kernel.
-LATENT_WIDE_FROM = 64
-LATENT_SHORT_PLAN = "latent_attention of short portions"
+def latent_wide_pays(tokens: int, position: int, heads: int, window: int) -> bool:
+    """Whether a portion of ``tokens`` tokens behind ``position`` others is faster head by head (``latent_wide``) than in the
+    latent's space, by what each takes on 256 CUs.  In the latent's space a workgroup of 16 tokens and four heads takes 3 us
+    for 32 rows, a CU holds one, and few tiles share out their rows; head by head a workgroup of 128 tokens of a head takes
+    1.15 us for 64 rows, two a CU, whoever is alone walks all of them, and the keys and values cost 0.52 ns a row and head and four
+    launches more.  (A layer with 16 heads: 2,048 tokens 430 us and 85; behind 2,048 others 830 and 175; 256 tokens behind 4,000
+    others 100 and 125; below some 700 tokens of a fresh prompt the launches weigh more than either.)"""
+    span = position + tokens if not window else min(position + tokens, window + tokens - 1)
+    latent = -(-tokens // 16) * -(-heads // 4) * -(-span // 32) * 3.0 / 256
+    wide = 20.0 + -(-span // 64) * 1.15 * -(-(-(-tokens // 128) * heads) // 512) + span * heads * 5.2e-4
+    return wide < latent
 
 
-def plan_latent_short(layout):
-    """As ``plan_latent_attention``, without the portions that attend head by head."""
-    keep = [r for r in range(layout.num_requests) if layout.q_start[r + 1] - layout.q_start[r] < LATENT_WIDE_FROM]
-    arrays, info = plan_latent_attention(layout)
-    if len(keep) < layout.num_requests:
-        tiles = arrays["tiles"][np.isin(arrays["tiles"][:, 2], keep)]
-        arrays = {"tiles": tiles if len(tiles) else np.zeros((1, 4), np.int32)}     # one that no launch reads
-        info = {"any_portion": bool((tiles[:, 1] > 1).any()), "any_lone": bool((tiles[:, 1] == 1).any()), "num_tiles": len(tiles)}
-    return arrays, info
+def latent_short_planner(heads: int, window: int):
+    """(key, planner) for a part whose long portions may attend head by head: ``plan_latent_attention`` for the others, and in
+    ``info["wide"]`` the requests that do."""
+    def plan(layout):
+        wide = [r for r in range(layout.num_requests)
+                if latent_wide_pays(layout.q_start[r + 1] - layout.q_start[r], layout.first_position[r], heads, window)]
+        arrays, info = plan_latent_attention(layout)
+        if wide:
+            tiles = arrays["tiles"][~np.isin(arrays["tiles"][:, 2], wide)]
+            arrays = {"tiles": tiles if len(tiles) else np.zeros((1, 4), np.int32)}     # one that no launch reads
+            info = {"any_portion": bool((tiles[:, 1] > 1).any()), "any_lone": bool((tiles[:, 1] == 1).any()), "num_tiles": len(tiles)}
+        return arrays, dict(info, wide=wide)
+    return ("latent attention of short portions", heads, window), plan
 
 
 def latent_wide_takes(rank: int, dim: int, rot: int, vdim: int, dtype: torch.dtype, device: torch.device) -> bool:
@@ -1362,11 +1374,9 @@ def latent_wide_takes(rank: int, dim: int, rot: int, vdim: int, dtype: torch.dty
     return bool(dtype == torch.bfloat16 and device.type == "cuda" and library().lc_latent_wide_supported(rank, dim, rot, vdim))
 
 
-def latent_wide_requests(batch) -> list:
+def latent_wide_requests(plan) -> list:
     """The requests of a step whose portions attend head by head (none with ``latent_matrix_cores(False)``)."""
-    if not _latent_fast.on or batch.num_tokens < LATENT_WIDE_FROM:
-        return []
-    return [r for r in range(batch.num_requests) if batch.q_start[r + 1] - batch.q_start[r] >= LATENT_WIDE_FROM]
+    return plan.info.get("wide", []) if plan is not None and _latent_fast.on else []
 
 
 def latent_wide(q: torch.Tensor, qa: torch.Tensor, heads: int, rank: int, dim: int, rot: int, vdim: int, uk: torch.Tensor,

@@ -108,7 +108,7 @@ class LatentAttention(Part):
 
     def batch_planner(self):
         if self.wide:
-            return ops.LATENT_SHORT_PLAN, ops.plan_latent_short
+            return ops.latent_short_planner(self.H, self.window or 0)
         return ops.LATENT_PLAN, ops.plan_latent_attention
 
     def tables_epoch(self) -> int:
@@ -140,13 +140,14 @@ class LatentAttention(Part):
         gate = None
         if self.gate:
             gate = ops.Strided(qdg, self.first_cols + rank + rot, 1 if self.gate_per_head else vdim)
-        long = ops.latent_wide_requests(batch) if self.wide else []
+        plan = batch.plans.get(self.batch_planner()[0])
+        long = ops.latent_wide_requests(plan) if self.wide else []
         if len(long) < batch.num_requests:
             if dim:
                 ops.grouped_gemm(ops.Strided(q, 0, dim + rot), self.uk_t, ops.Strided(qa, 0, rank + rot), T)
             latent = ops.latent_attention(qa, H, rank, rot, batch.tok_req, batch.positions, pages.block_table,
                                           site.cache, pages.page_size, self.scale, self.window or 0,
-                                          plan=batch.plans.get(self.batch_planner()[0]), max_ctx=batch.max_ctx, sink=self.sink)
+                                          plan=plan, max_ctx=batch.max_ctx, sink=self.sink)
             ops.grouped_gemm(ops.Strided(latent, 0, rank), self.uv, ops.Strided(heads, 0, vdim), T, gate=gate,
                              gate_per_group=self.gate_per_head)
         if long:        # over what the products above made of these tokens' rows, which nothing has attended for

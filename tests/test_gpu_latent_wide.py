@@ -84,15 +84,16 @@ def test_wide(heads, rank, page, window, gate, with_sink, requests):
 
 
 def test_short_portions_keep_their_tiles():
-    lengths, first = [1, 64, 63, 200, 1], [500, 0, 9, 100, 3]
+    lengths, first = [1, 1500, 63, 2000, 1], [500, 0, 9, 100, 3]
     q_start = [0]
     for n in lengths:
         q_start.append(q_start[-1] + n)
-    layout = HostLayout(5, q_start[-1], q_start, first, 16, False)
-    arrays, info = ops.plan_latent_short(layout)
-    assert sorted(set(arrays["tiles"][:, 2].tolist())) == [0, 2, 4]
-    assert int(arrays["tiles"][:, 1].sum()) == 65 and info == {"any_portion": True, "any_lone": True, "num_tiles": 6}
-    every, _ = ops.plan_latent_short(HostLayout(1, 90, [0, 90], [0], 16, False))
-    assert every["tiles"].shape == (1, 4)
-    assert torch.equal(torch.tensor(ops.plan_latent_short(HostLayout(1, 60, [0, 60], [5], 16, False))[0]["tiles"]),
-                       torch.tensor(ops.plan_latent_attention(HostLayout(1, 60, [0, 60], [5], 16, False))[0]["tiles"]))
+    key, plan = ops.latent_short_planner(16, 4096)
+    arrays, info = plan(HostLayout(5, q_start[-1], q_start, first, 16, False))
+    assert info == {"any_portion": True, "any_lone": True, "num_tiles": 6, "wide": [1, 3]}
+    assert sorted(set(arrays["tiles"][:, 2].tolist())) == [0, 2, 4] and int(arrays["tiles"][:, 1].sum()) == 65
+    every, info = plan(HostLayout(1, 2048, [0, 2048], [0], 16, False))
+    assert every["tiles"].shape == (1, 4) and info["wide"] == [0] and info["num_tiles"] == 0
+    short = HostLayout(2, 61, [0, 60, 61], [5, 9], 16, False)
+    assert plan(short)[0]["tiles"].tolist() == ops.plan_latent_attention(short)[0]["tiles"].tolist()
+    assert plan(short)[1]["wide"] == [] and key != ops.latent_short_planner(16, 0)[0]
