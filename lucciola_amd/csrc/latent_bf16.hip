@@ -40,7 +40,7 @@ template <int NR, int KS>
 __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     const bf16* __restrict__ qa, int H, int R, int rot, const bf16* __restrict__ cache,
     const int* __restrict__ tiles, const int* __restrict__ block_table, int max_blocks, int page_size,
-    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int by_tile,
+    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int per_tile,
     float* __restrict__ part_o, float* __restrict__ part_ml) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int Dk = R + rot, Dp = KS * 32;
@@ -270,8 +270,8 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
                 for (int r = 0; r < 4; ++r) dst[r] = static_cast<bf16>(o[d][r] * inv);
             }
     } else {
-        // a share's place: by token, or, where every tile is a lone token, by tile (the step may hold many other tokens)
-        const size_t place = by_tile ? (size_t)blockIdx.x * H + q_head : qi;
+        // a share's place goes by tile, not by token: the step may hold many tokens that are in no tile
+        const size_t place = ((size_t)blockIdx.x * per_tile + q_tok) * H + q_head;
         float* dst = part_o + (place * splits + blockIdx.z) * R;
 #pragma unroll
         for (int d = 0; d < NH; ++d)
@@ -285,13 +285,16 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     }
 }
 
-// One workgroup per (token, head), or (tiles given) per (tile of one token, head): the shares' sums, taken in from the first.
+// One workgroup per (tile, token of per_tile, head): the shares' sums, taken in from the first.
 __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                              int splits, int R, int H, const float* __restrict__ sink,
-                                             const int* __restrict__ tiles, bf16* __restrict__ out) {
+                                             const int* __restrict__ tiles, int per_tile, bf16* __restrict__ out) {
     __shared__ float weight[64];
     __shared__ float total;
     const size_t qi = blockIdx.x;
+    const int* tile = tiles + 4 * (qi / H / per_tile);
+    const int q_tok = (int)(qi / H) % per_tile;
+    if (q_tok >= tile[1]) return;
     if (threadIdx.x < 64) {
         const int z = threadIdx.x;
         const float m = z < splits ? part_ml[(qi * splits + z) * 2] : -INFINITY;
@@ -305,13 +308,20 @@ __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, c
     }
     __syncthreads();
     const float inv = 1.f / total;
-    const size_t row = tiles ? (size_t)tiles[4 * (qi / H)] * H + qi % H : qi;
+    const size_t row = (size_t)(tile[0] + q_tok) * H + qi % H;
     for (int d = threadIdx.x; d < R; d += blockDim.x) {
         float acc = 0.f;
         for (int z = 0; z < splits; ++z) acc = fmaf(part_o[(qi * splits + z) * R + d], weight[z], acc);
         out[row * R + d] = static_cast<bf16>(acc * inv);
     }
 }
+
+// latent_lone.hip: steps of lone tokens, rows of 512 + 64
+bool latent_lone_takes(int R, int rot);
+int launch_latent_lone(const void* qa, int H, const void* cache, const int* tiles, int num_tiles, const int* block_table, int max_blocks,
+                       int page_size, float scale, int window, const float* sink, void* out, int splits, float* part_o, float* part_ml,
+                       hipStream_t stream);
+static thread_local int g_lone = 1;
 
 static bool shape_of(int R, int rot, int* nr, int* ks) {
     const int Dk = R + rot;
@@ -333,6 +343,17 @@ LC_API int lc_latent_bf16_supported(int R, int rot) {
     return shape_of(R, rot, &nr, &ks) ? 1 : 0;
 }
 
+// Tests and tuning: whether steps of lone tokens may take the kernel of latent_lone.hip (1, the default), for the calling
+// thread.  Returns the setting before.
+LC_API int lc_latent_lone(int on) {
+    const int before = g_lone;
+    if (on >= 0) g_lone = on ? 1 : 0;
+    return before;
+}
+
+// Heads that a workgroup serves of a lone token.
+LC_API int lc_latent_lone_heads(int R, int rot) { return g_lone && latent_lone_takes(R, rot) ? 16 : 64; }
+
 // Shares the stages of a tile are cut into: from the number of workgroups without shares and
 // the most keys a tile can see.
 LC_API int lc_latent_bf16_splits(int workgroups, int max_keys) {
@@ -346,8 +367,8 @@ LC_API int lc_latent_bf16_splits(int workgroups, int max_keys) {
 
 // qa [T, H, R + rot], cache [slots, R + rot] -> out [T, H, R].  tiles [NT, 4]: first token row, tokens
 // (1 to 16), request, first position.  any_portion: whether a tile has more than one token (the
-// grid then has a workgroup per four heads).  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32,
-// n = T or, without a portion, num_tiles.
+// grid then has a workgroup per four heads).  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32, n the
+// tiles, times 16 where any has more than one token.
 LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot, const void* cache, const int* tiles,
                                     int num_tiles, int any_portion, const int* block_table, int max_blocks,
                                     int page_size, float scale, int window, const float* sink, void* out, int splits,
@@ -359,6 +380,20 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
     if (T == 0 || num_tiles == 0) return 0;
     LC_CHECK(qa && cache && tiles && block_table && out, "latent attention: null pointer");
     LC_CHECK(splits == 1 || (part_o && part_ml), "latent attention: shares need a workspace");
+    const int per_tile = any_portion ? 16 : 1;
+    auto join = [&]() {
+        if (splits > 1) {
+            latent_attention_join_kernel<<<num_tiles * per_tile * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink, tiles, per_tile,
+                                                                                      (bf16*)out);
+            LC_LAUNCH_CHECK("latent_attention_join");
+        }
+        return 0;
+    };
+    if (!any_portion && g_lone && latent_lone_takes(R, rot) && ((uintptr_t)qa | (uintptr_t)cache) % 16 == 0) {
+        const int rc = launch_latent_lone(qa, H, cache, tiles, num_tiles, block_table, max_blocks, page_size, scale, window, sink, out,
+                                          splits, part_o, part_ml, stream);
+        return rc ? rc : join();
+    }
     const int blocks_y = any_portion ? (H + 3) / 4 : (H + 63) / 64;
     LC_CHECK(blocks_y <= 65535, "latent attention: too many heads (%d)", H);
     const dim3 grid(num_tiles, blocks_y, splits);
@@ -372,7 +407,7 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
                      "latent attention: %zu bytes of LDS refused", lds);                                           \
         latent_attention_bf16_kernel<NR, KS><<<grid, LM_THREADS, lds, stream>>>(                                    \
             (const bf16*)qa, H, R, rot, (const bf16*)cache, tiles, block_table, max_blocks, page_size, scale, window, \
-            sink, (bf16*)out, splits, any_portion ? 0 : 1, part_o, part_ml);                                          \
+            sink, (bf16*)out, splits, per_tile, part_o, part_ml);                                                     \
     } while (0)
     if (nr == 4) LC_LM_LAUNCH(4, 4);
     else if (nr == 8) LC_LM_LAUNCH(8, 8);
@@ -380,10 +415,5 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
     else LC_LM_LAUNCH(32, 18);
 #undef LC_LM_LAUNCH
     LC_LAUNCH_CHECK("latent_attention_bf16");
-    if (splits > 1) {
-        latent_attention_join_kernel<<<(any_portion ? T : num_tiles) * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink,
-                                                                                          any_portion ? nullptr : tiles, (bf16*)out);
-        LC_LAUNCH_CHECK("latent_attention_join");
-    }
-    return 0;
+    return join();
 }

@@ -84,6 +84,8 @@ _SIGNATURES = {
     "lc_latent_prepare": "pqpiqiiiiipfppiipppp",
     "lc_latent_attention": "piiiiippppiifippp",
     "lc_latent_bf16_supported": "ii",
+    "lc_latent_lone": "i",
+    "lc_latent_lone_heads": "ii",
     "lc_latent_wide_supported": "iiii",
     "lc_latent_rows": "ppiiiiiippp",
     "lc_latent_wide": "pqpqqpppqiiiiifippqqpqp",
@@ -1454,12 +1456,11 @@ def latent_attention(qa: torch.Tensor, heads: int, rank: int, rot: int, tok_req:
             and lib.lc_latent_bf16_supported(rank, rot)):
         # the matrix-core kernel, over the planner's tiles; few tiles: their keys are shared out
         tiles, any_portion = plan.arrays["tiles"], plan.info["any_portion"]
-        workgroups = tiles.shape[0] * (-(-heads // 4) if any_portion else -(-heads // 64))
+        workgroups = tiles.shape[0] * -(-heads // (4 if any_portion else lib.lc_latent_lone_heads(rank, rot)))
         most = block_table.shape[1] * page_size if max_ctx <= 0 else max_ctx
         splits = lib.lc_latent_bf16_splits(workgroups, min(most, window) if window > 0 else most)
         part_o = part_ml = None
-        # the shares' places: by tile where all are lone tokens, else by token of the step, of which only few may have any
-        places = (T if any_portion else tiles.shape[0]) * heads
+        places = tiles.shape[0] * (LATENT_TILE if any_portion else 1) * heads
         if any_portion and splits > 1:
             splits = max(1, min(splits, (128 << 20) // (places * rank * 4)))
         if splits > 1:
