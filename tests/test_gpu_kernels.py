@@ -106,6 +106,39 @@ def test_gemm_generic_same_bits_for_any_number_of_rows(K):
         assert torch.equal(rows, whole[first:first + count]), (first, count)
 
 
+@pytest.mark.parametrize("dt_x,dt_w", [(torch.float32, torch.float32), (torch.float32, torch.bfloat16),
+                                       (torch.bfloat16, torch.bfloat16)])
+@pytest.mark.parametrize("M,N,K", [(1, 64, 32), (16, 65, 288), (17, 130, 1024), (64, 64, 256), (129, 200, 544),
+                                   (300, 16500, 96), (129, 4097, 224), (1025, 2300, 64)])
+def test_gemm_generic_whole_pieces_have_the_bits_of_single_elements(dt_x, dt_w, M, N, K):
+    """K of whole pairs of stages over aligned rows takes loads of whole pieces; the same rows an element off alignment take the
+    loads that test every k: the same products in the same order, so the same bits, in every tile shape, shared out or
+    not, and nothing is written behind the output."""
+    x, w = rnd(M, K, dtype=dt_x, seed=21), rnd(N, K, dtype=dt_w, seed=22)
+
+    def product(x, w):
+        out = torch.full((M * N + 64,), 7.0, device=DEV)
+        words = ops.library().lc_gemm_generic_workspace(M, N, K)
+        space = torch.empty((max(words, 1),), device=DEV)
+        ops._call("lc_gemm_generic", ops._ptr(x), ops._dt(x), ops._ptr(w), ops._dt(w), ops._ptr(out), ops._dt(out), M, N, K,
+                  ops._ptr(space), ops._stream())
+        assert bool((out[M * N:] == 7.0).all())
+        return out[:M * N].view(M, N)
+
+    def shifted(t):
+        room = torch.empty((t.numel() + 1,), dtype=t.dtype, device=DEV)
+        room[1:].copy_(t.flatten())
+        return room[1:].view(t.shape)
+
+    got = product(x, w)
+    assert torch.equal(got, product(shifted(x), w))
+    assert torch.equal(got, product(x, shifted(w)))
+    # K products of unit normals, each and their sums rounded to 24 bits: the error's deviation is below sqrt(K) roundings of a
+    # sum of size sqrt(K); 8 deviations
+    want = x.double() @ w.double().T
+    assert float((got.double() - want).abs().max()) <= 8 * K * 2.0 ** -24
+
+
 def make_rope_table(positions, rot, theta):
     i = torch.arange(rot // 2, dtype=torch.float64)
     inv = 1.0 / theta ** (2 * i / rot)
