@@ -906,12 +906,18 @@ static void launch_skinny(const bf16* x, const bf16* w, TO* out, int M, int N, i
 enum : int { SKINNY_DEEP = 0, SKINNY_PLAIN = 1, SKINNY_WIDE = 2, SKINNY_KEEP_X = 3 };
 constexpr int SK_KEEP_MAX = 3;   // k blocks of x per wave that fit in registers beside w's
 static thread_local int g_force_skinny = -1;
-static int skinny_shape(int M, int N, int K) {
+static int skinny_shape(int M, int N, int K, int epilogue) {
     if (g_force_skinny >= 0 && (g_force_skinny != SKINNY_KEEP_X || K <= SK_KEEP_MAX * 16 * SK_KBLOCK))
         return g_force_skinny;
     if (M <= 2) return SKINNY_DEEP;
     const int tiles = (N + 15) / 16;
-    if (K <= SK_KEEP_MAX * 16 * SK_KBLOCK && tiles > kCUs && (M >= 7 || tiles <= 2 * kCUs)) return SKINNY_KEEP_X;
+    // In a K of few blocks most of a workgroup's 16 waves have none or one: with x kept, a CU's second tile then waits for the
+    // first one's sums and hides nothing, while two workgroups a CU, or one with twice the rows, run side by side.  SwiGLU products
+    // at 8 rows, N = 6,144: K 512 7.3 us kept, 4.8 side by side; 1,024 7.4 and 6.1; 1,152 7.4 and 6.5; 1,280 7.5 and 7.0 (16 rows 8.1 and
+    // 8.0, and plain products 6.8 kept, 6.9); 1,536 7.6 and 7.7.
+    const bool keep_hides = K > 9 * SK_KBLOCK;
+    if (!keep_hides && epilogue == 1 && tiles > kCUs && tiles <= 2 * kCUs) return SKINNY_WIDE;   // (the others: skinny_plan)
+    if (keep_hides && K <= SK_KEEP_MAX * 16 * SK_KBLOCK && tiles > kCUs && (M >= 7 || tiles <= 2 * kCUs)) return SKINNY_KEEP_X;
     if (M >= 12 && N >= 32 * 2 * kCUs) return SKINNY_WIDE;
     return SKINNY_PLAIN;
 }
@@ -988,7 +994,7 @@ static SkinnyPlan skinny_plan(int M, int N, int K, int epilogue) {
         if (runs_keeps_x(p, K) || runs_ring_in_registers()) return p;
         p.runs = false;
     }
-    p.shape = skinny_shape(M, N, K);
+    p.shape = skinny_shape(M, N, K, epilogue);
     p.rows = p.shape == SKINNY_WIDE ? 32 : 16;
     p.items = (N + p.rows - 1) / p.rows;
     const bool keep = p.shape == SKINNY_KEEP_X;

@@ -738,6 +738,14 @@ def test_gemm_bf16_few_rows_every_shape(M, N, K, shape):
         ops.force_gemm_skinny(-1)
 
 
+@pytest.mark.parametrize("M,N,K", [(3, 4112, 128), (8, 6144, 1024), (16, 8192, 1152), (4, 8176, 1152), (5, 6160, 1280),
+                                   (12, 8208, 1152), (2, 6144, 1024)])
+def test_gemm_bf16_few_rows_of_short_k(M, N, K):
+    """Up to nine blocks of K, of which a workgroup's 16 waves have one or none: one to two tiles a CU go side by side or in items of
+    up to 32 rows instead of one behind the other with x in registers; the sizes on both sides of the rule."""
+    few_rows_case(M, N, K)
+
+
 @pytest.mark.parametrize("even", [True, False])
 @pytest.mark.parametrize("M,N,K", [(1, 5120, 256), (2, 6150, 384), (8, 5120, 8192), (16, 5136, 128), (5, 6150, 4096),
                                    (9, 10250, 5120), (3, 4100, 128), (12, 7170, 6272), (8, 16001, 256)])
