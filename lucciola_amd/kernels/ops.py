@@ -1355,12 +1355,23 @@ def latent_wide_pays(tokens: int, position: int, heads: int, window: int) -> boo
     return wide < latent
 
 
+# Entries of the keys of a step's requests that attend head by head, and of their values: 512 MB each.
+LATENT_WIDE_ENTRIES = 1 << 28
+
+
 def latent_short_planner(heads: int, window: int):
     """(key, planner) for a part whose long portions may attend head by head: ``plan_latent_attention`` for the others, and in
-    ``info["wide"]`` the requests that do."""
+    ``info["wide"]`` the requests that do.  These are taken in order as long as their visible rows' keys and values stay within
+    LATENT_WIDE_ENTRIES (16 heads: 131,072 rows); whoever does not fit stays in the latent's space, which needs no scratch by row."""
     def plan(layout):
-        wide = [r for r in range(layout.num_requests)
-                if latent_wide_pays(layout.q_start[r + 1] - layout.q_start[r], layout.first_position[r], heads, window)]
+        wide, rows = [], 0
+        for r in range(layout.num_requests):
+            tokens, position = layout.q_start[r + 1] - layout.q_start[r], layout.first_position[r]
+            if latent_wide_pays(tokens, position, heads, window):
+                visible = -(-(position + tokens - (max(0, position - window + 1) if window else 0)) // 64) * 64
+                if (rows + visible) * heads * 128 <= LATENT_WIDE_ENTRIES:
+                    wide.append(r)
+                    rows += visible
         arrays, info = plan_latent_attention(layout)
         if wide:
             tiles = arrays["tiles"][~np.isin(arrays["tiles"][:, 2], wide)]

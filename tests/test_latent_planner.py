@@ -1,0 +1,34 @@
+"""Which requests' portions attend head by head: the keys and values that this makes for every visible row are bounded."""
+from types import SimpleNamespace
+
+import pytest
+
+from lucciola_amd.kernels import ops
+
+
+def layout_of(requests):
+    q_start = [0]
+    for tokens, _ in requests:
+        q_start.append(q_start[-1] + tokens)
+    return SimpleNamespace(num_requests=len(requests), q_start=q_start, first_position=[p for _, p in requests], num_tokens=q_start[-1])
+
+
+@pytest.mark.parametrize("heads,window,requests,wide", [
+    (16, 0, [(2048, 0)], [0]),
+    (16, 0, [(1, 4000), (2048, 2048), (1, 5)], [1]),                     # lone tokens never
+    (16, 0, [(2048, 131072 - 2048)], [0]),                               # exactly what fits
+    (16, 0, [(2048, 131072 - 2047)], []),                                # one row more
+    (16, 4096, [(2048, 500000)], [0]),                                   # a window bounds the visible rows
+    (16, 0, [(1024, 100000), (1024, 100000), (1024, 20000)], [0, 2]),    # whoever does not fit stays, later ones may fit
+    (32, 0, [(1024, 64000), (1024, 64000)], [0]),
+])
+def test_requests_head_by_head_stay_within_the_scratch(heads, window, requests, wide):
+    layout = layout_of(requests)
+    _, plan = ops.latent_short_planner(heads, window)
+    arrays, info = plan(layout)
+    assert info["wide"] == wide
+    # every other token is in a tile of the latent's space, once
+    tiles = arrays["tiles"][:info["num_tiles"]]
+    others = sum(tokens for r, (tokens, _) in enumerate(requests) if r not in wide)
+    assert int(tiles[:, 1].sum()) == others if others else info["num_tiles"] == 0
+    assert not set(tiles[:, 2].tolist()) & set(wide)
