@@ -2,7 +2,7 @@
 //     S <- diag(decay) S - removal (probe^T S) + write v^T,    o = S^T read,
 // for portions of prompts, a chunk of SC = 32 tokens at a time on the float32 matrix instruction.  Token by token a step
 // is a chain of dependent vector instructions, 0.21 us a token without and 0.29 us with the removal term, on a wave that
-// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 105 and 180).
+// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 107 and 185).
 //
 // Inside a chunk, from the state S that the chunk before left, with a_i the product of the decays of tokens 0..i (key
 // channel by key channel), r_ij that of the tokens j+1..i, and y_i = probe_i^T S_(i-1) what token i takes out:
@@ -17,13 +17,15 @@
 // of 16 are made pair by pair, those between blocks are split at the border, so a decay of any size (0 too) is exact.
 // A token's sums are taken in another order than token by token and depend on where its chunk begins, so callers that
 // promise the same bits for every cut of a prompt (float32 models) and steps of few tokens keep the other kernel.
-// A chunk's products meet every value of the chunk: a NaN or an infinity in a token's vectors or values reaches the
-// chunk's earlier tokens too (never another request).
+// A chunk's products meet every token of the chunk, and zero times infinity is no number.  So a request with a vector of which
+// an entry is NaN, infinite or above SC_MOST goes token by token in the second kernel (walk_tokens), and a value that is not
+// finite meets no row of W - R T M above its own: such a token reaches what comes behind it and nothing before.
 #include "common.h"
 
 namespace lc {
 
 constexpr int SC = 32;                  // tokens of a chunk: two blocks of 16
+constexpr float SC_MOST = 0x1p40f;      // above that a chunk's products could overflow where a token's do not
 constexpr int SCP = SC + 4;             // floats of a row of a [SC x SC] matrix in LDS: b128 reads of 16 rows meet no bank twice
 
 typedef float f32x4 __attribute__((ext_vector_type(4)));
@@ -66,12 +68,14 @@ __device__ __forceinline__ f32x4 tile_product(A a, B b) {
     return c[0];
 }
 
-// grid (records, heads).  coef [5 or 3][T, heads DK] as delta_rule.hip has it.  2,048 tokens, 16 heads of 128: 26 us, and with
-// a removal term, where a workgroup fills its CU's LDS and its steps follow each other, 62 us.
+// grid (records, heads).  coef [5 or 3][T, heads DK] as delta_rule.hip has it.  alone [records][heads][8]: not all zero where the
+// chunk holds what has to go token by token, and its record is not to be used.  2,048 tokens, 16 heads of 128: 26 us, and with
+// a removal term, where a workgroup fills its CU's LDS and its steps follow each other, 63 us.
 template <int DK, bool REMOVE, int THREADS>
 __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float* __restrict__ coef,
                                                                      const int* __restrict__ q_offsets, int R, int T,
-                                                                     int heads, int least, float* __restrict__ records) {
+                                                                     int heads, int least, float* __restrict__ records,
+                                                                     unsigned char* __restrict__ alone) {
     typedef ChunkRecord<DK, REMOVE> Rec;
     constexpr int DKP = DK + 4, WAVES = THREADS / kWave, NP = REMOVE ? 5 : 3;
     constexpr int DECAY = 0, PROBE = 1, REMOVAL = 2, WRITE = REMOVE ? 3 : 1, READ = REMOVE ? 4 : 2;
@@ -95,13 +99,18 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
 
     // the chunk's vectors; a place behind the request's end keeps the state and adds nothing
+    unsigned most = 0;                                      // the largest entry's bits: NaN and infinity lie above all numbers
     for (int idx = tid; idx < NP * SC * (DK / 4); idx += THREADS) {
         const int i = idx % (DK / 4), t = idx / (DK / 4) % SC, p = idx / (DK / 4 * SC);
         const float pad = p == DECAY ? 1.f : 0.f;
         f32x4 x = {pad, pad, pad, pad};
         if (t < count) x = *reinterpret_cast<const f32x4*>(coef + ((size_t)p * T + t0 + t) * heads * DK + (size_t)head * DK + 4 * i);
+#pragma unroll
+        for (int e = 0; e < 4; ++e) most = max(most, __float_as_uint(x[e]) & 0x7FFFFFFFu);
         *reinterpret_cast<f32x4*>(&plane[p][t][4 * i]) = x;
     }
+    const bool odd = __builtin_amdgcn_ballot_w64(most > __float_as_uint(SC_MOST)) != 0;
+    if (lane < 8 / WAVES) alone[((size_t)record * heads + head) * 8 + wave * (8 / WAVES) + lane] = odd;
     __syncthreads();
 
     // every vector at its block's border.  A thread is a key channel of a block, and of the reading (read, probe) or the
@@ -332,19 +341,56 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     }
 }
 
+// The recurrence as it stands, for 16 value channels: 32 lanes a channel, DK / 32 key rows a lane.
+template <int DK, bool REMOVE>
+__device__ __forceinline__ void walk_tokens(const float* __restrict__ coef, const float* __restrict__ v, float* __restrict__ state,
+                                            float* __restrict__ out, int first, int last, int slot, int T, int heads, int head,
+                                            int dv, int block) {
+    constexpr int N = DK / 32, DECAY = 0, PROBE = 1, REMOVAL = 2, WRITE = REMOVE ? 3 : 1, READ = REMOVE ? 4 : 2;
+    const int j = block * 16 + threadIdx.x / 32, k0 = threadIdx.x % 32 * N;
+    if (j >= dv) return;
+    auto over_rows = [](float x) {
+        for (int n = 16; n >= 1; n /= 2) x += __shfl_xor(x, n, 32);
+        return x;
+    };
+    float* home = state + (((size_t)slot * heads + head) * dv + j) * DK + k0;
+    float S[N];
+    for (int i = 0; i < N; ++i) S[i] = home[i];
+    for (int t = first; t < last; ++t) {
+        const size_t at = ((size_t)t * heads + head) * dv + j;
+        const float value = v[at];
+        auto entry = [&](int p, int i) { return coef[(((size_t)p * T + t) * heads + head) * DK + k0 + i]; };
+        float held = 0.f, o = 0.f;
+        if constexpr (REMOVE) {
+            for (int i = 0; i < N; ++i) held = fmaf(entry(PROBE, i), S[i], held);
+            held = over_rows(held);
+        }
+        for (int i = 0; i < N; ++i) {
+            S[i] *= entry(DECAY, i);
+            if constexpr (REMOVE) S[i] = fmaf(-entry(REMOVAL, i), held, S[i]);
+            S[i] = fmaf(entry(WRITE, i), value, S[i]);
+            o = fmaf(entry(READ, i), S[i], o);
+        }
+        o = over_rows(o);
+        if (k0 == 0) out[at] = o;
+    }
+    for (int i = 0; i < N; ++i) home[i] = S[i];
+}
+
 // One workgroup per (16 value channels, head, request).  Four waves keep S, a quarter of the key rows each, as accumulators
 // (KT tiles of 16), which are B operands of the next products as they are, and take it from chunk to chunk; four others make
 // the chunks' read-outs from copies of S that the first leave in LDS, a chunk behind.  So a SIMD has two waves, and one's loads,
 // LDS trips and address arithmetic pass beside the other's products (with the read-outs made by the waves that keep S, one wave a
-// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 79 and 119).  What the
+// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 80 and 122).  What the
 // waves make of their key rows meets in LDS, two buffers in turn, one barrier a chunk.  A chunk's record is asked for two chunks
 // ahead.  Workgroups are numbered so that the blocks of one head, which read the same records, run on one XCD (workgroup
 // i on XCD i % 8) where the heads are a multiple of 8.
 template <int DK, bool REMOVE>
-__global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __restrict__ records, const float* __restrict__ v,
+__global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __restrict__ records, const uint2* __restrict__ alone,
+                                                              const float* __restrict__ coef, const float* __restrict__ v,
                                                               float* __restrict__ state, float* __restrict__ out,
                                                               const int* __restrict__ q_offsets,
-                                                              const int* __restrict__ slot_ids, int heads, int dv, int least) {
+                                                              const int* __restrict__ slot_ids, int T, int heads, int dv, int least) {
     typedef ChunkRecord<DK, REMOVE> Rec;
     constexpr int KT = DK / 64, TT = SC / 16, KEYS = DK / 16;
     __shared__ f32x4 states[2][4][KT][kWave], reads[2][4][TT][kWave], taken[REMOVE ? 2 : 1][4][TT][kWave];
@@ -355,6 +401,15 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     const int first = q_offsets[req], last = q_offsets[req + 1];
     if (last - first < least) return;
     const int chunks = (last - first + SC - 1) / SC;
+    bool by_token = false;
+    for (int c = lane; c < chunks; c += kWave) {
+        const uint2 waves = alone[(size_t)(first_record(q_offsets, req) + c) * heads + head];
+        by_token |= (waves.x | waves.y) != 0;
+    }
+    if (__builtin_amdgcn_ballot_w64(by_token) != 0) {       // in every wave alike
+        walk_tokens<DK, REMOVE>(coef, v, state, out, first, last, slot_ids[req], T, heads, head, dv, block);
+        return;
+    }
     const int j = block * 16 + row;                         // the value channel
     const bool mine = j < dv;                               // a channel behind dv works through the head's first one's values
     const int column = mine ? j : 0;
@@ -505,6 +560,22 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
 #pragma unroll
                     for (int t = 0; t < TT; ++t) o[t] = mfma4(l.read[t][k][i], S[i], o[t]);
             }
+            unsigned most = 0;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) most = max(most, __float_as_uint(l.value[i]) & 0x7FFFFFFFu);
+            if (__builtin_amdgcn_ballot_w64(most >= 0x7F800000u) != 0) {        // token by token, each for its own row and those behind it
+                mixed = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+                for (int s = 0; s < 16; ++s) {
+                    const float value = __shfl(l.value[s & 3], (s >> 2) * 16 + row, kWave);
+#pragma unroll
+                    for (int i = 0; i < 4; ++i) {
+                        const int to = 4 * quad + i;
+                        const float w = __shfl(l.mix[s & 3], (s >> 2) * 16 + to, kWave);
+                        if (s <= to + 16 * ((wave >> 1) - (wave & 1))) mixed[i] = fmaf(w, value, mixed[i]);
+                    }
+                }
+            }
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
 #pragma unroll
@@ -550,10 +621,12 @@ template <int DK, bool REMOVE>
 static void scan_chunks(const float* coef, const float* v, float* state, float* out, float* records, const int* q_offsets,
                         const int* slot_ids, int R, int T, int heads, int dv, int least, hipStream_t stream) {
     constexpr int THREADS = REMOVE ? 4 * DK : 2 * DK;
+    const int places = T / SC + R;
+    float* alone = records + (size_t)places * heads * ChunkRecord<DK, REMOVE>::SIZE;
     scan_chunk_prepare_kernel<DK, REMOVE, THREADS>
-        <<<dim3(T / SC + R, heads), THREADS, 0, stream>>>(coef, q_offsets, R, T, heads, least, records);
+        <<<dim3(places, heads), THREADS, 0, stream>>>(coef, q_offsets, R, T, heads, least, records, reinterpret_cast<unsigned char*>(alone));
     scan_chunk_walk_kernel<DK, REMOVE><<<dim3(heads * ((dv + 15) / 16), R), 512, 0, stream>>>(
-        records, v, state, out, q_offsets, slot_ids, heads, dv, least);
+        records, reinterpret_cast<const uint2*>(alone), coef, v, state, out, q_offsets, slot_ids, T, heads, dv, least);
 }
 
 }  // namespace lc
@@ -565,7 +638,7 @@ LC_API long long lc_scan_chunks_records(int planes, int R, int T, int heads, int
     if (R <= 0 || T <= 0 || heads <= 0 || dv <= 0 || (long long)heads * dv >= (1 << 23) || (planes != 3 && planes != 5) || (dk != 64 && dk != 128)) return 0;
     const long long size = dk == 64 ? (planes == 5 ? ChunkRecord<64, true>::SIZE : ChunkRecord<64, false>::SIZE)
                                     : (planes == 5 ? ChunkRecord<128, true>::SIZE : ChunkRecord<128, false>::SIZE);
-    return size * heads * (T / SC + R);
+    return (size + 2) * heads * (T / SC + R);
 }
 
 // The recurrence for the requests of at least `least` tokens; the others' states and rows of out are left alone.

@@ -2018,8 +2018,8 @@ def delta_scan_step(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, ba
     """The recurrence for a step's batch in a model of ``dtype``.  A float32 model's logits have the same bits for every cut
     of a prompt, so its tokens go one by one; a bfloat16 model's long portions go a chunk at a time, where the head's sizes
     are ones that the chunks' kernels take and the tensors begin at a whole 16 bytes.  16 heads of 128 x 128, one portion, us
-    token by token and in chunks: 48 tokens 12 and 15, 64 tokens 15 and 15, 96 tokens 21 and 15, 2,048 tokens 439 and 105; with
-    the removal term 15 and 19, 19 and 20, 30 and 23, 590 and 180."""
+    token by token and in chunks: 48 tokens 12 and 15, 64 tokens 15 and 15, 96 tokens 21 and 15, 2,048 tokens 439 and 107; with
+    the removal term 15 and 19, 19 and 20, 30 and 23, 590 and 185."""
     lists = (batch.q_offsets, batch.slot_ids, batch.num_requests, heads, key_dim, value_dim)
     if dtype != torch.float32 and key_dim in (64, 128) and v.is_cuda and batch.num_tokens >= SCAN_CHUNKS_FROM:
         lengths = [b - a for a, b in zip(batch.q_start, batch.q_start[1:])]

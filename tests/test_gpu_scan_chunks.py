@@ -83,3 +83,35 @@ def test_which_steps_go_in_chunks(monkeypatch, dtype, dk, lengths, chunked):
     assert bool(called) == chunked
     assert torch.equal(got, plain) or chunked
     assert float((got - plain).norm() / plain.norm()) < 1e-6
+
+
+@pytest.mark.parametrize("planes,where", [(5, p) for p in ("decay", "probe", "removal", "write", "read", "value")] +
+                         [(3, p) for p in ("decay", "write", "read", "value")])
+@pytest.mark.parametrize("bad,at", [(float("nan"), 45), (float("inf"), 99), (float("-inf"), 20), (2.0 ** 100, 3)])
+@pytest.mark.parametrize("dk,dv", [(128, 33), (64, 16)])
+def test_what_is_not_finite_reaches_later_tokens_only(planes, where, bad, at, dk, dv):
+    """One entry of one token: the chunks' products leave the very places finite that the token-by-token kernel does, and what
+    is finite is within 16 units of 2^-24 of that kernel's (both are within eight of the exact result where nothing is odd)."""
+    g = torch.Generator().manual_seed(dk + planes)
+    lengths, heads = [64, 100, 3], 2
+    T, R, token, head = sum(lengths), len(lengths), 64 + at, 1
+    coef = vectors("by channel", T, heads, dk, g)[0 if planes == 5 else 1].clone()
+    v = torch.randn(T, heads * dv, generator=g)
+    if where == "value":
+        v.view(T, heads, dv)[token, head, 5] = bad
+    else:
+        names = ("decay", "probe", "removal", "write", "read") if planes == 5 else ("decay", "write", "read")
+        coef.view(planes, T, heads, dk)[names.index(where), token, head, 7] = bad
+    state = torch.randn(R, heads, dv, dk, generator=g) * 0.2
+    starts = [0] + torch.tensor(lengths).cumsum(0).tolist()
+    lists = torch.tensor(starts, dtype=torch.int32, device=DEV), torch.arange(R, dtype=torch.int32, device=DEV)
+    results = []
+    for f in (lambda *a: ops.delta_scan(*a), lambda *a: ops.delta_scan_chunks(*a, some_short=True)):
+        s = state.to(DEV)
+        results.append((f(coef.to(DEV), v.to(DEV), s, *lists, R, heads, dk, dv).cpu(), s.cpu()))
+    for plain, got in zip(*results):
+        finite = torch.isfinite(plain)
+        assert torch.equal(torch.isfinite(got), finite)
+        usual = finite & (plain.abs() < 1e6)
+        assert float((got - plain)[usual].norm() / plain[usual].norm()) <= 16 * UNIT
+    assert bool(torch.isfinite(results[1][0][:token]).all())
