@@ -121,17 +121,22 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     float decay[16];
 #pragma unroll
     for (int i = 0; i < 16; ++i) decay[i] = plane[DECAY][16 * block + i][channel];
-    double through = 1.0;
+    double through = 1.0, least_through = 1.0, most_through = 1.0;
 #pragma unroll
-    for (int i = 0; i < 16; ++i) through *= (double)decay[i];
+    for (int i = 0; i < 16; ++i) {
+        through *= (double)decay[i];
+        least_through = fmin(least_through, through);
+        most_through = fmax(most_through, through);
+    }
     if (side == 0) {
         whole[block][channel] = through;
         total[block][channel] = (float)through;
     }
-    // Where no channel forgets more than 2^-60 of itself in 16 tokens, the pairs of a block are products of the vectors times
-    // and over the decays from the block's first token on, on the matrix instruction: a division by what is far from the
-    // smallest number loses nothing.  Else the pairs are made one by one, by vector instructions, several times as long.
-    const bool far = __syncthreads_or(!(through >= 0x1p-60 && through <= 0x1p60));
+    // Where no channel's decays multiply to less than 2^-60 or more than 2^60 anywhere in the 16 tokens, the pairs of a block are
+    // products of the vectors times and over the decays from the block's first token on, on the matrix instruction: a division
+    // by what is far from the smallest number loses nothing.  Else the pairs are made one by one, by vector instructions,
+    // several times as long.
+    const bool far = __syncthreads_or(!(least_through >= 0x1p-60 && most_through <= 0x1p60 && through == through));
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     auto put = [&](float (*to)[SCP], int r0, int c0, f32x4 v) {
 #pragma unroll

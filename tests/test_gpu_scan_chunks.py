@@ -115,3 +115,26 @@ def test_what_is_not_finite_reaches_later_tokens_only(planes, where, bad, at, dk
         usual = finite & (plain.abs() < 1e6)
         assert float((got - plain)[usual].norm() / plain[usual].norm()) <= 16 * UNIT
     assert bool(torch.isfinite(results[1][0][:token]).all())
+
+
+@pytest.mark.parametrize("planes", [5, 3])
+@pytest.mark.parametrize("steps", [(-66, -64, 62, 60), (50, 50, -50, -50), (-40, 30, -40, 50)])
+def test_decays_that_leave_the_range_inside_a_block(planes, steps):
+    """A block whose decays multiply to a common number, and to very small or large ones on the way: against float64, the
+    token-by-token kernel beside it."""
+    g = torch.Generator().manual_seed(planes)
+    T, heads, dk, dv = 64, 1, 64, 16
+    coef = vectors("by channel", T, heads, dk, g)[0 if planes == 5 else 1].clone()
+    decay = coef.view(planes, T, heads, dk)[0]
+    decay[19:23] = 2.0 ** torch.tensor(steps)[:, None, None].float()
+    if planes == 5:
+        coef.view(planes, T, heads, dk)[1] = torch.nn.functional.normalize(torch.randn(T, heads, dk, generator=g), dim=-1)
+    v, state = torch.randn(T, heads * dv, generator=g), torch.zeros(1, heads, dv, dk)
+    lists = torch.tensor([0, T], dtype=torch.int32), torch.zeros(1, dtype=torch.int32)
+    want = reference_ops.delta_scan(coef, v, state.double(), *lists, 1, heads, dk, dv).double()
+    on_gpu = coef.to(DEV), v.to(DEV)
+    plain = ops.delta_scan(*on_gpu, state.to(DEV), *(x.to(DEV) for x in lists), 1, heads, dk, dv).cpu().double()
+    got = ops.delta_scan_chunks(*on_gpu, state.to(DEV), *(x.to(DEV) for x in lists), 1, heads, dk, dv, some_short=False).cpu().double()
+    for t in range(T):      # token by token: one token's size says nothing of another's
+        off = [float((x[t] - want[t]).norm() / want[t].norm()) for x in (plain, got)]
+        assert off[1] <= max(4 * off[0], 64 * UNIT), (t, off)
