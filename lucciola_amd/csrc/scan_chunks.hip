@@ -43,8 +43,13 @@ struct ChunkRecord {
                          REMOVAL = PROBE + SC * DK, SIZE = REMOVE ? REMOVAL + SC * DK : PROBE;
 };
 
-// The records of request r's chunks begin at q_offsets[r] / SC + r: no two requests share one, whatever their lengths.
-__device__ __forceinline__ int first_record(const int* __restrict__ q_offsets, int r) { return q_offsets[r] / SC + r; }
+// Where the records of request r's chunks begin, for the requests of at least `least` tokens: no two of them share one, whatever
+// the lengths.  Behind such a request q / SC has grown by its whole chunks and the other term by one or more, for the rest of it.
+// The many lone tokens that a step may hold beside a portion take no record: their places are those that a request behind them has.
+__host__ __device__ __forceinline__ int record_place(int q, int r, int least) { return q / SC + min(r, q / least); }
+__device__ __forceinline__ int first_record(const int* __restrict__ q_offsets, int r, int least) {
+    return record_place(q_offsets[r], r, least);
+}
 
 // The [16 x 16] tile A B over 16 KT k, k = 16 t + 4 (lane / 16) + i: a(t) holds four neighbouring k of the lane's row of A, b(t)
 // of its column of B, so that rows are read 16 bytes at a time.  A lane gets rows 4 (lane / 16) .. + 3 of column lane % 16,
@@ -90,10 +95,10 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     int low = 0, high = R - 1;                              // the request whose records hold this one
     while (low < high) {
         const int mid = (low + high + 1) / 2;
-        if (first_record(q_offsets, mid) <= record) low = mid;
+        if (first_record(q_offsets, mid, least) <= record) low = mid;
         else high = mid - 1;
     }
-    const int last = q_offsets[low + 1], t0 = q_offsets[low] + (record - first_record(q_offsets, low)) * SC;
+    const int last = q_offsets[low + 1], t0 = q_offsets[low] + (record - first_record(q_offsets, low, least)) * SC;
     if (t0 >= last || last - q_offsets[low] < least) return;
     const int count = min(SC, last - t0);
     float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
@@ -408,7 +413,7 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     const int chunks = (last - first + SC - 1) / SC;
     bool by_token = false;
     for (int c = lane; c < chunks; c += kWave) {
-        const uint2 waves = alone[(size_t)(first_record(q_offsets, req) + c) * heads + head];
+        const uint2 waves = alone[(size_t)(first_record(q_offsets, req, least) + c) * heads + head];
         by_token |= (waves.x | waves.y) != 0;
     }
     if (__builtin_amdgcn_ballot_w64(by_token) != 0) {       // in every wave alike
@@ -420,7 +425,7 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     const int column = mine ? j : 0;
     const unsigned line = heads * dv;                       // floats from a token's values to the next one's, below 2^23
     const float* values = v + (size_t)first * line + (size_t)head * dv;
-    const float* record = records + ((size_t)first_record(q_offsets, req) * heads + head) * Rec::SIZE;
+    const float* record = records + ((size_t)first_record(q_offsets, req, least) * heads + head) * Rec::SIZE;
     // a chunk's record and values; behind the last chunk the last one's once more.  Entries that lie behind the request's
     // end are zero in the records, so such a token's value (the last token's) only has to be a number.
     auto record_of = [&](int c) { return record + (size_t)min(c, chunks - 1) * heads * Rec::SIZE; };
@@ -622,11 +627,14 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     }
 }
 
+// Records of a step, one at least: a list of short requests is taken too, and nothing is done for it.
+static int record_places(int T, int R, int least) { return max(1, record_place(T, R, least)); }
+
 template <int DK, bool REMOVE>
 static void scan_chunks(const float* coef, const float* v, float* state, float* out, float* records, const int* q_offsets,
                         const int* slot_ids, int R, int T, int heads, int dv, int least, hipStream_t stream) {
     constexpr int THREADS = REMOVE ? 4 * DK : 2 * DK;
-    const int places = T / SC + R;
+    const int places = record_places(T, R, least);
     float* alone = records + (size_t)places * heads * ChunkRecord<DK, REMOVE>::SIZE;
     scan_chunk_prepare_kernel<DK, REMOVE, THREADS>
         <<<dim3(places, heads), THREADS, 0, stream>>>(coef, q_offsets, R, T, heads, least, records, reinterpret_cast<unsigned char*>(alone));
@@ -639,11 +647,11 @@ static void scan_chunks(const float* coef, const float* v, float* state, float* 
 using namespace lc;
 
 // Floats that lc_scan_chunks wants as `records` for T tokens of R requests, or 0 where it does not take these sizes.
-LC_API long long lc_scan_chunks_records(int planes, int R, int T, int heads, int dk, int dv) {
-    if (R <= 0 || T <= 0 || heads <= 0 || dv <= 0 || (long long)heads * dv >= (1 << 23) || (planes != 3 && planes != 5) || (dk != 64 && dk != 128)) return 0;
+LC_API long long lc_scan_chunks_records(int planes, int R, int T, int heads, int dk, int dv, int least) {
+    if (least < 1 || R <= 0 || T <= 0 || heads <= 0 || dv <= 0 || (long long)heads * dv >= (1 << 23) || (planes != 3 && planes != 5) || (dk != 64 && dk != 128)) return 0;
     const long long size = dk == 64 ? (planes == 5 ? ChunkRecord<64, true>::SIZE : ChunkRecord<64, false>::SIZE)
                                     : (planes == 5 ? ChunkRecord<128, true>::SIZE : ChunkRecord<128, false>::SIZE);
-    return (size + 2) * heads * (T / SC + R);
+    return (size + 2) * heads * record_places(T, R, least);
 }
 
 // The recurrence for the requests of at least `least` tokens; the others' states and rows of out are left alone.
@@ -653,7 +661,7 @@ LC_API int lc_scan_chunks(const float* coef, int planes, const float* v, float* 
                           hipStream_t stream) {
     LC_CHECK(R >= 0 && T >= 0 && heads > 0 && dk > 0 && dv > 0 && slots >= 0 && least >= 1, "scan_chunks: bad sizes");
     if (R == 0 || T == 0) return 0;
-    LC_CHECK(lc_scan_chunks_records(planes, R, T, heads, dk, dv) > 0, "scan_chunks: sizes it does not take");
+    LC_CHECK(lc_scan_chunks_records(planes, R, T, heads, dk, dv, least) > 0, "scan_chunks: sizes it does not take");
     LC_CHECK(coef && v && state && out && records && q_offsets && slot_ids, "scan_chunks: null pointer");
     LC_CHECK(((uintptr_t)coef | (uintptr_t)state | (uintptr_t)records) % 16 == 0, "scan_chunks: not aligned to 16 bytes");
     LC_CHECK(R <= 65535 && heads <= 65535, "scan_chunks: too many requests or heads for the grid");

@@ -186,7 +186,7 @@ def library():
         lib.lc_attention_generic_workspace.restype = ctypes.c_longlong
         lib.lc_attention_generic_workspace.argtypes = [ctypes.c_int] * 5
         lib.lc_scan_chunks_records.restype = ctypes.c_longlong
-        lib.lc_scan_chunks_records.argtypes = [ctypes.c_int] * 6
+        lib.lc_scan_chunks_records.argtypes = [ctypes.c_int] * 7
         for name, sig in _SIGNATURES.items():
             _declare(lib, name, sig)
         if lib.lc_attn_page_granule() != ATTENTION_PAGE_GRANULE:
@@ -1992,7 +1992,7 @@ def delta_scan_chunks(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, 
     sums are taken in an order that depends on where its request's portion begins.  ``some_short``: there are requests of
     fewer tokens, which go token by token."""
     T = v.shape[0]
-    need = library().lc_scan_chunks_records(coef.shape[0], num_requests, T, heads, key_dim, value_dim)
+    need = library().lc_scan_chunks_records(coef.shape[0], num_requests, T, heads, key_dim, value_dim, SCAN_CHUNKS_FROM)
     if need <= 0:
         raise KernelError(f"delta_scan_chunks: heads of {key_dim} key channels are not 64 or 128")
     if tuple(coef.shape[1:]) != (T, heads * key_dim) or v.shape[1] != heads * value_dim or \

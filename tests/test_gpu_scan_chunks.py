@@ -138,3 +138,29 @@ def test_decays_that_leave_the_range_inside_a_block(planes, steps):
     for t in range(T):      # token by token: one token's size says nothing of another's
         off = [float((x[t] - want[t]).norm() / want[t].norm()) for x in (plain, got)]
         assert off[1] <= max(4 * off[0], 64 * UNIT), (t, off)
+
+
+@pytest.mark.parametrize("lengths", [[1] * 200 + [64] + [1] * 55, [64] + [1] * 255, [1] * 255 + [70], [63] * 9 + [64, 64, 65, 1, 127, 128, 2, 96],
+                                     [1, 2, 3] * 20 + [64, 1, 95, 1, 300], [20]])
+def test_requests_of_few_tokens_take_no_record(lengths):
+    """One portion beside many requests of few tokens: the right places, and scratch for the portions' chunks alone."""
+    g = torch.Generator().manual_seed(len(lengths))
+    heads, dk, dv, T, R = 2, 128, 16, sum(lengths), len(lengths)
+    coef = vectors("by channel", T, heads, dk, g)[0].to(DEV)
+    v, state = torch.randn(T, heads * dv, generator=g).to(DEV), torch.randn(R, heads, dv, dk, generator=g).to(DEV)
+    starts = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32, device=DEV)
+    lists = starts, torch.arange(R, dtype=torch.int32, device=DEV)
+    states = [state.clone(), state.clone()]
+    plain = ops.delta_scan(coef, v, states[0], *lists, R, heads, dk, dv)
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    got = ops.delta_scan_chunks(coef, v, states[1], *lists, R, heads, dk, dv, some_short=True)
+    scratch = torch.cuda.max_memory_allocated() - before - got.numel() * 4
+    # a chunk: four planes of vectors, the matrix and the decays; a portion of 64 tokens may waste one, the list half as many
+    chunk = (4 * 32 * dk + 2 * dk + 32 * 32 + 2) * 4 * heads
+    chunks = max(1, T // 32 + T // 64)
+    assert scratch <= chunks * chunk + 4096, (scratch, chunks * chunk)
+    for a, b in ((got, plain), (states[1], states[0])):
+        assert float((a - b).norm() / b.norm()) <= 16 * UNIT
+    short = torch.tensor([n < ops.SCAN_CHUNKS_FROM for n in lengths], device=DEV)
+    assert torch.equal(states[1][short], states[0][short])
