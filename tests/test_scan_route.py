@@ -1,0 +1,28 @@
+"""Which kernel a step's recurrence goes to (``ops.delta_scan_step``), without a GPU: the kernels are stand-ins."""
+from types import SimpleNamespace
+
+import pytest
+import torch
+
+from lucciola_amd.kernels import ops
+
+
+@pytest.fixture
+def route(monkeypatch):
+    def run(lengths, heads=2, key_dim=64, value_dim=16, dtype=torch.bfloat16, q_start=None):
+        went = []
+        monkeypatch.setattr(ops, "delta_scan", lambda *a, **k: went.append("tokens"))
+        monkeypatch.setattr(ops, "delta_scan_chunks", lambda *a, **k: went.append("chunks"))
+        starts = [0] + torch.tensor(lengths).cumsum(0).tolist()
+        batch = SimpleNamespace(num_tokens=starts[-1], num_requests=len(lengths), q_offsets=None, slot_ids=None,
+                                q_start=starts if q_start is None else q_start)
+        tensor = SimpleNamespace(is_cuda=True, data_ptr=lambda: 4096, shape=(3, starts[-1], heads * key_dim))
+        ops.delta_scan_step(tensor, tensor, tensor, batch, heads, key_dim, value_dim, dtype)
+        return went
+    return run
+
+
+@pytest.mark.parametrize("sizes,where", [(dict(), "chunks"), (dict(heads=1 << 15, value_dim=255), "chunks"), (dict(heads=1 << 15, value_dim=256), "tokens"),
+                                         (dict(key_dim=32), "tokens"), (dict(dtype=torch.float32), "tokens")])
+def test_sizes_that_the_chunks_refuse_go_token_by_token(route, sizes, where):
+    assert route([64, 2], **sizes) == [where]
