@@ -2021,8 +2021,10 @@ def delta_scan_step(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, ba
     token by token and in chunks: 48 tokens 12 and 15, 64 tokens 15 and 15, 96 tokens 21 and 15, 2,048 tokens 439 and 107; with
     the removal term 15 and 19, 19 and 20, 30 and 23, 590 and 185."""
     lists = (batch.q_offsets, batch.slot_ids, batch.num_requests, heads, key_dim, value_dim)
-    if dtype != torch.float32 and v.is_cuda and batch.num_tokens >= SCAN_CHUNKS_FROM and library().lc_scan_chunks_records(
-            coef.shape[0], batch.num_requests, batch.num_tokens, heads, key_dim, value_dim, SCAN_CHUNKS_FROM) > 0:
+    # (every request brings a token at least: where the others leave none for a portion, its length need not be looked for)
+    if dtype != torch.float32 and v.is_cuda and batch.num_tokens - batch.num_requests >= SCAN_CHUNKS_FROM - 1 and \
+            library().lc_scan_chunks_records(coef.shape[0], batch.num_requests, batch.num_tokens, heads, key_dim, value_dim,
+                                             SCAN_CHUNKS_FROM) > 0:
         lengths = [b - a for a, b in zip(batch.q_start, batch.q_start[1:])]
         if max(lengths) >= SCAN_CHUNKS_FROM and not (coef.data_ptr() | state.data_ptr()) % 16:
             return delta_scan_chunks(coef, v, state, *lists, some_short=min(lengths) < SCAN_CHUNKS_FROM)

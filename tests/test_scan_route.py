@@ -26,3 +26,21 @@ def route(monkeypatch):
                                          (dict(key_dim=32), "tokens"), (dict(dtype=torch.float32), "tokens")])
 def test_sizes_that_the_chunks_refuse_go_token_by_token(route, sizes, where):
     assert route([64, 2], **sizes) == [where]
+
+
+class _Unread(list):
+    def __iter__(self):
+        raise AssertionError("the lengths were walked")
+
+    __getitem__ = __iter__
+
+
+@pytest.mark.parametrize("lengths", [[1] * 64, [1] * 500, [60] + [1] * 40, [63] + [1] * 3])
+def test_steps_without_a_portion_look_for_none(route, lengths):
+    """The rule runs once a layer: a decode step of many requests must not pay for a walk over their lengths."""
+    assert route(lengths, q_start=_Unread()) == ["tokens"]
+
+
+def test_the_shortest_portion_is_found_among_lone_tokens(route):
+    assert route([1] * 40 + [64] + [1] * 9) == ["chunks"]
+    assert route([1] * 40 + [33] + [33] + [1] * 9) == ["tokens"]
