@@ -32,3 +32,18 @@ def test_requests_head_by_head_stay_within_the_scratch(heads, window, requests, 
     others = sum(tokens for r, (tokens, _) in enumerate(requests) if r not in wide)
     assert int(tiles[:, 1].sum()) == others if others else info["num_tiles"] == 0
     assert not set(tiles[:, 2].tolist()) & set(wide)
+
+
+def test_lone_tokens_are_not_asked(monkeypatch):
+    asked = []
+    pays = ops.latent_wide_pays
+    monkeypatch.setattr(ops, "latent_wide_pays", lambda *a: asked.append(a) or pays(*a))
+    _, plan = ops.latent_short_planner(16, 0)
+    assert plan(layout_of([(1, 2000 + i) for i in range(64)]))[1]["wide"] == [] and asked == []
+    assert plan(layout_of([(1, 4000), (2048, 2048), (1, 5)]))[1]["wide"] == [1] and [a[0] for a in asked] == [2048]
+
+
+@pytest.mark.parametrize("heads", [1, 3, 4, 5, 16, 128])
+@pytest.mark.parametrize("position", [0, 31, 2047, 131071, 10 ** 6])
+def test_a_lone_token_is_never_faster_head_by_head(heads, position):
+    assert not ops.latent_wide_pays(1, position, heads, 0)
