@@ -9,7 +9,7 @@ token and appends it to the sequences itself; here sampling is a stage of its ow
 from __future__ import annotations
 
 import time
-from typing import Dict, Hashable, List, Optional, Sequence
+from typing import Dict, Hashable, List, Optional, Sequence, Tuple
 
 import numpy as np
 import torch
@@ -28,16 +28,20 @@ class _CapturedStep:
 
 
 def blocks_from_free_memory(free: int, bytes_per_block: int, state_bytes: int,
-                            config: EngineConfig, max_positions: int = 0) -> int:
+                            config: EngineConfig, max_positions: int = 0, scratch: Tuple[int, int] = (0, 0)) -> int:
     """Pages for the cache when none are asked for, as the reference sizes its pools
     (src/qwen.cc:527-543): ``memory_fraction`` of the free memory less a reserve, divided by
     what a page costs over all layers.  Beyond the reference: the per-request state tensors
     come off first, and the count is capped at what ``max_seqs`` requests of the model's
     longest context can hold and at what a 32-bit slot id (page * block_size + offset) can
-    name."""
+    name.  ``scratch``: what a step may want for every cached token, and at most (``Part.step_scratch``).  What
+    the fraction leaves free is for it; where that is too little the rest is kept back, the whole of it or, on a card of few
+    pages, each page's share."""
     per_block = max(1, int(bytes_per_block))
-    usable = int(max(0, free - config.memory_reserve) * config.memory_fraction) - int(state_bytes)
-    blocks = usable // per_block
+    room = max(0, free - config.memory_reserve)
+    usable = int(room * config.memory_fraction) - int(state_bytes)
+    short = max(0, scratch[1] - int(room * (1.0 - config.memory_fraction)))
+    blocks = max((usable - short) // per_block, usable // (per_block + scratch[0] * config.block_size))
     if blocks <= 0:
         raise RuntimeError(f"no memory for the cache: {free} bytes free, a page of all "
                            f"layers takes {per_block}")
@@ -79,7 +83,7 @@ class ModelRunner:
         free, _ = torch.cuda.mem_get_info(self.device)
         return blocks_from_free_memory(
             free, probe.bytes_per_block(self.config.dtype), probe.state_bytes(self.config.dtype), self.config,
-            self.model.spec.max_positions)
+            self.model.spec.max_positions, self.model.step_scratch())
 
     # ------------------------------------------------------------------ the step
     def can_run(self, entries: Sequence[StepEntry]) -> bool:

@@ -1359,6 +1359,13 @@ def latent_wide_pays(tokens: int, position: int, heads: int, window: int) -> boo
 LATENT_WIDE_ENTRIES = 1 << 28
 
 
+def latent_wide_scratch(heads: int, rank: int, rot: int, dim: int, vdim: int) -> Tuple[int, int]:
+    """Bytes that ``latent_wide`` takes for a visible row (the row itself, its keys and its values), and at most for the requests
+    that ``latent_short_planner`` picks."""
+    row = 2 * (rank + rot + heads * (dim + vdim))
+    return row, LATENT_WIDE_ENTRIES // (heads * 128) * row
+
+
 def latent_short_planner(heads: int, window: int):
     """(key, planner) for a part whose long portions may attend head by head: ``plan_latent_attention`` for the others, and in
     ``info["wide"]`` the requests that do.  These are taken in order as long as their visible rows' keys and values stay within

@@ -12,7 +12,7 @@ from __future__ import annotations
 
 import math
 import sys
-from typing import Callable, Dict, List, Optional
+from typing import Callable, Dict, List, Optional, Tuple
 
 import torch
 
@@ -210,6 +210,12 @@ class CausalLM:
             if planner is not None:
                 planners.setdefault(planner[0], planner[1])
         return planners
+
+    def step_scratch(self) -> Tuple[int, int]:
+        """What a step may allocate for the cached tokens that it reads (``Part.step_scratch``): the parts run one after
+        the other, so the most of any."""
+        wanted = [part.step_scratch() for part in self._all_parts()]
+        return max((w[0] for w in wanted), default=0), max((w[1] for w in wanted), default=0)
 
     def portion_multiple(self) -> int:
         """Portions of a prompt, but for its last, must be multiples of this many tokens."""

@@ -26,7 +26,7 @@ Interfaces (all tensors on the GPU; "act" is the engine's activation dtype):
 from __future__ import annotations
 
 from dataclasses import dataclass, field
-from typing import Any, Dict
+from typing import Any, Dict, Tuple
 
 import torch
 
@@ -89,6 +89,11 @@ class Part:
         size).  A part that keeps several things (pages and a piece of state per request) returns a
         tuple of needs and finds the k-th as ``site.part(k)``."""
         return None
+
+    def step_scratch(self) -> Tuple[int, int]:
+        """Bytes that ``forward`` may allocate, for as long as it runs, for every cached token that a step's portions see,
+        and at most in all; nothing of what grows with the step's own tokens.  The cache's pages leave room for it."""
+        return 0, 0
 
     def tables_epoch(self) -> int:
         """A number that changes whenever this part has made a device table anew whose address

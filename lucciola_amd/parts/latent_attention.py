@@ -106,6 +106,9 @@ class LatentAttention(Part):
     def cache_need(self):
         return PagedLatent(self.rank + self.rot, self.window)
 
+    def step_scratch(self):
+        return ops.latent_wide_scratch(self.H, self.rank, self.rot, self.dim, self.vdim) if self.wide else (0, 0)
+
     def batch_planner(self):
         if self.wide:
             return ops.latent_short_planner(self.H, self.window or 0)

@@ -49,6 +49,10 @@ class ParallelMixers(Part):
     def batch_planner(self):
         return self.left.batch_planner() or self.right.batch_planner()
 
+    def step_scratch(self):     # one after the other
+        a, b = self.left.step_scratch(), self.right.step_scratch()
+        return max(a[0], b[0]), max(a[1], b[1])
+
     @property
     def portion_multiple(self) -> int:
         import math

@@ -97,3 +97,25 @@ def test_short_portions_keep_their_tiles():
     short = HostLayout(2, 61, [0, 60, 61], [5, 9], 16, False)
     assert plan(short)[0]["tiles"].tolist() == ops.plan_latent_attention(short)[0]["tiles"].tolist()
     assert plan(short)[1]["wide"] == [] and key != ops.latent_short_planner(16, 0)[0]
+
+
+def test_scratch_is_what_the_cache_leaves_room_for():
+    heads, rank, page, requests = 16, 512, 16, [(3000, 500), (0, 1100)]
+    g = torch.Generator().manual_seed(3)
+    T, pages = sum(n for _, n in requests), [-(-(p + n) // page) for p, n in requests]
+    cache = torch.randn(sum(pages) + 1, page, rank + ROT, generator=g).bfloat16().to(DEV)
+    table = torch.full((2, max(pages)), -1, dtype=torch.int32)
+    table[0, :pages[0]], table[1, :pages[1]] = torch.arange(pages[0]), pages[0] + torch.arange(pages[1])
+    q, qa = (torch.randn(T, heads * n, generator=g).bfloat16().to(DEV) for n in (DIM + ROT, rank + ROT))
+    uk, uv = (torch.randn(heads * n, rank, generator=g).bfloat16().to(DEV) for n in (DIM, VDIM))
+    out, table = torch.zeros(T, heads * VDIM, dtype=torch.bfloat16, device=DEV), table.to(DEV)
+    torch.cuda.synchronize()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.latent_wide(q, qa, heads, rank, DIM, ROT, VDIM, uk, uv, cache, table, page, [0, 1], [0, 500, T], [p for p, _ in requests],
+                    0.1, 0, None, None, False, out)
+    rows = sum(-(-(p + n) // 64) * 64 for p, n in requests)
+    partial = 4 * max(ops.library().lc_gemm_bf16_workspace(rows, heads * DIM, rank), ops.library().lc_gemm_bf16_workspace(heads * VDIM, rows, rank))
+    per_row, most = ops.latent_wide_scratch(heads, rank, ROT, DIM, VDIM)
+    assert 0 < torch.cuda.max_memory_allocated() - before <= rows * per_row + max(partial, 0) + 4096
+    assert rows * per_row <= most
