@@ -22,6 +22,9 @@ constexpr int LW_DIM = 128, LW_ROT = 64, LW_VDIM = 128;
 
 // grid (rows / 4): a wave a row.  Row i of the request's rows (position lo + i, its page's place in table) -> c [i][R], turned [i][rot];
 // zeros behind `count`.
+// A query that does not see a key gives it weight zero, and zero times what is not finite would be no number: the later token's row
+// would spoil up to a tile's 127 tokens before it.  So a latent with such an entry becomes a value of zeros and a key that is NaN
+// in its rotated part, whose score is NaN for the queries that see it and never asked for by the others.
 __global__ __launch_bounds__(256) void latent_rows_kernel(const bf16* __restrict__ cache, const int* __restrict__ table, int page_size,
                                                           int R, int rot, int lo, int count, int rows, bf16* __restrict__ c,
                                                           bf16* __restrict__ turned) {
@@ -29,14 +32,25 @@ __global__ __launch_bounds__(256) void latent_rows_kernel(const bf16* __restrict
     if (i >= rows) return;
     const int j = lo + i, pieces = (R + rot) / 8;
     const bool live = i < count;
+    bool odd = false;
     const bf16* row = cache + (size_t)(live ? table[j / page_size] * page_size + j % page_size : 0) * (R + rot);
     for (int p = lane; p < pieces; p += kWave) {
         bf16x8 v;
 #pragma unroll
         for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16>(0.f);
         if (live) v = *reinterpret_cast<const bf16x8*>(row + p * 8);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) odd |= p * 8 < R && (__builtin_bit_cast(unsigned short, static_cast<bf16>(v[e])) & 0x7F80) == 0x7F80;
         if (p * 8 < R) *reinterpret_cast<bf16x8*>(c + (size_t)i * R + p * 8) = v;
         else *reinterpret_cast<bf16x8*>(turned + (size_t)i * rot + (p * 8 - R)) = v;
+    }
+    if (__builtin_amdgcn_ballot_w64(odd) == 0) return;
+    for (int p = lane; p < pieces; p += kWave) {
+        const bool rotated = p * 8 >= R;
+        bf16x8 v;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = static_cast<bf16>(rotated ? __builtin_nanf("") : 0.f);
+        *reinterpret_cast<bf16x8*>(rotated ? turned + (size_t)i * rot + (p * 8 - R) : c + (size_t)i * R + p * 8) = v;
     }
 }
 

@@ -119,3 +119,28 @@ def test_scratch_is_what_the_cache_leaves_room_for():
     per_row, most = ops.latent_wide_scratch(heads, rank, ROT, DIM, VDIM)
     assert 0 < torch.cuda.max_memory_allocated() - before <= rows * per_row + max(partial, 0) + 4096
     assert rows * per_row <= most
+
+
+@pytest.mark.parametrize("bad", [float("nan"), float("inf"), float("-inf")])
+@pytest.mark.parametrize("entry", [5, 64 + 3])          # of the latent, of the rotated part
+@pytest.mark.parametrize("position,tokens,window,at", [(0, 130, 0, 100), (0, 130, 0, 129), (70, 200, 0, 200), (300, 150, 90, 380), (40, 64, 0, 10)])
+def test_a_row_that_is_not_finite_reaches_only_who_sees_it(bad, entry, position, tokens, window, at):
+    heads, rank, page, T = 2, 64, 16, tokens
+    g = torch.Generator().manual_seed(position + tokens)
+    pages = -(-(position + tokens) // page)
+    cache = torch.randn(pages, page, rank + ROT, generator=g).bfloat16().to(DEV)
+    q, qa = (torch.randn(T, heads * n, generator=g).bfloat16().to(DEV) for n in (DIM + ROT, rank + ROT))
+    uk, uv = (torch.randn(heads * n, rank, generator=g).mul(rank ** -0.5).bfloat16().to(DEV) for n in (DIM, VDIM))
+    table = torch.arange(pages, dtype=torch.int32, device=DEV)[None]
+    outs = []
+    for value in (0.25, bad):
+        cache.view(-1, rank + ROT)[at, entry] = value
+        outs.append(torch.zeros(T, heads * VDIM, dtype=torch.bfloat16, device=DEV))
+        ops.latent_wide(q, qa, heads, rank, DIM, ROT, VDIM, uk, uv, cache, table, page, [0], [0, T], [position], 0.1, window, None, None,
+                        False, outs[-1])
+    i = position + torch.arange(T, device=DEV)
+    sees = (i >= at) & ((i < at + window) if window else (i >= 0))
+    assert torch.equal(outs[1][~sees], outs[0][~sees])
+    assert bool(torch.isfinite(outs[0]).all())
+    if entry < 64:          # (a rotated part may make a score of minus infinity, which weighs nothing)
+        assert not bool(torch.isfinite(outs[1][sees]).any())
