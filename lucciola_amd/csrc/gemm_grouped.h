@@ -39,8 +39,10 @@ __device__ __forceinline__ bool find_tile(const GroupedArgs& a, int BM, GroupedT
     return true;
 }
 
-// Whether gemm_grouped_tiled.hip has a kernel for these bfloat16 operands (whole, aligned 16-byte pieces) and lists.
+// Whether gemm_grouped_tiled.hip has a kernel for these bfloat16 operands (whole, aligned 16-byte pieces) and lists, and whether it is
+// the faster one.
 bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows);
+bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows);
 int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, hipStream_t stream);
 
 }  // namespace lc

@@ -25,7 +25,12 @@ namespace lc {
 constexpr int GG_N = 64, GG_K = 16, GG_CHUNK = 256, GG_PAD = 16;
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
-static thread_local int g_grouped_fast = 1, g_grouped_tiled = 1;
+static thread_local int g_grouped_fast = 1, g_grouped_tiled = 2;
+
+// bfloat16 operands of whole, aligned pieces of eight
+static bool whole_pieces(const void* x, int x_dt, long long ldx, long long x_group, const void* w, int w_dt, int K) {
+    return x_dt == DT_BF16 && w_dt == DT_BF16 && K % 8 == 0 && ldx % 8 == 0 && x_group % 8 == 0 && ((uintptr_t)x | (uintptr_t)w) % 16 == 0;
+}
 
 template <typename TX, typename TW, typename TO, int BM, int WM, int WN>
 __global__ __launch_bounds__(256, 2) void gemm_grouped_kernel(GroupedArgs a) {
@@ -343,11 +348,27 @@ LC_API int lc_gemm_grouped_fast(int on) {
     return before;
 }
 
-// Tests and tuning: whether those products may take the kernels of gemm_grouped_tiled.hip, likewise.
+// Tests and tuning: whether those products take the kernels of gemm_grouped_tiled.hip: 2 (the default) where these are the faster
+// ones, 1 wherever they can, 0 nowhere.
 LC_API int lc_gemm_grouped_tiled(int on) {
     const int before = g_grouped_tiled;
-    if (on >= 0) g_grouped_tiled = on ? 1 : 0;
+    if (on >= 0) g_grouped_tiled = on < 2 ? on : 2;
     return before;
+}
+
+// Tests: whether the default is those kernels for whole, aligned bfloat16 operands of these sizes: max_tiles > 0 for the lists of experts
+// (M sorted rows), 0 for products per head.
+LC_API int lc_gemm_grouped_picks_tiled(int tile_rows, int M, int N, int K, int G, int max_tiles) {
+    static const int listed = 0;
+    GroupedArgs a{};
+    a.M = M; a.N = N; a.K = K; a.G = G;
+    a.row_start = max_tiles > 0 ? &listed : nullptr;
+    return grouped_tiled_takes(a, tile_rows) && grouped_tiled_pays(a, max_tiles, tile_rows) ? 1 : 0;
+}
+
+// Whether a product per head over so few rows that 16 go to a tile has the streaming kernel of gemm_grouped_tiled.hip.
+LC_API int lc_gemm_grouped_streams(const void* x, int x_dt, long long ldx, long long x_group, const void* w, int w_dt, int K) {
+    return whole_pieces(x, x_dt, ldx, x_group, w, w_dt, K) && K % 128 == 0 && g_grouped_fast ? 1 : 0;
 }
 
 // Whether tiles of `tile_rows` rows exist for these operand types (16 and 64: always; 128: the
@@ -378,9 +399,9 @@ LC_API int lc_gemm_grouped(const void* x, int x_dt, long long ldx, long long x_g
                   epilogue, gate, ldg, gate_group,
                   N % 2 == 0 && ldo % 2 == 0 && out_group % 2 == 0 && (uintptr_t)out % (out_dt == DT_BF16 ? 4 : 8) == 0};
     // bfloat16 operands whose pieces of 8 are whole and aligned: the bfloat16 matrix instruction
-    if (x_dt == DT_BF16 && w_dt == DT_BF16 && K % 8 == 0 && ldx % 8 == 0 && x_group % 8 == 0 &&
-        (uintptr_t)x % 16 == 0 && (uintptr_t)w % 16 == 0 && g_grouped_fast) {
-        if (g_grouped_tiled && (out_dt == DT_BF16 || out_dt == DT_F32) && grouped_tiled_takes(a, tile_rows))
+    if (whole_pieces(x, x_dt, ldx, x_group, w, w_dt, K) && g_grouped_fast) {
+        if (g_grouped_tiled && (out_dt == DT_BF16 || out_dt == DT_F32) && grouped_tiled_takes(a, tile_rows) &&
+            (g_grouped_tiled == 1 || grouped_tiled_pays(a, max_tiles, tile_rows)))
             return launch_grouped_tiled(a, max_tiles, tile_rows, out_dt == DT_BF16, stream);
         if (out_dt == DT_BF16) return launch_grouped_bf16<bf16>(a, max_tiles, tile_rows, stream);
         if (out_dt == DT_F32) return launch_grouped_bf16<float>(a, max_tiles, tile_rows, stream);

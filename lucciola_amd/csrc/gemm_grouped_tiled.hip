@@ -187,6 +187,28 @@ bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows) {
     return tile_rows == 16 ? a.K % STREAM_K == 0 : a.K % TL_K == 0;
 }
 
+// What these kernels are faster at is a K long enough to fill their rings; a tile of few blocks is mostly its first loads and its
+// stores, which the smaller workgroups of gemm_grouped.hip, of which a CU holds more, hide better.  From 512 k on they are as fast or
+// faster at every size tried; below it depends on how many workgroups there are (us, gemm_grouped.hip and these):
+//   stream   one round of two workgroups a CU gains (16 heads, 512 columns of 128 k, 64 rows 4.2 and 3.8), more lose: the same
+//            at 32 heads 5.1 and 5.4, 400 rows over 32 experts of 2,048 x 128 6.0 and 7.5.  Products per head from 256 k on gain too.
+//   128 rows likewise one round gains (8,192 rows, 32 experts of 512 x 256 19.0 and 16.2), more lose (8 of 2,048 x 256 24.8 and 27.1)
+//   64 rows  experts: 384 k and a workgroup for every CU (18.0 and 18.3 at the worst, 116 and 84 at the best); 256 k lose 10 % at
+//            few workgroups.  Per head: the shorter K, the more full tiles it takes: of 128 k 160 rows, 16 heads, 512 columns 5.8 and
+//            6.6, 2,048 rows 22.7 and 21.6; of 192 k 6.5 and 7.0, and 8.0 and 7.3 at 512 rows; of 64 k it mostly loses (10.1 and 12.4).
+bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows) {
+    const double columns = (a.N + (tile_rows == 16 ? STREAM_N : 128) - 1) / (tile_rows == 16 ? STREAM_N : 128);
+    const double workgroups =
+        columns * (a.row_start ? (max_tiles < a.M ? max_tiles : a.M) : (double)((a.M + tile_rows - 1) / tile_rows) * a.G);
+    const double round = 2 * device_cus();
+    if (a.K >= 512 || (tile_rows != 64 && workgroups <= round)) return a.K >= 128;
+    if (tile_rows == 128) return false;
+    if (a.row_start) return tile_rows == 64 && a.K >= 384 && workgroups >= device_cus();
+    if (tile_rows == 16) return a.K >= 256;
+    const double full = (double)a.M * a.N * a.G / (64 * 128), short_by = 512.0 / a.K;
+    return a.K >= 128 && full * full / workgroups >= 32 * short_by * short_by * short_by;
+}
+
 int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, hipStream_t stream) {
     return out_bf16 ? grouped_tiled<bf16>(a, max_tiles, tile_rows, stream) : grouped_tiled<float>(a, max_tiles, tile_rows, stream);
 }

@@ -80,6 +80,8 @@ _SIGNATURES = {
     "lc_gemm_grouped": "piqqpipiqqiiiipppiiipqqp",
     "lc_gemm_grouped_fast": "i",
     "lc_gemm_grouped_tiled": "i",
+    "lc_gemm_grouped_streams": "piqqpii",
+    "lc_gemm_grouped_picks_tiled": "iiiiii",
     "lc_gemm_grouped_takes_tile": "iii",
     "lc_latent_prepare": "pqpiqiiiiipfppiipppp",
     "lc_latent_attention": "piiiiippppiifippp",
@@ -1211,15 +1213,22 @@ def _check_strided(s: Strided, what: str, rows: int, groups: int, width: int, dt
                           f"and {rows} rows do not fit {tuple(s.tensor.shape)}")
 
 
-def _grouped_tile(rows: int, N: int, groups: int, x: torch.Tensor, w: torch.Tensor) -> int:
+def _grouped_tile(rows: int, N: int, groups: int, x: Strided, w: torch.Tensor) -> int:
     """Rows of the tiles of a product per head over ``rows`` rows: 16 for a step of few tokens, else 64; bfloat16 operands stay
     with 16 up to 1,024 workgroups (these products are short, K of 128 or 512 and as many columns, so what counts is many
     workgroups: 64 rows, 16 heads, 128 columns of 512 k: 4.2 us in tiles of 16 x 64, 8.4 to 8.9 in larger ones; 512 rows 8.0 and
-    8.5; 512 columns of 128 k, 160 rows 6.7 and 6.6, 512 rows 16 and 8)."""
+    8.5; 512 columns of 128 k, 160 rows 6.7 and 6.6, 512 rows 16 and 8), a longer K that the streaming kernel refuses up to 768 (256
+    rows, 32 heads, 128 columns of 320 k, 1,024 workgroups: 7.2 us in tiles of 16 x 64, 6.8 in 64 x 64; in rows that are not aligned,
+    512 rows, 16 heads, 128 columns of 512 k, 30 and 28)."""
     if rows <= 16:
         return 16
-    few = x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and -(-rows // 16) * -(-N // 64) * groups <= 1024
-    return 16 if few else 64
+    workgroups = -(-rows // 16) * -(-N // 64) * groups
+    if x.tensor.dtype != torch.bfloat16 or w.dtype != torch.bfloat16 or workgroups > 1024:
+        return 64
+    K = w.shape[2]
+    streams = workgroups <= 768 or K <= 192 or library().lc_gemm_grouped_streams(
+        x.pointer(), _dt(x.tensor), x.tensor.shape[1], x.group, _ptr(w), _dt(w), K)
+    return 16 if streams else 64
 
 
 def grouped_gemm(x: Strided, w: torch.Tensor, out: Strided, rows: int, gate: Optional[Strided] = None,
@@ -1243,7 +1252,7 @@ def grouped_gemm(x: Strided, w: torch.Tensor, out: Strided, rows: int, gate: Opt
         return
     _call("lc_gemm_grouped", x.pointer(), _dt(x.tensor), x.tensor.shape[1], x.group, _ptr(w), _dt(w),
           out.pointer(), _dt(out.tensor), out.tensor.shape[1], out.group, rows, N, K, G, None, None, None, 0,
-          _grouped_tile(rows, N, G, x.tensor, w), epilogue, gate.pointer() if gate is not None else None,
+          _grouped_tile(rows, N, G, x, w), epilogue, gate.pointer() if gate is not None else None,
           gate.tensor.shape[1] if gate is not None else 0, gate.group if gate is not None else 0, _stream())
 
 
