@@ -2000,7 +2000,7 @@ def delta_scan(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, q_offse
     return out
 
 
-# From this many tokens on a request's portion goes a chunk at a time (``delta_scan_step``).
+# From this many tokens on a request's portion goes a chunk at a time, in a step where that pays (``delta_scan_step``).
 SCAN_CHUNKS_FROM = 64
 
 
@@ -2031,21 +2031,70 @@ def delta_scan_chunks(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, 
     return out
 
 
+@dataclass
+class ScanPortions:
+    """What of a step's requests the choice between the two scans goes by: tokens of the longest, tokens in all and requests, of
+    those of SCAN_CHUNKS_FROM tokens and more and of the shorter ones."""
+
+    long: Tuple[int, int, int]
+    short: Tuple[int, int, int]
+
+    @staticmethod
+    def of(q_start: Sequence[int]) -> "ScanPortions":
+        lengths = [b - a for a, b in zip(q_start, q_start[1:])]
+        long = [n for n in lengths if n >= SCAN_CHUNKS_FROM]
+        short = [n for n in lengths if n < SCAN_CHUNKS_FROM]
+        return ScanPortions((max(long, default=0), sum(long), len(long)), (max(short, default=0), sum(short), len(short)))
+
+
+# (planes, key channels) -> us: token by token (before the first token, a token of the longest request, a token and 16 value channels
+# of a head, a million entries of state); in chunks (before the first chunk, a token of the longest request, a token and head, a token and
+# 16 value channels of a head).  Fitted to 1,876 steps of 64 to 2,600 tokens in portions of 64 to 640 beside none to 200 lone or short
+# requests, 2 to 32 heads of 16 to 257 value channels; eight of ten are within 13 % of their time.
+_SCAN_TIMES = {
+    (3, 64): ((4.4, 0.162, 2.25e-4, 1.69), (12.0, 0.0235, 4.24e-4, 1.00e-4)),
+    (3, 128): ((0.8, 0.249, 4.44e-4, 1.48), (14.2, 0.0392, 4.70e-4, 2.06e-4)),
+    (5, 64): ((4.7, 0.187, 4.39e-4, 2.57), (14.7, 0.0294, 1.11e-3, 1.61e-4)),
+    (5, 128): ((3.9, 0.283, 8.05e-4, 1.45), (17.1, 0.0604, 1.55e-3, 3.71e-4)),
+}
+
+
+def scan_chunks_pay(portions: ScanPortions, planes: int, heads: int, key_dim: int, value_dim: int) -> bool:
+    """Whether a step's portions of SCAN_CHUNKS_FROM tokens and more are faster in chunks, by an estimate of both forms' times on 256
+    CUs.  Token by token a step is its longest request's chain (half as long again a token where the requests bring fewer than 16 tokens
+    each: the shallower kernel), or the states' and tokens' trips where these are longer; the chunks' kernels take that one's place
+    for the portions, but the other requests then follow in a launch of their own.  16 heads of 128 x 128, five planes, us token by
+    token and in chunks: one portion of 64 tokens 19 and 21, of 96 31 and 24, of 2,048 590 and 185; beside 64 lone tokens 64 46 and 62, 128
+    68 and 63, 256 119 and 72; beside 200 lone tokens 192 120 and 142, 384 204 and 161; 16 portions of 64 120 and 100.  The chunks have
+    to gain an eighth: where decays leave their range (known to the kernel alone) their first pass takes up to twice its time."""
+    (start, token, work, state), (c_start, c_token, c_head, c_work) = _SCAN_TIMES[planes, key_dim]
+    blocks, entries = heads * -(-value_dim // 16), heads * value_dim * key_dim * 1e-6
+
+    def by_token(longest, tokens, requests):
+        chain = token * longest * (1.0 if tokens >= 16 * requests else 1.5)
+        return start + (chain ** 4 + (work * tokens * blocks + state * requests * entries) ** 4) ** 0.25 if requests else 0.0
+    (longest, tokens, requests), short = portions.long, portions.short
+    if not requests:
+        return False
+    chunks = c_start + max(c_token * longest, c_work * tokens * blocks) + c_head * tokens * heads + by_token(*short)
+    return 1.15 * chunks <= by_token(max(longest, short[0]), tokens + short[1], requests + short[2])
+
+
 def delta_scan_step(coef: torch.Tensor, v: torch.Tensor, state: torch.Tensor, batch, heads: int, key_dim: int,
                     value_dim: int, dtype: torch.dtype) -> torch.Tensor:
     """The recurrence for a step's batch in a model of ``dtype``.  A float32 model's logits have the same bits for every cut
     of a prompt, so its tokens go one by one; a bfloat16 model's long portions go a chunk at a time, where the head's sizes
-    are ones that the chunks' kernels take and the tensors begin at a whole 16 bytes.  16 heads of 128 x 128, one portion, us
-    token by token and in chunks: 48 tokens 12 and 15, 64 tokens 15 and 15, 96 tokens 21 and 15, 2,048 tokens 439 and 107; with
-    the removal term 15 and 19, 19 and 20, 30 and 23, 590 and 185."""
+    are ones that the chunks' kernels take, the tensors begin at a whole 16 bytes and it is the faster form (``scan_chunks_pay``)."""
     lists = (batch.q_offsets, batch.slot_ids, batch.num_requests, heads, key_dim, value_dim)
     # (every request brings a token at least: where the others leave none for a portion, its length need not be looked for)
     if dtype != torch.float32 and v.is_cuda and batch.num_tokens - batch.num_requests >= SCAN_CHUNKS_FROM - 1 and \
             library().lc_scan_chunks_records(coef.shape[0], batch.num_requests, batch.num_tokens, heads, key_dim, value_dim,
-                                             SCAN_CHUNKS_FROM) > 0:
-        lengths = [b - a for a, b in zip(batch.q_start, batch.q_start[1:])]
-        if max(lengths) >= SCAN_CHUNKS_FROM and not (coef.data_ptr() | state.data_ptr()) % 16:
-            return delta_scan_chunks(coef, v, state, *lists, some_short=min(lengths) < SCAN_CHUNKS_FROM)
+                                             SCAN_CHUNKS_FROM) > 0 and not (coef.data_ptr() | state.data_ptr()) % 16:
+        portions = getattr(batch, "scan_portions", None)
+        if portions is None:        # once a step, not once a layer
+            portions = batch.scan_portions = ScanPortions.of(batch.q_start)
+        if scan_chunks_pay(portions, coef.shape[0], heads, key_dim, value_dim):
+            return delta_scan_chunks(coef, v, state, *lists, some_short=portions.short[2] > 0)
     return delta_scan(coef, v, state, *lists)
 
 

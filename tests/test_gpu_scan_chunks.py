@@ -65,9 +65,10 @@ def test_chunks(planes, kind, heads, dk, dv, lengths):
             assert torch.equal(got[starts[r]:starts[r + 1]], plain[starts[r]:starts[r + 1]])
 
 
-@pytest.mark.parametrize("dtype,dk,lengths,chunked", [(torch.bfloat16, 128, [64, 2], True), (torch.float32, 128, [64, 2], False),
-                                                      (torch.bfloat16, 128, [63, 2], False), (torch.bfloat16, 32, [90], False),
-                                                      (torch.bfloat16, 64, [1, 70], True)])
+@pytest.mark.parametrize("dtype,dk,lengths,chunked", [(torch.bfloat16, 128, [160, 2], True), (torch.float32, 128, [160, 2], False),
+                                                      (torch.bfloat16, 128, [63, 2], False), (torch.bfloat16, 32, [190], False),
+                                                      (torch.bfloat16, 64, [1, 170], True), (torch.bfloat16, 64, [1, 70], False),
+                                                      (torch.bfloat16, 128, [64, 2], False)])
 def test_which_steps_go_in_chunks(monkeypatch, dtype, dk, lengths, chunked):
     g = torch.Generator().manual_seed(dk)
     T, heads, dv = sum(lengths), 2, 16
