@@ -1010,10 +1010,13 @@ static SkinnyPlan skinny_plan(int M, int N, int K, int epilogue) {
         }
         p.items = (N + p.rows - 1) / p.rows;
     }
-    if (g_even_rows && g_force_skinny < 0 && epilogue != 1 && !keep && p.shape != SKINNY_WIDE && p.items <= kCUs / 2) {
+    if (g_even_rows && g_force_skinny < 0 && epilogue != 1 && !keep && p.shape != SKINNY_WIDE && p.items <= kCUs / 2 &&
+        K >= 6 * SK_KBLOCK) {
         // so few tiles leave most CUs idle, and a CU's share of w comes no faster for that: an item for every CU, of four
         // rows at least (the output and down products of the smallest size, N = 1,024: a step of one token of 28 layers 1,054 us
-        // in 64 items of 16 rows, 1,015 in 128 of 8, 1,012 in 256 of 4; of eight 1,141, 1,107 and 1,091)
+        // in 64 items of 16 rows, 1,015 in 128 of 8, 1,012 in 256 of 4; of eight 1,141, 1,107 and 1,091).  A K of few blocks is no
+        // share to speak of, and the items' own starts weigh more: 1 row, N = 1,024, in items of 16 and of 4 rows: K 128 2.1 and 2.4 us, 512
+        // 2.5 and 2.6, 768 2.8 and 2.7, 2,048 4.6 and 3.8
         p.rows = (N + kCUs - 1) / kCUs;
         if (p.rows < 4) p.rows = 4;
         p.items = (N + p.rows - 1) / p.rows;
