@@ -53,8 +53,8 @@ template <> struct __attribute__((aligned(8))) Piece<bf16> {
 //
 // WHOLE: K is a multiple of two stages and x and w are aligned to 16 bytes, so that every load is a whole
 // piece.  Then nothing stands between a stage's loads and their use at the stage's end: no test of
-// k, no row set to zero (a row behind the last is the last one again: its products go nowhere),
-// no test whether there is a next stage (behind the last one it is the last one again).
+// k, and no test whether there is a next stage (behind the last one it is the last one again).  A row behind the
+// last is the last one again: its products go nowhere.
 template <typename TX, typename TW, typename TO, int BM, int BN, int WM, int WN, bool WHOLE, bool SHARED>
 __global__ __launch_bounds__(256, 2) void gemm_generic_kernel(const TX* __restrict__ x,
                                                            const TW* __restrict__ w,
@@ -90,25 +90,23 @@ __global__ __launch_bounds__(256, 2) void gemm_generic_kernel(const TX* __restri
     const bool vec = WHOLE || ((K & 3) == 0 && ((uintptr_t)x % 16 == 0) && ((uintptr_t)w % 16 == 0));
     Piece<TX> xr[XL];               // as they came: widened on the way to LDS, so that nothing waits for them before
     Piece<TW> wr[WL];
-    auto fetch_rows = [&](auto* rows_ptr, int first, int limit, int tile_rows, int count, auto* dst, int k0) {
+    auto fetch_rows = [&](auto* rows_ptr, int first, int limit, int count, auto* dst, int k0) {
         typedef std::remove_reference_t<decltype(*dst)> P;
 #pragma unroll
         for (int u = 0; u < count; ++u) {
             const int row = lrow + 64 * u;
-            const bool live = row < tile_rows && first + row < limit;
             const auto* p = rows_ptr + (size_t)min(first + row, limit - 1) * K + lk;
-            if (WHOLE || (vec && k0 + lk + 3 < K)) {
+            if (WHOLE || (vec && k0 + GB_K <= K)) {         // all four of a row's threads alike: one test a stage
                 dst[u] = *reinterpret_cast<const P*>(p + k0);
             } else {
 #pragma unroll
                 for (int j = 0; j < 4; ++j) dst[u].set(j, k0 + lk + j < K ? p + k0 + j : nullptr);
             }
-            if (!WHOLE && !live) dst[u] = P{};
         }
     };
     auto fetch = [&](int k0) {
-        fetch_rows(x, m0, M, BM, XL, xr, k0);
-        fetch_rows(w, n0, N, BN, WL, wr, k0);
+        fetch_rows(x, m0, M, XL, xr, k0);
+        fetch_rows(w, n0, N, WL, wr, k0);
     };
     // Where this lane writes entry j of its pieces, and where it reads: with wm and wn multiples of TM and TN tiles, tile i of
     // quarter q lies at ((wm / 16) ^ i ^ q ^ g), so that four addresses and constant offsets reach all of them.
@@ -145,8 +143,8 @@ __global__ __launch_bounds__(256, 2) void gemm_generic_kernel(const TX* __restri
     // product of its own: the matrix core is busy with it for 32 clocks, in which the wave issues other work,
     // and what the wave issues beyond that is the matrix core's idle time.
     const int k_begin = c_begin * GB_CHUNK, k_limit = min(K, c_end * GB_CHUNK);
-    // The last stage; stages go in pairs (a chunk but the last has 16), so that it may lie behind K: zeros, which add nothing.
-    const int k_last = k_begin + (k_limit - k_begin + 2 * GB_K - 1) / (2 * GB_K) * (2 * GB_K) - GB_K;
+    // The last stage.  Stages go in pairs (a chunk but the last has 16); a K that is not whole may end with half a pair.
+    const int k_last = k_begin + (k_limit - k_begin + GB_K - 1) / GB_K * GB_K - GB_K;
     fetch(k_begin);
 #pragma unroll
     for (int n = 0; n < PUTS; ++n) put_one(n, 0);
@@ -193,7 +191,7 @@ __global__ __launch_bounds__(256, 2) void gemm_generic_kernel(const TX* __restri
         const int k_end = min(K, (c + 1) * GB_CHUNK);
         for (int k0 = c * GB_CHUNK; k0 < k_end; k0 += 2 * GB_K) {
             step(k0, std::integral_constant<int, 0>{});
-            step(k0 + GB_K, std::integral_constant<int, 1>{});
+            if (WHOLE || k0 + GB_K < k_end) step(k0 + GB_K, std::integral_constant<int, 1>{});
         }
         // lane l holds the rows 4 (l / 16) + r and the column l % 16 of each of its tiles
 #pragma unroll
