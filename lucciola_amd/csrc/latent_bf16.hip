@@ -270,8 +270,8 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
                 for (int r = 0; r < 4; ++r) dst[r] = static_cast<bf16>(o[d][r] * inv);
             }
     } else {
-        // a share's place goes by tile, not by token: the step may hold many tokens that are in no tile
-        const size_t place = ((size_t)blockIdx.x * per_tile + q_tok) * H + q_head;
+        // a share's place goes by token, or (per_tile > 0) by tile, where the step holds tokens that are in no tile
+        const size_t place = per_tile ? ((size_t)blockIdx.x * per_tile + q_tok) * H + q_head : qi;
         float* dst = part_o + (place * splits + blockIdx.z) * R;
 #pragma unroll
         for (int d = 0; d < NH; ++d)
@@ -285,16 +285,20 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     }
 }
 
-// One workgroup per (tile, token of per_tile, head): the shares' sums, taken in from the first.
+// One workgroup per (token, head) or (per_tile > 0: tile, token of per_tile, head): the shares' sums, taken in from the first.
 __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                              int splits, int R, int H, const float* __restrict__ sink,
                                              const int* __restrict__ tiles, int per_tile, bf16* __restrict__ out) {
     __shared__ float weight[64];
     __shared__ float total;
     const size_t qi = blockIdx.x;
-    const int* tile = tiles + 4 * (qi / H / per_tile);
-    const int q_tok = (int)(qi / H) % per_tile;
-    if (q_tok >= tile[1]) return;
+    size_t row = qi;
+    if (per_tile) {
+        const int* tile = tiles + 4 * (qi / H / per_tile);
+        const int q_tok = (int)(qi / H) % per_tile;
+        if (q_tok >= tile[1]) return;
+        row = (size_t)(tile[0] + q_tok) * H + qi % H;
+    }
     if (threadIdx.x < 64) {
         const int z = threadIdx.x;
         const float m = z < splits ? part_ml[(qi * splits + z) * 2] : -INFINITY;
@@ -308,7 +312,6 @@ __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, c
     }
     __syncthreads();
     const float inv = 1.f / total;
-    const size_t row = (size_t)(tile[0] + q_tok) * H + qi % H;
     for (int d = threadIdx.x; d < R; d += blockDim.x) {
         float acc = 0.f;
         for (int z = 0; z < splits; ++z) acc = fmaf(part_o[(qi * splits + z) * R + d], weight[z], acc);
@@ -366,11 +369,12 @@ LC_API int lc_latent_bf16_splits(int workgroups, int max_keys) {
 }
 
 // qa [T, H, R + rot], cache [slots, R + rot] -> out [T, H, R].  tiles [NT, 4]: first token row, tokens
-// (1 to 16), request, first position.  any_portion: whether a tile has more than one token (the
-// grid then has a workgroup per four heads).  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32, n the
-// tiles, times 16 where any has more than one token.
+// (1 to 16), request, first position.  portions: 0 where every tile has one token, else (the grid then has a workgroup per four
+// heads) 1, and 2 if all T tokens are in a tile.  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32, n the tiles (0),
+// 16 times the tiles (1; the places of a tile's missing tokens are joined by workgroups that return at once: 16 tiles of 4 tokens
+// 47.0 us by token and 49.6 so) or T (2).
 LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot, const void* cache, const int* tiles,
-                                    int num_tiles, int any_portion, const int* block_table, int max_blocks,
+                                    int num_tiles, int portions, const int* block_table, int max_blocks,
                                     int page_size, float scale, int window, const float* sink, void* out, int splits,
                                     float* part_o, float* part_ml, hipStream_t stream) {
     int nr = 0, ks = 0;
@@ -380,21 +384,21 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
     if (T == 0 || num_tiles == 0) return 0;
     LC_CHECK(qa && cache && tiles && block_table && out, "latent attention: null pointer");
     LC_CHECK(splits == 1 || (part_o && part_ml), "latent attention: shares need a workspace");
-    const int per_tile = any_portion ? 16 : 1;
+    const int per_tile = portions == 2 ? 0 : portions ? 16 : 1;
     auto join = [&]() {
         if (splits > 1) {
-            latent_attention_join_kernel<<<num_tiles * per_tile * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink, tiles, per_tile,
-                                                                                      (bf16*)out);
+            latent_attention_join_kernel<<<(per_tile ? num_tiles * per_tile : T) * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink,
+                                                                                                       tiles, per_tile, (bf16*)out);
             LC_LAUNCH_CHECK("latent_attention_join");
         }
         return 0;
     };
-    if (!any_portion && g_lone && latent_lone_takes(R, rot) && ((uintptr_t)qa | (uintptr_t)cache) % 16 == 0) {
+    if (!portions && g_lone && latent_lone_takes(R, rot) && ((uintptr_t)qa | (uintptr_t)cache) % 16 == 0) {
         const int rc = launch_latent_lone(qa, H, cache, tiles, num_tiles, block_table, max_blocks, page_size, scale, window, sink, out,
                                           splits, part_o, part_ml, stream);
         return rc ? rc : join();
     }
-    const int blocks_y = any_portion ? (H + 3) / 4 : (H + 63) / 64;
+    const int blocks_y = portions ? (H + 3) / 4 : (H + 63) / 64;
     LC_CHECK(blocks_y <= 65535, "latent attention: too many heads (%d)", H);
     const dim3 grid(num_tiles, blocks_y, splits);
     const size_t lds = sizeof(bf16) * ((size_t)LM_STAGE * (ks * 32 + LM_KPAD) + (size_t)R * LM_VSTRIDE) +

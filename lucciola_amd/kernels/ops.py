@@ -1489,14 +1489,16 @@ def latent_attention(qa: torch.Tensor, heads: int, rank: int, rot: int, tok_req:
         most = block_table.shape[1] * page_size if max_ctx <= 0 else max_ctx
         splits = lib.lc_latent_bf16_splits(workgroups, min(most, window) if window > 0 else most)
         part_o = part_ml = None
-        places = tiles.shape[0] * (LATENT_TILE if any_portion else 1) * heads
-        if any_portion and splits > 1:
+        # where portions attend head by head the others' shares go by tile, whose missing tokens have a place too
+        portions = 0 if not any_portion else 1 if plan.info.get("wide") else 2
+        places = (tiles.shape[0], tiles.shape[0] * LATENT_TILE, T)[portions] * heads
+        if portions == 1 and splits > 1:
             splits = max(1, min(splits, (128 << 20) // (places * rank * 4)))
         if splits > 1:
             part_o = torch.empty((places * splits * rank,), dtype=torch.float32, device=qa.device)
             part_ml = torch.empty((places * splits * 2,), dtype=torch.float32, device=qa.device)
         _call("lc_latent_attention_bf16", _ptr(qa), T, heads, rank, rot, _ptr(cache), _ptr(tiles), tiles.shape[0],
-              1 if any_portion else 0, _ptr(block_table), block_table.shape[1], page_size, float(scale), int(window),
+              portions, _ptr(block_table), block_table.shape[1], page_size, float(scale), int(window),
               _ptr(sink), _ptr(out), splits, _ptr(part_o), _ptr(part_ml), _stream())
         return out
     if qa.dtype == torch.bfloat16 and plan is not None and _latent_fast.on and rank * heads >= 1024:

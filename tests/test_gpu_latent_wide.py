@@ -3,7 +3,7 @@ several requests, behind histories, windows and pages that were given back; and 
 import pytest
 import torch
 
-from lucciola_amd.engine.batch import HostLayout
+from lucciola_amd.engine.batch import HostLayout, Plan
 from lucciola_amd.kernels import ops
 
 pytestmark = pytest.mark.gpu
@@ -144,3 +144,48 @@ def test_a_row_that_is_not_finite_reaches_only_who_sees_it(bad, entry, position,
     assert bool(torch.isfinite(outs[0]).all())
     if entry < 64:          # (a rotated part may make a score of minus infinity, which weighs nothing)
         assert not bool(torch.isfinite(outs[1][sees]).any())
+
+
+@pytest.mark.parametrize("rank,heads,with_sink", [(512, 4, True), (256, 5, False)])
+@pytest.mark.parametrize("wide", [[], [1]])
+def test_shares_of_portions(monkeypatch, rank, heads, with_sink, wide):
+    """Short portions behind long histories, their keys shared out: shares by token where every token of the step is in a tile, by tile
+    beside a portion that attends head by head.  Against the general kernel in float32 arithmetic."""
+    requests, page = [(900, 40), (0, 1500), (700, 1), (500, 3)], 16
+    if not wide:
+        requests[1] = (1200, 17)
+    g = torch.Generator().manual_seed(rank + heads)
+    lengths, first = [n for _, n in requests], [p for p, _ in requests]
+    q_start = [0]
+    for n in lengths:
+        q_start.append(q_start[-1] + n)
+    T, R, pages = q_start[-1], len(requests), [-(-(p + n) // page) for p, n in requests]
+    cache = (torch.randn(sum(pages), page, rank + ROT, generator=g) * 0.5).bfloat16().to(DEV)
+    table, at = torch.full((R, max(pages)), -1, dtype=torch.int32), 0
+    for r, n in enumerate(pages):
+        table[r, :n] = torch.arange(at, at + n)
+        at += n
+    qa = (torch.randn(T, heads * (rank + ROT), generator=g) * 0.6).bfloat16().to(DEV)
+    positions = torch.cat([torch.arange(p, p + n) for p, n in requests]).to(torch.int32).to(DEV)
+    tok_req = torch.cat([torch.full((n,), r) for r, n in enumerate(lengths)]).to(torch.int32).to(DEV)
+    sink = torch.randn(heads, generator=g).to(DEV) if with_sink else None
+    layout = HostLayout(R, T, q_start, first, page, False)
+    monkeypatch.setattr(ops, "latent_wide_pays", lambda tokens, position, *a: tokens == 1500)
+    arrays, info = ops.latent_short_planner(heads, 0)[1](layout)
+    assert info["wide"] == wide
+    plan = Plan({k: torch.tensor(v, device=DEV) for k, v in arrays.items()}, info)
+    calls, call = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: calls.append((name, a)) or call(name, *a))
+    args = (qa, heads, rank, ROT, tok_req, positions, table.to(DEV), cache, page, (rank + ROT) ** -0.5 * 2.0)
+    got = ops.latent_attention(*args, plan=plan, max_ctx=max(p + n for p, n in requests), sink=sink)
+    (name, sent), = calls
+    assert name == "lc_latent_attention_bf16" and sent[8] == (1 if wide else 2) and sent[16] > 1, "form and shares"
+    before = ops.latent_matrix_cores(False)
+    try:
+        want = ops.latent_attention(*args, plan=plan, sink=sink)
+    finally:
+        ops.latent_matrix_cores(before)
+    for r in range(R):
+        if r not in wide:
+            a, b = (x[q_start[r]:q_start[r + 1]].double() for x in (got, want))
+            assert float((a - b).norm() / b.norm()) <= 2.0 ** -7, r       # weights and both results rounded to bfloat16
