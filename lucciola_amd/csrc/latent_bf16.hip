@@ -285,25 +285,27 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     }
 }
 
-// One workgroup per (token, head) or (per_tile > 0: tile, token of per_tile, head): the shares' sums, taken in from the first.
+// One workgroup per (token, head) or (PER > 0: tile, token of PER, head): the shares' sums, taken in from the first.
+template <int PER>
 __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, const float* __restrict__ part_ml,
                                              int splits, int R, int H, const float* __restrict__ sink,
-                                             const int* __restrict__ tiles, int per_tile, bf16* __restrict__ out) {
+                                             const int* __restrict__ tiles, bf16* __restrict__ out) {
     __shared__ float weight[64];
     __shared__ float total;
     const size_t qi = blockIdx.x;
+    const unsigned head = blockIdx.x % (unsigned)H;
     size_t row = qi;
-    if (per_tile) {
-        const int* tile = tiles + 4 * (qi / H / per_tile);
-        const int q_tok = (int)(qi / H) % per_tile;
-        if (q_tok >= tile[1]) return;
-        row = (size_t)(tile[0] + q_tok) * H + qi % H;
+    if constexpr (PER > 1) {
+        const unsigned place = blockIdx.x / (unsigned)H, q_tok = place % PER;
+        const int* tile = tiles + 4 * (place / PER);
+        if ((int)q_tok >= tile[1]) return;
+        row = (size_t)(tile[0] + q_tok) * H + head;
     }
     if (threadIdx.x < 64) {
         const int z = threadIdx.x;
         const float m = z < splits ? part_ml[(qi * splits + z) * 2] : -INFINITY;
         // the head's sink counts as one more share: maximum sink, sum 1, no row
-        const float s2 = sink ? sink[qi % H] * 1.4426950408889634f : -INFINITY;
+        const float s2 = sink ? sink[head] * 1.4426950408889634f : -INFINITY;
         const float M = fmaxf(wave_max(m), s2);
         const float w = m == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m - M);     // the maxima are in units of log 2
         weight[z] = w;
@@ -312,6 +314,7 @@ __global__ void latent_attention_join_kernel(const float* __restrict__ part_o, c
     }
     __syncthreads();
     const float inv = 1.f / total;
+    if constexpr (PER == 1) row = (size_t)tiles[4 * (blockIdx.x / (unsigned)H)] * H + head;     // not waited for before the shares
     for (int d = threadIdx.x; d < R; d += blockDim.x) {
         float acc = 0.f;
         for (int z = 0; z < splits; ++z) acc = fmaf(part_o[(qi * splits + z) * R + d], weight[z], acc);
@@ -324,7 +327,7 @@ bool latent_lone_takes(int R, int rot);
 int launch_latent_lone(const void* qa, int H, const void* cache, const int* tiles, int num_tiles, const int* block_table, int max_blocks,
                        int page_size, float scale, int window, const float* sink, void* out, int splits, float* part_o, float* part_ml,
                        hipStream_t stream);
-static thread_local int g_lone = 1;
+static thread_local int g_lone = 2;
 
 static bool shape_of(int R, int rot, int* nr, int* ks) {
     const int Dk = R + rot;
@@ -346,16 +349,46 @@ LC_API int lc_latent_bf16_supported(int R, int rot) {
     return shape_of(R, rot, &nr, &ks) ? 1 : 0;
 }
 
-// Tests and tuning: whether steps of lone tokens may take the kernel of latent_lone.hip (1, the default), for the calling
-// thread.  Returns the setting before.
+// Tests and tuning: whether steps of lone tokens take the kernel of latent_lone.hip: 2 (the default) where it is the faster one, 1
+// wherever it can, 0 never; for the calling thread.  Returns the setting before.
 LC_API int lc_latent_lone(int on) {
     const int before = g_lone;
-    if (on >= 0) g_lone = on ? 1 : 0;
+    if (on >= 0) g_lone = on < 2 ? on : 2;
     return before;
 }
 
-// Heads that a workgroup serves of a lone token.
-LC_API int lc_latent_lone_heads(int R, int rot) { return g_lone && latent_lone_takes(R, rot) ? 16 : 64; }
+// Shares for the kernel of latent_lone.hip, `workgroups` without shares (one to a CU: it takes a whole SIMD's registers a wave), of
+// which four waves share stages of 16 rows: those that cost least when the CUs take them in rounds, a round being its waves' stages and
+// what they cost to start and to bring together, 1.3 stages, and the second kernel 1.5; more than a round of whole tiles stays whole,
+// because what bounds it then is the rows' way from memory.  (Rounded up to fill every CU, as for
+// latent_attention_bf16_kernel, a few workgroups began a second round: 16 requests of 1,400 rows, 48 heads 41 us, so 27.)
+LC_API int lc_latent_lone_splits(int workgroups, int max_keys) {
+    const int cus = device_cus(), stages = (max_keys + 15) / 16;
+    int best = 1;
+    double least = 0.0;
+    for (int s = 1; s <= 64 && s <= (stages + 3) / 4 && (s == 1 || workgroups < cus); ++s) {
+        const int rounds = (int)(((long long)workgroups * s + cus - 1) / cus), share = (stages + s - 1) / s;
+        const double cost = rounds * ((share + 3) / 4 + 1.3) + (s > 1 ? 1.5 : 0.0);
+        if (s == 1 || cost < least) least = cost, best = s;
+    }
+    return best;
+}
+
+// Whether a step of `tiles` lone tokens that see up to max_keys rows takes the kernel of latent_lone.hip.  It needs rows enough to
+// pay for its end, where four waves' sums meet in LDS (16 heads, us here and there: 20 rows 9.4 and 7.1, 300 15.4 and 14.1, 64 requests of
+// 500 21.7 and 24.7, of 2,047 37 and 67).  Every 16 heads read the rows again, from a near cache as long as a tile's workgroups run
+// at once: 64 requests of 2,047, 64 heads 77 and 90 us, 256 of 2,000 426 and 277; 48 and 96 heads, whose workgroups do not go
+// into the CUs' rounds, 16 of 2,000 60 and 50.
+static bool latent_lone_pays(int H, int tiles, int max_keys) {
+    const int groups = (H + 15) / 16;
+    const long long workgroups = (long long)tiles * groups;
+    if (groups > 2 && workgroups > ((groups & (groups - 1)) ? 64 : 800)) return false;
+    if (groups == 1 && H > 8) return max_keys >= 1500 || (max_keys >= 256 && (long long)tiles * max_keys >= 16384);
+    return max_keys >= 256 || (max_keys > 64 && tiles <= 64);
+}
+LC_API int lc_latent_lone_picks(int R, int rot, int H, int tiles, int max_keys) {
+    return latent_lone_takes(R, rot) && (g_lone == 1 || (g_lone == 2 && latent_lone_pays(H, tiles, max_keys))) ? 1 : 0;
+}
 
 // Shares the stages of a tile are cut into: from the number of workgroups without shares and
 // the most keys a tile can see.
@@ -369,8 +402,8 @@ LC_API int lc_latent_bf16_splits(int workgroups, int max_keys) {
 }
 
 // qa [T, H, R + rot], cache [slots, R + rot] -> out [T, H, R].  tiles [NT, 4]: first token row, tokens
-// (1 to 16), request, first position.  portions: 0 where every tile has one token, else (the grid then has a workgroup per four
-// heads) 1, and 2 if all T tokens are in a tile.  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32, n the tiles (0),
+// (1 to 16), request, first position.  portions: 0 where every tile has one token (-1: and the kernel of latent_lone.hip serves them), else (the grid then has a workgroup per four
+// heads) 1, and 2 if all T tokens are in a tile.  splits > 1: part_o [n H splits R] and part_ml [n H splits 2] float32, n the tiles (0, -1),
 // 16 times the tiles (1; the places of a tile's missing tokens are joined by workgroups that return at once: 16 tiles of 4 tokens
 // 47.0 us by token and 49.6 so) or T (2).
 LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot, const void* cache, const int* tiles,
@@ -384,16 +417,18 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
     if (T == 0 || num_tiles == 0) return 0;
     LC_CHECK(qa && cache && tiles && block_table && out, "latent attention: null pointer");
     LC_CHECK(splits == 1 || (part_o && part_ml), "latent attention: shares need a workspace");
-    const int per_tile = portions == 2 ? 0 : portions ? 16 : 1;
+    const int per_tile = portions == 2 ? 0 : portions > 0 ? 16 : 1;
     auto join = [&]() {
         if (splits > 1) {
-            latent_attention_join_kernel<<<(per_tile ? num_tiles * per_tile : T) * H, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink,
-                                                                                                       tiles, per_tile, (bf16*)out);
+            const int blocks = (per_tile ? num_tiles * per_tile : T) * H;
+            (per_tile == 0 ? latent_attention_join_kernel<0> : per_tile == 1 ? latent_attention_join_kernel<1> : latent_attention_join_kernel<16>)
+                <<<blocks, 256, 0, stream>>>(part_o, part_ml, splits, R, H, sink, tiles, (bf16*)out);
             LC_LAUNCH_CHECK("latent_attention_join");
         }
         return 0;
     };
-    if (!portions && g_lone && latent_lone_takes(R, rot) && ((uintptr_t)qa | (uintptr_t)cache) % 16 == 0) {
+    if (portions < 0) {
+        LC_CHECK(latent_lone_takes(R, rot) && ((uintptr_t)qa | (uintptr_t)cache) % 16 == 0, "latent attention: rows that latent_lone refuses");
         const int rc = launch_latent_lone(qa, H, cache, tiles, num_tiles, block_table, max_blocks, page_size, scale, window, sink, out,
                                           splits, part_o, part_ml, stream);
         return rc ? rc : join();

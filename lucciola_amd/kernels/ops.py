@@ -87,7 +87,8 @@ _SIGNATURES = {
     "lc_latent_attention": "piiiiippppiifippp",
     "lc_latent_bf16_supported": "ii",
     "lc_latent_lone": "i",
-    "lc_latent_lone_heads": "ii",
+    "lc_latent_lone_picks": "iiiii",
+    "lc_latent_lone_splits": "ii",
     "lc_latent_wide_supported": "iiii",
     "lc_latent_rows": "ppiiiiiippp",
     "lc_latent_wide": "pqpqqpppqiiiiifippqqpqp",
@@ -1485,13 +1486,18 @@ def latent_attention(qa: torch.Tensor, heads: int, rank: int, rot: int, tok_req:
             and lib.lc_latent_bf16_supported(rank, rot)):
         # the matrix-core kernel, over the planner's tiles; few tiles: their keys are shared out
         tiles, any_portion = plan.arrays["tiles"], plan.info["any_portion"]
-        workgroups = tiles.shape[0] * -(-heads // (4 if any_portion else lib.lc_latent_lone_heads(rank, rot)))
         most = block_table.shape[1] * page_size if max_ctx <= 0 else max_ctx
-        splits = lib.lc_latent_bf16_splits(workgroups, min(most, window) if window > 0 else most)
+        most = min(most, window) if window > 0 else most
+        lone = not any_portion and not (qa.data_ptr() | cache.data_ptr()) % 16 and \
+            lib.lc_latent_lone_picks(rank, rot, heads, tiles.shape[0], most)
+        if lone:
+            splits = lib.lc_latent_lone_splits(tiles.shape[0] * -(-heads // 16), most)
+        else:
+            splits = lib.lc_latent_bf16_splits(tiles.shape[0] * -(-heads // (4 if any_portion else 64)), most)
         part_o = part_ml = None
         # where portions attend head by head the others' shares go by tile, whose missing tokens have a place too
-        portions = 0 if not any_portion else 1 if plan.info.get("wide") else 2
-        places = (tiles.shape[0], tiles.shape[0] * LATENT_TILE, T)[portions] * heads
+        portions = (-1 if lone else 0) if not any_portion else 1 if plan.info.get("wide") else 2
+        places = heads * (T if portions == 2 else tiles.shape[0] * (LATENT_TILE if any_portion else 1))
         if portions == 1 and splits > 1:
             splits = max(1, min(splits, (128 << 20) // (places * rank * 4)))
         if splits > 1:
