@@ -3,6 +3,12 @@ several requests, behind histories, windows and pages that were given back; and 
 import pytest
 import torch
 
+import kikunex_configs
+import plain_kikunex
+import plain_pubodra
+import pubodra_configs
+import traces
+from helpers import compare, make_runner, prompts_for, random_weights, replay
 from lucciola_amd.engine.batch import HostLayout, Plan
 from lucciola_amd.kernels import ops
 
@@ -189,3 +195,48 @@ def test_shares_of_portions(monkeypatch, rank, heads, with_sink, wide):
         if r not in wide:
             a, b = (x[q_start[r]:q_start[r + 1]].double() for x in (got, want))
             assert float((a - b).norm() / b.norm()) <= 2.0 ** -7, r       # weights and both results rounded to bfloat16
+
+
+def _pubodra():
+    """The queries out of the layer's input, a gate an entry, a window and none."""
+    mixers = [pubodra_configs._mixer(heads, DIM, ROT, VDIM, 512, 0.07, window) for heads, window in ((3, 100), (2, None))]
+    layers = [pubodra_configs._layer(mixers[0], None), pubodra_configs._layer(mixers[1], pubodra_configs._dense(96))]
+    cfg = {"architecture": "Pubodra", "vocab": 300, "width": 128, "norm": {"eps": 1e-6}, "layers": layers}
+    return cfg, random_weights(cfg, 5, std=0.1), plain_pubodra.forward
+
+
+def _kikunex():
+    """The queries out of a latent of their own, a gate a head, a sink, a window and none."""
+    mixers = [kikunex_configs.latent(8, DIM, ROT, VDIM, rank, 64, 0.07, window) for rank, window in ((512, None), (128, 90))]
+    cfg = {"architecture": "Kikunex", "vocab": 300, "width": 128, "norm": {"eps": 1e-6}, "layers": [kikunex_configs.layer(m, None) for m in mixers]}
+    weights, g = random_weights(dict(cfg, initializer_range=0.1), 6), torch.Generator().manual_seed(6)
+    for name, t in weights.items():
+        if name.endswith(".sink"):
+            weights[name] = (torch.randn(t.shape, generator=g) * 1.5).to(t.dtype)
+    return cfg, weights, plain_kikunex.forward
+
+
+@pytest.mark.parametrize("model", [_pubodra, _kikunex])
+def test_a_model_whose_portions_attend_head_by_head(monkeypatch, model):
+    """Steps of long portions only, of long ones beside short ones and lone tokens, behind what earlier steps have cached, and of
+    none: the logits at every place are the plain implementation's."""
+    cfg, weights, forward = model()
+    prompts = prompts_for({"vocab_size": cfg["vocab"]}, [281, 231, 122], 7)
+    refs = {n: forward(cfg, weights, ids) for n, ids in prompts.items()}
+    without = forward(cfg, {n: t * 0 if n.endswith(".uv") else t for n, t in weights.items()}, prompts["r0"])
+    moved = (without - refs["r0"]).abs().amax(1) / refs["r0"].abs().amax(1)
+    assert float(moved.median()) > 0.2, "the logits would not show a wrong attention"
+    steps, fed = [], dict.fromkeys(prompts, 0)
+    for sizes in ({"r0": 150, "r1": 128}, {"r0": 130, "r1": 1, "r2": 20}, {"r1": 1, "r2": 1}, {"r1": 101}, {"r2": 101, "r0": 1}):
+        entries = []
+        for name, n in sizes.items():
+            entries.append((name, prompts[name][fed[name]:fed[name] + n], list(range(n))))
+            fed[name] += n
+        steps.append((entries, [name for name in sizes if fed[name] == len(prompts[name])]))
+    monkeypatch.setattr(ops, "latent_wide_pays", lambda tokens, position, heads, window: tokens >= 100)
+    calls, call = [], ops._call
+    monkeypatch.setattr(ops, "_call", lambda name, *a: calls.append(name) or call(name, *a))
+    got = replay(make_runner(cfg, weights, 16, traces.max_live_tokens(steps, 16) // 16, "bfloat16", DEV), steps)
+    assert len(got) == sum(len(ids) for ids in prompts.values())
+    assert calls.count("lc_latent_wide") == 2 * 5, "two layers, five portions of 100 tokens and more"
+    print(f"{cfg['architecture']}: worst relative error {compare(got, cfg, weights, prompts, 4e-2, refs):.3e}")
