@@ -9,11 +9,17 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def off_by(got, want, K):
+def off_by(got, want, K, squared=False):
     """The largest error in units of what is allowed: float32 sums of K products of bfloat16 numbers (a unit of 2^-24 of the
-    terms' root mean square sum a term, on average far less), and half a unit of bfloat16 where the result is rounded."""
+    terms' root mean square sum a term, on average far less), and half a unit of bfloat16 where the result is rounded.
+    ``squared``: the result is the square of ``want``'s positive entries, whose error is the sum's times the slope, entry by entry,
+    and the square's own rounding."""
     want = want.to(DEV)
     allowed = K * 2.0 ** -24 * want.pow(2).mean().sqrt() + 1e-30
+    if squared:
+        want = torch.relu(want)
+        allowed = (2 * want + allowed) * allowed + want.pow(2) * 2.0 ** -24
+        want = want.pow(2)
     if got.dtype == torch.bfloat16:
         allowed = allowed + want.abs() * 2.0 ** -8
     return float(((got.float() - want).abs() / allowed).max())
@@ -45,7 +51,7 @@ def test_experts(out, tile, counts, N, K):
     routing = ops.Routing(ids, torch.ones(rows, 1, device=DEV), starts, tiles, token, entry, E, tile, rows // tile + E)
     x = torch.randn(rows, K, generator=g).bfloat16().to(DEV)
     w = torch.randn(E, N, K, generator=g).bfloat16().to(DEV)
-    for gather, act in ((True, "relu_squared"), (False, None)):
+    for gather, act in ((True, "relu_squared"), (True, None), (False, None)):
         got = switched(1, lambda: ops.moe_experts(x, w, routing, out, activation=act, gather=gather))
         plain = switched(0, lambda: ops.moe_experts(x, w, routing, out, activation=act, gather=gather))
         expert = ids[:, 0].long()[entry.argsort()] if gather else None
@@ -55,10 +61,8 @@ def test_experts(out, tile, counts, N, K):
         want = torch.empty(rows, N, device=DEV)
         for e in range(E):
             want[expert == e] = src[expert == e].float() @ w[e].float().T
-        z = torch.relu(want) ** 2 if act else want
-        scale = 1.0 if not act else 2.0 * float(want.abs().max())       # the square's slope
-        assert off_by(got, z, K) <= max(1.0, scale), (gather, act)
-        assert off_by(plain, z, K) <= max(1.0, scale), (gather, act)
+        assert off_by(got, want, K, squared=act is not None) <= 1.0, (gather, act)
+        assert off_by(plain, want, K, squared=act is not None) <= 1.0, (gather, act)
 
 
 @pytest.mark.parametrize("rows,G,N,K,gap", [(1, 3, 128, 128, 0), (16, 2, 65, 256, 8), (17, 4, 512, 128, 64), (64, 3, 128, 512, 0),
