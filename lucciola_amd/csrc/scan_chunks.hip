@@ -13,8 +13,13 @@
 //     S' = diag(a_last) S + (write~^T - removal~^T T M) V - removal~^T (T probe~ S)
 // All that does not hold S or V is made first, chunks and heads side by side (scan_chunk_prepare_kernel); then a workgroup
 // per 16 value channels and head walks a request's chunks in order (scan_chunk_walk_kernel), with S in the accumulators.
-// Everything is float32: operands, products and sums.  No decay is ever divided by: products between tokens of one block
-// of 16 are made pair by pair, those between blocks are split at the border, so a decay of any size (0 too) is exact.
+// Everything is float32: operands, products and sums; products of decays are made in 64 bits and rounded once.  Products between
+// blocks of 16 tokens are split at the border, where nothing is divided by.  Inside a block there are two ways.  Where no channel's
+// decays multiply to less than 2^-60 or more than 2^60 on the way through a block, the writing vectors are divided by what is left of the
+// block's decays and the reading ones multiplied, and a block's pairs are one product: the quotients stay far from float32's ends, so they
+// add two roundings a factor and no more (constant decays of 2^-3.74, 2^-59.8 a block: 1.9 to 2.2 units of 2^-24 of the result where token by
+// token has 1.3 to 1.5).  Elsewhere (a decay of 0, too) a chunk's pairs are made one by one, each decay multiplied in, none divided by
+// (2^-3.76: 1.6 to 2.1 units).
 // A token's sums are taken in another order than token by token and depend on where its chunk begins, so callers that
 // promise the same bits for every cut of a prompt (float32 models) and steps of few tokens keep the other kernel.
 // A chunk's products meet every token of the chunk, and zero times infinity is no number.  So a request with a vector of which
@@ -36,7 +41,8 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __bui
 // number in 32 bits and what that leaves out: a model's constant decay would be off by the same last bit in every chunk),
 // W^ [SC][SC], and with a removal term T probe~ [SC][DK] and -removal~^T [DK][SC].  The matrices lie as the operands that the
 // second kernel loads, 1 KB a [16 x 16] tile: lane (row, quad) has entries 4 quad .. + 3 of a row (in rows
-// the walk, whose loads then touch sixteen half lines each, took 109 us where it takes 95 and, removing, 199 us where 145).
+// the walk, whose loads then touch sixteen half lines each, took 109 us where it took 95 and, removing, 199 us where 145, in its form with
+// four waves; 80 and 122 now).
 template <int DK, bool REMOVE>
 struct ChunkRecord {
     static constexpr int READ = 0, Z = SC * DK, DECAY = 2 * SC * DK, MIX = DECAY + 2 * DK, PROBE = MIX + SC * SC,

@@ -165,3 +165,43 @@ def test_requests_of_few_tokens_take_no_record(lengths):
         assert float((a - b).norm() / b.norm()) <= 16 * UNIT
     short = torch.tensor([n < ops.SCAN_CHUNKS_FROM for n in lengths], device=DEV)
     assert torch.equal(states[1][short], states[0][short])
+
+
+@pytest.mark.parametrize("planes", [5, 3])
+@pytest.mark.parametrize("dk", [64, 128])
+# 16 tokens' decays multiply to 2^-60 at 2^-3.75 a token: just inside, where the pairs of a block are products of vectors scaled by up
+# to 2^60, just outside, where they are made one by one; every channel, one channel, one block, and blocks of both kinds
+@pytest.mark.parametrize("where", ["everywhere", "a channel", "a block"])
+@pytest.mark.parametrize("exponent", [-3.74, -3.76])
+def test_decays_around_the_range(planes, dk, where, exponent):
+    g = torch.Generator().manual_seed(planes + dk)
+    T, heads, dv = 112, 2, 32
+    coef = vectors("by channel", T, heads, dk, g)[0 if planes == 5 else 1].clone()
+    decay = coef.view(planes, T, heads, dk)[0]
+    decay[{"everywhere": slice(None), "a channel": (slice(None), 1, 7), "a block": slice(48, 64)}[where]] = 2.0 ** exponent
+    if planes == 5:     # the probe is the decay times a key, here the removal's
+        coef.view(planes, T, heads, dk)[1] = decay * coef.view(planes, T, heads, dk)[2]
+    v, state = torch.randn(T, heads * dv, generator=g), torch.randn(1, heads, dv, dk, generator=g) * 0.2
+    lists = torch.tensor([0, T], dtype=torch.int32), torch.zeros(1, dtype=torch.int32)
+    want_state, states = state.double(), [state.to(DEV), state.to(DEV)]
+    want = reference_ops.delta_scan(coef, v, want_state, *lists, 1, heads, dk, dv).double()
+    args = (coef.to(DEV), v.to(DEV)), tuple(x.to(DEV) for x in lists)
+    plain = ops.delta_scan(*args[0], states[0], *args[1], 1, heads, dk, dv).cpu().double()
+    got = ops.delta_scan_chunks(*args[0], states[1], *args[1], 1, heads, dk, dv, some_short=False).cpu().double()
+
+    def off(x, y):
+        return float((x - y).norm() / y.norm())
+    print(f"{off(got, want) / UNIT:.2f} {off(plain, want) / UNIT:.2f} units")
+    assert off(got, want) <= max(2 * off(plain, want), 8 * UNIT), "read-outs"
+    assert off(states[1].cpu().double(), want_state) <= max(2 * off(states[0].cpu().double(), want_state), 8 * UNIT), "states"
+    # Token by token, because none may hide behind another: a read-out is a sum of n = dk terms and more of either sign, whose sizes add
+    # up to `reach` (the recurrence over absolute values, what is removed added).  Its partial sums are some reach / sqrt(n) and the
+    # n roundings, half a unit of one each at the most, some sqrt(n) of them: half a unit of reach.  Four times that, or what
+    # the token-by-token kernel shows.
+    size = coef.abs().view(planes, T, heads * dk)
+    if planes == 5:
+        size[2] = -size[2]
+    reach = reference_ops.delta_scan(size, v.abs(), state.abs().double(), *lists, 1, heads, dk, dv).double()
+    for t in range(T):
+        error, beside = (float((x[t] - want[t]).norm()) for x in (got, plain))
+        assert error <= max(4 * beside, 2 * UNIT * float(reach[t].norm())), t
