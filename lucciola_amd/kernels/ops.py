@@ -1352,17 +1352,38 @@ def plan_latent_attention(layout):
              "num_tiles": len(tiles)})
 
 
-def latent_wide_pays(tokens: int, position: int, heads: int, window: int) -> bool:
-    """Whether a portion of ``tokens`` tokens behind ``position`` others is faster head by head (``latent_wide``) than in the
-    latent's space, by what each takes on 256 CUs.  In the latent's space a workgroup of 16 tokens and four heads takes 3 us
-    for 32 rows, a CU holds one, and few tiles share out their rows; head by head a workgroup of 128 tokens of a head takes
-    1.15 us for 64 rows, two a CU, whoever is alone walks all of them, and the keys and values cost 0.52 ns a row and head and four
-    launches more.  (A layer with 16 heads: 2,048 tokens 430 us and 85; behind 2,048 others 830 and 175; 256 tokens behind 4,000
-    others 100 and 125; below some 700 tokens of a fresh prompt the launches weigh more than either.)"""
+def latent_wide_time(tokens: int, position: int, heads: int, window: int) -> float:
+    """us that a portion of ``tokens`` tokens behind ``position`` others takes head by head (``latent_wide``) on 256 CUs: a workgroup
+    of 128 tokens of a head takes 1.15 us for 64 rows, two a CU, whoever is alone walks all of them, the keys and values cost 0.52
+    ns a row and head, and there are four launches more."""
     span = position + tokens if not window else min(position + tokens, window + tokens - 1)
-    latent = -(-tokens // 16) * -(-heads // 4) * -(-span // 32) * 3.0 / 256
-    wide = 20.0 + -(-span // 64) * 1.15 * -(-(-(-tokens // 128) * heads) // 512) + span * heads * 5.2e-4
-    return wide < latent
+    return 20.0 + -(-span // 64) * 1.15 * -(-(-(-tokens // 128) * heads) // 512) + span * heads * 5.2e-4
+
+
+def latent_wide_pays(tokens: int, position: int, heads: int, window: int) -> bool:
+    """Whether a portion alone is faster head by head than in the latent's space, where a workgroup of 16 tokens and four heads
+    takes 3 us for 32 rows, a CU holds one, and few tiles share out their rows.  (A layer with 16 heads: 2,048 tokens 430 us and
+    85; behind 2,048 others 830 and 175; 256 tokens behind 4,000 others 100 and 125; below some 700 tokens of a fresh prompt the
+    launches weigh more than either.)"""
+    span = position + tokens if not window else min(position + tokens, window + tokens - 1)
+    return latent_wide_time(tokens, position, heads, window) < -(-tokens // 16) * -(-heads // 4) * -(-span // 32) * 3.0 / 256
+
+
+def latent_wide_gains(wide_us: float, tiles: np.ndarray, rest: np.ndarray, heads: int, window: int, most: int) -> bool:
+    """Whether a step with ``tiles`` is faster when the portions that would take ``wide_us`` head by head leave it, for a ``rest``
+    that still holds a portion.  One longest tile may set the time of the latent's space, with the portion's work passing beside it
+    (16 heads, a window of 1,024: 1,024 tokens, 30 behind 3,000 others and 64 lone ones 248 us, 275 with the first head by head), and
+    whether it is shared out goes by how many tiles there are (the same beside 16 lone tokens 218 and 191).  A step's time is
+    estimated from its longest share and its work a CU; of 5,859 drawn steps, 4 to 64 heads, whose portions pay alone, 646 were over
+    5 % slower head by head (by up to 61 %), and 32 are with this (by up to 19 %); without a portion in the rest none was.  The gain
+    has to be a tenth of the estimate, because the estimate is off by that much.  31 of 3,894 other steps that it takes are over 5 % slower."""
+    def us(t):
+        stages = -(-(t[:, 3] + t[:, 1] - (np.maximum(0, t[:, 3] - window + 1) if window else 0)) // 32)
+        columns = -(-heads // 4)
+        splits = library().lc_latent_bf16_splits(len(t) * columns, min(most, window) if window else most)
+        longest, shared = -(-int(stages.max()) // splits), int(stages.sum()) * columns / 256
+        return 4.0 * (longest ** 3 + shared ** 3) ** (1 / 3) + (8.0 if splits > 1 else 0.0)
+    return wide_us + us(rest) < 0.9 * us(tiles)
 
 
 # Entries of the keys of a step's requests that attend head by head, and of their values: 512 MB each.
@@ -1383,19 +1404,24 @@ def latent_short_planner(heads: int, window: int):
     Lone tokens are not asked: a row costs them less in the latent's space than its key and value would (a decode step of 64: 52 us
     on the host, 83 when asked one by one)."""
     def plan(layout):
-        wide, rows = [], 0
+        wide, rows, us = [], 0, 0.0
         for r in range(layout.num_requests if layout.num_tokens > layout.num_requests else 0):
             tokens, position = layout.q_start[r + 1] - layout.q_start[r], layout.first_position[r]
             if tokens > 1 and latent_wide_pays(tokens, position, heads, window):
                 visible = -(-(position + tokens - (max(0, position - window + 1) if window else 0)) // 64) * 64
                 if (rows + visible) * heads * 128 <= LATENT_WIDE_ENTRIES:
+                    us += latent_wide_time(tokens, position, heads, window) - (14.0 if wide else 0.0)     # launches that they share
                     wide.append(r)
                     rows += visible
         arrays, info = plan_latent_attention(layout)
         if wide:
-            tiles = arrays["tiles"][~np.isin(arrays["tiles"][:, 2], wide)]
+            every = arrays["tiles"]
+            tiles = every[~np.isin(every[:, 2], wide)]
+            portions = bool((tiles[:, 1] > 1).any())
+            if portions and not latent_wide_gains(us, every, tiles, heads, window, int((every[:, 3] + every[:, 1]).max())):
+                return arrays, dict(info, wide=[])
             arrays = {"tiles": tiles if len(tiles) else np.zeros((1, 4), np.int32)}     # one that no launch reads
-            info = {"any_portion": bool((tiles[:, 1] > 1).any()), "any_lone": bool((tiles[:, 1] == 1).any()), "num_tiles": len(tiles)}
+            info = {"any_portion": portions, "any_lone": bool((tiles[:, 1] == 1).any()), "num_tiles": len(tiles)}
         return arrays, dict(info, wide=wide)
     return ("latent attention of short portions", heads, window), plan
 

@@ -177,6 +177,7 @@ def test_shares_of_portions(monkeypatch, rank, heads, with_sink, wide):
     sink = torch.randn(heads, generator=g).to(DEV) if with_sink else None
     layout = HostLayout(R, T, q_start, first, page, False)
     monkeypatch.setattr(ops, "latent_wide_pays", lambda tokens, position, *a: tokens == 1500)
+    monkeypatch.setattr(ops, "latent_wide_gains", lambda *a: True)
     arrays, info = ops.latent_short_planner(heads, 0)[1](layout)
     assert info["wide"] == wide
     plan = Plan({k: torch.tensor(v, device=DEV) for k, v in arrays.items()}, info)
@@ -234,6 +235,7 @@ def test_a_model_whose_portions_attend_head_by_head(monkeypatch, model):
             fed[name] += n
         steps.append((entries, [name for name in sizes if fed[name] == len(prompts[name])]))
     monkeypatch.setattr(ops, "latent_wide_pays", lambda tokens, position, heads, window: tokens >= 100)
+    monkeypatch.setattr(ops, "latent_wide_gains", lambda *a: True)
     calls, call = [], ops._call
     monkeypatch.setattr(ops, "_call", lambda name, *a: calls.append(name) or call(name, *a))
     got = replay(make_runner(cfg, weights, 16, traces.max_live_tokens(steps, 16) // 16, "bfloat16", DEV), steps)

@@ -47,3 +47,16 @@ def test_lone_tokens_are_not_asked(monkeypatch):
 @pytest.mark.parametrize("position", [0, 31, 2047, 131071, 10 ** 6])
 def test_a_lone_token_is_never_faster_head_by_head(heads, position):
     assert not ops.latent_wide_pays(1, position, heads, 0)
+
+
+# us of a layer that were measured with the first request head by head and with nobody: (tokens, position), times lone tokens
+@pytest.mark.parametrize("heads,window,portions,lone,head_by_head,nobody", [
+    (16, 1024, [(1024, 0), (40, 0), (30, 3000)], (64, 300), 275, 248), (16, 1024, [(1024, 0), (40, 0), (30, 3000)], (16, 300), 191, 218),
+    (16, 0, [(1024, 0), (40, 0), (30, 3000)], (64, 300), 513, 487), (16, 0, [(1024, 0), (40, 0), (30, 3000)], (16, 300), 248, 456),
+    (16, 1024, [(433, 2817), (4, 7378)], (64, 3500), 254, 189), (16, 1024, [(750, 0), (5, 820)], (64, 748), 241, 188),
+    (8, 1024, [(1189, 6156), (195, 2640), (119, 0)], (200, 52), 273, 212),
+    (16, 0, [(2056, 0), (5, 6966)], (0, 0), 272, 1162), (16, 0, [(1481, 0), (13, 5899), (3, 0)], (0, 0), 247, 896),
+    (16, 0, [(2048, 0)], (64, 2000), 285, 605), (16, 0, [(700, 0)], (1, 300), 141, 166)])
+def test_a_step_goes_head_by_head_where_the_whole_of_it_gains(heads, window, portions, lone, head_by_head, nobody):
+    wide = ops.latent_short_planner(heads, window)[1](layout_of(portions + [(1, lone[1])] * lone[0]))[1]["wide"]
+    assert wide == ([0] if head_by_head < nobody else [])
