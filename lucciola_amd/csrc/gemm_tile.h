@@ -65,11 +65,20 @@ __device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
 // else hides a stall.  Per k-step of 16 the wave issues its (BM/64)*(BN/64) products; between
 // them, one at a time, go the LDS reads of the NEXT k-step's operands (ds_read_b128 in inline
 // assembly with explicit waits: the compiler cannot tell the stages apart and would make every
-// load in flight land before any read) and, in a block's first k-step, the global loads of the
-// block TL_STAGES-1 ahead.  In a block's last k-step the wave waits for its own loads of the
-// next block, meets the others at a bare barrier (all waves' loads are then visible, and all
-// have finished reading the stage that the next loads overwrite) and reads the next block's
-// first operands while the rest of its products run.  sched_barrier pins that order.
+// load in flight land before any read) and the global loads.  In a block's last k-step the wave
+// waits for its own loads of the next block and meets the others at a bare barrier, the only one
+// of a block: behind it all waves' loads of the next block are visible, and all waves hold the
+// last operands of this block in registers, so that its stage is free.  From there on the wave
+// reads the next block's first operands and issues, a few products apart, the loads of the block
+// TL_STAGES ahead into the freed stage, on into the next block.  sched_barrier pins that order.
+//
+// The loads are spread because a CU takes them at 64 bytes a clock (58 measured for rows of 128
+// bytes that L2 holds): the 16 loads of a wave of the 256 x 256 tile, four waves at once, are a
+// thousand clocks in which a wave that issues them in a row issues no product.  In a row, behind
+// the barrier or in the first k-step (us; the same sums): 2,048 x 24576 x 4096 with SwiGLU 367,
+// 2,048 x 4096 x 12288 193, 2,048 x 2048 x 2048 26.3; spread: 328, 171 and 22.9 (the matrix cores
+// busy 69 % of the clocks instead of 56, at a clock that the power limit takes from 1.84 to
+// 1.64 GHz; 2.4 without load).
 constexpr int TL_K = 64;
 
 // BM x BN rows of x and of w, TL_STAGES stages, WM x WN waves, each owning (BM / WM) x (BN / WN) of the tile as TM x TN products
@@ -86,7 +95,7 @@ struct TileLoop {
     static constexpr int NM = TM * TN, NR = TM + TN;          // products and operand reads per k-step
     static constexpr int A_STAGE = BM * TL_K * 2, B_STAGE = BN * TL_K * 2;   // bytes
     static constexpr int LDS = S * (A_STAGE + B_STAGE);       // A stages, then B stages, aligned to 1,024
-    static_assert(S >= 2 && (S == 2 ? 2 : S - 1) * LP <= 63, "the load counter holds 63");
+    static_assert(S >= 2, "a stage is loaded while another is read");
     static_assert(LDS <= 160 * 1024, "LDS");
 
     __device__ static __forceinline__ int swz(int row) { return (row >> 1) & 7; }
@@ -111,18 +120,28 @@ struct TileLoop {
             __builtin_amdgcn_global_load_lds((glb_ptr_t)(wg[idx - LPA] + kb * TL_K),
                 (lds_ptr_t)(lds + S * A_STAGE + stage * B_STAGE + ((idx - LPA) * NW + wave) * 1024), 16, 0, 0);
     };
-    // With two stages, a block's loads are issued a block early: in the last k-step of block it,
-    // once every wave has read the last of the stage, block it + 2 goes into it, behind block
-    // it + 1 that is still arriving.  (Issued only after block it + 1 has landed, the loads
-    // would start with nothing in flight: their first data would be a whole latency away, and
-    // the way from L2 into the CU, which bounds these kernels, would stand idle meanwhile.)
-    constexpr bool EARLY = S == 2;
-    constexpr int AHEAD = EARLY ? 2 : S - 1;                  // blocks in flight at the start
+    // Where the loads of a block sit among the products: position 0 is the first product behind the barrier that frees their
+    // stage.  With two stages they have to be back at the next barrier and are issued in the first half; with more they are spread
+    // over the whole block but its end (from a third to the whole of it: within 2 %; two stages and three quarters: 345 us
+    // where 328 stand above).
+    constexpr int BAR = NM / 4;                                // the product after which a block's last k-step syncs
+    constexpr int WIN = KS * NM;                               // products between two barriers
+    constexpr int NA = NM - 1 - BAR;                           // of them in the block that frees the stage
+    constexpr int SPAN = S == 2 ? WIN / 2 : WIN * 7 / 8;
+    static_assert(SPAN >= 1 && SPAN < WIN, "all loads of a block are issued before the next barrier");
+    struct At { static constexpr int of(int l) { return l * SPAN / LP; } };      // load l's position
+    // Tiles of two stages with few products a block are several to a CU and bound by how much is on its way, and issue a whole
+    // block's loads behind a barrier of their own before they wait for the block before it (8,192 rows over 32 matrices of
+    // 2,048 x 2,048 in tiles of 128 x 128: 127 us, 141 spread).
+        constexpr bool EARLY = S == 2 && NM <= 4;
+    constexpr int PA = EARLY ? LP : [] { int n = 0; for (int l = 0; l < LP; ++l) n += l * SPAN / LP < NA; return n; }();   // loads in that block
+    static_assert((S - 1) * LP + PA <= 63, "the load counter holds 63");
 #pragma unroll
-    for (int s = 0; s < AHEAD; ++s)
+    for (int s = 0; s < S; ++s)
         if (s < nk) {
 #pragma unroll
-            for (int i = 0; i < LP; ++i) issue_one(i, s, s);
+            for (int i = 0; i < LP; ++i)
+                if (s < S - 1 || i < PA) issue_one(i, s, s);
         }
 
 #pragma unroll
@@ -169,22 +188,20 @@ struct TileLoop {
         acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0);
     };
 
-    // where the reads and loads sit among the NM products of a k-step
+    // where the reads sit among the NM products of a k-step
     constexpr int QR = (2 * NR + NM - 1) / NM;                 // reads after each product, from the first on
-    constexpr int RS = (NR + QR - 1) / QR;                     // products that the reads take
-    constexpr int QL = NM > RS ? (LP + (NM - RS) - 1) / (NM - RS) : LP;   // loads after each later product
-    constexpr int BAR = NM / 4;                                // the product after which a block's last k-step syncs
     constexpr int QT = NM - BAR - 1 > 0 ? (NR + (NM - BAR - 1) - 1) / (NM - BAR - 1) : NR;
 
-    // block 0 has landed when at most the younger blocks are still in flight
-    if (nk >= AHEAD) wait_vmcnt<(AHEAD - 1) * LP>(); else wait_vmcnt<0>();
+    if (nk >= S) wait_vmcnt<(S - 2) * LP + PA>(); else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
 #pragma unroll
     for (int r = 0; r < NR; ++r) read_one(r, 0, 0, 0);
 
-    int stage = 0, lstage = S - 1;   // the stage of block `it`; the stage that block it+S-1 goes to
-    auto block = [&](int it, auto load_tag) {
-        constexpr bool LOAD = decltype(load_tag)::value;       // block it+S-1 exists and is loaded here
+    int stage = 0, pstage = S - 1;   // the stages of blocks `it` and `it - 1`
+    // FREE: block it + S exists, its first loads go into this block's stage once it is free; REST: block it + S - 1 exists, its other
+    // loads go where block it - 1 was
+    auto block = [&](int it, auto free_tag, auto rest_tag) {
+        constexpr bool FREE = decltype(free_tag)::value, REST = decltype(rest_tag)::value;
         const int nstage = stage + 1 == S ? 0 : stage + 1;
 #pragma unroll
         for (int ks = 0; ks < KS; ++ks) {
@@ -192,64 +209,57 @@ struct TileLoop {
             wait_lgkmcnt<0>();
             tie(cur);
             __builtin_amdgcn_sched_barrier(0);
-            if (ks < KS - 1) {
 #pragma unroll
-                for (int k = 0; k < NM; ++k) {
-                    product(k, cur);
-                    __builtin_amdgcn_sched_barrier(0);
+            for (int k = 0; k < NM; ++k) {
+                product(k, cur);
+                __builtin_amdgcn_sched_barrier(0);
+                if (ks < KS - 1) {
 #pragma unroll
                     for (int r = k * QR; r < (k + 1) * QR; ++r)
                         if (r < NR) read_one(r, stage, ks + 1, nxt);
-                    if (LOAD && !EARLY && ks == 0 && (k >= RS || NM == RS)) {
-                        const int first = NM == RS ? k * QL : (k - RS) * QL;
-#pragma unroll
-                        for (int l = first; l < first + QL; ++l)
-                            if (l < LP) issue_one(l, it + S - 1, lstage);
-                    }
-                    __builtin_amdgcn_sched_barrier(0);
                 }
-            } else {
+                if (REST && (ks < KS - 1 || k <= BAR)) {
 #pragma unroll
-                for (int k = 0; k < NM; ++k) {
-                    product(k, cur);
-                    __builtin_amdgcn_sched_barrier(0);
-                    if (LOAD) {
-                        if (k == BAR && EARLY) {
-                            __builtin_amdgcn_s_barrier();          // nobody reads this stage any more
-#pragma unroll
-                            for (int l = 0; l < LP; ++l) issue_one(l, it + 2, stage);
-                            wait_vmcnt<LP>();                      // block it + 1 has landed
+                    for (int l = PA; l < LP; ++l)
+                        if (At::of(l) - NA == ks * NM + k) issue_one(l, it + S - 1, pstage);
+                }
+                if (ks == KS - 1) {
+                    if (k == BAR && (REST || it + 1 < nk)) {
+                        // block it + 1 has landed (this wave's part, then everybody's), and nobody reads this stage any more
+                        if (EARLY && FREE) {
                             __builtin_amdgcn_s_barrier();
-                        } else if (k == BAR) {
-                            wait_vmcnt<(S - 2) * LP>();
-                            __builtin_amdgcn_s_barrier();
-                        }
-                        if (NM - BAR - 1 > 0) {
 #pragma unroll
-                            for (int r = (k - BAR - 1) * QT; r < (k - BAR) * QT; ++r)
-                                if (k > BAR && r < NR) read_one(r, nstage, 0, nxt);
-                        } else if (k == BAR) {
-#pragma unroll
-                            for (int r = 0; r < NR; ++r) read_one(r, nstage, 0, nxt);
-                        }
-                    } else if (k == BAR) {
-                        if (it + 1 < nk) {
-                            wait_vmcnt<0>();
-                            __builtin_amdgcn_s_barrier();
+                            for (int l = 0; l < LP; ++l) issue_one(l, it + S, stage);
+                            wait_vmcnt<LP>();
+                        } else if (REST) wait_vmcnt<(S - 2) * LP>();
+                        else wait_vmcnt<0>();
+                        __builtin_amdgcn_s_barrier();
+                        if (NM - BAR - 1 == 0) {
 #pragma unroll
                             for (int r = 0; r < NR; ++r) read_one(r, nstage, 0, nxt);
                         }
                     }
-                    __builtin_amdgcn_sched_barrier(0);
+                    if (k > BAR && (REST || it + 1 < nk)) {
+#pragma unroll
+                        for (int r = (k - BAR - 1) * QT; r < (k - BAR) * QT; ++r)
+                            if (r < NR) read_one(r, nstage, 0, nxt);
+                    }
+                    if (FREE && !EARLY && k > BAR) {
+#pragma unroll
+                        for (int l = 0; l < PA; ++l)
+                            if (At::of(l) == k - BAR - 1) issue_one(l, it + S, stage);
+                    }
                 }
+                __builtin_amdgcn_sched_barrier(0);
             }
         }
+        pstage = stage;
         stage = nstage;
-        lstage = lstage + 1 == S ? 0 : lstage + 1;
     };
     int it = 0;
-    for (; it + AHEAD < nk; ++it) block(it, std::true_type{});
-    for (; it < nk; ++it) block(it, std::false_type{});
+    for (; it + S < nk; ++it) block(it, std::true_type{}, std::true_type{});
+    if (it + S - 1 < nk) { block(it, std::false_type{}, std::true_type{}); ++it; }
+    for (; it < nk; ++it) block(it, std::false_type{}, std::false_type{});
 
     }
 };
