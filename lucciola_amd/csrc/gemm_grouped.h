@@ -43,6 +43,7 @@ __device__ __forceinline__ bool find_tile(const GroupedArgs& a, int BM, GroupedT
 // the faster one.
 bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows);
 bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows);
-int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, hipStream_t stream);
+// forced: tests ask for the kernel of even tiles wherever it can run
+int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, bool forced, hipStream_t stream);
 
 }  // namespace lc

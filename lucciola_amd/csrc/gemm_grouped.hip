@@ -402,7 +402,7 @@ LC_API int lc_gemm_grouped(const void* x, int x_dt, long long ldx, long long x_g
     if (whole_pieces(x, x_dt, ldx, x_group, w, w_dt, K) && g_grouped_fast) {
         if (g_grouped_tiled && (out_dt == DT_BF16 || out_dt == DT_F32) && grouped_tiled_takes(a, tile_rows) &&
             (g_grouped_tiled == 1 || grouped_tiled_pays(a, max_tiles, tile_rows)))
-            return launch_grouped_tiled(a, max_tiles, tile_rows, out_dt == DT_BF16, stream);
+            return launch_grouped_tiled(a, max_tiles, tile_rows, out_dt == DT_BF16, g_grouped_tiled == 1, stream);
         if (out_dt == DT_BF16) return launch_grouped_bf16<bf16>(a, max_tiles, tile_rows, stream);
         if (out_dt == DT_F32) return launch_grouped_bf16<float>(a, max_tiles, tile_rows, stream);
     }

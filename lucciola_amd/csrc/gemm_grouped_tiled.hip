@@ -1,11 +1,15 @@
-// The grouped products of gemm_grouped.hip for bfloat16 operands, in two shapes of their own:
+// The grouped products of gemm_grouped.hip for bfloat16 operands, in three shapes of their own:
 //
-//   tiles    many rows a group (prompts): tiles of 64 or 128 rows by 128 columns through the loop of the dense products
-//            (gemm_tile.h): direct loads to LDS, v_mfma_f32_32x32x16_bf16, scheduled by hand.  Bound by the CUs' way from L2,
-//            18 to 23 bytes a clock each.  Two or three workgroups a CU, because a group's K is short (32 blocks) and
-//            a tile's first loads and its stores pass beside another's products: 8,192 rows over 32 matrices of 2,048 x 2,048
-//            take 125 us (through registers in tiles of 128 x 128, as in gemm_grouped.hip: 175), where the tiles of 128 x 256,
-//            which ask L2 for a third less and have a CU to themselves, take 172; 4,096 x 2,048: 278 -> 221 us.
+//   even     experts with many rows (prompts): tiles of 256 columns whose height follows from the group's rows, one workgroup a CU,
+//            through the loop of the dense products (gemm_tile.h): direct loads to LDS, v_mfma_f32_32x32x16_bf16, scheduled by
+//            hand.  8,192 rows over 32 matrices of 2,048 x 2,048 (256 rows each, more or less): 128 us in tiles of 128 x 128,
+//            90 (0.76 PFLOP/s); 6,092 rows 102 and 71; 4,096 x 2,048: 258 and 202.  A third of that is that no tile is mostly
+//            empty, a third that workgroups do not all ask the same memory channels (below), a third that the tile is found with
+//            one trip to memory and stored in whole lines without a test of the epilogue an entry.  What bounds them now is the
+//            start (the matrices come from memory once, 45 to 50 us of it) and end of a tile, some 11 us a round, which nothing
+//            hides, and 1.0 us a block of 64 k at 160 rows, where LDS is read and written at 0.7 of what it can.
+//   tiles    shorter K, fewer columns, products per head: 64 rows by 128 columns through the same loop, four workgroups a CU, because
+//            a tile is short and its first loads and its stores pass beside another's products.
 //   stream   few rows a group (decoding: 16 rows a tile): bound by reading every group's matrix once, so what counts is
 //            how much of it is on its way.  256 rows over 32 matrices of 2,048 x 2,048 (268 MB): 68 -> 51 us (5.3 TB/s); 32 rows,
 //            21 matrices: 51 -> 31; 512 rows, 32 matrices of 4,096 x 2,048: 156 -> 98.
@@ -84,6 +88,174 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_grouped_tiled_kernel(Groupe
                     const int m = m0 + i * 32 + (v >> 2) * 8 + (v & 3), n = c0 + j * 32;
                     if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish(a, gate, m, n, acc[i][j][v]));
                 }
+    }
+}
+
+// Experts with many rows: tiles of 256 columns whose height follows from the group.  A group's rows, in units of 32, are cut into the
+// fewest tiles of at most `most` units and evenly (257 rows are two tiles of 160 rows' room and not three of 128, the last of
+// one row), and `most`, 1 to 8, is what lets the product end first by an estimate: a tile costs its units and two more (its
+// columns of w, its first loads and its stores), and the CUs, which hold a workgroup each, take the tiles in rounds.  Every
+// workgroup works this out by itself from row_start, a lane per candidate and share of the groups, so that the host need not
+// know the routing.
+struct EvenTile {
+    int group, first, end, units, column;      // units 0: there is none
+};
+
+__device__ __forceinline__ int even_tiles(int units, int most) { return units ? (units + most - 1) / most : 0; }
+
+__device__ __forceinline__ EvenTile find_even_tile(const int* row_start, int G, int id, int columns, int room, int cus, int lane) {
+    const int sub = lane >> 3, most = (lane & 7) + 1;
+    int tiles = 0, highest = 0, cost = 0;
+    for (int g = sub; g < G; g += 8) {
+        const int units = (row_start[g + 1] - row_start[g] + 31) / 32, n = even_tiles(units, most), h = n ? (units + n - 1) / n : 0;
+        tiles += n;
+        cost += n * (h + 2);
+        highest = max(highest, h);
+    }
+#pragma unroll
+    for (int d = 8; d < 64; d *= 2) {
+        tiles += __shfl_xor(tiles, d);
+        cost += __shfl_xor(cost, d);
+        highest = max(highest, __shfl_xor(highest, d));
+    }
+    const int rounds = (tiles * columns + cus - 1) / cus;
+    float until = tiles > room ? INFINITY : tiles ? (float)(rounds - 1) * cost / tiles + (highest + 2) : 0.f;     // `most` 8 always has room
+    int best = most;
+#pragma unroll
+    for (int d = 1; d < 8; d *= 2) {
+        const float other = __shfl_xor(until, d);
+        const int its = __shfl_xor(best, d);
+        if (other < until || (other == until && its > best)) { until = other; best = its; }
+    }
+    best = __builtin_amdgcn_readfirstlane(best);
+    tiles = __shfl(tiles, best - 1);
+
+    // An XCD (workgroup id % 8) takes neighbouring tiles, a group's column by column: its L2 then serves one group's rows to all of its
+    // columns and a column of w to all of the group's tiles, and memory is asked for each once.
+    const int items = tiles * columns, per = (items + 7) / 8;
+    const int item = (id & 7) * per + (id >> 3);
+    EvenTile t{0, 0, 0, 0, 0};
+    if ((id >> 3) >= per || item >= items) return t;
+    int before = 0;
+    for (int g0 = 0; g0 < G; g0 += 64) {
+        const int g = g0 + lane;
+        const int from = g < G ? row_start[g] : 0, to = g < G ? row_start[g + 1] : 0;
+        const int units = (to - from + 31) / 32, n = even_tiles(units, best);
+        int upto = n;
+#pragma unroll
+        for (int d = 1; d < 64; d *= 2) {
+            const int v = __shfl_up(upto, d);
+            upto += lane >= d ? v : 0;
+        }
+        const unsigned long long past = __ballot(item < (before + upto) * columns);
+        if (past) {
+            const int at = __builtin_ctzll(past);
+            const int count = __builtin_amdgcn_readfirstlane(__shfl(n, at)), first = __builtin_amdgcn_readfirstlane(__shfl(from, at));
+            const int end = __builtin_amdgcn_readfirstlane(__shfl(to, at)), all = __builtin_amdgcn_readfirstlane(__shfl(units, at));
+            const int place = __builtin_amdgcn_readfirstlane(item - (before + __shfl(upto, at) - count) * columns);
+            t.group = g0 + at;
+            t.units = (all + count - 1) / count;
+            t.column = place / count;
+            t.first = first + (place - t.column * count) * t.units * 32;
+            t.end = min(end, t.first + t.units * 32);
+            return t;
+        }
+        before += __builtin_amdgcn_readfirstlane(__shfl(upto, 63));
+    }
+    return t;
+}
+
+constexpr int EVEN_GROUPS = 4096;
+constexpr int EVEN_N = 256, EVEN_LDS = 3 * (160 + EVEN_N) * TL_K * 2;
+
+// BM rows from tile.first on by the 256 columns of tile.column.
+template <typename TO, int BM, int STAGES, int WM, int WN>
+__device__ __forceinline__ void even_tile(const GroupedArgs& a, const EvenTile& tile, char* lds, int wave, int lane) {
+    typedef TileLoop<BM, EVEN_N, STAGES, WM, WN> Loop;
+    static_assert(Loop::LDS <= EVEN_LDS, "LDS");
+    constexpr int TM = Loop::TM, TN = Loop::TN;
+    const int n0 = tile.column * EVEN_N, N = a.N, K = a.K, blocks = K / TL_K;
+    const bf16* x = reinterpret_cast<const bf16*>(a.x);
+    const bf16* w = reinterpret_cast<const bf16*>(a.w) + (size_t)tile.group * N * K;
+    const bf16* xg[Loop::LPA];
+    const bf16* wg[Loop::LPB];
+#pragma unroll
+    for (int i = 0; i < Loop::LPA; ++i) {
+        const int m = min(tile.first + Loop::row_of(i, wave, lane), tile.end - 1);      // a row behind the tile's end is its last one
+        xg[i] = x + (size_t)(a.gather ? a.gather[m] : m) * a.ldx + Loop::chunk_of(i, wave, lane) * 8;
+    }
+#pragma unroll
+    for (int i = 0; i < Loop::LPB; ++i)
+        wg[i] = w + (size_t)min(n0 + Loop::row_of(i, wave, lane), N - 1) * K + Loop::chunk_of(i, wave, lane) * 8;
+    floatx16 acc[TM][TN];
+    // Rows of w lie 2 K bytes apart, so workgroups that walk k in step ask the same few memory channels at every moment: each group
+    // starts at a block of its own and wraps around.  Its tiles and columns start together, because they share rows in L2.
+    Loop::run(lds, xg, wg, blocks, (int)((unsigned)tile.group * 13u % (unsigned)blocks), wave, lane, acc);
+
+    // 32 rows at a time pass through the wave's part of the ring, so that a lane gets 8 neighbouring columns
+    // (acc[i][j][v]: row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32 of the 32 x 32 tile)
+    constexpr int WIDTH = 32 * TN, STRIDE = WIDTH + 4;
+    static_assert(4 * 32 * STRIDE * 4 <= EVEN_LDS, "a strip of every wave");
+    float* strip = reinterpret_cast<float*>(lds) + wave * 32 * STRIDE;
+    TO* out = reinterpret_cast<TO*>(a.out);
+    const int m0 = tile.first + (wave / WN) * (BM / WM), c0 = n0 + (wave % WN) * WIDTH;
+    constexpr int LANES = WIDTH / 8, ROWS = 64 / LANES;         // lanes a row, rows a pass
+    const int r0 = lane / LANES, c = lane % LANES * 8, n = c0 + c;
+    auto store = [&](int i, int r, auto finish) {
+        const int m = m0 + i * 32 + r;
+        const float4 lo = *reinterpret_cast<const float4*>(strip + r * STRIDE + c);
+        const float4 hi = *reinterpret_cast<const float4*>(strip + r * STRIDE + c + 4);
+        if (m >= tile.end || n >= N) return;                    // N % 8 == 0
+        const float v[8] = {finish(lo.x), finish(lo.y), finish(lo.z), finish(lo.w), finish(hi.x), finish(hi.y), finish(hi.z), finish(hi.w)};
+        TO* to = out + (size_t)m * a.ldo + n;
+        if constexpr (sizeof(TO) == 2) {
+            bf16x8 packed;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) packed[e] = static_cast<bf16>(v[e]);
+            *reinterpret_cast<bf16x8*>(to) = packed;
+        } else {
+            *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
+            *reinterpret_cast<float4*>(to + 4) = make_float4(v[4], v[5], v[6], v[7]);
+        }
+    };
+    __syncthreads();
+#pragma unroll
+    for (int i = 0; i < TM; ++i) {
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v)
+                strip[((v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)) * STRIDE + j * 32 + (lane & 31)] = acc[i][j][v];
+        __builtin_amdgcn_wave_barrier();
+        if (a.epilogue == ACT_NONE) {
+#pragma unroll
+            for (int r = 0; r < 32; r += ROWS) store(i, r0 + r, [](float z) { return z; });
+        } else {
+#pragma unroll 1
+            for (int r = 0; r < 32; r += ROWS) store(i, r0 + r, [&](float z) { return activate(z, a.epilogue); });
+        }
+        __builtin_amdgcn_wave_barrier();
+    }
+}
+
+template <typename TO>
+__global__ __launch_bounds__(256) void gemm_grouped_even_kernel(GroupedArgs a, int columns, int room, int cus) {
+    __shared__ __attribute__((aligned(1024))) char lds[EVEN_LDS];
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    int* row_start = reinterpret_cast<int*>(lds);       // G <= EVEN_GROUPS
+    for (int g = threadIdx.x; g <= a.G; g += 256) row_start[g] = a.row_start[g];
+    __syncthreads();
+    const EvenTile tile = find_even_tile(row_start, a.G, blockIdx.x, columns, room, cus, lane);
+    __syncthreads();
+    switch (tile.units) {
+        case 0: return;
+        case 1: return even_tile<TO, 32, 3, 1, 4>(a, tile, lds, wave, lane);
+        case 2: return even_tile<TO, 64, 3, 1, 4>(a, tile, lds, wave, lane);
+        case 3: return even_tile<TO, 96, 3, 1, 4>(a, tile, lds, wave, lane);
+        case 4: return even_tile<TO, 128, 3, 2, 2>(a, tile, lds, wave, lane);
+        case 5: return even_tile<TO, 160, 3, 1, 4>(a, tile, lds, wave, lane);
+        case 6: return even_tile<TO, 192, 2, 2, 2>(a, tile, lds, wave, lane);
+        default: return even_tile<TO, 256, 2, 2, 2>(a, tile, lds, wave, lane);
     }
 }
 
@@ -171,20 +343,41 @@ __global__ __launch_bounds__(256) void gemm_grouped_stream_kernel(GroupedArgs a)
     }
 }
 
+// Whether gemm_grouped_even_kernel takes these operands: lists, no gates, whole pieces of 8 columns that it stores at once.
+static bool even_takes(const GroupedArgs& a) {
+    const long long columns = (a.N + EVEN_N - 1) / EVEN_N, room = a.M / 128 + a.G;
+    return a.row_start && a.K % TL_K == 0 && a.N % 8 == 0 && a.ldo % 8 == 0 && (uintptr_t)a.out % 16 == 0 && a.G < EVEN_GROUPS &&
+           a.epilogue != ACT_SIGMOID_GATE && a.epilogue != ACT_SIGMOID_GROUP_GATE && room * columns < 1 << 30;
+}
+
+// Lists for tiles of 128 rows have no other kernel here.  With fewer rows an expert (lists for tiles of 64 rows) the tiles of 64 x 128, of
+// which a CU holds four, are as fast or faster where the tile is short or there are few columns (us, 64 x 128 and these: 8,192 rows over
+// 64 matrices of 2,048 x 512 52 and 53, 2,048 rows 34 and 41, over 16 of 256 x 2,048 21 and 25, over 256 of 512 x 512 35 and 55); from 1,024
+// k and 512 columns on these are faster at every size tried (64 matrices of 512 x 2,048, 2,048 rows 41 and 35; 32 of 4,096 x 1,024,
+// 8,192 rows 129 and 113; 32 of 2,048 x 2,048, 520 rows 71 and 51, 3,000 73 and 57, 6,092 103 and 71).
+static bool even_pays(const GroupedArgs& a, int tile_rows) {
+    return tile_rows == 128 || (tile_rows == 64 && a.K >= 1024 && a.N >= 512);
+}
+
 template <typename TO>
-static int grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, hipStream_t stream) {
+static int grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool forced, hipStream_t stream) {
     auto grid = [&](int bm, int bn) {
         return dim3((a.N + bn - 1) / bn, a.row_start ? max_tiles : (a.M + bm - 1) / bm, a.row_start ? 1 : a.G);
     };
-    if (tile_rows == 16) gemm_grouped_stream_kernel<TO><<<grid(16, STREAM_N), 256, 0, stream>>>(a);
-    else if (tile_rows == 64) gemm_grouped_tiled_kernel<TO, 64, 128, 2, 2, 2><<<grid(64, 128), 256, 0, stream>>>(a);
-    else gemm_grouped_tiled_kernel<TO, 128, 128, 2, 4, 1><<<grid(128, 128), 256, 0, stream>>>(a);
+    if (tile_rows == 16) {
+        gemm_grouped_stream_kernel<TO><<<grid(16, STREAM_N), 256, 0, stream>>>(a);
+    } else if (even_takes(a) && (forced || even_pays(a, tile_rows))) {
+        const int columns = (a.N + EVEN_N - 1) / EVEN_N, room = a.M / 128 + a.G;
+        gemm_grouped_even_kernel<TO><<<(room * columns + 7) / 8 * 8, 256, 0, stream>>>(a, columns, room, device_cus());
+    } else {
+        gemm_grouped_tiled_kernel<TO, 64, 128, 2, 2, 2><<<grid(64, 128), 256, 0, stream>>>(a);
+    }
     LC_LAUNCH_CHECK("gemm_grouped_tiled");
     return 0;
 }
 
 bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows) {
-    return tile_rows == 16 ? a.K % STREAM_K == 0 : a.K % TL_K == 0;
+    return tile_rows == 16 ? a.K % STREAM_K == 0 : tile_rows == 128 ? even_takes(a) : a.K % TL_K == 0;
 }
 
 // What these kernels are faster at is a K long enough to fill their rings; a tile of few blocks is mostly its first loads and its
@@ -209,8 +402,9 @@ bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows) {
     return a.K >= 128 && full * full / workgroups >= 32 * short_by * short_by * short_by;
 }
 
-int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, hipStream_t stream) {
-    return out_bf16 ? grouped_tiled<bf16>(a, max_tiles, tile_rows, stream) : grouped_tiled<float>(a, max_tiles, tile_rows, stream);
+int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, bool forced, hipStream_t stream) {
+    return out_bf16 ? grouped_tiled<bf16>(a, max_tiles, tile_rows, forced, stream)
+                    : grouped_tiled<float>(a, max_tiles, tile_rows, forced, stream);
 }
 
 }  // namespace lc

@@ -133,7 +133,7 @@ struct TileLoop {
     // Tiles of two stages with few products a block are several to a CU and bound by how much is on its way, and issue a whole
     // block's loads behind a barrier of their own before they wait for the block before it (8,192 rows over 32 matrices of
     // 2,048 x 2,048 in tiles of 128 x 128: 127 us, 141 spread).
-        constexpr bool EARLY = S == 2 && NM <= 4;
+    constexpr bool EARLY = S == 2 && NM <= 4;
     constexpr int PA = EARLY ? LP : [] { int n = 0; for (int l = 0; l < LP; ++l) n += l * SPAN / LP < NA; return n; }();   // loads in that block
     static_assert((S - 1) * LP + PA <= 63, "the load counter holds 63");
 #pragma unroll

@@ -1565,9 +1565,8 @@ class Routing:
 def _routed_tile(rows: int, experts: int, large_tiles: bool) -> int:
     """Rows of the experts' tiles for ``rows`` (token, choice) pairs: 16 where an expert has that many on average, which reads
     every matrix at the memory's rate (32 experts of 4,096 x 2,048, 16 rows each: 98 us against 119 in tiles of 64, the
-    matrices alone 98); 128 where it has more than one tile of 128 and the caller's products take them, else 64 (2,048 x 2,048
-    matrices, 75, 190 and 256 rows an expert: 75, 104 and 125 us in tiles of 64, 78, 102 and 125 in tiles of 128; 6,144 x 4,096,
-    256 rows: 751 and 644, since the larger tile asks L2 for less)."""
+    matrices alone 98); 128 where it has more than one tile of 128 and the caller's products take them, else 64.  From 1,024 k and
+    512 columns on both mean the same kernel, which cuts an expert's rows by itself."""
     return 16 if rows <= 16 * experts else 128 if large_tiles and rows >= 192 * experts else 64
 
 

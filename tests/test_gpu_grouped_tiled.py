@@ -65,6 +65,32 @@ def test_experts(out, tile, counts, N, K):
         assert off_by(plain, want, K, squared=act is not None) <= 1.0, (gather, act)
 
 
+# Tiles of every height: 64 experts' columns fill the CUs once, so that an expert of up to 256 rows is one tile of the fewest units of 32 that
+# hold it; several tiles an expert; experts without rows and more experts than a wave has lanes; columns that end inside a tile.
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("counts,N,K", [
+    ([32 * h - (7 * e + h) % 32 for e in range(64)], 1024, 64 * blocks) for h, blocks in ((1, 1), (2, 2), (3, 3), (4, 4), (5, 5), (6, 2), (7, 3), (8, 1))] + [
+    ([(e * e * 7) % 301 for e in range(40)], 520, 192), ([0, 1, 0, 31] * 33 + [257], 264, 128), ([0] * 70 + [900], 8, 256), ([1], 256, 64)])
+def test_even_tiles(out, counts, N, K):
+    g = torch.Generator().manual_seed(len(counts) + N + K)
+    E, rows = len(counts), sum(counts)
+    expert = torch.cat([torch.full((n,), e, dtype=torch.int32) for e, n in enumerate(counts)])
+    ids = expert[torch.randperm(rows, generator=g)].to(DEV)[:, None].contiguous()
+    lists = torch.empty(2 * (E + 1) + 2 * rows, dtype=torch.int32, device=DEV)
+    starts, tiles = lists[:E + 1], lists[E + 1:2 * (E + 1)]
+    token, entry = lists[2 * (E + 1):2 * (E + 1) + rows], lists[2 * (E + 1) + rows:]
+    ops._call("lc_moe_lists", ops._ptr(ids), rows, 1, E, 64, ops._ptr(starts), ops._ptr(tiles), ops._ptr(token), ops._ptr(entry),
+              ops._stream())
+    routing = ops.Routing(ids, torch.ones(rows, 1, device=DEV), starts, tiles, token, entry, E, 64, rows // 64 + E)
+    x = torch.randn(rows, K, generator=g).bfloat16().to(DEV)
+    w = torch.randn(E, N, K, generator=g).bfloat16().to(DEV)
+    for gather, act in ((True, "relu_squared"), (False, None)):
+        got = switched(1, lambda: ops.moe_experts(x, w, routing, out, activation=act, gather=gather))
+        src = x[token.long()] if gather else x
+        want = torch.cat([src[starts[e]:starts[e + 1]].float() @ w[e].float().T for e in range(E)])
+        assert off_by(got, want, K, squared=act is not None) <= 1.0, (gather, act)
+
+
 @pytest.mark.parametrize("rows,G,N,K,gap", [(1, 3, 128, 128, 0), (16, 2, 65, 256, 8), (17, 4, 512, 128, 64), (64, 3, 128, 512, 0),
                                             (65, 2, 33, 64, 8), (200, 5, 130, 192, 0)])
 def test_heads(rows, G, N, K, gap):
