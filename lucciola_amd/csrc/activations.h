@@ -24,6 +24,13 @@ __device__ __forceinline__ float activate(float z, int kind) {
     return z;
 }
 
+// The tanh form for results that are rounded to bfloat16: (1 + tanh y) / 2 = 1 / (1 + e^-2y), which loses nothing where tanh is next to -1,
+// with the hardware's exp and reciprocal (a unit in the last place each).
+__device__ __forceinline__ float gelu_tanh_fast(float z) {
+    const float inner = 0.7978845608028654f * fmaf(0.044715f * z, z * z, z);
+    return z * __builtin_amdgcn_rcpf(1.f + __expf(-2.f * inner));
+}
+
 __device__ __forceinline__ float sigmoid(float z) { return 1.f / (1.f + expf(-z)); }
 
 // xIELU with its two numbers already through softplus: z > 0: a z^2 + z/2;  z <= 0: b (e^z - 1 - z) + z/2

@@ -39,11 +39,22 @@ __device__ __forceinline__ bool find_tile(const GroupedArgs& a, int BM, GroupedT
     return true;
 }
 
+// What a gated expert makes of its first product's sums (gate rows of w, then as many up rows): act(gate) * up, both first times the
+// weight of the row's (token, choice) where weights are given.
+struct GroupedGate {
+    const float* weights; const int* entry_row;     // [tokens * top]: the choice's weight, the choice's sorted row; null: no weights
+    int top;
+    int kind;                                       // 0: silu, 1: gelu (tanh form)
+};
+
 // Whether gemm_grouped_tiled.hip has a kernel for these bfloat16 operands (whole, aligned 16-byte pieces) and lists, and whether it is
 // the faster one.
 bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows);
 bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows);
 // forced: tests ask for the kernel of even tiles wherever it can run
 int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, bool forced, hipStream_t stream);
+
+bool grouped_gates(const GroupedArgs& a, int tile_rows);
+int launch_grouped_gated(const GroupedArgs& a, const GroupedGate& gate, hipStream_t stream);
 
 }  // namespace lc

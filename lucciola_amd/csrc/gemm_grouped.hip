@@ -421,3 +421,27 @@ LC_API int lc_gemm_grouped(const void* x, int x_dt, long long ldx, long long x_g
     }
     return 0;
 }
+
+// The first product of gated experts with act(gate) * up in its epilogue: w [G, 2 I, K] holds gate rows, then up rows.
+static GroupedArgs gated_args(const void* x, const void* w, void* out, int M, int I, int K, int G, const int* gather, const int* row_start) {
+    return GroupedArgs{x, K, 0, w, out, I, 0, M, 2 * I, K, G, gather, row_start, row_start, ACT_NONE, nullptr, 0, 0, true};
+}
+
+// Whether lc_gemm_grouped_gated takes these operands, and is the faster way: 1 or 0.
+LC_API int lc_gemm_grouped_gates(const void* x, int x_dt, const void* w, int w_dt, int M, int I, int K, int G, int tile_rows) {
+    static const int listed = 0;
+    if (!g_grouped_fast || !g_grouped_tiled || M <= 0 || I <= 0 || K <= 0 || G <= 0 || !whole_pieces(x, x_dt, K, 0, w, w_dt, K)) return 0;
+    return grouped_gates(gated_args(x, w, nullptr, M, I, K, G, nullptr, &listed), tile_rows) ? 1 : 0;
+}
+
+// x, w, out: bfloat16, out [M, I] (16-byte aligned); gather: a sorted row's token; weights, entry_row [tokens * top] or both null;
+// kind 0: silu, 1: gelu (tanh form)
+LC_API int lc_gemm_grouped_gated(const void* x, const void* w, void* out, int M, int I, int K, int G, const int* gather,
+                                 const int* row_start, int tile_rows, const float* weights, const int* entry_row, int top, int kind,
+                                 hipStream_t stream) {
+    LC_CHECK(x && w && out && gather && row_start, "gated grouped product: null pointer");
+    LC_CHECK((weights == nullptr) == (entry_row == nullptr) && top > 0 && (kind == 0 || kind == 1), "gated grouped product: bad arguments");
+    LC_CHECK((uintptr_t)out % 16 == 0 && lc_gemm_grouped_gates(x, DT_BF16, w, DT_BF16, M, I, K, G, tile_rows),
+             "gated grouped product: %d rows over %d matrices of 2 x %d x %d are not its case", M, G, I, K);
+    return launch_grouped_gated(gated_args(x, w, out, M, I, K, G, gather, row_start), GroupedGate{weights, entry_row, top, kind}, stream);
+}

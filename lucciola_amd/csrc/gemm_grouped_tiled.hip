@@ -168,9 +168,12 @@ __device__ __forceinline__ EvenTile find_even_tile(const int* row_start, int G, 
 constexpr int EVEN_GROUPS = 4096;
 constexpr int EVEN_N = 256, EVEN_LDS = 3 * (160 + EVEN_N) * TL_K * 2;
 
-// BM rows from tile.first on by the 256 columns of tile.column.
-template <typename TO, int BM, int STAGES, int WM, int WN>
-__device__ __forceinline__ void even_tile(const GroupedArgs& a, const EvenTile& tile, char* lds, int wave, int lane) {
+// BM rows from tile.first on by the 256 columns of tile.column.  GATED: these are 128 gate and the 128 up columns that belong to them,
+// 32 of each in turn, so that a wave has both of a pair, and 128 columns are stored: 8,192 rows by 4,096 columns would be written
+// and read again by a kernel of 49 us (2,048 columns stored, K of 2,048, four choices of 32 weighed: 198 + 49 -> 209 us).
+template <typename TO, bool GATED, int BM, int STAGES, int WM, int WN>
+__device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGate& gate, const EvenTile& tile, char* lds,
+                                          const float* row_weight, int wave, int lane) {
     typedef TileLoop<BM, EVEN_N, STAGES, WM, WN> Loop;
     static_assert(Loop::LDS <= EVEN_LDS, "LDS");
     constexpr int TM = Loop::TM, TN = Loop::TN;
@@ -185,8 +188,11 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const EvenTile& 
         xg[i] = x + (size_t)(a.gather ? a.gather[m] : m) * a.ldx + Loop::chunk_of(i, wave, lane) * 8;
     }
 #pragma unroll
-    for (int i = 0; i < Loop::LPB; ++i)
-        wg[i] = w + (size_t)min(n0 + Loop::row_of(i, wave, lane), N - 1) * K + Loop::chunk_of(i, wave, lane) * 8;
+    for (int i = 0; i < Loop::LPB; ++i) {
+        const int r = Loop::row_of(i, wave, lane);
+        const int n = GATED ? min(n0 / 2 + (r >> 6) * 32 + (r & 31), N / 2 - 1) + ((r >> 5) & 1) * (N / 2) : min(n0 + r, N - 1);
+        wg[i] = w + (size_t)n * K + Loop::chunk_of(i, wave, lane) * 8;
+    }
     floatx16 acc[TM][TN];
     // Rows of w lie 2 K bytes apart, so workgroups that walk k in step ask the same few memory channels at every moment: each group
     // starts at a block of its own and wraps around.  Its tiles and columns start together, because they share rows in L2.
@@ -197,16 +203,26 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const EvenTile& 
     constexpr int WIDTH = 32 * TN, STRIDE = WIDTH + 4;
     static_assert(4 * 32 * STRIDE * 4 <= EVEN_LDS, "a strip of every wave");
     float* strip = reinterpret_cast<float*>(lds) + wave * 32 * STRIDE;
+    constexpr int OUT = GATED ? WIDTH / 2 : WIDTH, LANES = OUT / 8, ROWS = 64 / LANES;      // stored columns, lanes a row, rows a pass
     TO* out = reinterpret_cast<TO*>(a.out);
-    const int m0 = tile.first + (wave / WN) * (BM / WM), c0 = n0 + (wave % WN) * WIDTH;
-    constexpr int LANES = WIDTH / 8, ROWS = 64 / LANES;         // lanes a row, rows a pass
-    const int r0 = lane / LANES, c = lane % LANES * 8, n = c0 + c;
+    const int top_row = (wave / WN) * (BM / WM), columns = GATED ? N / 2 : N;
+    const int r0 = lane / LANES, c = lane % LANES * 8, n = (GATED ? n0 / 2 : n0) + (wave % WN) * OUT + c;
+    const int place = GATED ? c / 32 * 64 + c % 32 : c;         // in the strip; GATED: the up entries stand 32 behind
+    // finish: a sum (GATED: a gate's and an up column's) to the stored entry
     auto store = [&](int i, int r, auto finish) {
-        const int m = m0 + i * 32 + r;
-        const float4 lo = *reinterpret_cast<const float4*>(strip + r * STRIDE + c);
-        const float4 hi = *reinterpret_cast<const float4*>(strip + r * STRIDE + c + 4);
-        if (m >= tile.end || n >= N) return;                    // N % 8 == 0
-        const float v[8] = {finish(lo.x), finish(lo.y), finish(lo.z), finish(lo.w), finish(hi.x), finish(hi.y), finish(hi.z), finish(hi.w)};
+        const int m = tile.first + top_row + i * 32 + r;
+        const float* from = strip + r * STRIDE + place;
+        float v[8], u[8];
+        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(from);
+        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(from + 4);
+        if (GATED) {
+            *reinterpret_cast<float4*>(u) = *reinterpret_cast<const float4*>(from + 32);
+            *reinterpret_cast<float4*>(u + 4) = *reinterpret_cast<const float4*>(from + 36);
+        }
+        if (m >= tile.end || n >= columns) return;              // columns % 8 == 0
+        const float weight = GATED && gate.weights ? row_weight[top_row + i * 32 + r] : 1.f;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] = GATED ? finish(weight * v[e], weight * u[e]) : finish(v[e], 0.f);
         TO* to = out + (size_t)m * a.ldo + n;
         if constexpr (sizeof(TO) == 2) {
             bf16x8 packed;
@@ -218,6 +234,30 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const EvenTile& 
             *reinterpret_cast<float4*>(to + 4) = make_float4(v[4], v[5], v[6], v[7]);
         }
     };
+    // one test of the epilogue for 32 rows (one an entry cost 10 to 30 us of a product of 8,192 rows); the long forms stay rolled
+    auto finish = [&](int i) {
+        auto rolled = [&](auto f) {
+#pragma unroll 1
+            for (int r = 0; r < 32; r += ROWS) store(i, r0 + r, f);
+        };
+        auto unrolled = [&](auto f) {
+#pragma unroll
+            for (int r = 0; r < 32; r += ROWS) store(i, r0 + r, f);
+        };
+        if constexpr (GATED) {
+            if (gate.kind == 0) unrolled([](float g, float u) { return gated_f(g, u, kSilu); });
+            else unrolled([](float g, float u) { return gelu_tanh_fast(g) * u; });
+        } else {
+            switch (a.epilogue) {
+                case ACT_NONE: unrolled([](float z, float) { return z; }); break;
+                case ACT_RELU_SQUARED: unrolled([](float z, float) { return activate(z, ACT_RELU_SQUARED); }); break;
+                case ACT_GELU_ERF: rolled([](float z, float) { return activate(z, ACT_GELU_ERF); }); break;
+                default:
+                    if constexpr (sizeof(TO) == 2) unrolled([](float z, float) { return gelu_tanh_fast(z); });
+                    else rolled([](float z, float) { return activate(z, ACT_GELU_TANH); });
+            }
+        }
+    };
     __syncthreads();
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
@@ -227,35 +267,35 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const EvenTile& 
             for (int v = 0; v < 16; ++v)
                 strip[((v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)) * STRIDE + j * 32 + (lane & 31)] = acc[i][j][v];
         __builtin_amdgcn_wave_barrier();
-        if (a.epilogue == ACT_NONE) {
-#pragma unroll
-            for (int r = 0; r < 32; r += ROWS) store(i, r0 + r, [](float z) { return z; });
-        } else {
-#pragma unroll 1
-            for (int r = 0; r < 32; r += ROWS) store(i, r0 + r, [&](float z) { return activate(z, a.epilogue); });
-        }
+        finish(i);
         __builtin_amdgcn_wave_barrier();
     }
 }
 
-template <typename TO>
-__global__ __launch_bounds__(256) void gemm_grouped_even_kernel(GroupedArgs a, int columns, int room, int cus) {
+template <typename TO, bool GATED>
+__global__ __launch_bounds__(256) void gemm_grouped_even_kernel(GroupedArgs a, GroupedGate gate, int columns, int room, int cus) {
     __shared__ __attribute__((aligned(1024))) char lds[EVEN_LDS];
+    __shared__ float row_weight[GATED ? 256 : 1];
     const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    int* row_start = reinterpret_cast<int*>(lds);       // G <= EVEN_GROUPS
+    int* row_start = reinterpret_cast<int*>(lds);       // G < EVEN_GROUPS
     for (int g = threadIdx.x; g <= a.G; g += 256) row_start[g] = a.row_start[g];
     __syncthreads();
     const EvenTile tile = find_even_tile(row_start, a.G, blockIdx.x, columns, room, cus, lane);
+    if (GATED && gate.weights && tile.first + (int)threadIdx.x < tile.end) {
+        const int m = tile.first + threadIdx.x, token = a.gather[m];        // one of the token's choices is row m
+        for (int k = 0; k < gate.top; ++k)
+            if (gate.entry_row[(size_t)token * gate.top + k] == m) row_weight[threadIdx.x] = gate.weights[(size_t)token * gate.top + k];
+    }
     __syncthreads();
     switch (tile.units) {
         case 0: return;
-        case 1: return even_tile<TO, 32, 3, 1, 4>(a, tile, lds, wave, lane);
-        case 2: return even_tile<TO, 64, 3, 1, 4>(a, tile, lds, wave, lane);
-        case 3: return even_tile<TO, 96, 3, 1, 4>(a, tile, lds, wave, lane);
-        case 4: return even_tile<TO, 128, 3, 2, 2>(a, tile, lds, wave, lane);
-        case 5: return even_tile<TO, 160, 3, 1, 4>(a, tile, lds, wave, lane);
-        case 6: return even_tile<TO, 192, 2, 2, 2>(a, tile, lds, wave, lane);
-        default: return even_tile<TO, 256, 2, 2, 2>(a, tile, lds, wave, lane);
+        case 1: return even_tile<TO, GATED, 32, 3, 1, 4>(a, gate, tile, lds, row_weight, wave, lane);
+        case 2: return even_tile<TO, GATED, 64, 3, 1, 4>(a, gate, tile, lds, row_weight, wave, lane);
+        case 3: return even_tile<TO, GATED, 96, 3, 1, 4>(a, gate, tile, lds, row_weight, wave, lane);
+        case 4: return even_tile<TO, GATED, 128, 3, 2, 2>(a, gate, tile, lds, row_weight, wave, lane);
+        case 5: return even_tile<TO, GATED, 160, 3, 1, 4>(a, gate, tile, lds, row_weight, wave, lane);
+        case 6: return even_tile<TO, GATED, 192, 2, 2, 2>(a, gate, tile, lds, row_weight, wave, lane);
+        default: return even_tile<TO, GATED, 256, 2, 2, 2>(a, gate, tile, lds, row_weight, wave, lane);
     }
 }
 
@@ -359,6 +399,12 @@ static bool even_pays(const GroupedArgs& a, int tile_rows) {
     return tile_rows == 128 || (tile_rows == 64 && a.K >= 1024 && a.N >= 512);
 }
 
+template <typename TO, bool GATED>
+static void launch_even(const GroupedArgs& a, const GroupedGate& gate, hipStream_t stream) {
+    const int columns = (a.N + EVEN_N - 1) / EVEN_N, room = a.M / 128 + a.G;
+    gemm_grouped_even_kernel<TO, GATED><<<(room * columns + 7) / 8 * 8, 256, 0, stream>>>(a, gate, columns, room, device_cus());
+}
+
 template <typename TO>
 static int grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool forced, hipStream_t stream) {
     auto grid = [&](int bm, int bn) {
@@ -367,8 +413,7 @@ static int grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, boo
     if (tile_rows == 16) {
         gemm_grouped_stream_kernel<TO><<<grid(16, STREAM_N), 256, 0, stream>>>(a);
     } else if (even_takes(a) && (forced || even_pays(a, tile_rows))) {
-        const int columns = (a.N + EVEN_N - 1) / EVEN_N, room = a.M / 128 + a.G;
-        gemm_grouped_even_kernel<TO><<<(room * columns + 7) / 8 * 8, 256, 0, stream>>>(a, columns, room, device_cus());
+        launch_even<TO, false>(a, GroupedGate{}, stream);
     } else {
         gemm_grouped_tiled_kernel<TO, 64, 128, 2, 2, 2><<<grid(64, 128), 256, 0, stream>>>(a);
     }
@@ -405,6 +450,17 @@ bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows) {
 int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, bool forced, hipStream_t stream) {
     return out_bf16 ? grouped_tiled<bf16>(a, max_tiles, tile_rows, forced, stream)
                     : grouped_tiled<float>(a, max_tiles, tile_rows, forced, stream);
+}
+
+// a.N: gate and up columns together
+bool grouped_gates(const GroupedArgs& a, int tile_rows) {
+    return tile_rows != 16 && a.N % 16 == 0 && even_takes(a) && even_pays(a, tile_rows) && grouped_tiled_pays(a, a.M / tile_rows + a.G, tile_rows);
+}
+
+int launch_grouped_gated(const GroupedArgs& a, const GroupedGate& gate, hipStream_t stream) {
+    launch_even<bf16, true>(a, gate, stream);
+    LC_LAUNCH_CHECK("gemm_grouped_gated");
+    return 0;
 }
 
 }  // namespace lc

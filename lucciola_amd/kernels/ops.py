@@ -78,6 +78,8 @@ _SIGNATURES = {
     "lc_token_shift": "pippppppiip",
     "lc_rms_shift": "ppipffppppppiiip",
     "lc_gemm_grouped": "piqqpipiqqiiiipppiiipqqp",
+    "lc_gemm_grouped_gates": "pipiiiiii",
+    "lc_gemm_grouped_gated": "pppiiiippippiip",
     "lc_gemm_grouped_fast": "i",
     "lc_gemm_grouped_tiled": "i",
     "lc_gemm_grouped_streams": "piqqpii",
@@ -1646,6 +1648,27 @@ def moe_experts(x: torch.Tensor, w: torch.Tensor, routing: Routing, out_dtype: t
               routing.max_tiles, routing.tile, _EPILOGUES[activation] if activation else 0,
               None, 0, 0, _stream())
     return out
+
+
+def moe_experts_gated(x: torch.Tensor, w: torch.Tensor, routing: Routing, kind: str, weighted: bool, out_dtype: torch.dtype) -> torch.Tensor:
+    """The first product of gated experts and what follows it: sorted row m, of expert e and token t, becomes
+    ``act(x[t] . gate[e]^T) * (x[t] . up[e]^T)`` with ``w`` [E, 2 I, K], gate rows first; ``weighted``: both factors first times
+    the weight of the row's (token, choice) pair.  -> [T top, I]"""
+    if x.is_cuda and out_dtype == torch.bfloat16:
+        _need(x, "moe_experts_gated x", None, 2)
+        _need(w, "moe_experts_gated w", None, 3)
+        E, N, K = w.shape
+        rows = routing.sorted_token.shape[0]
+        if E != routing.experts or x.shape[1] != K or N % 2:
+            raise KernelError(f"moe_experts_gated: x {tuple(x.shape)} and w {tuple(w.shape)} do not fit the routing")
+        if library().lc_gemm_grouped_gates(_ptr(x), _dt(x), _ptr(w), _dt(w), rows, N // 2, K, E, routing.tile):
+            out = torch.empty((rows, N // 2), dtype=out_dtype, device=x.device)
+            _call("lc_gemm_grouped_gated", _ptr(x), _ptr(w), _ptr(out), rows, N // 2, K, E, _ptr(routing.sorted_token),
+                  _ptr(routing.row_start), routing.tile, _ptr(routing.weights if weighted else None),
+                  _ptr(routing.entry_row if weighted else None), routing.ids.shape[1], GATE_ACTIVATIONS[kind], _stream())
+            return out
+    both = moe_experts(x, w, routing, out_dtype, gather=True)
+    return gated_activation_weighted(both, kind, routing) if weighted else gated_activation(both, kind)
 
 
 def moe_combine(y: torch.Tensor, routing: Routing, out_dtype: torch.dtype) -> torch.Tensor:

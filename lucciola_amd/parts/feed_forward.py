@@ -287,11 +287,7 @@ class RoutedGatedMLP(Part):
             routing = ops.moe_route_sigmoid(logits, self.top, large_tiles=self.large_tiles)
         else:
             routing = ops.moe_route_logits(logits, self.E, self.top, self.bias, large_tiles=self.large_tiles)
-        both = ops.moe_experts(x, self.gate_up, routing, self.dtype, gather=True)
-        if self.weigh == "input":
-            hidden = ops.gated_activation_weighted(both, self.activation, routing)
-        else:
-            hidden = ops.gated_activation(both, self.activation)
+        hidden = ops.moe_experts_gated(x, self.gate_up, routing, self.activation, self.weigh == "input", self.dtype)
         y = ops.moe_experts(hidden, self.down, routing, torch.float32)
         weighted = self.weigh == "output"
         if self.shared is None:

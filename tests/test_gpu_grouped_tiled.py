@@ -91,6 +91,32 @@ def test_even_tiles(out, counts, N, K):
         assert off_by(got, want, K, squared=act is not None) <= 1.0, (gather, act)
 
 
+# act(gate) * up formed where the sums are: tokens of several choices, experts without rows, columns that end inside a tile.  An error of the
+# sums (off_by's bound) reaches the result through both factors, whose slopes are at most 1.13 |up| and |act(gate)| <= |gate|, and the weight.
+@pytest.mark.parametrize("tokens,E,top,I,K", [(700, 8, 2, 264, 1024), (300, 40, 3, 1000, 1088), (1100, 3, 3, 256, 1024)])
+@pytest.mark.parametrize("kind", ["silu", "gelu_tanh"])
+@pytest.mark.parametrize("weighted", [False, True])
+def test_gated_tiles(tokens, E, top, I, K, kind, weighted):
+    g = torch.Generator().manual_seed(tokens + I + K)
+    logits = (torch.randn(tokens, E, generator=g) * 2).to(DEV)
+    routing = ops.moe_route(logits, top, True, large_tiles=True)
+    x = torch.randn(tokens, K, generator=g).bfloat16().to(DEV)
+    w = (torch.randn(E, 2 * I, K, generator=g) * K ** -0.5).bfloat16().to(DEV)
+    assert ops.library().lc_gemm_grouped_gates(ops._ptr(x), ops._dt(x), ops._ptr(w), ops._dt(w), tokens * top, I, K, E, routing.tile) == 1
+    got = ops.moe_experts_gated(x, w, routing, kind, weighted, torch.bfloat16)
+    token, starts = routing.sorted_token.long(), routing.row_start.tolist()
+    both = torch.cat([x[token[starts[e]:starts[e + 1]]].double() @ w[e].double().T for e in range(E)])
+    if weighted:
+        weight = torch.empty(tokens * top, dtype=torch.float64, device=DEV)
+        weight[routing.entry_row.long()] = routing.weights.double().reshape(-1)
+        both = both * weight[:, None]
+    gate, up = both[:, :I], both[:, I:]
+    act = torch.nn.functional.silu(gate) if kind == "silu" else torch.nn.functional.gelu(gate, approximate="tanh")
+    want = act * up
+    allowed = K * 2.0 ** -24 * (1.13 * up.abs() + gate.abs()) + want.abs() * 2.0 ** -8 + 1e-30
+    assert float(((got.double() - want).abs() / allowed).max()) <= 1.0
+
+
 @pytest.mark.parametrize("rows,G,N,K,gap", [(1, 3, 128, 128, 0), (16, 2, 65, 256, 8), (17, 4, 512, 128, 64), (64, 3, 128, 512, 0),
                                             (65, 2, 33, 64, 8), (200, 5, 130, 192, 0)])
 def test_heads(rows, G, N, K, gap):
