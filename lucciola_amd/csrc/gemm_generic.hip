@@ -14,12 +14,16 @@
 // them in the same order: a row's result has the same bits whether it is computed alone or
 // among thousands.
 //
+// float32 x by bfloat16 w in whole steps of 32 k has kernels of its own, twice as fast (gemm_split.hip); this entry's workspace and the sum
+// of shared chunks serve both.
+//
 // Bound by the matrix instruction: 143 TFLOP/s from registers alone on this card.  What kept the first form of the loop
 // at 88 (2,048 x 4,096 x 1,024, bfloat16 w, 195 us) was what stood between the products: loads behind a test of k each, whose rows
 // were set to zero right behind them, so that each waited for its own trip; LDS writes four to a bank; and all of a stage's LDS work
 // in one heap, in which the matrix core had nothing to do.  Now 156 us (110).  566 rows: N 6,144, K 1,024 110 -> 79 us, N 1,024, K 3,072
 // 61 -> 46, N 151,936 2,272 -> 1,728; 8 rows, N 6,144 13.6 -> 9.0.
 #include "common.h"
+#include "gemm_split.h"
 
 #include <type_traits>
 
@@ -260,6 +264,8 @@ static int chunks_per_workgroup(int M, int N, int K) {
     return (int)((chunks + shares - 1) / shares);
 }
 
+static thread_local bool g_generic_plain = false;     // tests: float32 x by bfloat16 w here too
+
 template <typename TX, typename TW, typename TO>
 static int launch_generic(const void* x, const void* w, void* out, int M, int N, int K, float* workspace,
                           hipStream_t stream) {
@@ -294,8 +300,15 @@ static int launch_generic(const void* x, const void* w, void* out, int M, int N,
         else if (part) launch(Tile{}, Tile{}, two, is_whole, std::true_type{});
         else launch(Tile{}, Tile{}, two, is_whole, std::false_type{});
     };
-    if (whole) with_shape(std::true_type{});
-    else with_shape(std::false_type{});
+    bool split = false;
+    if constexpr (std::is_same_v<TX, float> && std::is_same_v<TW, bf16> && std::is_same_v<TO, float>) {
+        split = !g_generic_plain && gemm_split_takes(K);
+        if (split) launch_gemm_split((const float*)x, (const bf16*)w, (float*)out, M, N, K, part, per, shares, stream);
+    }
+    if (!split) {
+        if (whole) with_shape(std::true_type{});
+        else with_shape(std::false_type{});
+    }
     LC_LAUNCH_CHECK("gemm_generic");
     if (per > 0) {
         const size_t MN = (size_t)M * N;
@@ -311,6 +324,14 @@ static int launch_generic(const void* x, const void* w, void* out, int M, int N,
 }  // namespace lc
 
 using namespace lc;
+
+// Tests: whether float32 x by bfloat16 w stays with the float32 instruction (1) or is cut in three (0, the default).  Returns the setting
+// before.
+LC_API int lc_gemm_generic_plain(int on) {
+    const int before = g_generic_plain ? 1 : 0;
+    if (on >= 0) g_generic_plain = on != 0;
+    return before;
+}
 
 // float32 words of workspace that lc_gemm_generic needs for these sizes (0: none)
 LC_API long long lc_gemm_generic_workspace(int M, int N, int K) {

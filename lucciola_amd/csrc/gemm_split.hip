@@ -1,0 +1,326 @@
+// out[M, N] = x[M, K] . w[N, K]^T for float32 x and bfloat16 w as a true 32-bit product on the bfloat16 matrix instruction: a float32
+// number is the sum of three bfloat16 numbers, cut off after 8 bits each (24 in all, so nothing is left over), the product of two
+// bfloat16 numbers is exact in float32, and v_mfma_f32_32x32x16_bf16 adds in float32.  Three such products cost 3/16 of what
+// v_mfma_f32_16x16x4_f32 takes for the same sums (gemm_generic.hip, which serves float32 w and a K that is not whole).
+//
+// The order of the additions is a function of the output element alone: K goes in steps of 16, the smallest third of x first, in
+// chunks of 256 that are summed from zero and added one after the other; with few tiles the chunks are shared out over workgroups
+// that leave their sums in a workspace, and a second kernel adds them in the same order.  A row has the same bits alone and among
+// thousands.
+//
+// us, gemm_generic.hip and these (weights of several products in turn): 566 rows, 6,144 x 1,024 77 and 38, 1,024 x 3,072 45 and 31, 151,936 x
+// 1,024 1,541 and 878; 2,048 rows, 24,576 x 4,096 3,025 and 1,627 (253 TFLOP/s, 0.76 of 10^15 products a second); 64 rows, 24,576 x 4,096 146
+// and 99; 8 rows 78 and 56 (bound by w: 201 MB); 1 row, 6,144 x 1,024 17 and 13.  Errors against 64 bits 2.9e-7 and 1.7e-7, because
+// 16 products are added at a time.  What bounds the tiles is the vector unit, which cuts x once for every 64 columns (5.5
+// instructions an entry), and LDS, where the parts are written and read; larger tiles of w need more registers than there
+// are (128 x 128 spills), x in the operands' layout past LDS is cut by every wave (566 rows, 6,144 x 1,024 85 us in tiles of 64 x 64), and
+// blocks of 64 k or loads two blocks ahead are slower (64 and 63).
+//
+// x is cut on its way from registers to LDS.  Infinite entries have no such parts (inf - inf), and three parts of x times an
+// infinite w are not x times it; both give NaN, and a chunk's sum that is NaN is made again from x and w as they are.
+#include "common.h"
+
+#include "gemm_split.h"
+#include "gemm_tile.h"
+
+namespace lc {
+
+constexpr int GS_CHUNK = 256;
+
+// Eight neighbouring entries of x -> their three parts, operands of a product each.
+__device__ __forceinline__ void cut_in_three(const float4& lo, const float4& hi, bf16x8 (&parts)[3]) {
+    float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
+#pragma unroll
+    for (int part = 0; part < 3; ++part) {
+        unsigned pairs[4];
+#pragma unroll
+        for (int e = 0; e < 8; e += 2)              // the upper halves of two entries
+            pairs[e / 2] = __builtin_amdgcn_perm(__float_as_uint(v[e + 1]), __float_as_uint(v[e]), 0x07060302u);
+        parts[part] = __builtin_bit_cast(bf16x8, make_uint4(pairs[0], pairs[1], pairs[2], pairs[3]));
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v[e] -= __uint_as_float(__float_as_uint(v[e]) & 0xFFFF0000u);
+    }
+}
+
+// Eight neighbouring entries; WHOLE: aligned to 16 bytes, else one by one.
+template <bool WHOLE>
+__device__ __forceinline__ void load8(float4& lo, float4& hi, const float* from) {
+    if (WHOLE) {
+        lo = *reinterpret_cast<const float4*>(from);
+        hi = *reinterpret_cast<const float4*>(from + 4);
+    } else {
+        lo = make_float4(from[0], from[1], from[2], from[3]);
+        hi = make_float4(from[4], from[5], from[6], from[7]);
+    }
+}
+template <bool WHOLE>
+__device__ __forceinline__ bf16x8 load8(const bf16* from) {
+    if (WHOLE) return *reinterpret_cast<const bf16x8*>(from);
+    bf16x8 v;
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = from[e];
+    return v;
+}
+
+// A chunk's sum that is NaN, from x and w as they are.
+__device__ __forceinline__ float plain_sum(const float* x, const bf16* w, int k0, int k1) {
+    float sum = 0.f;
+#pragma unroll 1
+    for (int k = k0; k < k1; ++k) sum = fmaf(x[k], to_f32(w[k]), sum);
+    return sum;
+}
+
+// Tile BM x BN, WM x WN waves, KB k a block.  SHARED: blockIdx.z owns the chunks [z * per, (z + 1) * per) and leaves each chunk's sums in
+// part[chunk][M][N].
+template <int BM, int BN, int WM, int WN, int KB, bool WHOLE, bool SHARED>
+__global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(const float* __restrict__ x, const bf16* __restrict__ w, float* __restrict__ out,
+                                                            int M, int N, int K, float* __restrict__ part, int per) {
+    static_assert(GS_CHUNK % KB == 0, "whole blocks a chunk");
+    constexpr int THREADS = 64 * WM * WN;
+    constexpr int TM = BM / 32 / WM, TN = BN / 32 / WN;
+    constexpr int PIECES = KB / 8, ROWS = THREADS / PIECES;          // 16-byte pieces a row and block, rows that the threads bring at once
+    constexpr int XL = (BM + ROWS - 1) / ROWS, WL = BN / ROWS;
+    constexpr int PLANE = BM * KB, STAGE = 3 * PLANE + BN * KB;  // entries
+    __shared__ __attribute__((aligned(1024))) unsigned short lds[2 * STAGE];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int m0 = blockIdx.y * BM, n0 = blockIdx.x * BN;
+    const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
+    const int chunks = (K + GS_CHUNK - 1) / GS_CHUNK;
+    const int c_begin = SHARED ? blockIdx.z * per : 0, c_end = SHARED ? min(c_begin + per, chunks) : chunks;
+    if (c_begin >= c_end) return;
+
+    // Piece c of row r lies at place c ^ swizzle(r), so that the 16 rows that LDS serves together meet no bank twice.  A row behind the
+    // last is the last one again: its products go nowhere.
+    auto swizzle = [](int r) { return (r / (128 / KB)) & (PIECES - 1); };
+    const int row = tid / PIECES, piece = tid % PIECES;
+    const float* xg[XL];
+    const bf16* wg[WL];
+#pragma unroll
+    for (int i = 0; i < XL; ++i) xg[i] = x + (size_t)min(m0 + row + ROWS * i, M - 1) * K + piece * 8;
+#pragma unroll
+    for (int i = 0; i < WL; ++i) wg[i] = w + (size_t)min(n0 + row + ROWS * i, N - 1) * K + piece * 8;
+    float4 xr[XL][2];
+    bf16x8 wr[WL];
+    auto fetch = [&](int k) {
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+            if (BM % ROWS == 0 || row < BM) load8<WHOLE>(xr[i][0], xr[i][1], xg[i] + k);
+#pragma unroll
+        for (int i = 0; i < WL; ++i) wr[i] = load8<WHOLE>(wg[i] + k);
+    };
+    auto put = [&](int stage) {
+        unsigned short* to = lds + stage * STAGE;
+#pragma unroll
+        for (int i = 0; i < WL; ++i) {
+            const int r = row + ROWS * i;
+            *reinterpret_cast<bf16x8*>(to + 3 * PLANE + r * KB + (piece ^ swizzle(r)) * 8) = wr[i];
+        }
+#pragma unroll
+        for (int i = 0; i < XL; ++i)
+            if (BM % ROWS == 0 || row < BM) {
+                const int r = row + ROWS * i;
+                bf16x8 parts[3];
+                cut_in_three(xr[i][0], xr[i][1], parts);
+#pragma unroll
+                for (int p = 0; p < 3; ++p) *reinterpret_cast<bf16x8*>(to + p * PLANE + r * KB + (piece ^ swizzle(r)) * 8) = parts[p];
+            }
+    };
+    const int lr = lane & 31, kg = lane >> 5;
+    auto operand = [&](const unsigned short* from, int r, int ks) {
+        return *reinterpret_cast<const bf16x8*>(from + r * KB + ((2 * ks + kg) ^ swizzle(r)) * 8);
+    };
+
+    // K is a multiple of KB: every block is whole
+    const int k_begin = c_begin * GS_CHUNK, k_limit = min(K, c_end * GS_CHUNK);
+    floatx16 total[TM][TN];
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) total[i][j][v] = 0.f;
+    fetch(k_begin);
+    put(0);
+    fetch(min(k_begin + KB, k_limit - KB));
+    int stage = 0;
+    for (int c = c_begin; c < c_end; ++c) {
+        floatx16 acc[TM][TN];
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+        const int k_end = min(K, (c + 1) * GS_CHUNK);
+        for (int k = c * GS_CHUNK; k < k_end; k += KB) {
+            __syncthreads();                    // this block is written by everybody, and the other stage read
+            const unsigned short* from = lds + stage * STAGE;
+#pragma unroll
+            for (int ks = 0; ks < KB / 16; ++ks) {
+                bf16x8 a[3][TM], b[TN];
+#pragma unroll
+                for (int j = 0; j < TN; ++j) b[j] = operand(from + 3 * PLANE, wn + 32 * j + lr, ks);
+#pragma unroll
+                for (int p = 2; p >= 0; --p)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i) a[p][i] = operand(from + p * PLANE, wm + 32 * i + lr, ks);
+                if (ks == 0) {
+                    put(stage ^ 1);             // the next block (behind the last one: some block once more)
+                    fetch(min(k + 2 * KB, k_limit - KB));
+                }
+#pragma unroll
+                for (int p = 2; p >= 0; --p)
+#pragma unroll
+                    for (int i = 0; i < TM; ++i)
+#pragma unroll
+                        for (int j = 0; j < TN; ++j)
+                            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[p][i], b[j], acc[i][j], 0, 0, 0);
+            }
+            stage ^= 1;
+        }
+        // lane l holds the rows (v / 4) * 8 + (l / 32) * 4 + v % 4 and column l % 32 of each of its products
+        auto m_of = [&](int i, int v) { return m0 + wm + 32 * i + (v >> 2) * 8 + kg * 4 + (v & 3); };
+        auto n_of = [&](int j) { return n0 + wn + 32 * j + lr; };
+        bool bad = false;
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) bad = bad || acc[i][j][v] != acc[i][j][v];
+        if (__any(bad)) {
+#pragma unroll
+            for (int i = 0; i < TM; ++i)
+#pragma unroll
+                for (int j = 0; j < TN; ++j)
+#pragma unroll
+                    for (int v = 0; v < 16; ++v)
+                        if (acc[i][j][v] != acc[i][j][v])
+                            acc[i][j][v] = plain_sum(x + (size_t)min(m_of(i, v), M - 1) * K, w + (size_t)min(n_of(j), N - 1) * K,
+                                                     c * GS_CHUNK, k_end);
+        }
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    if (SHARED) {
+                        if (m_of(i, v) < M && n_of(j) < N) part[((size_t)c * M + m_of(i, v)) * N + n_of(j)] = acc[i][j][v];
+                    } else {
+                        total[i][j][v] = __fadd_rn(total[i][j][v], acc[i][j][v]);
+                    }
+                }
+    }
+    if (SHARED) return;
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const int m = m0 + wm + 32 * i + (v >> 2) * 8 + kg * 4 + (v & 3), n = n0 + wn + 32 * j + lr;
+                if (m < M && n < N) out[(size_t)m * N + n] = total[i][j][v];
+            }
+}
+
+// Up to 16 rows: a chunk of x lies in LDS in its three parts, and each of the four waves streams its 32 rows of w past it, a chunk's 16
+// loads asked for together in the operands' own layout: nothing is staged and nothing waited for in between.  The products and
+// their order are those of the tiles; rows 16 to 31 of a product are the first 16 once more.
+constexpr int GS_FEW = 16, GS_FEW_N = 128;
+
+template <bool WHOLE, bool SHARED>
+__global__ __launch_bounds__(256, 2) void gemm_split_few_kernel(const float* __restrict__ x, const bf16* __restrict__ w, float* __restrict__ out,
+                                                                int M, int N, int K, float* __restrict__ part, int per) {
+    constexpr int STEPS = GS_CHUNK / 16, PIECES = GS_CHUNK / 8;
+    __shared__ __attribute__((aligned(16))) unsigned short lds[3 * GS_FEW * GS_CHUNK];
+    const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), lr = lane & 31, kg = lane >> 5;
+    const int n0 = blockIdx.x * GS_FEW_N + wave * 32, n = n0 + lr;
+    const int chunks = (K + GS_CHUNK - 1) / GS_CHUNK;
+    const int c_begin = SHARED ? blockIdx.z * per : 0, c_end = SHARED ? min(c_begin + per, chunks) : chunks;
+    const bf16* wg = w + (size_t)min(n, N - 1) * K + 8 * kg;
+    const int row = tid / 16;
+    const float* xg = x + (size_t)min(row, M - 1) * K;
+    floatx16 total;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) total[v] = 0.f;
+    for (int c = c_begin; c < c_end; ++c) {
+        const int k0 = c * GS_CHUNK, k_end = min(K, k0 + GS_CHUNK), steps = (k_end - k0) / 16;      // K is a multiple of 32
+        bf16x8 b[STEPS];
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s) b[s] = load8<WHOLE>(wg + k0 + 16 * min(s, steps - 1));
+        if (c > c_begin) __syncthreads();       // the chunk before is read by everybody
+#pragma unroll
+        for (int i = 0; i < PIECES / 16; ++i) {
+            // piece p of row r lies at place p ^ r: the 16 rows that LDS serves together meet no bank twice
+            const int piece = tid % 16 + 16 * i;
+            if (k0 + 8 * piece < k_end) {
+                bf16x8 parts[3];
+                float4 lo, hi;
+                load8<WHOLE>(lo, hi, xg + k0 + 8 * piece);
+                cut_in_three(lo, hi, parts);
+#pragma unroll
+                for (int p = 0; p < 3; ++p)
+                    *reinterpret_cast<bf16x8*>(lds + (p * GS_FEW + row) * GS_CHUNK + (piece ^ row) * 8) = parts[p];
+            }
+        }
+        __syncthreads();
+        floatx16 acc;
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[v] = 0.f;
+#pragma unroll
+        for (int s = 0; s < STEPS; ++s)
+            if (s < steps)
+#pragma unroll
+                for (int p = 2; p >= 0; --p) {
+                    const int r = lr & (GS_FEW - 1);
+                    const bf16x8 a = *reinterpret_cast<const bf16x8*>(lds + (p * GS_FEW + r) * GS_CHUNK + ((2 * s + kg) ^ r) * 8);
+                    acc = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b[s], acc, 0, 0, 0);
+                }
+        bool bad = false;
+#pragma unroll
+        for (int v = 0; v < 8; ++v) bad = bad || acc[v] != acc[v];      // the rows up to 15
+        if (__any(bad)) {
+#pragma unroll
+            for (int v = 0; v < 8; ++v)
+                if (acc[v] != acc[v])
+                    acc[v] = plain_sum(x + (size_t)min((v >> 2) * 8 + kg * 4 + (v & 3), M - 1) * K, w + (size_t)min(n, N - 1) * K, k0, k_end);
+        }
+#pragma unroll
+        for (int v = 0; v < 8; ++v) {
+            const int m = (v >> 2) * 8 + kg * 4 + (v & 3);
+            if (SHARED) {
+                if (m < M && n < N) part[((size_t)c * M + m) * N + n] = acc[v];
+            } else {
+                total[v] = __fadd_rn(total[v], acc[v]);
+            }
+        }
+    }
+    if (SHARED) return;
+#pragma unroll
+    for (int v = 0; v < 8; ++v) {
+        const int m = (v >> 2) * 8 + kg * 4 + (v & 3);
+        if (m < M && n < N) out[(size_t)m * N + n] = total[v];
+    }
+}
+
+bool gemm_split_takes(int K) { return K % 32 == 0; }
+
+template <bool WHOLE, bool SHARED>
+static void launch_split(const float* x, const bf16* w, float* out, int M, int N, int K, float* part, int per, int shares, hipStream_t stream) {
+    if (M <= GS_FEW)
+        gemm_split_few_kernel<WHOLE, SHARED><<<dim3((N + GS_FEW_N - 1) / GS_FEW_N, 1, shares), 256, 0, stream>>>(x, w, out, M, N, K, part, per);
+    else
+        gemm_split_kernel<64, 64, 2, 2, 32, WHOLE, SHARED><<<dim3((N + 63) / 64, (M + 63) / 64, shares), 256, 0, stream>>>(x, w, out, M, N, K,
+                                                                                                                    part, per);
+}
+
+void launch_gemm_split(const float* x, const bf16* w, float* out, int M, int N, int K, float* part, int per, int shares, hipStream_t stream) {
+    const bool whole = ((uintptr_t)x | (uintptr_t)w) % 16 == 0;
+    if (whole && part) launch_split<true, true>(x, w, out, M, N, K, part, per, shares, stream);
+    else if (whole) launch_split<true, false>(x, w, out, M, N, K, part, per, shares, stream);
+    else if (part) launch_split<false, true>(x, w, out, M, N, K, part, per, shares, stream);
+    else launch_split<false, false>(x, w, out, M, N, K, part, per, shares, stream);
+}
+
+}  // namespace lc

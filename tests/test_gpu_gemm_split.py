@@ -1,0 +1,54 @@
+"""float32 x by bfloat16 w as three products of bfloat16 numbers (``csrc/gemm_split.hip``): edges of tiles, blocks and chunks, the same bits
+for every number of rows, errors no larger than the float32 instruction's, and entries that have no three parts."""
+import pytest
+import torch
+
+from lucciola_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+
+
+def product(x, w, plain=0):
+    ops.library().lc_gemm_generic_plain(plain)
+    try:
+        return ops.gemm(x, w, torch.float32)
+    finally:
+        ops.library().lc_gemm_generic_plain(0)
+
+
+@pytest.mark.parametrize("M", [1, 15, 16, 17, 63, 65, 200])
+@pytest.mark.parametrize("N,K", [(1, 32), (63, 224), (129, 256), (300, 288), (1000, 1024), (40000, 96)])
+def test_edges(M, N, K):
+    g = torch.Generator().manual_seed(M + N + K)
+    x = (torch.randn(M, K, generator=g) * torch.exp(3 * torch.randn(M, K, generator=g))).to(DEV)
+    w = torch.randn(N, K, generator=g).bfloat16().to(DEV)
+    got, want = product(x, w), x.double() @ w.double().T
+    # K products, exact, added in float32: each addition is off by 2^-24 of a sum that is no larger than the terms' absolute values
+    allowed = 2.0 ** -24 * K * (x.double().abs() @ w.double().abs().T)
+    assert bool(((got.double() - want).abs() <= allowed).all())
+    plain = product(x, w, plain=1)
+    if M * N >= 10000:      # a root mean square over n errors is itself off by some 1 / sqrt(2 n) of it: 0.7 % here, 20 % at 15 entries
+        assert float((got.double() - want).norm()) <= 1.05 * float((plain.double() - want).norm())
+    # a row alone, few rows and many have the same bits
+    many = product(x.repeat(-(-700 // M), 1), w)
+    assert torch.equal(many[:M], got) and torch.equal(many[-M:], got)
+    assert torch.equal(product(x[M // 2:M // 2 + 1].contiguous(), w)[0], got[M // 2])
+
+
+@pytest.mark.parametrize("M", [3, 40])
+@pytest.mark.parametrize("K", [288, 4096])
+def test_entries_without_parts(M, K):
+    """Infinite and not-a-number entries, the largest and the smallest numbers: what the float32 instruction makes of them."""
+    g = torch.Generator().manual_seed(K)
+    x, w = torch.randn(M, K, generator=g).to(DEV), torch.randn(130, K, generator=g).bfloat16().to(DEV)
+    x[0, 5], x[1, 270], x[2, 7] = float("inf"), float("nan"), -float("inf")
+    w[3, 9], w[4, 271] = float("inf"), float("nan")
+    w[5, 5] = 0.0
+    x[2, 20:24] = torch.tensor([3.4028235e38, -3.4028235e38, 1e-40, -1.1754944e-38])
+    w[:, 20:22] = 0.0
+    got, plain = product(x, w), product(x, w, plain=1)
+    same = torch.isfinite(plain)
+    assert torch.equal(torch.isnan(got), torch.isnan(plain)) and torch.equal(torch.isposinf(got), torch.isposinf(plain))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(plain))
+    torch.testing.assert_close(got[same], plain[same], rtol=1e-5, atol=1e-4)
