@@ -220,35 +220,58 @@ __global__ __launch_bounds__(MA_THREADS) void attention_prepare_kernel(
         }
 }
 
-// The same for steps without the unit norm, where nothing is summed over a head: a thread per pair of neighbouring
-// entries of the whole row (head sizes and the row's stride even), the pair's inputs and taps in wide loads.  The sums
-// and the rotation are written as in the kernel above, so both give the same bits.
+// Two neighbouring entries, in one store where p is aligned to the pair.
 template <typename T>
-__global__ void attention_prepare_pairs_kernel(
+__device__ __forceinline__ void put_pair(T* p, float a, float b) {
+    typedef T pair_t __attribute__((ext_vector_type(2)));
+    if ((uintptr_t)p % (2 * sizeof(T)) == 0) {
+        pair_t v;
+        v[0] = from_f32<T>(a);
+        v[1] = from_f32<T>(b);
+        *reinterpret_cast<pair_t*>(p) = v;
+    } else {
+        p[0] = from_f32<T>(a);
+        p[1] = from_f32<T>(b);
+    }
+}
+
+// The same for steps without the unit norm, where nothing is summed over a head: a thread per pair of neighbouring entries of the
+// row (head sizes and the row's stride even) and run of TOKENS tokens.  KT: taps (0: as many as K says; no convolution: -1).  The sums and
+// the rotation are written as in the kernel above, so both give the same bits.  Values of a run that fill a page's 16-byte piece are
+// stored as one: they lie transposed in their page, 2 bytes of every row otherwise.  2,048 tokens, 16 heads of 2 x 64 over 4, values
+// of 128, 4 taps: 63 us with a thread per (token, pair), a 64-bit division and four inputs each; 16 us.
+template <typename T, int KT, int TOKENS>
+__global__ __launch_bounds__(256) void attention_prepare_pairs_kernel(
     const float* __restrict__ proj, int cols, int T_, int nq, int nk, int nv, int d, int dv,
     const float* __restrict__ taps, int K, const float* __restrict__ tails, const int* __restrict__ tok_req,
     const int* __restrict__ q_offsets, const int* __restrict__ slot_ids, const float* __restrict__ table, int rot,
     const int* __restrict__ positions, T* __restrict__ q_out, T* __restrict__ k_cache, T* __restrict__ v_cache,
     const int* __restrict__ rows, int page_size) {
-    const int C = (nq + nk) * d + nv * dv, pairs = C / 2, q_cols = nq * d, qk_cols = (nq + nk) * d;
-    const size_t total = (size_t)T_ * pairs;
-    for (size_t idx = (size_t)blockIdx.x * blockDim.x + threadIdx.x; idx < total;
-         idx += (size_t)gridDim.x * blockDim.x) {
-        const int t = (int)(idx / pairs), c = 2 * (int)(idx % pairs);
-        const bool is_v = c >= qk_cols;
-        const int at = is_v ? (c - qk_cols) % dv : c % d;          // the pair's place in its head
+    const int C = (nq + nk) * d + nv * dv, q_cols = nq * d, qk_cols = (nq + nk) * d;
+    const int c = 2 * (blockIdx.y * 256 + threadIdx.x), t0 = blockIdx.x * TOKENS;
+    if (c >= C) return;
+    const bool is_v = c >= qk_cols;
+    const int at = is_v ? (c - qk_cols) % dv : c % d;          // the pair's place in its head
+    ShortConvRun<KT < 0 ? 0 : KT> first, second;
+    if (KT > 0) {
+        first.start(taps, c);
+        second.start(taps, c + 1);
+    }
+    constexpr int PIECE = 16 / sizeof(T);
+    float va[TOKENS], vb[TOKENS];
+    int before = -1;
+#pragma unroll
+    for (int i = 0; i < TOKENS; ++i) {
+        const int t = t0 + i;
+        va[i] = vb[i] = 0.f;
+        if (t >= T_) continue;
         float a, b;
-        if (taps) {
-            const int r = tok_req[t];
-            const int local = t - q_offsets[r];
+        if constexpr (KT >= 0) {
+            const int r = tok_req[t], local = t - q_offsets[r];
             const float* tail = tails + (size_t)slot_ids[r] * (K - 1) * C;
-            a = b = 0.f;
-            for (int back = K - 1; back >= 0; --back) {         // oldest input first
-                const float2 in = *reinterpret_cast<const float2*>(
-                    back <= local ? proj + (size_t)(t - back) * cols + c : tail + (size_t)((K - 1) - (back - local)) * C + c);
-                a = fmaf(taps[(size_t)c * K + (K - 1 - back)], in.x, a);
-                b = fmaf(taps[(size_t)(c + 1) * K + (K - 1 - back)], in.y, b);
-            }
+            a = first.at(proj, cols, t, local, c, taps, K, tail, C, r != before);
+            b = second.at(proj, cols, t, local, c + 1, taps, K, tail, C, r != before);
+            before = r;
         } else {
             const float2 in = *reinterpret_cast<const float2*>(proj + (size_t)t * cols + c);
             a = in.x;
@@ -261,20 +284,48 @@ __global__ void attention_prepare_pairs_kernel(
             a = a0 * cs - b0 * sn;
             b = fmaf(b0, cs, a0 * sn);
         }
-        if (c < q_cols) {
-            q_out[(size_t)t * q_cols + c] = from_f32<T>(a);
-            q_out[(size_t)t * q_cols + c + 1] = from_f32<T>(b);
-        } else if (rows && rows[t] >= 0) {
-            if (is_v) {
-                T* dst = v_cache + ((size_t)(rows[t] / page_size) * nv * dv + (c - qk_cols)) * page_size + rows[t] % page_size;
-                dst[0] = from_f32<T>(a);
-                dst[page_size] = from_f32<T>(b);
-            } else {
-                T* dst = k_cache + (size_t)rows[t] * nk * d + (c - q_cols);
-                dst[0] = from_f32<T>(a);
-                dst[1] = from_f32<T>(b);
+        va[i] = a;
+        vb[i] = b;
+        if (c < q_cols) put_pair(q_out + (size_t)t * q_cols + c, a, b);
+        else if (!is_v && rows && rows[t] >= 0) put_pair(k_cache + (size_t)rows[t] * nk * d + (c - q_cols), a, b);
+    }
+    if (!is_v || !rows) return;
+    auto to = [&](int row) { return v_cache + ((size_t)(row / page_size) * nv * dv + (c - qk_cols)) * page_size + row % page_size; };
+    if constexpr (TOKENS % PIECE == 0) {
+        typedef T piece_t __attribute__((ext_vector_type(PIECE)));
+#pragma unroll
+        for (int i0 = 0; i0 < TOKENS; i0 += PIECE) {
+            const int row = t0 + i0 < T_ ? rows[t0 + i0] : -1;
+            bool whole = row >= 0 && row % PIECE == 0 && page_size % PIECE == 0 && t0 + i0 + PIECE <= T_ && (uintptr_t)v_cache % 16 == 0;
+#pragma unroll
+            for (int i = 1; i < PIECE; ++i) whole = whole && rows[min(t0 + i0 + i, T_ - 1)] == row + i;
+            if (whole) {
+                piece_t a, b;
+#pragma unroll
+                for (int i = 0; i < PIECE; ++i) {
+                    a[i] = from_f32<T>(va[i0 + i]);
+                    b[i] = from_f32<T>(vb[i0 + i]);
+                }
+                *reinterpret_cast<piece_t*>(to(row)) = a;
+                *reinterpret_cast<piece_t*>(to(row) + page_size) = b;
+                continue;
             }
+#pragma unroll
+            for (int i = 0; i < PIECE; ++i)
+                if (t0 + i0 + i < T_ && rows[t0 + i0 + i] >= 0) {
+                    T* dst = to(rows[t0 + i0 + i]);
+                    dst[0] = from_f32<T>(va[i0 + i]);
+                    dst[page_size] = from_f32<T>(vb[i0 + i]);
+                }
         }
+    } else {
+#pragma unroll
+        for (int i = 0; i < TOKENS; ++i)
+            if (t0 + i < T_ && rows[t0 + i] >= 0) {
+                T* dst = to(rows[t0 + i]);
+                dst[0] = from_f32<T>(va[i]);
+                dst[page_size] = from_f32<T>(vb[i]);
+            }
     }
 }
 
@@ -341,18 +392,24 @@ LC_API int lc_attention_prepare(const float* proj, int cols, int T, int nq, int 
     LC_CHECK(!table || (rot > 0 && rot % 2 == 0 && rot <= d && positions), "attention prepare: bad rotation");
     LC_CHECK(!rows || (k_cache && v_cache && page_size > 0), "attention prepare: rows without a cache");
     if (!unit && d % 2 == 0 && dv % 2 == 0 && cols % 2 == 0 && g_prepare_pairs) {
-        const size_t total = (size_t)T * (((nq + nk) * d + nv * dv) / 2);
-        const int blocks = (int)((total + 255) / 256 < 16384 ? (total + 255) / 256 : 16384);
-        if (dt == DT_F32)
-            attention_prepare_pairs_kernel<float><<<blocks, 256, 0, stream>>>(
-                proj, cols, T, nq, nk, nv, d, dv, taps, K, tails, tok_req, q_offsets, slot_ids, table, rot, positions,
-                (float*)q_out, (float*)k_cache, (float*)v_cache, rows, page_size > 0 ? page_size : 1);
-        else if (dt == DT_BF16)
-            attention_prepare_pairs_kernel<bf16><<<blocks, 256, 0, stream>>>(
-                proj, cols, T, nq, nk, nv, d, dv, taps, K, tails, tok_req, q_offsets, slot_ids, table, rot, positions,
-                (bf16*)q_out, (bf16*)k_cache, (bf16*)v_cache, rows, page_size > 0 ? page_size : 1);
-        else
-            LC_CHECK(false, "attention prepare: unknown dtype %d", dt);
+        const int pair_blocks = (((nq + nk) * d + nv * dv) / 2 + 255) / 256;
+        LC_CHECK(pair_blocks <= 65535, "attention prepare: too many heads");
+#define LC_PAIRS_AS(TT, KT, TOKENS)                                                                                                     \
+    attention_prepare_pairs_kernel<TT, KT, TOKENS><<<dim3((T + TOKENS - 1) / TOKENS, pair_blocks), 256, 0, stream>>>(                   \
+        proj, cols, T, nq, nk, nv, d, dv, taps, K, tails, tok_req, q_offsets, slot_ids, table, rot, positions, (TT*)q_out, (TT*)k_cache, \
+        (TT*)v_cache, rows, page_size > 0 ? page_size : 1)
+        // runs of tokens where there are many; a step of few keeps a thread a token and pair
+#define LC_PAIRS(TT)                                                                  \
+    do {                                                                              \
+        if (!taps) { if (T >= 1024) LC_PAIRS_AS(TT, -1, 8); else LC_PAIRS_AS(TT, -1, 1); } \
+        else if (K == 4) { if (T >= 1024) LC_PAIRS_AS(TT, 4, 8); else LC_PAIRS_AS(TT, 4, 1); } \
+        else LC_PAIRS_AS(TT, 0, 1);                                                   \
+    } while (0)
+        if (dt == DT_F32) LC_PAIRS(float);
+        else if (dt == DT_BF16) LC_PAIRS(bf16);
+        else LC_CHECK(false, "attention prepare: unknown dtype %d", dt);
+#undef LC_PAIRS
+#undef LC_PAIRS_AS
         LC_LAUNCH_CHECK("attention_prepare");
         return 0;
     }

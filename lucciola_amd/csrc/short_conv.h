@@ -25,4 +25,40 @@ __device__ __forceinline__ float short_conv(const float* __restrict__ proj, size
     return y;
 }
 
+// The same for tokens that follow one another: a thread keeps its channel's taps and last inputs, so that each input is read once and
+// not once a tap.  KT: the number of taps, or 0 where it is known at run time alone (then every token reads all of its inputs).  The
+// sums are short_conv's, to the bit.
+template <int KT>
+struct ShortConvRun {
+    float w[KT > 0 ? KT : 1], in[KT > 0 ? KT : 1];      // the taps; the inputs up to the token, the oldest first
+
+    __device__ __forceinline__ void start(const float* __restrict__ taps, int c) {
+#pragma unroll
+        for (int j = 0; j < KT; ++j) w[j] = taps[(size_t)c * KT + j];
+    }
+
+    // fresh: the token before was not this request's, or not this thread's
+    __device__ __forceinline__ float at(const float* __restrict__ proj, size_t cols, int t, int local, int c, const float* __restrict__ taps,
+                                        int K, const float* __restrict__ tail, int C, bool fresh) {
+        if constexpr (KT == 0) {
+            return short_conv(proj, cols, t, local, c, taps, K, tail, C);
+        } else {
+#pragma unroll
+            for (int j = 0; j < KT - 1; ++j) {
+                if (fresh) {
+                    const int back = KT - 1 - j;
+                    in[j] = back <= local ? proj[(size_t)(t - back) * cols + c] : tail[(size_t)((KT - 1) - (back - local)) * C + c];
+                } else {
+                    in[j] = in[j + 1];
+                }
+            }
+            in[KT - 1] = proj[(size_t)t * cols + c];
+            float y = 0.f;
+#pragma unroll
+            for (int j = 0; j < KT; ++j) y = fmaf(w[j], in[j], y);
+            return y;
+        }
+    }
+};
+
 }  // namespace lc
