@@ -19,6 +19,9 @@
 // in a row of a key, straight from memory) leaves a lane with four keys of one query column, which is the
 // operand P^T of O^T += V^T P^T (16x16x16; V^T's operand is four neighbouring keys of one value entry, 8
 // bytes in a row of the transposed page), so the weights never leave the registers.
+// The workgroups go tile by tile, a tile's kv heads beside each other, and the list has the longest tiles first: with all tiles of
+// one kv head before the next head's, the last head's longest tile began when half of the card had run dry (2,048 tokens, four kv
+// heads, a workgroup a CU: 202 -> 136 us for two maps of 64, 207 -> 143 for one of 128 with the bias; 1,523 tokens 102 -> 78).
 #include "common.h"
 
 namespace lc {
@@ -82,36 +85,52 @@ struct ColumnState {
     floatx4 o[MAPS][DVB];       // O^T: value entries 16 t + 4 (lane / 16) + i of the lane's query column
 };
 
-// One block of 16 keys for the lane's column: scores from the keys' and the queries' operands, mask, bias, the
-// reference point and the sum, and the weighted values taken into O^T.
-template <int DSTEPS, int DVB, int MAPS>
+// The upper halves of two float32 numbers side by side.
+__device__ __forceinline__ unsigned upper_halves(float first, float second) {
+    return __builtin_amdgcn_perm(__float_as_uint(second), __float_as_uint(first), 0x07060302u);
+}
+
+// NB blocks of 16 keys for the lane's column: scores from the keys' and the queries' operands, mask, bias, the
+// reference point and the sum, and the weighted values taken into O^T.  Two blocks at once take their values with products over 32
+// keys (a lane's operand is its four keys of the one and its four of the other), which cost what products over 16 do: 2,048 tokens, 16
+// heads over 4, two maps of 64 224 -> 202 us, one of 128 with the bias 210 -> 207.
+template <int NB, int DSTEPS, int DVB, int MAPS>
 __device__ __forceinline__ void block_step(ColumnState<DVB, MAPS>& st, const MaskedArgs& a,
-                                           const bf16x8 (&bq)[MAPS][DSTEPS], const bf16x8 (&ka)[MAPS][DSTEPS],
-                                           const short4v (&va)[DVB], int key0, int pos, int lo, float bias1, float bias2,
-                                           bool all_seen, int lane) {
+                                           const bf16x8 (&bq)[MAPS][DSTEPS], const bf16x8 (&ka)[NB][MAPS][DSTEPS],
+                                           const short4v (&va)[NB][DVB], const int (&key0)[NB], int pos, int lo, float bias1, float bias2,
+                                           const bool (&all_seen)[NB], int lane) {
     const int quad = lane >> 4;
-    const int j0 = key0 + quad * 4;
-    float far[4];
+    float far[NB][4];
 #pragma unroll
-    for (int v = 0; v < 4; ++v) far[v] = a.r1 ? bias1 * __logf(1.f + bias2 * (float)max(pos - (j0 + v), 0)) : 0.f;
+    for (int b = 0; b < NB; ++b)
+#pragma unroll
+        for (int v = 0; v < 4; ++v)
+            far[b][v] = a.r1 ? bias1 * __logf(1.f + bias2 * (float)max(pos - (key0[b] + quad * 4 + v), 0)) : 0.f;
 #pragma unroll
     for (int m = 0; m < MAPS; ++m) {
-        floatx4 s = {0.f, 0.f, 0.f, 0.f};
+        floatx4 s[NB];
 #pragma unroll
-        for (int i = 0; i < DSTEPS; ++i) s = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[m][i], bq[m][i], s, 0, 0, 0);
+        for (int b = 0; b < NB; ++b) s[b] = floatx4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int i = 0; i < DSTEPS; ++i)
+#pragma unroll
+            for (int b = 0; b < NB; ++b) s[b] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(ka[b][m][i], bq[m][i], s[b], 0, 0, 0);
         float mx = -INFINITY;
-        if (all_seen) {             // every column of the wave sees the whole block: nothing to mask
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                s[v] = held(fmaf(s[v], a.scale, -far[v]), a.cap);
-                mx = fmaxf(mx, s[v]);
-            }
-        } else {
+        for (int b = 0; b < NB; ++b) {
+            if (all_seen[b]) {             // every column of the wave sees the whole block: nothing to mask
 #pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const int j = j0 + v;
-                s[v] = ((j >= lo || j < a.keep) && j <= pos) ? held(fmaf(s[v], a.scale, -far[v]), a.cap) : -INFINITY;
-                mx = fmaxf(mx, s[v]);
+                for (int v = 0; v < 4; ++v) {
+                    s[b][v] = held(fmaf(s[b][v], a.scale, -far[b][v]), a.cap);
+                    mx = fmaxf(mx, s[b][v]);
+                }
+            } else {
+#pragma unroll
+                for (int v = 0; v < 4; ++v) {
+                    const int j = key0[b] + quad * 4 + v;
+                    s[b][v] = ((j >= lo || j < a.keep) && j <= pos) ? held(fmaf(s[b][v], a.scale, -far[b][v]), a.cap) : -INFINITY;
+                    mx = fmaxf(mx, s[b][v]);
+                }
             }
         }
         // The column's reference point st.m moves only when a score outgrows it by e^8 (or it has none yet): until
@@ -130,25 +149,43 @@ __device__ __forceinline__ void block_step(ColumnState<DVB, MAPS>& st, const Mas
         // A weight p >= 0 as two bfloat16 numbers: its upper 16 bits, and the upper 16 bits of what they leave
         // (p minus them is exact in float32): together p to 2^-15 of itself.
         float psum = 0.f;
-        unsigned hi_bits[4], lw_bits[4];
+        unsigned hi[2 * NB], lw[2 * NB];
 #pragma unroll
-        for (int v = 0; v < 4; ++v) {
-            const float p = __expf(s[v] - base);
-            psum += p;
-            const unsigned whole = __float_as_uint(p), upper = whole & 0xffff0000u;
-            hi_bits[v] = whole >> 16;
-            lw_bits[v] = __float_as_uint(p - __uint_as_float(upper)) >> 16;
+        for (int b = 0; b < NB; ++b) {
+            float p[4], left[4];
+#pragma unroll
+            for (int v = 0; v < 4; ++v) {
+                p[v] = __expf(s[b][v] - base);
+                psum += p[v];
+                left[v] = p[v] - __uint_as_float(__float_as_uint(p[v]) & 0xffff0000u);
+            }
+            hi[2 * b] = upper_halves(p[0], p[1]);
+            hi[2 * b + 1] = upper_halves(p[2], p[3]);
+            lw[2 * b] = upper_halves(left[0], left[1]);
+            lw[2 * b + 1] = upper_halves(left[2], left[3]);
         }
-        typedef unsigned uint2v __attribute__((ext_vector_type(2)));
-        const short4v hi = __builtin_bit_cast(short4v, uint2v{hi_bits[0] | (hi_bits[1] << 16), hi_bits[2] | (hi_bits[3] << 16)});
-        const short4v lw = __builtin_bit_cast(short4v, uint2v{lw_bits[0] | (lw_bits[1] << 16), lw_bits[2] | (lw_bits[3] << 16)});
         st.l[m] += psum;
         // the weights' upper halves into every block of value entries first, then the remainders: no product waits
         // for the one before it
+        if constexpr (NB == 2) {
+            typedef unsigned uint4v __attribute__((ext_vector_type(4)));
+            auto both = [&](int t) {
+                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(va[0][t], va[1][t], 0, 1, 2, 3, 4, 5, 6, 7));
+            };
+            const bf16x8 hi8 = __builtin_bit_cast(bf16x8, uint4v{hi[0], hi[1], hi[2], hi[3]});
+            const bf16x8 lw8 = __builtin_bit_cast(bf16x8, uint4v{lw[0], lw[1], lw[2], lw[3]});
 #pragma unroll
-        for (int t = 0; t < DVB; ++t) st.o[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[t], hi, st.o[m][t], 0, 0, 0);
+            for (int t = 0; t < DVB; ++t) st.o[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(both(t), hi8, st.o[m][t], 0, 0, 0);
 #pragma unroll
-        for (int t = 0; t < DVB; ++t) st.o[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[t], lw, st.o[m][t], 0, 0, 0);
+            for (int t = 0; t < DVB; ++t) st.o[m][t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(both(t), lw8, st.o[m][t], 0, 0, 0);
+        } else {
+            typedef unsigned uint2v __attribute__((ext_vector_type(2)));
+            const short4v hi4 = __builtin_bit_cast(short4v, uint2v{hi[0], hi[1]}), lw4 = __builtin_bit_cast(short4v, uint2v{lw[0], lw[1]});
+#pragma unroll
+            for (int t = 0; t < DVB; ++t) st.o[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[0][t], hi4, st.o[m][t], 0, 0, 0);
+#pragma unroll
+            for (int t = 0; t < DVB; ++t) st.o[m][t] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(va[0][t], lw4, st.o[m][t], 0, 0, 0);
+        }
     }
 }
 
@@ -231,28 +268,28 @@ __device__ __forceinline__ void attend_blocks(ColumnState<DVB, MAPS>& st, const 
     };
     // the next block's values travel ahead as well where the registers hold them
     constexpr bool VALUES_AHEAD = DSTEPS * MAPS * 4 + DVB * MAPS * 4 + DVB * 4 <= 120;
-    bf16x8 ka[MAPS][DSTEPS], kn[MAPS][DSTEPS];
-    short4v va[DVB], vn[DVB];
+    bf16x8 ka[1][MAPS][DSTEPS], kn[MAPS][DSTEPS];
+    short4v va[1][DVB], vn[DVB];
     if (at < blocks.count) {
-        load_keys(ka, blocks.block(at));
-        if constexpr (VALUES_AHEAD) load_values(va, blocks.block(at));
+        load_keys(ka[0], blocks.block(at));
+        if constexpr (VALUES_AHEAD) load_values(va[0], blocks.block(at));
     }
     for (int i = at; i < blocks.count; i += stride) {
         const int b = blocks.block(i), key0 = b * 16;
-        if constexpr (!VALUES_AHEAD) load_values(va, b);
+        if constexpr (!VALUES_AHEAD) load_values(va[0], b);
         if (i + stride < blocks.count) {            // on their way while this block is worked on
             load_keys(kn, blocks.block(i + stride));
             if constexpr (VALUES_AHEAD) load_values(vn, blocks.block(i + stride));
         }
-        block_step<DSTEPS, DVB, MAPS>(st, a, bq, ka, va, key0, pos, lo, bias1, bias2,
-                                      (key0 >= seen_from || key0 + 15 < a.keep) && key0 + 15 <= seen_to, lane);
+        block_step<1, DSTEPS, DVB, MAPS>(st, a, bq, ka, va, {key0}, pos, lo, bias1, bias2,
+                                         {(key0 >= seen_from || key0 + 15 < a.keep) && key0 + 15 <= seen_to}, lane);
 #pragma unroll
         for (int m = 0; m < MAPS; ++m)
 #pragma unroll
-            for (int i = 0; i < DSTEPS; ++i) ka[m][i] = kn[m][i];
+            for (int i = 0; i < DSTEPS; ++i) ka[0][m][i] = kn[m][i];
         if constexpr (VALUES_AHEAD)
 #pragma unroll
-            for (int t = 0; t < DVB; ++t) va[t] = vn[t];
+            for (int t = 0; t < DVB; ++t) va[0][t] = vn[t];
     }
 }
 
@@ -308,9 +345,10 @@ __device__ __forceinline__ void finish_column(const ColumnState<DVB, MAPS>& st, 
 template <int DSTEPS, int DVB, int MAPS>
 __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(MaskedArgs a) {
     __shared__ float meet[MB_WAVES - 1][kWave][DVB * 4 + 2];
-    const int* tile = a.tiles + 4 * blockIdx.x;
+    const int tile_at = blockIdx.x / a.kv_heads;      // a tile's kv heads are neighbours: the longest tiles of all heads start first
+    const int* tile = a.tiles + 4 * tile_at;
     const int t0 = tile[0], n = tile[1], r = tile[2], p0 = tile[3];
-    const int g = blockIdx.y, group = a.heads / a.kv_heads;
+    const int g = blockIdx.x - tile_at * a.kv_heads, group = a.heads / a.kv_heads;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), col = lane & 15;
     const int* table = a.block_table + (size_t)r * a.max_blocks;
     auto first_key = [&](int p) {
@@ -381,7 +419,7 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(Maske
             if (zsplits > 1) {
                 const int passes = (group + 15) / 16;
                 // [share][lane][map][numbers]: a lane's numbers in a row, which it reads back in wide loads
-                float* mine = a.shares + ((((size_t)blockIdx.x * a.kv_heads + g) * passes + h0 / 16) * zsplits + z)
+                float* mine = a.shares + (((size_t)blockIdx.x * passes + h0 / 16) * zsplits + z)
                                              * kWave * MAPS * share_floats<DVB>() + (size_t)lane * MAPS * share_floats<DVB>();
 #pragma unroll
                 for (int m = 0; m < MAPS; ++m) {
@@ -412,10 +450,11 @@ template <int DSTEPS, int DVB, int MAPS>
 __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kernel(MaskedArgs a) {
     extern __shared__ __align__(16) unsigned char staged[];       // a stage; afterwards where split key ranges meet
     float (*meet)[kWave][DVB * 4 + 2] = reinterpret_cast<float (*)[kWave][DVB * 4 + 2]>(staged);
-    const int* tile = a.tiles + 4 * blockIdx.x;
+    const int tile_at = blockIdx.x / a.kv_heads;      // a tile's kv heads are neighbours: the longest tiles of all heads start first
+    const int* tile = a.tiles + 4 * tile_at;
     const int t0 = tile[0], n = tile[1], r = tile[2], p0 = tile[3];
     if (n == 1) return;
-    const int g = blockIdx.y, group = a.heads / a.kv_heads;
+    const int g = blockIdx.x - tile_at * a.kv_heads, group = a.heads / a.kv_heads;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), col = lane & 15, quad = lane >> 4;
     const int* table = a.block_table + (size_t)r * a.max_blocks;
     auto first_key = [&](int p) {
@@ -514,12 +553,7 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
         __syncthreads();
         for (int stage = 0; stage < stages; ++stage) {
             if (stage + 1 < stages) fetch(stage + 1);       // on its way while this stage is worked on
-            for (int j = 0; j < a.wave_blocks; ++j) {
-                const int blk = j * splits + split, place_of = stage * stage_blocks + blk;
-                if (!wave_on || place_of >= blocks.count) continue;
-                const int b = blocks.block(place_of);
-                bf16x8 ka[MAPS][DSTEPS];
-                short4v va[DVB];
+            auto operands = [&](int blk, bf16x8 (&ka)[MAPS][DSTEPS], short4v (&va)[DVB]) {
                 const unsigned char* krow = staged + (blk * 16 + col) * k_pitch + quad * 16;
                 const unsigned char* vrow = staged + k_bytes + col * v_pitch + blk * 32 + quad * 8;
                 if (full_sizes) {           // the sizes the kernel is built for: no operand has empty places
@@ -546,8 +580,31 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
                         if (t * 16 < a.dv) va[t] = *reinterpret_cast<const short4v*>(vrow + t * 16 * v_pitch);
                     }
                 }
-                block_step<DSTEPS, DVB, MAPS>(st, a, bq, ka, va, b * 16, pos, lo, bias1, bias2,
-                                              (b * 16 >= seen_from || b * 16 + 15 < a.keep) && b * 16 + 15 <= p0, lane);
+            };
+            auto seen = [&](int b) { return (b * 16 >= seen_from || b * 16 + 15 < a.keep) && b * 16 + 15 <= p0; };
+            const int at0 = stage * stage_blocks + split, at1 = at0 + splits;       // this wave's one or two blocks of the stage
+            // both at once where their operands and sums find room in registers
+            constexpr bool PAIRS = 2 * MAPS * DSTEPS * 4 + 2 * DVB * 2 + MAPS * DVB * 4 + MAPS * DSTEPS * 4 <= 160;
+            bool done = false;
+            if constexpr (PAIRS) {
+                done = wave_on && a.wave_blocks == 2 && at1 < blocks.count;
+                if (done) {
+                    const int b0 = blocks.block(at0), b1 = blocks.block(at1);
+                    bf16x8 ka[2][MAPS][DSTEPS];
+                    short4v va[2][DVB];
+                    operands(split, ka[0], va[0]);
+                    operands(splits + split, ka[1], va[1]);
+                    block_step<2, DSTEPS, DVB, MAPS>(st, a, bq, ka, va, {b0 * 16, b1 * 16}, pos, lo, bias1, bias2, {seen(b0), seen(b1)}, lane);
+                }
+            }
+            if (!done && wave_on) {
+                for (int at = at0, blk = split; at < min(stage * stage_blocks + stage_blocks, blocks.count); at += splits, blk += splits) {
+                    const int b0 = blocks.block(at);
+                    bf16x8 ka[1][MAPS][DSTEPS];
+                    short4v va[1][DVB];
+                    operands(blk, ka[0], va[0]);
+                    block_step<1, DSTEPS, DVB, MAPS>(st, a, bq, ka, va, {b0 * 16}, pos, lo, bias1, bias2, {seen(b0)}, lane);
+                }
             }
             __syncthreads();                    // every wave has read the stage
             if (stage + 1 < stages) store();
@@ -588,10 +645,11 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
 // One wave per lone token and kv head: the workgroups' shares taken in, in their order; then the columns' end.
 template <int DVB, int MAPS>
 __global__ __launch_bounds__(kWave) void masked_attention_bf16_join_kernel(MaskedArgs a) {
-    const int* tile = a.tiles + 4 * blockIdx.x;
+    const int tile_at = blockIdx.x / a.kv_heads;      // a tile's kv heads are neighbours: the longest tiles of all heads start first
+    const int* tile = a.tiles + 4 * tile_at;
     const int t0 = tile[0], n = tile[1], p0 = tile[3];
     if (n != 1) return;
-    const int g = blockIdx.y, group = a.heads / a.kv_heads, lane = threadIdx.x, col = lane & 15;
+    const int g = blockIdx.x - tile_at * a.kv_heads, group = a.heads / a.kv_heads, lane = threadIdx.x, col = lane & 15;
     const int passes = (group + 15) / 16;
     for (int h0 = 0; h0 < group; h0 += 16) {
         const bool on = h0 + col < group;
@@ -605,7 +663,7 @@ __global__ __launch_bounds__(kWave) void masked_attention_bf16_join_kernel(Maske
             for (int t = 0; t < DVB; ++t) st.o[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
         for (int z = 0; z < a.zsplits; ++z) {
-            const float* its = a.shares + ((((size_t)blockIdx.x * a.kv_heads + g) * passes + h0 / 16) * a.zsplits + z)
+            const float* its = a.shares + (((size_t)blockIdx.x * passes + h0 / 16) * a.zsplits + z)
                                               * kWave * MAPS * share_floats<DVB>() + (size_t)lane * MAPS * share_floats<DVB>();
 #pragma unroll
             for (int m = 0; m < MAPS; ++m) {
@@ -693,7 +751,8 @@ LC_API int lc_masked_attention_bf16(const void* q, const void* k_cache, const vo
     if (staged_lds < meet_lds) staged_lds = meet_lds;
     a.lone_only = staged ? 1 : 0;
     const bool main_kernel = !staged || any_lone;
-    const dim3 grid(num_tiles, kv_heads, zsplits), join_grid(num_tiles, kv_heads);
+    LC_CHECK((long long)num_tiles * kv_heads < 1ll << 31, "masked attention: too many tiles");
+    const dim3 grid(num_tiles * kv_heads, 1, zsplits), join_grid(num_tiles * kv_heads);
     const int dsteps = (d + 31) / 32, dvb = dv / 16;
 #define LC_MB_AS(DS, VB, MP)                                                                                            \
     do {                                                                                                                \
