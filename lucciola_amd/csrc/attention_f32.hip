@@ -8,11 +8,11 @@
 //   O^T += V^T P^T: instruction r takes the keys 4 g + r, so those four weights are its operands as they stand and a lane's four
 //   keys of a dim are one 16-byte load.
 // Each product costs what the instruction costs (16 columns by 16 keys by 128 entries, both products: 2,048 clocks of a SIMD); float32
-// multiply-adds with a lane a key spend four instructions on one.  Against that kernel (us, heads of 128, rows cold in the caches of one
-// layer): 566 rows of three prompts of up to 333 tokens, 16 heads over 8, 119 -> 34; 2,048 rows, 32 over 8, 1,373 -> 515 (67 TFLOP/s
+// multiply-adds with a lane a key spend four instructions on one.  Against that kernel (us, heads of 128, the keys of one layer hot in the
+// caches): 566 rows of three prompts of up to 333 tokens, 16 heads over 8, 119 -> 27; 2,048 rows, 32 over 8, 1,373 -> 489 (70 TFLOP/s
 // of 157 over the keys that are seen; the rest is the weights between the products and the units that a row sees in part); 576 rows
-// after 8,192 tokens 2,806 -> 1,078; lone tokens, which wait for memory: 8 at 8,192 126 -> 110 (4.9 TB/s), 64 at 1,024 123 -> 111,
-// 1 at 8,192 39 -> 28.  Its errors against 64 bits are 5 to 30 % smaller, because sums are made in shorter chains.
+// after 8,192 tokens 2,806 -> 1,097; lone tokens, which wait for memory: 8 at 8,192 126 -> 112 (4.8 TB/s), 64 at 1,024 123 -> 105,
+// 1 at 8,192 39 -> 29.  Its errors against 64 bits are 5 to 30 % smaller, because sums are made in shorter chains.
 //
 // The order of the additions is a function of the column's query alone.  Keys go in units of 16 at multiples of 16 and in spans of 512
 // at multiples of 512; wave w of the four of a workgroup takes the units u % 4 == w.  A wave's maximum, sum and P.V of a span are
@@ -280,21 +280,22 @@ __device__ __forceinline__ void attend_columns(const F32Attention& a, int t0, in
     }
 }
 
-// grid (groups of rows, then lone rows; kv heads by batches of 16 query heads; spans).  A group's rows are worked together when they
+// grid (groups of rows, then lone rows, each with its kv heads by batches of 16 query heads side by side; 1; spans).  A group's rows are worked together when they
 // belong to one request, else request by request.
 template <int DB>
 __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_kernel(F32Attention a) {
     __shared__ __attribute__((aligned(16))) float lds[DB * 256 + AF_WAVES * (2 * AF_COLUMNS + DB * 256)];
     const int group = a.nh / a.nkv, per = min(group, AF_COLUMNS), batches = (group + per - 1) / per;
-    const int kvh = blockIdx.y / batches, h0 = kvh * group + blockIdx.y % batches * per;
+    const int columns = a.nkv * batches, at = blockIdx.x / columns, batch = blockIdx.x - at * columns;
+    const int kvh = batch / batches, h0 = kvh * group + batch % batches * per;
     const int heads = min(per, (kvh + 1) * group - h0);
-    if ((int)blockIdx.x >= a.groups) {
-        const int4 row = a.lone[blockIdx.x - a.groups];
+    if (at >= a.groups) {
+        const int4 row = a.lone[at - a.groups];
         attend_columns<DB>(a, row.x, 1, row.y, row.z, kvh, h0, heads, per, lds);
         return;
     }
     // the last groups, which mostly see the most keys, first
-    const int first = (a.groups - 1 - blockIdx.x) * a.rows, end = min(first + a.rows, a.T);
+    const int first = (a.groups - 1 - at) * a.rows, end = min(first + a.rows, a.T);
     for (int t = first; t < end;) {
         const int request = a.tok_req[t];
         int n = 1;
@@ -367,7 +368,7 @@ static int f32_spans(int T, int nh, int nkv, int d, int max_blocks, int page_siz
 template <int DB>
 static void launch_f32(const F32Attention& a, int lone, hipStream_t stream) {
     const int group = a.nh / a.nkv, batches = (group + AF_COLUMNS - 1) / AF_COLUMNS;
-    attention_f32_kernel<DB><<<dim3(a.groups + lone, a.nkv * batches, a.spans > 0 ? a.spans : 1), 64 * AF_WAVES, 0, stream>>>(a);
+    attention_f32_kernel<DB><<<dim3((a.groups + lone) * a.nkv * batches, 1, a.spans > 0 ? a.spans : 1), 64 * AF_WAVES, 0, stream>>>(a);
     if (a.spans > 0) attention_f32_join_kernel<DB><<<dim3(a.T, a.nh), 64 * AF_WAVES, 0, stream>>>(a);
 }
 
@@ -400,7 +401,7 @@ LC_API int lc_attention_f32(const void* q, int q_stride, const void* k_cache, co
     LC_CHECK(q && k_cache && v_cache && out && tok_req && positions && block_table && (lone == 0 || lone_rows), "attention: null pointer");
     LC_CHECK(lc_attention_f32_takes(q, q_stride, k_cache, v_cache, nh, nkv, d, page_size) && ((uintptr_t)out | (uintptr_t)lone_rows) % 16 == 0,
              "attention: heads of %d and pages of %d tokens, or unaligned operands, are the general kernel's", d, page_size);
-    LC_CHECK(nh <= 65535, "attention: too many heads (%d)", nh);
+    LC_CHECK(nh <= 65535 && 2ll * T * nh < 1ll << 31, "attention: too many heads (%d) for %d tokens", nh, T);
     const F32Cut cut = f32_cut(T, nh, nkv, together != 0, lone);
     const int spans = f32_spans(T, nh, nkv, d, max_blocks, page_size, cut);
     LC_CHECK(spans == 0 || (workspace && (uintptr_t)workspace % 16 == 0), "attention: T=%d with %d blocks needs a workspace", T, max_blocks);

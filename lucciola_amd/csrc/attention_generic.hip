@@ -2,7 +2,7 @@
 // float32 arithmetic throughout (scores, max, exp, sum, P.V).  One workgroup per token (per two
 // tokens of one request where a batch is mostly rows of prompts) and up to four query heads of
 // one kv head, which share every key and value they load.  (float32 heads of 16, 32, ... 128 in pages of whole groups of four tokens
-// have a kernel on the matrix instruction, attention_f32.hip: 566 rows of three prompts 119 -> 34 us, 8 lone tokens at 8,192 126 -> 110.)
+// have a kernel on the matrix instruction, attention_f32.hip: 566 rows of three prompts 119 -> 27 us, 8 lone tokens at 8,192 126 -> 112.)
 //
 // Formulas (reference: plain form src/kernels/attention.cu:51-67,84-107,129-144; paged decode
 // src/kernels/attention_paged.cu:68-140):

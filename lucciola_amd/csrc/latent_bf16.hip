@@ -40,7 +40,7 @@ template <int NR, int KS>
 __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     const bf16* __restrict__ qa, int H, int R, int rot, const bf16* __restrict__ cache,
     const int* __restrict__ tiles, const int* __restrict__ block_table, int max_blocks, int page_size,
-    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int per_tile,
+    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int per_tile, int blocks_y,
     float* __restrict__ part_o, float* __restrict__ part_ml) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int Dk = R + rot, Dp = KS * 32;
@@ -54,10 +54,11 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     // waves share every SIMD
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 7, half = (tid >> 6) & 1, col = lane & 15, g = lane >> 4;
     constexpr int NH = NR / 2;
-    const int* tile = tiles + 4 * blockIdx.x;
+    const int tile_at = blockIdx.x / blocks_y;      // a tile's heads are neighbours: the longest tiles start first, with all of their heads
+    const int* tile = tiles + 4 * tile_at;
     const int t0 = tile[0], ntok = tile[1], req = tile[2], p0 = tile[3];
     const bool lone = ntok == 1;
-    const int h0 = blockIdx.y * (lone ? 64 : 4);
+    const int h0 = (int)(blockIdx.x - tile_at * blocks_y) * (lone ? 64 : 4);
     if (h0 >= H) return;
     // this lane's query column
     const int q_tok = lone ? 0 : col, q_head = lone ? h0 + 16 * wave + col : h0 + wave;
@@ -271,7 +272,7 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
             }
     } else {
         // a share's place goes by token, or (per_tile > 0) by tile, where the step holds tokens that are in no tile
-        const size_t place = per_tile ? ((size_t)blockIdx.x * per_tile + q_tok) * H + q_head : qi;
+        const size_t place = per_tile ? ((size_t)tile_at * per_tile + q_tok) * H + q_head : qi;
         float* dst = part_o + (place * splits + blockIdx.z) * R;
 #pragma unroll
         for (int d = 0; d < NH; ++d)
@@ -435,7 +436,8 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
     }
     const int blocks_y = portions ? (H + 3) / 4 : (H + 63) / 64;
     LC_CHECK(blocks_y <= 65535, "latent attention: too many heads (%d)", H);
-    const dim3 grid(num_tiles, blocks_y, splits);
+    LC_CHECK((long long)num_tiles * blocks_y < 1ll << 31, "latent attention: too many tiles");
+    const dim3 grid(num_tiles * blocks_y, 1, splits);
     const size_t lds = sizeof(bf16) * ((size_t)LM_STAGE * (ks * 32 + LM_KPAD) + (size_t)R * LM_VSTRIDE) +
                        sizeof(int) * 2 * LM_STAGE;
 #define LC_LM_LAUNCH(NR, KS)                                                                                       \
@@ -446,7 +448,7 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
                      "latent attention: %zu bytes of LDS refused", lds);                                           \
         latent_attention_bf16_kernel<NR, KS><<<grid, LM_THREADS, lds, stream>>>(                                    \
             (const bf16*)qa, H, R, rot, (const bf16*)cache, tiles, block_table, max_blocks, page_size, scale, window, \
-            sink, (bf16*)out, splits, per_tile, part_o, part_ml);                                                     \
+            sink, (bf16*)out, splits, per_tile, blocks_y, part_o, part_ml);                                           \
     } while (0)
     if (nr == 4) LC_LM_LAUNCH(4, 4);
     else if (nr == 8) LC_LM_LAUNCH(8, 8);
