@@ -81,11 +81,21 @@ __device__ __forceinline__ void lds_four(bf16x8 (&r)[4], unsigned a, unsigned b,
 // base 2 against a reference point that moves when a score outgrows it by 2^8; O^T += V^T P^T.  A stage of 64 keys (40 KB) comes
 // straight into LDS while the one before is worked through; 16-byte chunks lie at places xor the row, so that no operand's 16
 // rows meet a bank twice.  Two workgroups a CU, whose waves fill each other's waits.
-__global__ __launch_bounds__(256, 2) void latent_wide_kernel(WideArgs a) {
+//
+// HALVES 2: eight waves, of which four take every other stage of the same queries, with a ring of their own; their sums are joined at the
+// end.  A stage keeps a wave busy for 2.2 us where it is alone on its SIMD (its loads, products and weights wait for each other) and
+// two waves for little more, so where there are no more workgroups than two a CU the halves are the second wave, and they halve the
+// longest chain (us, one and two halves: 2,048 tokens of 16 heads 67 and 52, behind 2,048 others 129 and 98, 512 behind 4,000 129 and
+// 97; 4,000 tokens, 512 workgroups, 133 and 107).  With more workgroups a CU has its second wave anyway, and the halves only wait for
+// each other (768 workgroups 93 and 124, 1,024 354 and 380).
+template <int HALVES>
+__global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a) {
     constexpr int KB = LW_KEYS * LW_DIM * 2, TB = LW_KEYS * LW_ROT * 2, VB = LW_VDIM * LW_KEYS * 2, STAGE = KB + TB + VB;
     constexpr int KS = (LW_DIM + LW_ROT) / 16, VT = LW_VDIM / 32;
-    __shared__ __attribute__((aligned(1024))) char lds[2 * STAGE];
-    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), col = lane & 31, half = lane >> 5;
+    __shared__ __attribute__((aligned(1024))) char all_lds[HALVES * 2 * STAGE];
+    const int lane = threadIdx.x & 63, col = lane & 31, half = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) & 3, part = __builtin_amdgcn_readfirstlane(threadIdx.x >> 8);
+    char* lds = all_lds + part * 2 * STAGE;
     const int head = blockIdx.x, tile = gridDim.y - 1 - blockIdx.y;
     const int row = tile * LW_TOKENS + wave * 32 + col;     // the lane's token of the portion
     const bool live = row < a.tokens;
@@ -124,8 +134,8 @@ __global__ __launch_bounds__(256, 2) void latent_wide_kernel(WideArgs a) {
         const int key = 16 * wave + 8 * i + r8;
         t_from[i] = a.turned + (size_t)key * LW_ROT + (((lane & 7) ^ ((key >> 1) & 7)) * 8);
     }
-    auto issue = [&](int s) {
-        char* stage = lds + (s & 1) * STAGE;
+    auto issue = [&](int s, int turn) {
+        char* stage = lds + (turn & 1) * STAGE;
 #pragma unroll
         for (int i = 0; i < 4; ++i)
             __builtin_amdgcn_global_load_lds((glb_ptr_t)(k_from[i] + (size_t)s * LW_KEYS * a.H * LW_DIM),
@@ -152,15 +162,17 @@ __global__ __launch_bounds__(256, 2) void latent_wide_kernel(WideArgs a) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[i][v] = 0.f;
     float m_ref = -INFINITY, l = 0.f;
-    if (s_begin < s_end) issue(s_begin);
-    for (int s = s_begin; s < s_end; ++s) {
+    if (s_begin + part < s_end) issue(s_begin + part, 0);
+    const int turns = (s_end - s_begin + HALVES - 1) / HALVES;
+    for (int turn = 0; turn < turns; ++turn) {
+        const int s = s_begin + part + turn * HALVES;
         wait_vmcnt<0>();                                    // this wave's loads of the stage have landed
         __builtin_amdgcn_s_barrier();                       // everybody's have; nobody reads the other stage any more
         asm volatile("" ::: "memory");
-        if (s + 1 < s_end) issue(s + 1);
+        if (s + HALVES < s_end) issue(s + HALVES, turn + 1);
         const int c0 = s * LW_KEYS;
-        if (!wave_live || c0 > wave_hi || c0 + LW_KEYS <= wave_lo) continue;
-        const unsigned stage = (s & 1) * STAGE;
+        if (!wave_live || s >= s_end || c0 > wave_hi || c0 + LW_KEYS <= wave_lo) continue;
+        const unsigned stage = (turn & 1) * STAGE;
         floatx16 sc[2];
 #pragma unroll
         for (int t = 0; t < 2; ++t) {
@@ -228,6 +240,30 @@ __global__ __launch_bounds__(256, 2) void latent_wide_kernel(WideArgs a) {
             for (int b = 0; b < 4; ++b) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[b], p[b], o[i], 0, 0, 0);
         }
     }
+    if constexpr (HALVES == 2) {
+        static_assert((VT * 16 + 2) * 256 * 4 <= HALVES * 2 * STAGE, "the second half's sums");
+        float* its = reinterpret_cast<float*>(all_lds) + (threadIdx.x & 255);       // [m, l, the sums][thread]
+        __syncthreads();                                    // nobody reads a stage any more
+        if (part == 1) {
+            its[0] = m_ref;
+            its[256] = l;
+#pragma unroll
+            for (int i = 0; i < VT; ++i)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) its[(2 + 16 * i + v) * 256] = o[i][v];
+        }
+        __syncthreads();
+        if (part == 1) return;
+        const float m_its = its[0], m_all = fmaxf(m_ref, m_its);
+        const float mine = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_all);
+        const float by = m_its == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_its - m_all);
+        l = fmaf(l, mine, its[256] * by);
+#pragma unroll
+        for (int i = 0; i < VT; ++i)
+#pragma unroll
+            for (int v = 0; v < 16; ++v) o[i][v] = fmaf(o[i][v], mine, its[(2 + 16 * i + v) * 256] * by);
+        m_ref = m_all;
+    }
     if (!live) return;
     l += __shfl_xor(l, 32, kWave);
     float inv = 1.f / l;
@@ -259,6 +295,15 @@ __global__ __launch_bounds__(256, 2) void latent_wide_kernel(WideArgs a) {
 }  // namespace lc
 
 using namespace lc;
+
+static thread_local int g_wide_halves = 0;
+
+// Tests and tuning: 1 or 2 halves for the calling thread's launches, 0 lets the size decide.  Returns the setting before.
+LC_API int lc_latent_wide_halves(int halves) {
+    const int before = g_wide_halves;
+    if (halves >= 0 && halves <= 2) g_wide_halves = halves;
+    return before;
+}
 
 // Whether these heads have a kernel.
 LC_API int lc_latent_wide_supported(int R, int dim, int rot, int vdim) {
@@ -297,7 +342,9 @@ LC_API int lc_latent_wide(const void* q, long long ldq, const void* q_turned, lo
     WideArgs a{(const bf16*)q, ldq, (const bf16*)q_turned, q_row, q_head, (const bf16*)keys, (const bf16*)turned, (const bf16*)values, ldv,
                H, first, tokens, position, lo, scale * 1.4426950408889634f, window, sink, (const bf16*)gate, ldg, gate_head,
                (bf16*)out, ldo};
-    latent_wide_kernel<<<dim3(H, tiles), 256, 0, stream>>>(a);
+    const int halves = g_wide_halves ? g_wide_halves : (long long)H * tiles <= 2 * device_cus() ? 2 : 1;
+    if (halves == 2) latent_wide_kernel<2><<<dim3(H, tiles), 512, 0, stream>>>(a);
+    else latent_wide_kernel<1><<<dim3(H, tiles), 256, 0, stream>>>(a);
     LC_LAUNCH_CHECK("latent_wide");
     return 0;
 }

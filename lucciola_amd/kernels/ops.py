@@ -95,6 +95,7 @@ _SIGNATURES = {
     "lc_latent_lone_picks": "iiiii",
     "lc_latent_lone_splits": "ii",
     "lc_latent_wide_supported": "iiii",
+    "lc_latent_wide_halves": "i",
     "lc_latent_rows": "ppiiiiiippp",
     "lc_latent_wide": "pqpqqpppqiiiiifippqqpqp",
     "lc_latent_bf16_splits": "ii",

@@ -34,10 +34,13 @@ def reference(q, turned_q, c, turned, uk, uv, position, scale, window, sink):
     return e @ v / (e.sum(1, keepdim=True) + (torch.exp(sink - top) if sink is not None else 0.0))
 
 
-@pytest.mark.parametrize("heads,rank,page,window,gate,with_sink,requests", [
+WIDE_CASES = [
     (2, 512, 16, 0, "entry", False, [(0, 64)]), (3, 64, 16, 0, "head", True, [(0, 65), (63, 127), (100, 128)]),
     (1, 128, 4, 50, "none", True, [(0, 129), (200, 300)]), (2, 192, 32, 64, "entry", False, [(7, 191), (64, 64)]),
-    (1, 512, 16, 0, "none", False, [(1000, 257)])])
+    (1, 512, 16, 0, "none", False, [(1000, 257)])]
+
+
+@pytest.mark.parametrize("heads,rank,page,window,gate,with_sink,requests", WIDE_CASES)
 def test_wide(heads, rank, page, window, gate, with_sink, requests):
     g = torch.Generator().manual_seed(heads * 1000 + rank + window)
     def made(*shape):
@@ -87,6 +90,18 @@ def test_wide(heads, rank, page, window, gate, with_sink, requests):
             bound = 3 * 2.0 ** -9 * float(rows.abs().max().clamp(min=4.0))
             assert float((got - want).abs().max()) <= bound, (r, h)
             assert float((got - want).norm() / want.norm()) <= 2.0 ** -8, (r, h)
+
+
+@pytest.mark.parametrize("halves", [1, 2])
+def test_wide_in_halves(halves):
+    """Both forms of the kernel, whatever the size would choose: stages in one row, and every other stage for each half, with a last
+    one that only one half has, windows that begin inside a stage and waves whose queries see none."""
+    before = ops.library().lc_latent_wide_halves(halves)
+    try:
+        for case in WIDE_CASES:
+            test_wide(*case)
+    finally:
+        ops.library().lc_latent_wide_halves(before)
 
 
 def test_short_portions_keep_their_tiles():
