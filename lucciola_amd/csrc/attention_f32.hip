@@ -46,10 +46,11 @@ __device__ __forceinline__ size_t part_at(const F32Attention& a, int D, int t, i
     return ((((size_t)t * a.nh + h) * a.spans + span) * AF_WAVES + wave) * (D + 4);
 }
 
-// The running (M, L, O) takes in (m, l, o); m = -inf: there were no keys.  Explicit operations, so that all who use it round alike.
+// The running (M, L, O) takes in (m, l, o); m = -inf and l = 0: there were no keys.  (Scores that are all NaN leave m at -inf too, for a
+// maximum passes NaN by, but their weights make l NaN.)  Explicit operations, so that all who use it round alike.
 template <int N>
 __device__ __forceinline__ void take_sums(float& M, float& L, floatx4 (&O)[N], float m, float l, const floatx4 (&o)[N]) {
-    if (m == -INFINITY) return;
+    if (m == -INFINITY && l == 0.f) return;
     const float top = fmaxf(M, m), a = expf(M - top), b = expf(m - top);
     L = fmaf(L, a, __fmul_rn(l, b));
 #pragma unroll

@@ -61,3 +61,25 @@ def test_a_value_that_is_not_finite_reaches_only_who_sees_it(bad, window):
     sees = sees.view(length, nh * d)
     assert torch.equal(got[~sees], clean[~sees])
     assert not torch.isfinite(got[sees]).any()
+
+
+@pytest.mark.parametrize("spoilt", [(16, 32), (0, 16), (48, 60), (512, 1024), (530, 531)])
+@pytest.mark.parametrize("rows", [1, 4])
+def test_keys_that_are_not_a_number_are_not_passed_by(spoilt, rows):
+    """All keys that a wave (of a unit of 16) or a workgroup (of a span of 512) sees are NaN: their scores leave no maximum, and the query that
+    sees them gets NaN and not the other keys' mean."""
+    nh, nkv, d, page, length = 4, 2, 32, 16, 60 if spoilt[1] <= 60 else 1100
+    qkv, batch, kc, vc = paged_case([length], [length if length < 100 else 700], nh, nkv, d, page, torch.float32, seed=9)
+    clean = run(qkv, batch, kc, vc, nh, nkv, d, page, 0, rows=rows)
+    for j in range(*spoilt):
+        kc[batch.block_table[0, j // page].item(), 1, j % page] = float("nan")
+    got = run(qkv, batch, kc, vc, nh, nkv, d, page, 0, rows=rows)
+    sees = torch.zeros(qkv.shape[0], nh, d, dtype=torch.bool, device=DEV)
+    sees[batch.positions >= spoilt[0], 2:] = True
+    sees = sees.view(got.shape)
+    assert torch.equal(got[~sees], clean[~sees])
+    assert torch.isnan(got[sees]).all()
+    # lone tokens, their spans shared out
+    alone, last, k2, v2 = paged_case([length], [1], nh, nkv, d, page, torch.float32, seed=9)
+    got = run(qkv[-1:].contiguous(), last, kc, vc, nh, nkv, d, page, 0)
+    assert torch.isnan(got[0, 2 * d:]).all() and torch.isfinite(got[0, :2 * d]).all()
