@@ -1,6 +1,8 @@
 // out[M, N] = x[M, K] . w[N, K]^T for float32 x and bfloat16 w as a true 32-bit product on the bfloat16 matrix instruction: a float32
 // number is the sum of three bfloat16 numbers, cut off after 8 bits each (24 in all, so nothing is left over), the product of two
-// bfloat16 numbers is exact in float32, and v_mfma_f32_32x32x16_bf16 adds in float32.  Three such products cost 3/16 of what
+// bfloat16 numbers is exact in float32, and v_mfma_f32_32x32x16_bf16 adds in float32.  x is cut times 2^40: the last bit of the smallest
+// float32, 2^-149, then stands at 2^-109, inside bfloat16's range (as they stand, entries below 2^-110 lose their last bits: 2e-5 of one at
+// 1e-36), and a chunk's sum is taken times 2^-40.  Three such products cost 3/16 of what
 // v_mfma_f32_16x16x4_f32 takes for the same sums (gemm_generic.hip, which serves float32 w and a K that is not whole).
 //
 // The order of the additions is a function of the output element alone: K goes in steps of 16, the smallest third of x first, in
@@ -11,13 +13,15 @@
 // us, gemm_generic.hip and these (weights of several products in turn): 566 rows, 6,144 x 1,024 77 and 38, 1,024 x 3,072 45 and 31, 151,936 x
 // 1,024 1,541 and 878; 2,048 rows, 24,576 x 4,096 3,025 and 1,627 (253 TFLOP/s, 0.76 of 10^15 products a second); 64 rows, 24,576 x 4,096 146
 // and 99; 8 rows 78 and 56 (bound by w: 201 MB); 1 row, 6,144 x 1,024 17 and 13.  Errors against 64 bits 2.9e-7 and 1.7e-7, because
-// 16 products are added at a time.  What bounds the tiles is the vector unit, which cuts x once for every 64 columns (5.5
+// 16 products are added at a time.  What bounds the tiles is the vector unit, which cuts x once for every 64 columns (4.5
 // instructions an entry), and LDS, where the parts are written and read; larger tiles of w need more registers than there
 // are (128 x 128 spills), x in the operands' layout past LDS is cut by every wave (566 rows, 6,144 x 1,024 85 us in tiles of 64 x 64), and
 // blocks of 64 k or loads two blocks ahead are slower (64 and 63).
 //
-// x is cut on its way from registers to LDS.  Infinite entries have no such parts (inf - inf), and three parts of x times an
-// infinite w are not x times it; both give NaN, and a chunk's sum that is NaN is made again from x and w as they are.
+// x is cut on its way from registers to LDS (an entry's remainder is one v_dot2_f32_bf16 with its pair of upper halves; a pair with an
+// infinite entry spoils both of its entries, which are one row's).  Infinite entries have no such parts (inf - inf), nor have those of 2^88 and more, three parts
+// of x times an infinite w are not x times it, and sums of 2^88 leave the range; all of them give infinity or NaN, and a chunk's sum that is
+// not finite is made again from x and w as they are.
 #include "common.h"
 
 #include "gemm_split.h"
@@ -27,18 +31,30 @@ namespace lc {
 
 constexpr int GS_CHUNK = 256;
 
-// Eight neighbouring entries of x -> their three parts, operands of a product each.
+typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+constexpr float GS_UP = 0x1p40f, GS_DOWN = 0x1p-40f;
+
+// Eight neighbouring entries of x, times GS_UP -> their three parts, operands of a product each.
 __device__ __forceinline__ void cut_in_three(const float4& lo, const float4& hi, bf16x8 (&parts)[3]) {
     float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
 #pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] *= GS_UP;
+    // (-1, 0) and (0, -1), from registers: as a constant of the instruction -1 is read into the upper half
+    unsigned first_bits = 0x0000BF80u, second_bits = 0xBF800000u;
+    asm("" : "+s"(first_bits), "+s"(second_bits));
+    const bf16x2 first = __builtin_bit_cast(bf16x2, first_bits), second = __builtin_bit_cast(bf16x2, second_bits);
+#pragma unroll
     for (int part = 0; part < 3; ++part) {
-        unsigned pairs[4];
+        bf16x2 pairs[4];
 #pragma unroll
-        for (int e = 0; e < 8; e += 2)              // the upper halves of two entries
-            pairs[e / 2] = __builtin_amdgcn_perm(__float_as_uint(v[e + 1]), __float_as_uint(v[e]), 0x07060302u);
-        parts[part] = __builtin_bit_cast(bf16x8, make_uint4(pairs[0], pairs[1], pairs[2], pairs[3]));
-#pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] -= __uint_as_float(__float_as_uint(v[e]) & 0xFFFF0000u);
+        for (int e = 0; e < 8; e += 2) {            // the upper halves of two entries, and what they leave: one instruction an entry
+            pairs[e / 2] = __builtin_bit_cast(bf16x2, __builtin_amdgcn_perm(__float_as_uint(v[e + 1]), __float_as_uint(v[e]), 0x07060302u));
+            if (part < 2) {
+                v[e] = __builtin_amdgcn_fdot2_f32_bf16(pairs[e / 2], first, v[e], false);
+                v[e + 1] = __builtin_amdgcn_fdot2_f32_bf16(pairs[e / 2], second, v[e + 1], false);
+            }
+        }
+        parts[part] = __builtin_bit_cast(bf16x8, pairs);
     }
 }
 
@@ -62,7 +78,7 @@ __device__ __forceinline__ bf16x8 load8(const bf16* from) {
     return v;
 }
 
-// A chunk's sum that is NaN, from x and w as they are.
+// A chunk's sum that is not finite, from x and w as they are.
 __device__ __forceinline__ float plain_sum(const float* x, const bf16* w, int k0, int k1) {
     float sum = 0.f;
 #pragma unroll 1
@@ -187,7 +203,10 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(const float
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) bad = bad || acc[i][j][v] != acc[i][j][v];
+                for (int v = 0; v < 16; ++v) {
+                    acc[i][j][v] *= GS_DOWN;
+                    bad = bad || !(fabsf(acc[i][j][v]) < INFINITY);
+                }
         if (__any(bad)) {
 #pragma unroll
             for (int i = 0; i < TM; ++i)
@@ -195,7 +214,7 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_split_kernel(const float
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
                     for (int v = 0; v < 16; ++v)
-                        if (acc[i][j][v] != acc[i][j][v])
+                        if (!(fabsf(acc[i][j][v]) < INFINITY))
                             acc[i][j][v] = plain_sum(x + (size_t)min(m_of(i, v), M - 1) * K, w + (size_t)min(n_of(j), N - 1) * K,
                                                      c * GS_CHUNK, k_end);
         }
@@ -279,11 +298,14 @@ __global__ __launch_bounds__(256, 2) void gemm_split_few_kernel(const float* __r
                 }
         bool bad = false;
 #pragma unroll
-        for (int v = 0; v < 8; ++v) bad = bad || acc[v] != acc[v];      // the rows up to 15
+        for (int v = 0; v < 8; ++v) {           // the rows up to 15
+            acc[v] *= GS_DOWN;
+            bad = bad || !(fabsf(acc[v]) < INFINITY);
+        }
         if (__any(bad)) {
 #pragma unroll
             for (int v = 0; v < 8; ++v)
-                if (acc[v] != acc[v])
+                if (!(fabsf(acc[v]) < INFINITY))
                     acc[v] = plain_sum(x + (size_t)min((v >> 2) * 8 + kg * 4 + (v & 3), M - 1) * K, w + (size_t)min(n, N - 1) * K, k0, k_end);
         }
 #pragma unroll

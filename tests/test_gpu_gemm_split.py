@@ -36,19 +36,27 @@ def test_edges(M, N, K):
     assert torch.equal(product(x[M // 2:M // 2 + 1].contiguous(), w)[0], got[M // 2])
 
 
-@pytest.mark.parametrize("M", [3, 40])
+@pytest.mark.parametrize("M", [7, 40])
 @pytest.mark.parametrize("K", [288, 4096])
 def test_entries_without_parts(M, K):
-    """Infinite and not-a-number entries, the largest and the smallest numbers: what the float32 instruction makes of them."""
+    """Infinite and not-a-number entries reach the outputs that 64 bits give them to; the largest and the smallest numbers, each with rows of
+    their own that hold nothing larger, lose nothing."""
     g = torch.Generator().manual_seed(K)
     x, w = torch.randn(M, K, generator=g).to(DEV), torch.randn(130, K, generator=g).bfloat16().to(DEV)
     x[0, 5], x[1, 270], x[2, 7] = float("inf"), float("nan"), -float("inf")
     w[3, 9], w[4, 271] = float("inf"), float("nan")
     w[5, 5] = 0.0
-    x[2, 20:24] = torch.tensor([3.4028235e38, -3.4028235e38, 1e-40, -1.1754944e-38])
-    w[:, 20:22] = 0.0
-    got, plain = product(x, w), product(x, w, plain=1)
-    same = torch.isfinite(plain)
-    assert torch.equal(torch.isnan(got), torch.isnan(plain)) and torch.equal(torch.isposinf(got), torch.isposinf(plain))
-    assert torch.equal(torch.isneginf(got), torch.isneginf(plain))
-    torch.testing.assert_close(got[same], plain[same], rtol=1e-5, atol=1e-4)
+    x[3, 20:22] = torch.tensor([3.4028235e38, -3.4028235e38])
+    w[:, 20] = 2.0 ** -10
+    w[:, 21] = 2.0 ** -12
+    x[4] *= 1e-36
+    x[5] *= 1.2e-38
+    x[6] *= 1e-41
+    got, want = product(x, w).double(), x.double() @ w.double().T
+    same = torch.isfinite(want)
+    assert torch.equal(torch.isnan(got), torch.isnan(want)) and torch.equal(torch.isposinf(got), torch.isposinf(want))
+    assert torch.equal(torch.isneginf(got), torch.isneginf(want))
+    assert bool(same[3:].any(dim=1).all()), "every row has outputs to compare"
+    # as in test_edges, and the results, chunk by chunk, rounded to multiples of 2^-149
+    allowed = 2.0 ** -24 * K * (x.double().abs() @ w.double().abs().T) + 2.0 ** -149 * (1 + K // 256)
+    assert bool(((got - want).abs()[same] <= allowed[same]).all())
