@@ -180,7 +180,7 @@ __global__ __launch_bounds__(256, 2) void gemm_grouped_kernel(GroupedArgs a) {
                     float v = total[i][j][r];
                     if (a.epilogue == ACT_SIGMOID_GATE) v *= sigmoid(to_f32(gate[(size_t)m * a.ldg + n]));
                     else if (a.epilogue == ACT_SIGMOID_GROUP_GATE) v *= sigmoid(to_f32(gate[(size_t)m * a.ldg]));
-                    else v = activate(v, a.epilogue);
+                    else v = activate<TO>(v, a.epilogue);
                     out[(size_t)m * a.ldo + n] = from_f32<TO>(v);
                 }
             }
@@ -300,7 +300,7 @@ __global__ __launch_bounds__(256, 2) void gemm_grouped_bf16_kernel(GroupedArgs a
                     float v = acc[i][j][r];
                     if (a.epilogue == ACT_SIGMOID_GATE) v *= sigmoid(to_f32(gate[(size_t)m * a.ldg + n]));
                     else if (a.epilogue == ACT_SIGMOID_GROUP_GATE) v *= sigmoid(to_f32(gate[(size_t)m * a.ldg]));
-                    else v = activate(v, a.epilogue);
+                    else v = activate<TO>(v, a.epilogue);
                     out[(size_t)m * a.ldo + n] = from_f32<TO>(v);
                 }
             }

@@ -23,11 +23,12 @@
 
 namespace lc {
 
-// One element's epilogue.
+// One element's epilogue, for a result of type TO.
+template <typename TO>
 __device__ __forceinline__ float grouped_finish(const GroupedArgs& a, const bf16* gate, int m, int n, float v) {
     if (a.epilogue == ACT_SIGMOID_GATE) return v * sigmoid(to_f32(gate[(size_t)m * a.ldg + n]));
     if (a.epilogue == ACT_SIGMOID_GROUP_GATE) return v * sigmoid(to_f32(gate[(size_t)m * a.ldg]));
-    return activate(v, a.epilogue);
+    return activate<TO>(v, a.epilogue);
 }
 
 // grid (column tiles, row tiles, groups or 1): neighbouring workgroups, which go to different XCDs, take different columns
@@ -75,8 +76,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_grouped_tiled_kernel(Groupe
                     const float got = lane_swap<0xB1>(odd ? first : second);    // lane ^ 1
                     const int row = m + (odd ? 1 : 0);
                     if (row < tile.end && pair < N)
-                        store_pair<TO>(out + (size_t)row * a.ldo + pair, grouped_finish(a, gate, row, pair, odd ? got : first),
-                                       grouped_finish(a, gate, row, pair + 1, odd ? second : got));
+                        store_pair<TO>(out + (size_t)row * a.ldo + pair, grouped_finish<TO>(a, gate, row, pair, odd ? got : first),
+                                       grouped_finish<TO>(a, gate, row, pair + 1, odd ? second : got));
                 }
     } else {
 #pragma unroll
@@ -86,7 +87,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_grouped_tiled_kernel(Groupe
 #pragma unroll
                 for (int v = 0; v < 16; ++v) {
                     const int m = m0 + i * 32 + (v >> 2) * 8 + (v & 3), n = c0 + j * 32;
-                    if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish(a, gate, m, n, acc[i][j][v]));
+                    if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish<TO>(a, gate, m, n, acc[i][j][v]));
                 }
     }
 }
@@ -246,15 +247,15 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGat
         };
         if constexpr (GATED) {
             if (gate.kind == 0) unrolled([](float g, float u) { return gated_f(g, u, kSilu); });
-            else unrolled([](float g, float u) { return gelu_tanh_fast(g) * u; });
+            else unrolled([](float g, float u) { return gelu_tanh<bf16>(g) * u; });
         } else {
             switch (a.epilogue) {
                 case ACT_NONE: unrolled([](float z, float) { return z; }); break;
-                case ACT_RELU_SQUARED: unrolled([](float z, float) { return activate(z, ACT_RELU_SQUARED); }); break;
-                case ACT_GELU_ERF: rolled([](float z, float) { return activate(z, ACT_GELU_ERF); }); break;
+                case ACT_RELU_SQUARED: unrolled([](float z, float) { return activate<TO>(z, ACT_RELU_SQUARED); }); break;
+                case ACT_GELU_ERF: rolled([](float z, float) { return activate<TO>(z, ACT_GELU_ERF); }); break;
                 default:
-                    if constexpr (sizeof(TO) == 2) unrolled([](float z, float) { return gelu_tanh_fast(z); });
-                    else rolled([](float z, float) { return activate(z, ACT_GELU_TANH); });
+                    if constexpr (sizeof(TO) == 2) unrolled([](float z, float) { return gelu_tanh<TO>(z); });
+                    else rolled([](float z, float) { return gelu_tanh<TO>(z); });
             }
         }
     };
@@ -379,7 +380,7 @@ __global__ __launch_bounds__(256) void gemm_grouped_stream_kernel(GroupedArgs a)
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
         const int m = tile.first + 4 * quad + i;
-        if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish(a, gate, m, n, acc[i]));
+        if (m < tile.end && n < N) store_out<TO>(out + (size_t)m * a.ldo + n, grouped_finish<TO>(a, gate, m, n, acc[i]));
     }
 }
 

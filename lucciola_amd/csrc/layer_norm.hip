@@ -161,8 +161,8 @@ __global__ void embedding_sinusoid_kernel(const int* __restrict__ ids, const int
     }
 }
 
-// A thread per VEC neighbouring entries of a row (grid: pieces of a row, rows).  Results in bfloat16 take the hardware's exp and reciprocal:
-// 2,039 rows of 2 x 8,192 with the tanh form 34 us with a thread an entry, a 64-bit division and tanhf, 17 now.
+// A thread per VEC neighbouring entries of a row (grid: pieces of a row, rows).  2,039 rows of 2 x 8,192 with the tanh form 34 us with a
+// thread an entry, a 64-bit division and tanhf, 17 now.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void gated_activation_kernel(const T* __restrict__ gu, T* __restrict__ out, int I, int kind, float limit,
                                                                float slope, float shift, int rows) {
@@ -183,7 +183,7 @@ __global__ __launch_bounds__(256) void gated_activation_kernel(const T* __restri
             } else if (kind == 0) {
                 y[e] = from_f32<T>(silu(g) * u);
             } else {
-                y[e] = from_f32<T>((sizeof(T) == 2 ? gelu_tanh_fast(g) : activate(g, ACT_GELU_TANH)) * u);
+                y[e] = from_f32<T>(gelu_tanh<T>(g) * u);
             }
         }
         *reinterpret_cast<piece*>(out + (size_t)t * I + i) = y;

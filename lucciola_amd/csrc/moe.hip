@@ -295,7 +295,7 @@ __global__ void gated_activation_weighted_kernel(const T* __restrict__ gu, T* __
         const size_t row = (size_t)entry_row[e];
         const float w = weights[e];
         const float g = w * to_f32(gu[row * 2 * I + i]), u = w * to_f32(gu[row * 2 * I + I + i]);
-        out[row * I + i] = from_f32<T>((kind == 0 ? g * sigmoid(g) : activate(g, ACT_GELU_TANH)) * u);
+        out[row * I + i] = from_f32<T>((kind == 0 ? g * sigmoid(g) : gelu_tanh<T>(g)) * u);
     }
 }
 

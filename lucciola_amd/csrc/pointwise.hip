@@ -52,8 +52,8 @@ __global__ void stream_add_kernel(float* __restrict__ h, const T* __restrict__ d
     }
 }
 
-// VEC entries a thread and turn (total is a multiple).  The tanh form of bfloat16 entries takes the hardware's exp and reciprocal: 2,048 x
-// 8,192 21 us with an entry a thread and tanhf, 14 now.
+// VEC entries a thread and turn (total is a multiple): 2,048 x 8,192 bfloat16 entries, tanh form, 21 us with an entry a thread and tanhf, 14
+// now.
 template <typename T, int VEC>
 __global__ __launch_bounds__(256) void activation_kernel(T* __restrict__ x, int kind, float a, float b, size_t total) {
     typedef T piece __attribute__((ext_vector_type(VEC)));
@@ -63,7 +63,7 @@ __global__ __launch_bounds__(256) void activation_kernel(T* __restrict__ x, int 
         for (int e = 0; e < VEC; ++e) {
             const float z = to_f32(v[e]);
             v[e] = from_f32<T>(kind == ACT_XIELU ? xielu(z, a, b)
-                               : kind == ACT_GELU_TANH && sizeof(T) == 2 ? gelu_tanh_fast(z) : activate(z, kind));
+                               : activate<T>(z, kind));
         }
         *reinterpret_cast<piece*>(x + idx) = v;
     }

@@ -137,3 +137,31 @@ def test_heads(rows, G, N, K, gap):
             want = plain * torch.sigmoid(gate[:, 2:2 + G].float())[:, :, None]
         assert off_by(out[:, 3:], want.reshape(rows, G * N), K) <= 1.0, kind
         assert float(out[:, :3].abs().max()) == 0.0, "columns before the first group were written"
+
+
+@pytest.mark.parametrize("out", [torch.float32, torch.bfloat16])
+def test_one_gelu(out):
+    """The tanh form rounds alike in every product's epilogue and in the element-wise kernels, also where 1 + tanh cancels: a batch's size
+    decides which of them a token meets.  The sums are single products with one and so the same everywhere."""
+    z = torch.cat([torch.linspace(-12, 4, 500), torch.tensor([0.0, -40.0, 40.0, 1e4])]).bfloat16().to(DEV)
+    N, K, rows, E = z.shape[0], 128, 300, 2
+    x = torch.zeros(rows, K, dtype=torch.bfloat16, device=DEV)
+    x[:, 5] = 1
+    w = torch.zeros(E, N, K, dtype=torch.bfloat16, device=DEV)
+    w[:, :, 5] = z
+    alone = z.to(out).clone()[None].contiguous()
+    ops.activation(alone, "gelu_tanh")
+    ids = (torch.arange(rows, dtype=torch.int32, device=DEV) % E)[:, None].contiguous()
+    for tile in (16, 64, 128):
+        lists = torch.empty(2 * (E + 1) + 2 * rows, dtype=torch.int32, device=DEV)
+        starts, tiles = lists[:E + 1], lists[E + 1:2 * (E + 1)]
+        token, entry = lists[2 * (E + 1):2 * (E + 1) + rows], lists[2 * (E + 1) + rows:]
+        ops._call("lc_moe_lists", ops._ptr(ids), rows, 1, E, tile, ops._ptr(starts), ops._ptr(tiles), ops._ptr(token), ops._ptr(entry),
+                  ops._stream())
+        routing = ops.Routing(ids, torch.ones(rows, 1, device=DEV), starts, tiles, token, entry, E, tile, rows // tile + E)
+        for on in (0, 1, 2):
+            got = switched(on, lambda: ops.moe_experts(x, w, routing, out, activation="gelu_tanh", gather=True))
+            assert torch.equal(got, alone.expand(rows, N)), (tile, on)
+    both = torch.cat([z, torch.ones_like(z)]).to(out).expand(rows, 2 * N).contiguous()
+    assert torch.equal(ops.gated_activation(both, "gelu_tanh"), alone.expand(rows, N))
+    assert torch.equal(ops.gated_activation_weighted(both, "gelu_tanh", routing), alone.expand(rows, N))
