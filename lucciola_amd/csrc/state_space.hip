@@ -18,22 +18,24 @@ __device__ __forceinline__ float ss_softplus(float z) { return fmaxf(z, 0.f) + l
 // A thread per convolved entry and run of `tokens` tokens.  proj [T, cols]: x (heads dv) | B (groups N) | C (groups N) | z (heads dv) | dt
 // (heads); the first C = heads dv + 2 groups N columns pass the convolution.  The first x_blocks workgroups of a run take the channels of
 // x; the threads of the others a (group, n) pair each, make B and C at n and write them for every head of the group with the head's
-// own step and decay, which the workgroup makes once a (token, head) in LDS.  coef [3, T, heads N]; x_out [T, heads dv].
+// own step and decay, which the workgroup makes once a (token, head) in LDS (KEPT; else, where so many heads do not fit, every thread makes
+// those that it needs).  coef [3, T, heads N]; x_out [T, heads dv].
 // 2,048 tokens, 16 heads of 128, 4 groups of 128 entries: 83 us with a thread per (token, entry), a 64-bit division, four inputs
 // and every head's two exponentials each; 34 us.
-template <int KT>
+template <int KT, bool KEPT>
 __global__ __launch_bounds__(256) void state_space_prepare_kernel(
     const float* __restrict__ proj, int cols, int T, int heads, int groups, int N, int dv, const float* __restrict__ taps,
     const float* __restrict__ bias, int K, const float* __restrict__ tails, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
     const int* __restrict__ tok_req, const int* __restrict__ q_offsets, const int* __restrict__ slot_ids, float* __restrict__ coef,
-    float* __restrict__ x_out, int tokens, int x_blocks) {
+    float* __restrict__ x_out, int tokens, int x_blocks, int blocks) {
     extern __shared__ float rates[];                // [tokens][heads] steps, then as many decays
     const int inner = heads * dv, C = inner + 2 * groups * N, per_group = heads / groups;
-    const int t0 = blockIdx.x * tokens, t1 = min(t0 + tokens, T);
+    const int run_at = blockIdx.x / blocks, block = blockIdx.x - run_at * blocks;
+    const int t0 = run_at * tokens, t1 = min(t0 + tokens, T);
     const size_t plane = (size_t)T * heads * N;
     auto tail_of = [&](int r) { return K > 1 ? tails + (size_t)slot_ids[r] * (K - 1) * C : nullptr; };
-    if ((int)blockIdx.y < x_blocks) {
-        const int i = blockIdx.y * 256 + threadIdx.x;
+    if (block < x_blocks) {
+        const int i = block * 256 + threadIdx.x;
         if (i >= inner) return;
         ShortConvRun<KT> run;
         run.start(taps, i);
@@ -45,14 +47,18 @@ __global__ __launch_bounds__(256) void state_space_prepare_kernel(
         }
         return;
     }
-    for (int e = threadIdx.x; e < (t1 - t0) * heads; e += 256) {
-        const int t = t0 + e / heads, head = e % heads;
-        const float step = ss_softplus(proj[(size_t)t * cols + C + inner + head] + dt_bias[head]);
-        rates[e] = step;
-        rates[tokens * heads + e] = expf(-expf(a_log[head]) * step);
+    auto step_of = [&](int t, int head) { return ss_softplus(proj[(size_t)t * cols + C + inner + head] + dt_bias[head]); };
+    auto decay_of = [&](int head, float step) { return expf(-expf(a_log[head]) * step); };
+    if constexpr (KEPT) {
+        for (int e = threadIdx.x; e < (t1 - t0) * heads; e += 256) {
+            const int head = e % heads;
+            const float step = step_of(t0 + e / heads, head);
+            rates[e] = step;
+            rates[tokens * heads + e] = decay_of(head, step);
+        }
+        __syncthreads();
     }
-    __syncthreads();
-    const int i = (blockIdx.y - x_blocks) * 256 + threadIdx.x;
+    const int i = (block - x_blocks) * 256 + threadIdx.x;
     if (i >= groups * N) return;
     const int g = i / N, n = i % N, cb = inner + i, cc = inner + groups * N + i;
     ShortConvRun<KT> run_b, run_c;
@@ -68,8 +74,9 @@ __global__ __launch_bounds__(256) void state_space_prepare_kernel(
         for (int k = 0; k < per_group; ++k) {
             const int head = g * per_group + k, e = (t - t0) * heads + head;
             const size_t at = ((size_t)t * heads + head) * N + n;
-            coef[at] = rates[tokens * heads + e];
-            coef[plane + at] = rates[e] * b;
+            const float step = KEPT ? rates[e] : step_of(t, head);
+            coef[at] = KEPT ? rates[tokens * heads + e] : decay_of(head, step);
+            coef[plane + at] = step * b;
             coef[2 * plane + at] = c;
         }
     }
@@ -123,19 +130,19 @@ LC_API int lc_state_space_prepare(const float* proj, int cols, int T, int heads,
     int tokens = T >= 1024 ? 8 : T >= 256 ? 4 : 1;
     while (tokens > 1 && tokens * heads > 4096) tokens /= 2;
     const size_t lds = (size_t)2 * tokens * heads * sizeof(float);
-    LC_CHECK(lds <= 64 * 1024, "state space prepare: %d heads are too many", heads);
-    const int x_blocks = (heads * dv + 255) / 256;
-    const dim3 grid((T + tokens - 1) / tokens, x_blocks + (groups * N + 255) / 256);
-    LC_CHECK(grid.y <= 65535, "state space prepare: too many channels");
-#define LC_SS_PREPARE(KT)                                                                                                              \
-    state_space_prepare_kernel<KT><<<grid, 256, lds, stream>>>(proj, cols, T, heads, groups, N, dv, taps, bias, K, tails, dt_bias, a_log, \
-                                                               tok_req, q_offsets, slot_ids, coef, x_out, tokens, x_blocks)
-    switch (K) {
-        case 2: LC_SS_PREPARE(2); break;
-        case 3: LC_SS_PREPARE(3); break;
-        case 4: LC_SS_PREPARE(4); break;
-        default: LC_SS_PREPARE(0);
-    }
+    const bool kept = lds <= 64 * 1024;
+    const int x_blocks = (heads * dv + 255) / 256, blocks = x_blocks + (groups * N + 255) / 256;
+    const long long grid = (long long)((T + tokens - 1) / tokens) * blocks;
+    LC_CHECK(grid * 256 < 1ll << 32, "state space prepare: %d tokens of %d columns are too many", T, cols);
+#define LC_SS_PREPARE(KT, KEPT)                                                                                                           \
+    state_space_prepare_kernel<KT, KEPT><<<(int)grid, 256, KEPT ? lds : 0, stream>>>(proj, cols, T, heads, groups, N, dv, taps, bias, K,  \
+                                                                                     tails, dt_bias, a_log, tok_req, q_offsets, slot_ids, \
+                                                                                     coef, x_out, tokens, x_blocks, blocks)
+    if (!kept) LC_SS_PREPARE(0, false);
+    else if (K == 2) LC_SS_PREPARE(2, true);
+    else if (K == 3) LC_SS_PREPARE(3, true);
+    else if (K == 4) LC_SS_PREPARE(4, true);
+    else LC_SS_PREPARE(0, true);
 #undef LC_SS_PREPARE
     LC_LAUNCH_CHECK("state_space_prepare");
     return 0;

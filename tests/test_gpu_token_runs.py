@@ -78,3 +78,20 @@ def test_state_space_inputs(heads, groups, N, dv, taps):
         for a, b in zip(one, got):
             b = b.view(-1, T, b.shape[-1])[:, first:first + few] if b.dim() == 3 else b[first:first + few]
             assert torch.equal(a.reshape(b.shape), b)
+
+
+@pytest.mark.parametrize("heads,groups,taps", [(8192, 2, 4), (8193, 1, 4), (20000, 4, 1)])
+def test_state_space_of_many_heads(heads, groups, taps):
+    """More heads than a workgroup's LDS has room for a step and a decay of."""
+    g = torch.Generator().manual_seed(heads)
+    T, N, dv = 5, 3, 1
+    C = heads * dv + 2 * groups * N
+    given = [torch.randn(T, C + heads * dv + heads, generator=g), torch.randn(C, taps, generator=g) * 0.5, torch.randn(C, generator=g) * 0.3,
+             torch.randn(2, taps - 1, C, generator=g) if taps > 1 else None, torch.randn(heads, generator=g), torch.randn(heads, generator=g) - 1,
+             torch.tensor([0, 0, 0, 1, 1], dtype=torch.int32), torch.tensor([0, 3, 5], dtype=torch.int32), torch.tensor([1, 0], dtype=torch.int32)]
+    proj, conv, bias, tail, dt_bias, a_log, *rest = given
+    want = reference_ops.state_space_prepare(proj, heads, groups, N, dv, conv, bias, tail, dt_bias, a_log, *rest)
+    proj, conv, bias, tail, dt_bias, a_log, *rest = [None if t is None else t.to(DEV) for t in given]
+    got = ops.state_space_prepare(proj, heads, groups, N, dv, conv, bias, tail, dt_bias, a_log, *rest)
+    for a, b in zip(got, want):
+        torch.testing.assert_close(a.cpu(), b, rtol=2e-6, atol=2e-6)
