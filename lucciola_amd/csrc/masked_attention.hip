@@ -391,9 +391,8 @@ LC_API int lc_attention_prepare(const float* proj, int cols, int T, int nq, int 
              "attention prepare: a convolution needs 1 to %d taps, the tails and the request lists", SHORT_CONV_MAX_TAPS);
     LC_CHECK(!table || (rot > 0 && rot % 2 == 0 && rot <= d && positions), "attention prepare: bad rotation");
     LC_CHECK(!rows || (k_cache && v_cache && page_size > 0), "attention prepare: rows without a cache");
-    if (!unit && d % 2 == 0 && dv % 2 == 0 && cols % 2 == 0 && g_prepare_pairs) {
-        const int pair_blocks = (((nq + nk) * d + nv * dv) / 2 + 255) / 256;
-        LC_CHECK(pair_blocks <= 65535, "attention prepare: too many heads");
+    const int pair_blocks = (((nq + nk) * d + nv * dv) / 2 + 255) / 256;
+    if (!unit && d % 2 == 0 && dv % 2 == 0 && cols % 2 == 0 && pair_blocks <= 65535 && g_prepare_pairs) {
 #define LC_PAIRS_AS(TT, KT, TOKENS)                                                                                                     \
     attention_prepare_pairs_kernel<TT, KT, TOKENS><<<dim3((T + TOKENS - 1) / TOKENS, pair_blocks), 256, 0, stream>>>(                   \
         proj, cols, T, nq, nk, nv, d, dv, taps, K, tails, tok_req, q_offsets, slot_ids, table, rot, positions, (TT*)q_out, (TT*)k_cache, \
