@@ -27,11 +27,11 @@ __global__ __launch_bounds__(256) void state_space_prepare_kernel(
     const float* __restrict__ proj, int cols, int T, int heads, int groups, int N, int dv, const float* __restrict__ taps,
     const float* __restrict__ bias, int K, const float* __restrict__ tails, const float* __restrict__ dt_bias, const float* __restrict__ a_log,
     const int* __restrict__ tok_req, const int* __restrict__ q_offsets, const int* __restrict__ slot_ids, float* __restrict__ coef,
-    float* __restrict__ x_out, int tokens, int x_blocks, int blocks) {
+    float* __restrict__ x_out, int tokens, int x_blocks) {
     extern __shared__ float rates[];                // [tokens][heads] steps, then as many decays
     const int inner = heads * dv, C = inner + 2 * groups * N, per_group = heads / groups;
-    const int run_at = blockIdx.x / blocks, block = blockIdx.x - run_at * blocks;
-    const int t0 = run_at * tokens, t1 = min(t0 + tokens, T);
+    const int block = blockIdx.y + blockIdx.z * gridDim.y;
+    const int t0 = blockIdx.x * tokens, t1 = min(t0 + tokens, T);
     const size_t plane = (size_t)T * heads * N;
     auto tail_of = [&](int r) { return K > 1 ? tails + (size_t)slot_ids[r] * (K - 1) * C : nullptr; };
     if (block < x_blocks) {
@@ -126,18 +126,22 @@ LC_API int lc_state_space_prepare(const float* proj, int cols, int T, int heads,
     if (T == 0) return 0;
     LC_CHECK(proj && taps && bias && dt_bias && a_log && tok_req && q_offsets && slot_ids && coef && x_out && (K == 1 || tails),
              "state space prepare: null pointer");
-    // runs of tokens where there are many; a step of few keeps a thread a token and entry
-    int tokens = T >= 1024 ? 8 : T >= 256 ? 4 : 1;
+    const int x_blocks = (heads * dv + 255) / 256, blocks = x_blocks + (groups * N + 255) / 256;
+    // Runs of tokens where they leave five workgroups a CU (eight tokens: eight workgroups, and taps whose inputs are kept).  Runs that empty
+    // the card only make its threads' chains longer: 4 heads of 32, a group of 16, 1,024 tokens, two workgroups a run: 256 of eight tokens 9.1 us,
+    // 6 taps 16.0, 2,048 of one 5.6 and 6.2; 16 heads of 128, 4 groups of 128, 512 tokens in runs of one, two and four 21, 11.5 and 9.7.
+    int tokens = 1;
+    auto leaves = [&](int run) { return (long long)((T + run - 1) / run) * blocks / device_cus(); };
+    while (tokens < 4 && leaves(2 * tokens) >= 5) tokens *= 2;
+    if (K >= 2 && K <= 4 && leaves(8) >= 8) tokens = 8;
     while (tokens > 1 && tokens * heads > 4096) tokens /= 2;
     const size_t lds = (size_t)2 * tokens * heads * sizeof(float);
     const bool kept = lds <= 64 * 1024;
-    const int x_blocks = (heads * dv + 255) / 256, blocks = x_blocks + (groups * N + 255) / 256;
-    const long long grid = (long long)((T + tokens - 1) / tokens) * blocks;
-    LC_CHECK(grid * 256 < 1ll << 32, "state space prepare: %d tokens of %d columns are too many", T, cols);
-#define LC_SS_PREPARE(KT, KEPT)                                                                                                           \
-    state_space_prepare_kernel<KT, KEPT><<<(int)grid, 256, KEPT ? lds : 0, stream>>>(proj, cols, T, heads, groups, N, dv, taps, bias, K,  \
-                                                                                     tails, dt_bias, a_log, tok_req, q_offsets, slot_ids, \
-                                                                                     coef, x_out, tokens, x_blocks, blocks)
+    const dim3 grid((T + tokens - 1) / tokens, blocks < 65535 ? blocks : 65535, (blocks + 65534) / 65535);
+#define LC_SS_PREPARE(KT, KEPT)                                                                                                       \
+    state_space_prepare_kernel<KT, KEPT><<<grid, 256, KEPT ? lds : 0, stream>>>(proj, cols, T, heads, groups, N, dv, taps, bias, K,   \
+                                                                                tails, dt_bias, a_log, tok_req, q_offsets, slot_ids,  \
+                                                                                coef, x_out, tokens, x_blocks)
     if (!kept) LC_SS_PREPARE(0, false);
     else if (K == 2) LC_SS_PREPARE(2, true);
     else if (K == 3) LC_SS_PREPARE(3, true);

@@ -52,7 +52,8 @@ def test_attention_inputs(dtype, nq, nk, nv, d, dv, taps, rot, page):
         assert torch.equal(got, want)
 
 
-@pytest.mark.parametrize("heads,groups,N,dv,taps", [(4, 2, 16, 32, 4), (3, 1, 7, 100, 3), (2, 2, 130, 3, 2), (6, 3, 5, 64, 1), (2, 1, 16, 16, 6)])
+@pytest.mark.parametrize("heads,groups,N,dv,taps", [(4, 2, 16, 32, 4), (3, 1, 7, 100, 3), (2, 2, 130, 3, 2), (6, 3, 5, 64, 1), (2, 1, 16, 16, 6),
+                                                      (4, 2, 130, 2000, 4), (3, 1, 7, 1300, 2), (4, 2, 130, 1000, 6)])       # runs of eight and four
 def test_state_space_inputs(heads, groups, N, dv, taps):
     g = torch.Generator().manual_seed(heads + N + taps)
     T, inner = sum(LENGTHS), heads * dv
@@ -71,7 +72,7 @@ def test_state_space_inputs(heads, groups, N, dv, taps):
     tok_req, q_offsets, slots = rest
     for r, n in enumerate(LENGTHS):
         first = int(q_offsets[r])
-        few = min(n, 200)
+        few = min(n, 200 if heads * dv < 3000 else 20)
         one = ops.state_space_prepare(proj[first:first + few].contiguous(), heads, groups, N, dv, conv, bias, tail, dt_bias, a_log,
                                       torch.zeros(few, dtype=torch.int32, device=DEV), torch.tensor([0, few], dtype=torch.int32, device=DEV),
                                       slots[r:r + 1].contiguous())
