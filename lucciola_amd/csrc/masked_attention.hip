@@ -253,7 +253,7 @@ __global__ __launch_bounds__(256) void attention_prepare_pairs_kernel(
     const bool is_v = c >= qk_cols;
     const int at = is_v ? (c - qk_cols) % dv : c % d;          // the pair's place in its head
     ShortConvRun<KT < 0 ? 0 : KT> first, second;
-    if (KT > 0) {
+    if constexpr (KT > 0) {
         first.start(taps, c);
         second.start(taps, c + 1);
     }
@@ -266,7 +266,18 @@ __global__ __launch_bounds__(256) void attention_prepare_pairs_kernel(
         va[i] = vb[i] = 0.f;
         if (t >= T_) continue;
         float a, b;
-        if constexpr (KT >= 0) {
+        if constexpr (KT == 0) {                // nothing is kept from token to token: both inputs in one load
+            const int r = tok_req[t], local = t - q_offsets[r];
+            const float* tail = tails + (size_t)slot_ids[r] * (K - 1) * C;
+            a = b = 0.f;
+#pragma unroll 4
+            for (int back = K - 1; back >= 0; --back) {         // oldest input first
+                const float2 in = *reinterpret_cast<const float2*>(
+                    back <= local ? proj + (size_t)(t - back) * cols + c : tail + (size_t)((K - 1) - (back - local)) * C + c);
+                a = fmaf(taps[(size_t)c * K + (K - 1 - back)], in.x, a);
+                b = fmaf(taps[(size_t)(c + 1) * K + (K - 1 - back)], in.y, b);
+            }
+        } else if constexpr (KT > 0) {
             const int r = tok_req[t], local = t - q_offsets[r];
             const float* tail = tails + (size_t)slot_ids[r] * (K - 1) * C;
             a = first.at(proj, cols, t, local, c, taps, K, tail, C, r != before);
@@ -397,11 +408,13 @@ LC_API int lc_attention_prepare(const float* proj, int cols, int T, int nq, int 
     attention_prepare_pairs_kernel<TT, KT, TOKENS><<<dim3((T + TOKENS - 1) / TOKENS, pair_blocks), 256, 0, stream>>>(                   \
         proj, cols, T, nq, nk, nv, d, dv, taps, K, tails, tok_req, q_offsets, slot_ids, table, rot, positions, (TT*)q_out, (TT*)k_cache, \
         (TT*)v_cache, rows, page_size > 0 ? page_size : 1)
-        // runs of tokens where there are many; a step of few keeps a thread a token and pair
+        // Runs of tokens where they leave two workgroups a CU; else a thread a token and pair (8 heads of 64 over 2, two blocks of pairs, no
+        // convolution, 1,024 tokens: 256 workgroups 5.5 us, 2,048 4.4; 2,048 tokens, 512 workgroups of runs 5.7 and 6.6 before there were any).
+        const bool runs = T >= 1024 && (long long)(T / 8) * pair_blocks >= 2 * device_cus();
 #define LC_PAIRS(TT)                                                                  \
     do {                                                                              \
-        if (!taps) { if (T >= 1024) LC_PAIRS_AS(TT, -1, 8); else LC_PAIRS_AS(TT, -1, 1); } \
-        else if (K == 4) { if (T >= 1024) LC_PAIRS_AS(TT, 4, 8); else LC_PAIRS_AS(TT, 4, 1); } \
+        if (!taps) { if (runs) LC_PAIRS_AS(TT, -1, 8); else LC_PAIRS_AS(TT, -1, 1); } \
+        else if (K == 4) { if (runs) LC_PAIRS_AS(TT, 4, 8); else LC_PAIRS_AS(TT, 4, 1); } \
         else LC_PAIRS_AS(TT, 0, 1);                                                   \
     } while (0)
         if (dt == DT_F32) LC_PAIRS(float);

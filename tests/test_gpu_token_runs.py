@@ -19,7 +19,9 @@ def lists():
 
 @pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
 @pytest.mark.parametrize("nq,nk,nv,d,dv,taps,rot,page", [
-    (4, 2, 2, 64, 64, 4, 32, 16), (3, 1, 2, 6, 10, 4, 4, 12), (2, 2, 1, 130, 8, 0, 0, 16), (5, 1, 1, 32, 34, 3, 32, 24), (2, 0, 0, 16, 2, 4, 0, 16)])
+    (4, 2, 2, 64, 64, 4, 32, 16), (3, 1, 2, 6, 10, 4, 4, 12), (2, 2, 1, 130, 8, 0, 0, 16), (5, 1, 1, 32, 34, 3, 32, 24), (2, 0, 0, 16, 2, 4, 0, 16),
+    (3, 1, 2, 6, 10, 8, 4, 12), (5, 1, 1, 32, 34, 1, 32, 24), (30, 3, 2, 66, 34, 4, 4, 12), (16, 8, 4, 64, 128, 0, 0, 24), (12, 6, 6, 130, 34, 4, 0, 16),
+    (16, 8, 4, 64, 128, 4, 32, 16)])       # the last four wide enough for runs of tokens
 def test_attention_inputs(dtype, nq, nk, nv, d, dv, taps, rot, page):
     g = torch.Generator().manual_seed(nq + d + dv + taps)
     T, C = sum(LENGTHS), (nq + nk) * d + nv * dv
