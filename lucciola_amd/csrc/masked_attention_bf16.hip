@@ -38,6 +38,7 @@ struct MaskedArgs {
     const bf16* k_cache;
     const bf16* v_cache;
     const int* tiles;
+    int num_tiles;
     const int* block_table;
     int max_blocks, page_size, heads, kv_heads, d, dv;
     float scale;
@@ -56,6 +57,7 @@ struct MaskedArgs {
     int zsplits;
     int lone_only;      // the tiles of several tokens are another kernel's
     int wave_blocks;    // blocks of a stage for every wave that shares a head's keys, in the kernel that stages them
+    int at_once;        // the order of the workgroups (below)
 };
 
 // floats a wave leaves per lane and map where key ranges are joined: maximum, sum, the lane's part of O^T
@@ -342,13 +344,22 @@ __device__ __forceinline__ void finish_column(const ColumnState<DVB, MAPS>& st, 
     }
 }
 
+// The order in which workgroups start.  Grid (kv heads; tiles; a layer for every 65,535 tiles): a tile's kv heads are neighbours and the longest
+// tiles of all heads come first.  Where all workgroups are on the card at once there is nothing to gain by that, and a tile's kv heads, whose
+// keys are neighbours in memory, are better read by one XCD (workgroup number % 8) than by several at once: grid (tiles; kv heads; zsplits).
+// Lone tokens, 16 heads over 4, keys of 64 and values of 128: 64 at 2,048, 256 workgroups, 51 and 37 us, 8 at 2,048 20.3 and 15.6; keys and values
+// of 128, heads over 16, 64 tokens at 128 to 2,047, 1,024 workgroups, 98 and 147.
+constexpr int MB_GRID = 65535;
+
 template <int DSTEPS, int DVB, int MAPS>
 __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(MaskedArgs a) {
     __shared__ float meet[MB_WAVES - 1][kWave][DVB * 4 + 2];
-    const int tile_at = blockIdx.x / a.kv_heads;      // a tile's kv heads are neighbours: the longest tiles of all heads start first
+    const int tile_at = a.at_once ? blockIdx.x : blockIdx.y + blockIdx.z * MB_GRID;
+    const int g = a.at_once ? blockIdx.y : blockIdx.x, z = a.at_once ? blockIdx.z : 0;
+    if (tile_at >= a.num_tiles) return;
     const int* tile = a.tiles + 4 * tile_at;
     const int t0 = tile[0], n = tile[1], r = tile[2], p0 = tile[3];
-    const int g = blockIdx.x - tile_at * a.kv_heads, group = a.heads / a.kv_heads;
+    const int group = a.heads / a.kv_heads;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), col = lane & 15;
     const int* table = a.block_table + (size_t)r * a.max_blocks;
     auto first_key = [&](int p) {
@@ -358,7 +369,7 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(Maske
         return lo;
     };
     const bool lone = n == 1;
-    const int z = blockIdx.z, zsplits = lone ? a.zsplits : 1;
+    const int zsplits = lone ? a.zsplits : 1;
     if (!lone && (z > 0 || a.lone_only)) return;
     // head places of a pass (a power of two up to the waves), and the waves that share a place's keys
     int places = 1;
@@ -419,7 +430,7 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(Maske
             if (zsplits > 1) {
                 const int passes = (group + 15) / 16;
                 // [share][lane][map][numbers]: a lane's numbers in a row, which it reads back in wide loads
-                float* mine = a.shares + (((size_t)blockIdx.x * passes + h0 / 16) * zsplits + z)
+                float* mine = a.shares + ((((size_t)tile_at * a.kv_heads + g) * passes + h0 / 16) * zsplits + z)
                                              * kWave * MAPS * share_floats<DVB>() + (size_t)lane * MAPS * share_floats<DVB>();
 #pragma unroll
                 for (int m = 0; m < MAPS; ++m) {
@@ -446,15 +457,27 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(Maske
 // of padding): every operand is one read without bank conflicts.  Lone tokens are left to the kernel above.
 constexpr int MB_STAGE_BLOCKS = 2;
 
+// PAIRS: a wave takes its two blocks of a stage at once.  That needs room for both blocks' operands in registers (MB_ROOM), and those
+// take waves off a SIMD: two are left of four with keys and values of 64.  It pays where the products over values are most of the work
+// (MB_VALUES: keys and values of 128, 128 1.09 times as fast, 64, 128 1.04, 64, 64 in two maps 1.04), and elsewhere where four heads or more
+// share the waves' stage (64, 64 and 64, 32 1.03 over 4 of 16 heads, 32, 32 over 1 of 8 1.07).  With fewer the waves are what is missing, for
+// one head leaves half of them idle: 16 heads over 16, 576 to 2,048 tokens after up to 3,000: 64, 64 and 64, 32 0.66 times as fast, 128, 32 0.70;
+// over 8, 64, 64 0.75; and 128, 64 in two maps 0.94 with any number.
 template <int DSTEPS, int DVB, int MAPS>
+constexpr bool MB_ROOM = 2 * MAPS * DSTEPS * 4 + 2 * DVB * 2 + MAPS * DVB * 4 + MAPS * DSTEPS * 4 <= 160;
+template <int DSTEPS, int DVB, int MAPS>
+constexpr bool MB_VALUES = DVB == 8 || (DVB == 4 && MAPS * DSTEPS == 4);
+
+template <int DSTEPS, int DVB, int MAPS, bool PAIRS>
 __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kernel(MaskedArgs a) {
     extern __shared__ __align__(16) unsigned char staged[];       // a stage; afterwards where split key ranges meet
     float (*meet)[kWave][DVB * 4 + 2] = reinterpret_cast<float (*)[kWave][DVB * 4 + 2]>(staged);
-    const int tile_at = blockIdx.x / a.kv_heads;      // a tile's kv heads are neighbours: the longest tiles of all heads start first
+    const int tile_at = blockIdx.y + blockIdx.z * MB_GRID;
+    if (tile_at >= a.num_tiles) return;
     const int* tile = a.tiles + 4 * tile_at;
     const int t0 = tile[0], n = tile[1], r = tile[2], p0 = tile[3];
     if (n == 1) return;
-    const int g = blockIdx.x - tile_at * a.kv_heads, group = a.heads / a.kv_heads;
+    const int g = blockIdx.x, group = a.heads / a.kv_heads;
     const int wave = threadIdx.x / kWave, lane = threadIdx.x & (kWave - 1), col = lane & 15, quad = lane >> 4;
     const int* table = a.block_table + (size_t)r * a.max_blocks;
     auto first_key = [&](int p) {
@@ -583,8 +606,6 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
             };
             auto seen = [&](int b) { return (b * 16 >= seen_from || b * 16 + 15 < a.keep) && b * 16 + 15 <= p0; };
             const int at0 = stage * stage_blocks + split, at1 = at0 + splits;       // this wave's one or two blocks of the stage
-            // both at once where their operands and sums find room in registers
-            constexpr bool PAIRS = 2 * MAPS * DSTEPS * 4 + 2 * DVB * 2 + MAPS * DVB * 4 + MAPS * DSTEPS * 4 <= 160;
             bool done = false;
             if constexpr (PAIRS) {
                 done = wave_on && a.wave_blocks == 2 && at1 < blocks.count;
@@ -645,11 +666,11 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
 // One wave per lone token and kv head: the workgroups' shares taken in, in their order; then the columns' end.
 template <int DVB, int MAPS>
 __global__ __launch_bounds__(kWave) void masked_attention_bf16_join_kernel(MaskedArgs a) {
-    const int tile_at = blockIdx.x / a.kv_heads;      // a tile's kv heads are neighbours: the longest tiles of all heads start first
+    const int tile_at = blockIdx.x;
     const int* tile = a.tiles + 4 * tile_at;
     const int t0 = tile[0], n = tile[1], p0 = tile[3];
     if (n != 1) return;
-    const int g = blockIdx.x - tile_at * a.kv_heads, group = a.heads / a.kv_heads, lane = threadIdx.x, col = lane & 15;
+    const int g = blockIdx.y, group = a.heads / a.kv_heads, lane = threadIdx.x, col = lane & 15;
     const int passes = (group + 15) / 16;
     for (int h0 = 0; h0 < group; h0 += 16) {
         const bool on = h0 + col < group;
@@ -663,7 +684,7 @@ __global__ __launch_bounds__(kWave) void masked_attention_bf16_join_kernel(Maske
             for (int t = 0; t < DVB; ++t) st.o[m][t] = floatx4{0.f, 0.f, 0.f, 0.f};
         }
         for (int z = 0; z < a.zsplits; ++z) {
-            const float* its = a.shares + (((size_t)blockIdx.x * passes + h0 / 16) * a.zsplits + z)
+            const float* its = a.shares + ((((size_t)tile_at * a.kv_heads + g) * passes + h0 / 16) * a.zsplits + z)
                                               * kWave * MAPS * share_floats<DVB>() + (size_t)lane * MAPS * share_floats<DVB>();
 #pragma unroll
             for (int m = 0; m < MAPS; ++m) {
@@ -730,9 +751,9 @@ LC_API int lc_masked_attention_bf16(const void* q, const void* k_cache, const vo
     LC_CHECK((r1 == nullptr) == (r2 == nullptr), "masked attention: the bias needs both of its vectors");
     LC_CHECK(kv_heads <= 65535, "masked attention: too many kv heads");
     LC_CHECK(chunk >= 0 && window >= 0 && keep >= 0 && cap >= 0.f, "masked attention: bad mask or cap");
-    MaskedArgs a{(const bf16*)q, (const bf16*)k_cache, (const bf16*)v_cache, tiles, block_table, max_blocks, page_size,
+    MaskedArgs a{(const bf16*)q, (const bf16*)k_cache, (const bf16*)v_cache, tiles, num_tiles, block_table, max_blocks, page_size,
                  heads, kv_heads, d, dv, scale, chunk, window, keep, cap, r1, r2, sink, lambda, unit_out, eps, out_scale, gate,
-                 gate_stride, gate_column, (bf16*)out, shares, zsplits, 0, 1};
+                 gate_stride, gate_column, (bf16*)out, shares, zsplits, 0, 1, 0};
     // tiles of several tokens go through the kernel that stages keys and values in LDS where a stage fits a thread's
     // two pieces of each kind
     const int group = heads / kv_heads;
@@ -751,12 +772,19 @@ LC_API int lc_masked_attention_bf16(const void* q, const void* k_cache, const vo
     if (staged_lds < meet_lds) staged_lds = meet_lds;
     a.lone_only = staged ? 1 : 0;
     const bool main_kernel = !staged || any_lone;
-    LC_CHECK((long long)num_tiles * kv_heads < 1ll << 31, "masked attention: too many tiles");
-    const dim3 grid(num_tiles * kv_heads, 1, zsplits), join_grid(num_tiles * kv_heads);
+    a.at_once = zsplits > 1 || (long long)num_tiles * kv_heads <= 2 * device_cus() ? 1 : 0;
+    const dim3 portions_grid(kv_heads, num_tiles < MB_GRID ? num_tiles : MB_GRID, (num_tiles + MB_GRID - 1) / MB_GRID);
+    const dim3 grid = a.at_once ? dim3(num_tiles, kv_heads, zsplits) : portions_grid;
+    const dim3 join_grid(num_tiles, kv_heads);         // on the XCDs that left the shares
     const int dsteps = (d + 31) / 32, dvb = dv / 16;
 #define LC_MB_AS(DS, VB, MP)                                                                                            \
     do {                                                                                                                \
-        if (staged) masked_attention_bf16_staged_kernel<DS, VB, MP><<<join_grid, MB_THREADS, staged_lds, stream>>>(a);  \
+        if (staged && (MB_VALUES<DS, VB, MP> || (group >= 4 && MP * DS < 8)))                                           \
+            masked_attention_bf16_staged_kernel<DS, VB, MP, MB_ROOM<DS, VB, MP>>                                        \
+                <<<portions_grid, MB_THREADS, staged_lds, stream>>>(a);                                                 \
+        else if (staged)                                                                                                \
+            masked_attention_bf16_staged_kernel<DS, VB, MP, MB_ROOM<DS, VB, MP> && MB_VALUES<DS, VB, MP>>               \
+                <<<portions_grid, MB_THREADS, staged_lds, stream>>>(a);                                                 \
         if (main_kernel) masked_attention_bf16_kernel<DS, VB, MP><<<grid, MB_THREADS, 0, stream>>>(a);                  \
         if (zsplits > 1) masked_attention_bf16_join_kernel<VB, MP><<<join_grid, kWave, 0, stream>>>(a);                 \
     } while (0)
