@@ -102,13 +102,21 @@ struct EvenTile {
     int group, first, end, units, column;      // units 0: there is none
 };
 
-__device__ __forceinline__ int even_tiles(int units, int most) { return units ? (units + most - 1) / most : 0; }
+// units divided by `most`, rounded up; inverse: 2^32 divided by `most`, rounded up (0 for 1).  Exact below 2^28 units, for the inverse is too large
+// by less than 8.
+__device__ __forceinline__ int even_tiles(int units, int most, unsigned inverse) {
+    return most == 1 ? units : (int)__umulhi((unsigned)(units + most - 1), inverse);
+}
+__device__ __forceinline__ unsigned even_inverse(int most) { return most == 1 ? 0u : 0xFFFFFFFFu / (unsigned)most + 1u; }
 
 __device__ __forceinline__ EvenTile find_even_tile(const int* row_start, int G, int id, int columns, int room, int cus, int lane) {
     const int sub = lane >> 3, most = (lane & 7) + 1;
+    const unsigned inverse = even_inverse(most);
     int tiles = 0, highest = 0, cost = 0;
     for (int g = sub; g < G; g += 8) {
-        const int units = (row_start[g + 1] - row_start[g] + 31) / 32, n = even_tiles(units, most), h = n ? (units + n - 1) / n : 0;
+        // (divisions of integers, some eighty instructions a group, were a quarter of a short product of 256 experts)
+        const int units = (row_start[g + 1] - row_start[g] + 31) >> 5, n = even_tiles(units, most, inverse);
+        const int h = n ? (int)ceilf((float)units * __builtin_amdgcn_rcpf((float)n) - 0.001f) : 0;
         tiles += n;
         cost += n * (h + 2);
         highest = max(highest, h);
@@ -130,6 +138,7 @@ __device__ __forceinline__ EvenTile find_even_tile(const int* row_start, int G, 
     }
     best = __builtin_amdgcn_readfirstlane(best);
     tiles = __shfl(tiles, best - 1);
+    const unsigned best_inverse = even_inverse(best);
 
     // An XCD (workgroup id % 8) takes neighbouring tiles, a group's column by column: its L2 then serves one group's rows to all of its
     // columns and a column of w to all of the group's tiles, and memory is asked for each once.
@@ -141,7 +150,7 @@ __device__ __forceinline__ EvenTile find_even_tile(const int* row_start, int G, 
     for (int g0 = 0; g0 < G; g0 += 64) {
         const int g = g0 + lane;
         const int from = g < G ? row_start[g] : 0, to = g < G ? row_start[g + 1] : 0;
-        const int units = (to - from + 31) / 32, n = even_tiles(units, best);
+        const int units = (to - from + 31) >> 5, n = even_tiles(units, best, best_inverse);
         int upto = n;
 #pragma unroll
         for (int d = 1; d < 64; d *= 2) {
