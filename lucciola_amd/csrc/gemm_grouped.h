@@ -54,7 +54,9 @@ bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows);
 // forced: tests ask for the kernel of even tiles wherever it can run
 int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, bool forced, hipStream_t stream);
 
-bool grouped_gates(const GroupedArgs& a, int tile_rows);
+// whether the gated product is for these sizes (forced: wherever it can run); whether an experts' product goes to the kernel of even tiles
+bool grouped_gates(const GroupedArgs& a, int tile_rows, bool forced);
+bool grouped_evens(const GroupedArgs& a, int max_tiles, int tile_rows);
 int launch_grouped_gated(const GroupedArgs& a, const GroupedGate& gate, hipStream_t stream);
 
 }  // namespace lc

@@ -366,6 +366,16 @@ LC_API int lc_gemm_grouped_picks_tiled(int tile_rows, int M, int N, int K, int G
     return grouped_tiled_takes(a, tile_rows) && grouped_tiled_pays(a, max_tiles, tile_rows) ? 1 : 0;
 }
 
+// Tests: whether the default for experts' products (M sorted rows over G matrices of N x K) is the kernel of even tiles; gated: of 2 x N x K,
+// with the gated epilogue.
+LC_API int lc_gemm_grouped_picks_even(int tile_rows, int M, int N, int K, int G, int gated) {
+    static const int listed = 0;
+    GroupedArgs a{};
+    a.M = M; a.N = gated ? 2 * N : N; a.K = K; a.G = G;
+    a.row_start = &listed;
+    return (gated ? grouped_gates(a, tile_rows, false) : grouped_evens(a, M / tile_rows + G, tile_rows)) ? 1 : 0;
+}
+
 // Whether a product per head over so few rows that 16 go to a tile has the streaming kernel of gemm_grouped_tiled.hip.
 LC_API int lc_gemm_grouped_streams(const void* x, int x_dt, long long ldx, long long x_group, const void* w, int w_dt, int K) {
     return whole_pieces(x, x_dt, ldx, x_group, w, w_dt, K) && K % 128 == 0 && g_grouped_fast ? 1 : 0;
@@ -427,11 +437,11 @@ static GroupedArgs gated_args(const void* x, const void* w, void* out, int M, in
     return GroupedArgs{x, K, 0, w, out, I, 0, M, 2 * I, K, G, gather, row_start, row_start, ACT_NONE, nullptr, 0, 0, true};
 }
 
-// Whether lc_gemm_grouped_gated takes these operands, and is the faster way: 1 or 0.
+// Whether lc_gemm_grouped_gated takes these operands, and is the faster way (lc_gemm_grouped_tiled(1): takes them): 1 or 0.
 LC_API int lc_gemm_grouped_gates(const void* x, int x_dt, const void* w, int w_dt, int M, int I, int K, int G, int tile_rows) {
     static const int listed = 0;
     if (!g_grouped_fast || !g_grouped_tiled || M <= 0 || I <= 0 || K <= 0 || G <= 0 || !whole_pieces(x, x_dt, K, 0, w, w_dt, K)) return 0;
-    return grouped_gates(gated_args(x, w, nullptr, M, I, K, G, nullptr, &listed), tile_rows) ? 1 : 0;
+    return grouped_gates(gated_args(x, w, nullptr, M, I, K, G, nullptr, &listed), tile_rows, g_grouped_tiled == 1) ? 1 : 0;
 }
 
 // x, w, out: bfloat16, out [M, I] (16-byte aligned); gather: a sorted row's token; weights, entry_row [tokens * top] or both null;

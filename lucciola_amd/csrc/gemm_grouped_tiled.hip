@@ -17,6 +17,8 @@
 // Which rows are whose, the gather list and the epilogues are as described there.
 #include "common.h"
 
+#include <cmath>
+
 #include "activations.h"
 #include "gemm_grouped.h"
 #include "gemm_tile.h"
@@ -400,13 +402,34 @@ static bool even_takes(const GroupedArgs& a) {
            a.epilogue != ACT_SIGMOID_GATE && a.epilogue != ACT_SIGMOID_GROUP_GATE && room * columns < 1 << 30;
 }
 
-// Lists for tiles of 128 rows have no other kernel here.  With fewer rows an expert (lists for tiles of 64 rows) the tiles of 64 x 128, of
-// which a CU holds four, are as fast or faster where the tile is short or there are few columns (us, 64 x 128 and these: 8,192 rows over
-// 64 matrices of 2,048 x 512 52 and 53, 2,048 rows 34 and 41, over 16 of 256 x 2,048 21 and 25, over 256 of 512 x 512 35 and 55); from 1,024
-// k and 512 columns on these are faster at every size tried (64 matrices of 512 x 2,048, 2,048 rows 41 and 35; 32 of 4,096 x 1,024,
-// 8,192 rows 129 and 113; 32 of 2,048 x 2,048, 520 rows 71 and 51, 3,000 73 and 57, 6,092 103 and 71).
-static bool even_pays(const GroupedArgs& a, int tile_rows) {
-    return tile_rows == 128 || (tile_rows == 64 && a.K >= 1024 && a.N >= 512);
+// Tiles of 64 rows that the experts' rows make, as routers deal them out: about evenly, some sqrt(p) more or fewer than the p rows of each.
+static double tiles_of_64(const GroupedArgs& a) {
+    const double p = (double)a.M / a.G, spread = sqrt(p);
+    double tiles = 1.0 - exp(-p);
+    if (p > 1024) tiles = p / 64 + 0.5;
+    else
+        for (int rows = 64; rows < p + 4 * spread + 1; rows += 64) tiles += 0.5 * erfc((rows - p) / (spread * M_SQRT2));
+    return tiles * a.G;
+}
+
+// Whether the kernel of even tiles is the faster one of this file's.  Lists for tiles of 128 rows have no other.  With fewer rows an expert
+// (lists for tiles of 64 rows, whole K in 64 x 128) it needs 1,024 k and 512 columns (us, 64 x 128 and these, weights cold here and below:
+// 2,048 rows over 16 matrices of 512 x 256 8.8 and 9.8, 256 x 1,024 11.6 and 14.4), and what decides then is how many workgroups the tiles of
+// 64 x 128 make.  One a CU and fewer bring a CU less per product than a single wide tile does (400 rows, 4 matrices of 1,024 x 2,048 25 and 31;
+// 1,520 rows, 8 of them 24 and 31; 1,600 rows, 16 26 and 34; K 4,096 47 and 59), unless w is so large that memory's rate counts, at which
+// these are better (640 rows, 32 matrices of 1,024 x 2,048 37 and 33, K 1,024 17.6 and 20.2; 800 rows, 8 of 4,096 x 2,048 37 and 32).  More of
+// them share CUs, and the wide tiles win (2,240 rows, 16 of 768 x 2,048 38 and 31; 6,080 rows, 32 of 1,024 x 2,048 58 and 39), but for a short
+// K with a tile an expert and many experts, where both wait for w (1,280 rows, 64 of 1,024 x 1,024 30.8 and 32.3, 480 rows, 24 of 2,048 x 1,024
+// 25.1 and 23.7).  gated: these save a pass besides, and win
+// from one workgroup a CU on (320 rows, 16 of 2 x 1,024 x 1,024 20.9 and 19.1, 1,280 rows, 64 of 2 x 512 x 1,024 32.9 and 31.9), but not
+// below (1,120 rows, 8 of 2 x 512 x 2,048 26.7 and 29.8).
+static bool even_pays(const GroupedArgs& a, int tile_rows, bool gated) {
+    if (tile_rows != 64) return tile_rows == 128;
+    if (a.K < 1024 || a.N < 512) return false;
+    const double experts = tiles_of_64(a), tiles = experts * ((a.N + 127) / 128), cus = device_cus();
+    if (gated) return tiles > 0.98 * cus;
+    if (tiles > 1.02 * cus) return a.K >= 1536 || experts > 1.05 * a.G || a.G < 48;
+    return (double)a.G * a.N > cus * (80 + 50.0 * 1024 / a.K);
 }
 
 template <typename TO, bool GATED>
@@ -422,7 +445,7 @@ static int grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, boo
     };
     if (tile_rows == 16) {
         gemm_grouped_stream_kernel<TO><<<grid(16, STREAM_N), 256, 0, stream>>>(a);
-    } else if (even_takes(a) && (forced || even_pays(a, tile_rows))) {
+    } else if (even_takes(a) && (forced || even_pays(a, tile_rows, false))) {
         launch_even<TO, false>(a, GroupedGate{}, stream);
     } else {
         gemm_grouped_tiled_kernel<TO, 64, 128, 2, 2, 2><<<grid(64, 128), 256, 0, stream>>>(a);
@@ -463,8 +486,13 @@ int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, boo
 }
 
 // a.N: gate and up columns together
-bool grouped_gates(const GroupedArgs& a, int tile_rows) {
-    return tile_rows != 16 && a.N % 16 == 0 && even_takes(a) && even_pays(a, tile_rows) && grouped_tiled_pays(a, a.M / tile_rows + a.G, tile_rows);
+bool grouped_gates(const GroupedArgs& a, int tile_rows, bool forced) {
+    if (tile_rows == 16 || a.N % 16 || !even_takes(a)) return false;
+    return forced || (even_pays(a, tile_rows, true) && grouped_tiled_pays(a, a.M / tile_rows + a.G, tile_rows));
+}
+
+bool grouped_evens(const GroupedArgs& a, int max_tiles, int tile_rows) {
+    return tile_rows != 16 && even_takes(a) && even_pays(a, tile_rows, false) && grouped_tiled_pays(a, max_tiles, tile_rows);
 }
 
 int launch_grouped_gated(const GroupedArgs& a, const GroupedGate& gate, hipStream_t stream) {

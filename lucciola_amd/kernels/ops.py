@@ -85,6 +85,7 @@ _SIGNATURES = {
     "lc_gemm_grouped_gated": "pppiiiippippiip",
     "lc_gemm_grouped_fast": "i",
     "lc_gemm_grouped_tiled": "i",
+    "lc_gemm_grouped_picks_even": "iiiiii",
     "lc_gemm_grouped_streams": "piqqpii",
     "lc_gemm_grouped_picks_tiled": "iiiiii",
     "lc_gemm_grouped_takes_tile": "iii",
@@ -1588,8 +1589,8 @@ class Routing:
 def _routed_tile(rows: int, experts: int, large_tiles: bool) -> int:
     """Rows of the experts' tiles for ``rows`` (token, choice) pairs: 16 where an expert has that many on average, which reads
     every matrix at the memory's rate (32 experts of 4,096 x 2,048, 16 rows each: 98 us against 119 in tiles of 64, the
-    matrices alone 98); 128 where it has more than one tile of 128 and the caller's products take them, else 64.  From 1,024 k and
-    512 columns on both mean the same kernel, which cuts an expert's rows by itself."""
+    matrices alone 98); 128 where it has more than one tile of 128 and the caller's products take them, else 64.  Where the workgroups
+    fill the card both mean the same kernel, which cuts an expert's rows by itself."""
     return 16 if rows <= 16 * experts else 128 if large_tiles and rows >= 192 * experts else 64
 
 

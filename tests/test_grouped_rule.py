@@ -26,6 +26,22 @@ def test_experts(tile, tokens, top, experts, columns, K, tiled):
     assert bool(ops.library().lc_gemm_grouped_picks_tiled(tile, rows, columns, K, experts, rows // tile + experts)) == tiled
 
 
+# lists for tiles of 64 rows: one workgroup of 64 x 128 a CU and fewer, more of them, w so large that memory counts, a short K
+@pytest.mark.parametrize("rows,experts,columns,K,even", [
+    (400, 4, 1024, 2048, False), (1520, 8, 1024, 4096, False), (1600, 16, 1024, 2048, False), (800, 4, 512, 1024, False), (2240, 16, 768, 2048, True),
+    (6080, 32, 1024, 2048, True), (140, 1, 512, 2048, False), (640, 32, 1024, 2048, True), (640, 32, 1024, 1024, False), (1280, 64, 1024, 1024, False), (480, 24, 2048, 1024, True),
+    (1280, 64, 1024, 2048, True), (6080, 32, 511, 2048, False), (6080, 32, 1024, 960, False), (8960, 64, 512, 1024, True), (8960, 64, 2048, 1024, True)])
+def test_even_tiles(rows, experts, columns, K, even):
+    assert bool(ops.library().lc_gemm_grouped_picks_even(64, rows, columns, K, experts, 0)) == even
+
+
+@pytest.mark.parametrize("rows,experts,I,K,fused", [
+    (1120, 8, 512, 2048, False), (560, 4, 256, 2048, False), (320, 16, 1024, 1024, True), (1280, 64, 512, 1024, True), (2240, 16, 512, 2048, True),
+    (8960, 64, 256, 2048, True), (8960, 64, 128, 2048, False)])
+def test_gated_experts(rows, experts, I, K, fused):
+    assert bool(ops.library().lc_gemm_grouped_picks_even(64, rows, I, K, experts, 1)) == fused
+
+
 @pytest.mark.parametrize("rows,columns,K,heads,gap,dtype,tile", [
     (16, 128, 512, 16, 0, torch.bfloat16, 16), (512, 128, 512, 16, 0, torch.bfloat16, 16), (513, 128, 512, 16, 0, torch.bfloat16, 64),
     (256, 128, 320, 32, 0, torch.bfloat16, 64), (192, 128, 320, 32, 0, torch.bfloat16, 16), (512, 128, 512, 16, 4, torch.bfloat16, 64),
