@@ -19,7 +19,7 @@ def gelu(z):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("T,I", [(1, 8), (3, 24), (5, 25), (70, 2048), (300, 2056), (2, 4100)])
+@pytest.mark.parametrize("T,I", [(1, 8), (3, 24), (5, 25), (70, 2048), (300, 2056), (2, 4100), (9001, 64), (33000, 24), (4000, 136)])
 def test_gated(dtype, T, I):
     g = torch.Generator().manual_seed(T + I)
     gu = (torch.randn(T, 2 * I, generator=g) * 4).to(dtype).to(DEV)
