@@ -228,14 +228,14 @@ __global__ __launch_bounds__(1024) void moe_lists_kernel(const int* __restrict__
 
 // VEC neighbouring entries a thread: the choices' weights and rows are looked up once for them, and rows come in wide loads (2,048 tokens,
 // four choices of 2,048 entries: 16 us with an entry a thread, 13 now; with the shared rows 27 and 16).
-template <int VEC>
+template <int VEC, bool WEIGHTED>
 __device__ __forceinline__ void combine_rows(float (&total)[VEC], const float* __restrict__ y, const float* __restrict__ weights,
                                              const int* __restrict__ entry_row, int t, int top, int n, int i) {
     typedef float piece __attribute__((ext_vector_type(VEC)));
 #pragma unroll
     for (int e = 0; e < VEC; ++e) total[e] = 0.f;
     for (int k = 0; k < top; ++k) {
-        const float w = weights ? weights[(size_t)t * top + k] : 1.f;
+        const float w = WEIGHTED ? weights[(size_t)t * top + k] : 1.f;
         const piece v = *reinterpret_cast<const piece*>(y + (size_t)entry_row[(size_t)t * top + k] * n + i);
 #pragma unroll
         for (int e = 0; e < VEC; ++e) total[e] = fmaf(w, v[e], total[e]);
@@ -249,7 +249,7 @@ __global__ void moe_combine_kernel(const float* __restrict__ y, const float* __r
     const int t = blockIdx.x;
     for (int i = threadIdx.x * VEC; i < n; i += blockDim.x * VEC) {
         float total[VEC];
-        combine_rows<VEC>(total, y, weights, entry_row, t, top, n, i);
+        combine_rows<VEC, true>(total, y, weights, entry_row, t, top, n, i);
         piece v;
 #pragma unroll
         for (int e = 0; e < VEC; ++e) v[e] = from_f32<T>(total[e]);
@@ -270,7 +270,8 @@ __global__ void moe_combine_shared_kernel(const float* __restrict__ y, const flo
     const float g = gates ? 1.f / (1.f + expf(-gates[(size_t)t * gate_cols + gate_column])) : 1.f;
     for (int i = threadIdx.x * VEC; i < n; i += blockDim.x * VEC) {
         float total[VEC];
-        combine_rows<VEC>(total, y, weights, entry_row, t, top, n, i);
+        if (weights) combine_rows<VEC, true>(total, y, weights, entry_row, t, top, n, i);
+        else combine_rows<VEC, false>(total, y, weights, entry_row, t, top, n, i);
         if (shared) {
             const shared_piece more = *reinterpret_cast<const shared_piece*>(shared + (size_t)t * n + i);
 #pragma unroll
@@ -356,7 +357,7 @@ LC_API int lc_moe_combine(const float* y, const float* weights, const int* entry
     LC_CHECK(T >= 0 && top > 0 && n > 0, "moe combine: bad sizes");
     if (T == 0) return 0;
     LC_CHECK(y && weights && entry_row && out, "moe combine: null pointer");
-    const bool whole = n % 4 == 0 && ((uintptr_t)y | (uintptr_t)out) % 16 == 0;
+    const bool whole = n % 4 == 0 && n >= 256 && ((uintptr_t)y | (uintptr_t)out) % 16 == 0;      // (fewer entries have a thread each anyway)
     const int pieces = whole ? n / 4 : n, threads = pieces >= 256 ? 256 : (pieces >= 128 ? 128 : 64);
     LC_CHECK(dt == DT_F32 || dt == DT_BF16, "moe combine: unknown dtype %d", dt);
 #define LC_COMBINE(TT, VEC) moe_combine_kernel<TT, VEC><<<T, threads, 0, stream>>>(y, weights, entry_row, top, n, (TT*)out)
@@ -389,7 +390,7 @@ LC_API int lc_moe_combine_shared(const float* y, const float* weights, const int
              "moe combine: bad sizes");
     if (T == 0) return 0;
     LC_CHECK(y && entry_row && out && (shared || !gates), "moe combine: null pointer");
-    const bool whole = n % 4 == 0 && ((uintptr_t)y | (uintptr_t)out | (uintptr_t)shared) % 16 == 0;
+    const bool whole = n % 4 == 0 && n >= 256 && ((uintptr_t)y | (uintptr_t)out | (uintptr_t)shared) % 16 == 0;
     const int pieces = whole ? n / 4 : n, threads = pieces >= 256 ? 256 : (pieces >= 128 ? 128 : 64);
 #define LC_COMBINE_AS(TO, TS, VEC)                                                                                  \
     moe_combine_shared_kernel<TO, TS, VEC><<<T, threads, 0, stream>>>(y, weights, entry_row, top, n, (const TS*)shared, \

@@ -33,7 +33,7 @@ def test_gated(dtype, T, I):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("n", [1, 8, 31, 4096, 100003])
+@pytest.mark.parametrize("n", [1, 8, 31, 4096, 100003, 1 << 20, (1 << 20) + 8, (1 << 20) + 9])
 def test_activation(dtype, n):
     x = (torch.randn(1, n, generator=torch.Generator().manual_seed(n)) * 4).to(dtype).to(DEV)
     for kind, f in ((1, gelu), (2, lambda z: torch.relu(z) ** 2), (6, torch.nn.functional.gelu)):
@@ -43,7 +43,7 @@ def test_activation(dtype, n):
 
 
 @pytest.mark.parametrize("dtype", DTYPES)
-@pytest.mark.parametrize("T,top,n", [(1, 1, 4), (7, 3, 66), (40, 4, 2048), (5, 2, 4100), (9, 2, 301)])
+@pytest.mark.parametrize("T,top,n", [(1, 1, 4), (7, 3, 66), (40, 4, 2048), (5, 2, 4100), (9, 2, 301), (6, 8, 2050), (3, 7, 512)])
 def test_combine(dtype, T, top, n):
     g = torch.Generator().manual_seed(T + n)
     E = top + 2
