@@ -24,6 +24,8 @@
 
 #include "gemm_tile.h"
 
+LC_API int lc_attention_generic_rows(int rows);        // attention_generic.hip
+
 namespace lc {
 
 constexpr int AF_UNIT = 16, AF_SPAN = 512, AF_WAVES = 4;
@@ -281,14 +283,13 @@ __device__ __forceinline__ void attend_columns(const F32Attention& a, int t0, in
     }
 }
 
-// grid (groups of rows, then lone rows, each with its kv heads by batches of 16 query heads side by side; 1; spans).  A group's rows are worked together when they
-// belong to one request, else request by request.
+// grid (kv heads by batches of 16 query heads; groups of rows, then lone rows; spans), so that a group's heads start side by side.  A group's
+// rows are worked together when they belong to one request, else request by request.
 template <int DB>
 __global__ __launch_bounds__(64 * AF_WAVES, 2) void attention_f32_kernel(F32Attention a) {
     __shared__ __attribute__((aligned(16))) float lds[DB * 256 + AF_WAVES * (2 * AF_COLUMNS + DB * 256)];
     const int group = a.nh / a.nkv, per = min(group, AF_COLUMNS), batches = (group + per - 1) / per;
-    const int columns = a.nkv * batches, at = blockIdx.x / columns, batch = blockIdx.x - at * columns;
-    const int kvh = batch / batches, h0 = kvh * group + batch % batches * per;
+    const int at = blockIdx.y, kvh = batches == 1 ? blockIdx.x : blockIdx.x / batches, h0 = kvh * group + (blockIdx.x - kvh * batches) * per;
     const int heads = min(per, (kvh + 1) * group - h0);
     if (at >= a.groups) {
         const int4 row = a.lone[at - a.groups];
@@ -346,12 +347,17 @@ __global__ __launch_bounds__(64 * AF_WAVES) void attention_f32_join_kernel(F32At
         make_float4(O4[0][0] / L4, O4[0][1] / L4, O4[0][2] / L4, O4[0][3] / L4);
 }
 
-// How a batch's rows are cut: `together` (rows that follow one another are mostly of one request) and how many lone rows have
-// workgroups of their own.
+// How a batch's rows are cut: rows a workgroup takes, workgroups that take rows, lone rows with a workgroup of their own.  A workgroup's rows
+// of several requests are worked one request after the other, so it takes no more than a portion has on average (64 portions of two rows, 8
+// heads over 8 of 128: 16 rows a workgroup 42.7 us, two 8.4; 40 of three after 600, 4 heads over 4 of 16: 57.5 and 15.5).
 struct F32Cut { int rows, groups, lone; };
 
-static F32Cut f32_cut(int T, int nh, int nkv, bool together, int lone) {
-    const int per = nh / nkv < AF_COLUMNS ? nh / nkv : AF_COLUMNS, rows = together ? AF_COLUMNS / per : 1;
+static F32Cut f32_cut(int T, int nh, int nkv, int requests, int lone) {
+    const int forced = lc_attention_generic_rows(-1);       // tests: one row, or as many as there is room for; no lone rows then
+    if (forced) lone = 0;
+    const int per = nh / nkv < AF_COLUMNS ? nh / nkv : AF_COLUMNS, most = AF_COLUMNS / per;
+    const int portions = requests - lone > 1 ? requests - lone : 1, mean = (T - lone) / portions;
+    const int rows = forced == 1 ? 1 : forced || mean >= most ? most : mean > 1 ? mean : 1;
     return {rows, lone == T ? 0 : (T + rows - 1) / rows, lone};
 }
 
@@ -369,7 +375,7 @@ static int f32_spans(int T, int nh, int nkv, int d, int max_blocks, int page_siz
 template <int DB>
 static void launch_f32(const F32Attention& a, int lone, hipStream_t stream) {
     const int group = a.nh / a.nkv, batches = (group + AF_COLUMNS - 1) / AF_COLUMNS;
-    attention_f32_kernel<DB><<<dim3((a.groups + lone) * a.nkv * batches, 1, a.spans > 0 ? a.spans : 1), 64 * AF_WAVES, 0, stream>>>(a);
+    attention_f32_kernel<DB><<<dim3(a.nkv * batches, a.groups + lone, a.spans > 0 ? a.spans : 1), 64 * AF_WAVES, 0, stream>>>(a);
     if (a.spans > 0) attention_f32_join_kernel<DB><<<dim3(a.T, a.nh), 64 * AF_WAVES, 0, stream>>>(a);
 }
 
@@ -384,17 +390,21 @@ LC_API int lc_attention_f32_takes(const void* q, int q_stride, const void* k_cac
            ((uintptr_t)q | (uintptr_t)k_cache | (uintptr_t)v_cache) % 16 == 0;
 }
 
-// float32 words of workspace that it needs (0: none)
-LC_API long long lc_attention_f32_workspace(int T, int nh, int nkv, int d, int max_blocks, int page_size, int together, int lone) {
-    if (T <= 0 || nh <= 0 || nkv <= 0 || nh % nkv || d <= 0 || max_blocks <= 0 || page_size <= 0 || lone < 0 || lone > T) return 0;
-    return (long long)T * nh * f32_spans(T, nh, nkv, d, max_blocks, page_size, f32_cut(T, nh, nkv, together != 0, lone)) * AF_WAVES * (d + 4);
+// float32 words of workspace that lc_attention_f32 needs (0: none) for T rows of `requests` requests, `lone` of which have a row and a list
+// entry each; -1: these sizes or operands are the general kernel's (grids are cut for up to 65,535 groups of rows and heads).
+LC_API long long lc_attention_f32_workspace(const void* q, int q_stride, const void* k_cache, const void* v_cache, int T, int nh, int nkv, int d,
+                                            int max_blocks, int page_size, int requests, int lone) {
+    if (!lc_attention_f32_takes(q, q_stride, k_cache, v_cache, nh, nkv, d, page_size) || T <= 0 || max_blocks <= 0 || lone < 0 || lone > T) return -1;
+    const F32Cut cut = f32_cut(T, nh, nkv, requests, lone);
+    if (nh > 65535 || (long long)cut.groups + cut.lone > 65535) return -1;
+    return (long long)T * nh * f32_spans(T, nh, nkv, d, max_blocks, page_size, cut) * AF_WAVES * (d + 4);
 }
 
-// together: rows that follow one another are mostly of one request, and worked together then.  lone_rows [lone, 4] (row, request, position,
+// requests: rows of the block table, which tells portions of many rows from portions of few.  lone_rows [lone, 4] (row, request, position,
 // any): all requests that have a single row, or none at all (lone 0).
 LC_API int lc_attention_f32(const void* q, int q_stride, const void* k_cache, const void* v_cache, void* out, const int* tok_req,
                             const int* positions, const int* block_table, int max_blocks, int T, int nh, int nkv, int d, int page_size,
-                            float scale, int window, int together, const int* lone_rows, int lone, float* workspace, hipStream_t stream) {
+                            float scale, int window, int requests, const int* lone_rows, int lone, float* workspace, hipStream_t stream) {
     LC_CHECK(T >= 0 && nh > 0 && nkv > 0 && d > 0 && page_size > 0 && max_blocks > 0 && lone >= 0 && lone <= T,
              "attention: bad sizes T=%d nh=%d nkv=%d d=%d page=%d blocks=%d lone=%d", T, nh, nkv, d, page_size, max_blocks, lone);
     if (T == 0) return 0;
@@ -402,22 +412,22 @@ LC_API int lc_attention_f32(const void* q, int q_stride, const void* k_cache, co
     LC_CHECK(q && k_cache && v_cache && out && tok_req && positions && block_table && (lone == 0 || lone_rows), "attention: null pointer");
     LC_CHECK(lc_attention_f32_takes(q, q_stride, k_cache, v_cache, nh, nkv, d, page_size) && ((uintptr_t)out | (uintptr_t)lone_rows) % 16 == 0,
              "attention: heads of %d and pages of %d tokens, or unaligned operands, are the general kernel's", d, page_size);
-    LC_CHECK(nh <= 65535 && 2ll * T * nh < 1ll << 31, "attention: too many heads (%d) for %d tokens", nh, T);
-    const F32Cut cut = f32_cut(T, nh, nkv, together != 0, lone);
+    const F32Cut cut = f32_cut(T, nh, nkv, requests, lone);
+    LC_CHECK(nh <= 65535 && (long long)cut.groups + cut.lone <= 65535, "attention: too many heads (%d) or rows (%d)", nh, T);
     const int spans = f32_spans(T, nh, nkv, d, max_blocks, page_size, cut);
     LC_CHECK(spans == 0 || (workspace && (uintptr_t)workspace % 16 == 0), "attention: T=%d with %d blocks needs a workspace", T, max_blocks);
     const F32Attention a{(const float*)q, q_stride, (const float*)k_cache, (const float*)v_cache, (float*)out, tok_req, positions, block_table,
                          max_blocks, T, nh, nkv, page_size, scale, window, workspace, spans, cut.rows, cut.groups,
-                         lone > 0 ? (const int4*)lone_rows : nullptr};
+                         cut.lone > 0 ? (const int4*)lone_rows : nullptr};
     switch (d / 16) {
-        case 1: launch_f32<1>(a, lone, stream); break;
-        case 2: launch_f32<2>(a, lone, stream); break;
-        case 3: launch_f32<3>(a, lone, stream); break;
-        case 4: launch_f32<4>(a, lone, stream); break;
-        case 5: launch_f32<5>(a, lone, stream); break;
-        case 6: launch_f32<6>(a, lone, stream); break;
-        case 7: launch_f32<7>(a, lone, stream); break;
-        default: launch_f32<8>(a, lone, stream);
+        case 1: launch_f32<1>(a, cut.lone, stream); break;
+        case 2: launch_f32<2>(a, cut.lone, stream); break;
+        case 3: launch_f32<3>(a, cut.lone, stream); break;
+        case 4: launch_f32<4>(a, cut.lone, stream); break;
+        case 5: launch_f32<5>(a, cut.lone, stream); break;
+        case 6: launch_f32<6>(a, cut.lone, stream); break;
+        case 7: launch_f32<7>(a, cut.lone, stream); break;
+        default: launch_f32<8>(a, cut.lone, stream);
     }
     LC_LAUNCH_CHECK("attention_f32");
     return 0;

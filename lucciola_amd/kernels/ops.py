@@ -194,7 +194,7 @@ def library():
         lib.lc_gemm_generic_workspace.restype = ctypes.c_longlong
         lib.lc_gemm_generic_workspace.argtypes = [ctypes.c_int] * 3
         lib.lc_attention_f32_workspace.restype = ctypes.c_longlong
-        lib.lc_attention_f32_workspace.argtypes = [ctypes.c_int] * 8
+        lib.lc_attention_f32_workspace.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int] * 8
         lib.lc_attention_generic_workspace.restype = ctypes.c_longlong
         lib.lc_attention_generic_workspace.argtypes = [ctypes.c_int] * 5
         lib.lc_scan_chunks_records.restype = ctypes.c_longlong
@@ -1065,21 +1065,20 @@ def attention(qkv, batch: AttentionBatch, k_cache: torch.Tensor,
                   _c_float(prologue.eps if own_q else 0.0), _ptr(rope if own_q else None),
                   rot if own_q else 0, pf_splits, _ptr(pf_o), _ptr(pf_ml), _stream())
         return out
-    if qkv.dtype == torch.float32 and lib.lc_attention_f32_takes(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), nh, nkv, d, page_size):
+    if qkv.dtype == torch.float32:
         # the requests' portions go several rows together, lone tokens (where the planner listed them) each by itself
-        forced = lib.lc_attention_generic_rows(-1)
-        lone = batch.decode_rows if batch.num_decode and not forced else None
+        lone = batch.decode_rows if batch.num_decode else None
         if lone is not None and lone.data_ptr() % 16:
             lone = None
         singles = batch.num_decode if lone is not None else 0
-        together = 1 if forced > 1 or (not forced and batch.num_decode < T) else 0
-        mb = batch.block_table.shape[1]
-        words = lib.lc_attention_f32_workspace(T, nh, nkv, d, mb, page_size, together, singles)
-        workspace = torch.empty((words,), dtype=torch.float32, device=qkv.device) if words else None
-        _call("lc_attention_f32", _ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(batch.tok_req),
-              _ptr(batch.positions), _ptr(batch.block_table), mb, T, nh, nkv, d, page_size, scale, window, together, _ptr(lone), singles,
-              _ptr(workspace), _stream())
-        return out
+        R, mb = batch.block_table.shape
+        words = lib.lc_attention_f32_workspace(_ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), T, nh, nkv, d, mb, page_size, R, singles)
+        if words >= 0:
+            workspace = torch.empty((words,), dtype=torch.float32, device=qkv.device) if words else None
+            _call("lc_attention_f32", _ptr(qkv), qkv.shape[1], _ptr(k_cache), _ptr(v_cache), _ptr(out), _ptr(batch.tok_req),
+                  _ptr(batch.positions), _ptr(batch.block_table), mb, T, nh, nkv, d, page_size, scale, window, R, _ptr(lone), singles,
+                  _ptr(workspace), _stream())
+            return out
     words = lib.lc_attention_generic_workspace(T, nh, nkv, batch.block_table.shape[1], page_size)
     workspace = torch.empty((words,), dtype=torch.float32, device=qkv.device) if words else None
     _call("lc_attention_generic", _ptr(qkv), _c_int(qkv.shape[1]), _ptr(k_cache), _ptr(v_cache),

@@ -47,6 +47,19 @@ def test_edges(nh, nkv, d, page, window):
         assert torch.equal(run(qkv.repeat(times, 1), many, kc, vc, nh, nkv, d, page, window, rows=rows), got.repeat(times, 1))
 
 
+@pytest.mark.parametrize("nh,nkv", [(2, 2), (4, 1), (6, 2), (17, 1)])
+@pytest.mark.parametrize("lengths,new", [([2] * 30, [2] * 30), ([600, 3, 40, 520] * 3, [3] * 12), ([50, 9, 700], [2, 9, 1]), ([5] * 9, [1, 2, 3] * 3)])
+def test_short_portions(nh, nkv, lengths, new):
+    """A workgroup takes as many rows as a portion has on average: the same bits as row by row and as with all that it has room for."""
+    d, page = 32, 16
+    qkv, batch, kc, vc = paged_case(lengths, new, nh, nkv, d, page, torch.float32, seed=nh)
+    got = run(qkv, batch, kc, vc, nh, nkv, d, page, 0)
+    plain = AttentionBatch(batch.tok_req.cpu(), batch.positions.cpu(), batch.block_table.cpu())
+    close(got, ref.attention(qkv.cpu().double(), plain, kc.cpu().double(), vc.cpu().double(), nh, nkv, d, page, d ** -0.5, 0), torch.float32)
+    for rows in (1, 4):
+        assert torch.equal(run(qkv, batch, kc, vc, nh, nkv, d, page, 0, rows=rows), got)
+
+
 @pytest.mark.parametrize("bad", [float("inf"), float("nan")])
 @pytest.mark.parametrize("window", [0, 9])
 def test_a_value_that_is_not_finite_reaches_only_who_sees_it(bad, window):
