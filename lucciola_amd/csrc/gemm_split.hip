@@ -282,8 +282,14 @@ __global__ __launch_bounds__(256, 2) void gemm_split_few_kernel(const float* __r
     for (int c = c_begin; c < c_end; ++c) {
         const int k0 = c * GS_CHUNK, k_end = min(K, k0 + GS_CHUNK), steps = (k_end - k0) / 16;      // K is a multiple of 32
         bf16x8 b[STEPS];
+        if (steps == STEPS) {
 #pragma unroll
-        for (int s = 0; s < STEPS; ++s) b[s] = load8<WHOLE>(wg + k0 + 16 * min(s, steps - 1));
+            for (int s = 0; s < STEPS; ++s) b[s] = load8<WHOLE>(wg + k0 + 16 * s);
+        } else {
+#pragma unroll
+            for (int s = 0; s < STEPS; ++s)
+                if (s < steps) b[s] = load8<WHOLE>(wg + k0 + 16 * s);
+        }
         if (c > c_begin) __syncthreads();       // the chunk before is read by everybody
 #pragma unroll
         for (int i = 0; i < PIECES / 16; ++i) {
