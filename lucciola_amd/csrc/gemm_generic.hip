@@ -17,6 +17,9 @@
 // float32 x by bfloat16 w in whole steps of 32 k has kernels of its own, twice as fast (gemm_split.hip); this entry's workspace and the sum
 // of shared chunks serve both.
 //
+// The figures here are of what those kernels replaced, the product with bfloat16 w on the float32 instruction; the loop is the one
+// that float32 w, float32 x of a broken K and 16-bit x of a broken K still run.
+//
 // Bound by the matrix instruction: 143 TFLOP/s from registers alone on this card.  What kept the first form of the loop
 // at 88 (2,048 x 4,096 x 1,024, bfloat16 w, 195 us) was what stood between the products: loads behind a test of k each, whose rows
 // were set to zero right behind them, so that each waited for its own trip; LDS writes four to a bank; and all of a stage's LDS work
@@ -264,8 +267,6 @@ static int chunks_per_workgroup(int M, int N, int K) {
     return (int)((chunks + shares - 1) / shares);
 }
 
-static thread_local bool g_generic_plain = false;     // tests: float32 x by bfloat16 w here too
-
 template <typename TX, typename TW, typename TO>
 static int launch_generic(const void* x, const void* w, void* out, int M, int N, int K, float* workspace,
                           hipStream_t stream) {
@@ -300,12 +301,11 @@ static int launch_generic(const void* x, const void* w, void* out, int M, int N,
         else if (part) launch(Tile{}, Tile{}, two, is_whole, std::true_type{});
         else launch(Tile{}, Tile{}, two, is_whole, std::false_type{});
     };
-    bool split = false;
-    if constexpr (std::is_same_v<TX, float> && std::is_same_v<TW, bf16> && std::is_same_v<TO, float>) {
-        split = !g_generic_plain && gemm_split_takes(K);
-        if (split) launch_gemm_split((const float*)x, (const bf16*)w, (float*)out, M, N, K, part, per, shares, stream);
-    }
-    if (!split) {
+    constexpr bool SPLITS = std::is_same_v<TX, float> && std::is_same_v<TW, bf16> && std::is_same_v<TO, float>;
+    if constexpr (SPLITS) {             // a K that is whole has kernels of its own
+        if (gemm_split_takes(K)) launch_gemm_split((const float*)x, (const bf16*)w, (float*)out, M, N, K, part, per, shares, stream);
+        else with_shape(std::false_type{});
+    } else {
         if (whole) with_shape(std::true_type{});
         else with_shape(std::false_type{});
     }
@@ -324,14 +324,6 @@ static int launch_generic(const void* x, const void* w, void* out, int M, int N,
 }  // namespace lc
 
 using namespace lc;
-
-// Tests: whether float32 x by bfloat16 w stays with the float32 instruction (1) or is cut in three (0, the default).  Returns the setting
-// before.
-LC_API int lc_gemm_generic_plain(int on) {
-    const int before = g_generic_plain ? 1 : 0;
-    if (on >= 0) g_generic_plain = on != 0;
-    return before;
-}
 
 // float32 words of workspace that lc_gemm_generic needs for these sizes (0: none)
 LC_API long long lc_gemm_generic_workspace(int M, int N, int K) {

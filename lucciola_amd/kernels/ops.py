@@ -29,7 +29,6 @@ _SIGNATURES = {
     "lc_rmsnorm": "ppppfpiiiipiipp",
     "lc_rmsnorm_act": "pqpfpiiip",
     "lc_gemm_generic": "pipipiiiipp",
-    "lc_gemm_generic_plain": "i",
     "lc_gemm_bf16": "pppiiiiipp",
     "lc_gemm_bf16_gated": "pppiiiifffpp",
     "lc_gemm_bf16_supported": "iii",

@@ -9,12 +9,8 @@ pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
 
 
-def product(x, w, plain=0):
-    ops.library().lc_gemm_generic_plain(plain)
-    try:
-        return ops.gemm(x, w, torch.float32)
-    finally:
-        ops.library().lc_gemm_generic_plain(0)
+def product(x, w):
+    return ops.gemm(x, w, torch.float32)
 
 
 @pytest.mark.parametrize("M", [1, 15, 16, 17, 63, 65, 200])
@@ -27,7 +23,7 @@ def test_edges(M, N, K):
     # K products, exact, added in float32: each addition is off by 2^-24 of a sum that is no larger than the terms' absolute values
     allowed = 2.0 ** -24 * K * (x.double().abs() @ w.double().abs().T)
     assert bool(((got.double() - want).abs() <= allowed).all())
-    plain = product(x, w, plain=1)
+    plain = product(x, w.float())           # float32 by float32, on the float32 instruction
     if M * N >= 10000:      # a root mean square over n errors is itself off by some 1 / sqrt(2 n) of it: 0.7 % here, 20 % at 15 entries
         assert float((got.double() - want).norm()) <= 1.05 * float((plain.double() - want).norm())
     # a row alone, few rows and many have the same bits
