@@ -29,6 +29,7 @@ typedef float floatx4 __attribute__((ext_vector_type(4)));
 constexpr int LM_THREADS = 512;       // eight waves: four pairs, a pair shares its query columns
 constexpr int LM_STAGE = 32;          // keys of a stage
 constexpr int LM_ROT_MOST = 128;      // rotated entries of a row, at most
+constexpr int LM_TILES = 65535;       // rows of tiles of a grid's layer
 constexpr int LM_KPAD = 8;            // bf16 of padding behind a staged row
 constexpr int LM_VSTRIDE = LM_STAGE + 8;   // bf16 between two entries' key runs in the transposed stage
 
@@ -40,7 +41,7 @@ template <int NR, int KS>
 __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     const bf16* __restrict__ qa, int H, int R, int rot, const bf16* __restrict__ cache,
     const int* __restrict__ tiles, const int* __restrict__ block_table, int max_blocks, int page_size,
-    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int per_tile, int blocks_y,
+    float scale, int window, const float* __restrict__ sink, bf16* __restrict__ out, int splits, int per_tile, int num_tiles, int near_bits,
     float* __restrict__ part_o, float* __restrict__ part_ml) {
     extern __shared__ __align__(16) unsigned char lds_raw[];
     const int Dk = R + rot, Dp = KS * 32;
@@ -54,11 +55,22 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     // waves share every SIMD
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 7, half = (tid >> 6) & 1, col = lane & 15, g = lane >> 4;
     constexpr int NH = NR / 2;
-    const int tile_at = blockIdx.x / blocks_y;      // a tile's heads are neighbours: the longest tiles start first, with all of their heads
+    // grid (2^near_bits tiles for each group of heads; the rows of so many tiles; the shares, once for every 65,535 rows).  A tile's
+    // groups of heads begin close to each other, so that the longest tiles start first with all of their heads, and, from 64 tiles,
+    // eight workgroups apart, so that they read the tile's keys through the same L2 (an XCD takes every eighth workgroup).  us, rank 512,
+    // group by group of heads (each begins when all tiles of the one before have) and so: 2,048 tokens, 16 heads 434 -> 277, 32 heads
+    // 745 -> 540, behind 2,048 others 892 -> 751 and 1,678 -> 1,489.  Side by side, not eight apart: rank 256, 8 heads 139 -> 136 and
+    // behind 2,048 others 278 -> 268, 16 x 64 tokens behind 500 46.0 -> 44.4; the rest within 1 %.
+    int split = blockIdx.z, tile_at = (int)(blockIdx.y << near_bits) + (int)(blockIdx.x & ((1u << near_bits) - 1));
+    while (split >= splits) {
+        split -= splits;
+        tile_at += LM_TILES << near_bits;
+    }
+    if (tile_at >= num_tiles) return;
     const int* tile = tiles + 4 * tile_at;
     const int t0 = tile[0], ntok = tile[1], req = tile[2], p0 = tile[3];
     const bool lone = ntok == 1;
-    const int h0 = (int)(blockIdx.x - tile_at * blocks_y) * (lone ? 64 : 4);
+    const int h0 = (int)(blockIdx.x >> near_bits) * (lone ? 64 : 4);
     if (h0 >= H) return;
     // this lane's query column
     const int q_tok = lone ? 0 : col, q_head = lone ? h0 + 16 * wave + col : h0 + wave;
@@ -73,7 +85,7 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     const int j_lo = (window > 0 && p0 - window + 1 > 0) ? p0 - window + 1 : 0;
     const int stages = (p_last - j_lo) / LM_STAGE + 1;
     const int per = (stages + splits - 1) / splits;
-    const int s_begin = blockIdx.z * per, s_end = min(stages, s_begin + per);
+    const int s_begin = split * per, s_end = min(stages, s_begin + per);
     const int* table = block_table + (size_t)req * max_blocks;
 
     // the queries as operands: entries 32 ks + 8 g ... of the lane's column
@@ -273,15 +285,15 @@ __global__ __launch_bounds__(LM_THREADS) void latent_attention_bf16_kernel(
     } else {
         // a share's place goes by token, or (per_tile > 0) by tile, where the step holds tokens that are in no tile
         const size_t place = per_tile ? ((size_t)tile_at * per_tile + q_tok) * H + q_head : qi;
-        float* dst = part_o + (place * splits + blockIdx.z) * R;
+        float* dst = part_o + (place * splits + split) * R;
 #pragma unroll
         for (int d = 0; d < NH; ++d)
             if ((half * NH + d) * 16 < R)
 #pragma unroll
                 for (int r = 0; r < 4; ++r) dst[(half * NH + d) * 16 + 4 * g + r] = o[d][r];
         if (g == 0 && half == 0) {
-            part_ml[(place * splits + blockIdx.z) * 2] = m_run;
-            part_ml[(place * splits + blockIdx.z) * 2 + 1] = l_run;
+            part_ml[(place * splits + split) * 2] = m_run;
+            part_ml[(place * splits + split) * 2 + 1] = l_run;
         }
     }
 }
@@ -434,10 +446,12 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
                                           splits, part_o, part_ml, stream);
         return rc ? rc : join();
     }
-    const int blocks_y = portions ? (H + 3) / 4 : (H + 63) / 64;
-    LC_CHECK(blocks_y <= 65535, "latent attention: too many heads (%d)", H);
-    LC_CHECK((long long)num_tiles * blocks_y < 1ll << 31, "latent attention: too many tiles");
-    const dim3 grid(num_tiles * blocks_y, 1, splits);
+    const int groups = portions ? (H + 3) / 4 : (H + 63) / 64;
+    LC_CHECK(groups <= 65535, "latent attention: too many heads (%d)", H);
+    const int near_bits = num_tiles >= 64 ? 3 : 0;
+    const long long rows = ((long long)num_tiles + (1 << near_bits) - 1) >> near_bits, layers = (rows + LM_TILES - 1) / LM_TILES;
+    LC_CHECK((long long)num_tiles * groups < 1ll << 31 && layers * splits <= 65535, "latent attention: too many tiles");
+    const dim3 grid(groups << near_bits, (unsigned)(rows < LM_TILES ? rows : LM_TILES), (unsigned)(layers * splits));
     const size_t lds = sizeof(bf16) * ((size_t)LM_STAGE * (ks * 32 + LM_KPAD) + (size_t)R * LM_VSTRIDE) +
                        sizeof(int) * 2 * LM_STAGE;
 #define LC_LM_LAUNCH(NR, KS)                                                                                       \
@@ -448,7 +462,7 @@ LC_API int lc_latent_attention_bf16(const void* qa, int T, int H, int R, int rot
                      "latent attention: %zu bytes of LDS refused", lds);                                           \
         latent_attention_bf16_kernel<NR, KS><<<grid, LM_THREADS, lds, stream>>>(                                    \
             (const bf16*)qa, H, R, rot, (const bf16*)cache, tiles, block_table, max_blocks, page_size, scale, window, \
-            sink, (bf16*)out, splits, per_tile, blocks_y, part_o, part_ml);                                           \
+            sink, (bf16*)out, splits, per_tile, num_tiles, near_bits, part_o, part_ml);                               \
     } while (0)
     if (nr == 4) LC_LM_LAUNCH(4, 4);
     else if (nr == 8) LC_LM_LAUNCH(8, 8);
