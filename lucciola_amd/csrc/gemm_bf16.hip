@@ -800,8 +800,12 @@ static int shares_for(int t, int M, int N, int K, bool partials_wanted = false) 
 
 // The tile for a product with M > 16.  Up to 64 rows: a 64-row tile.  Beyond: the shape with
 // the least estimated time in microseconds.  A CU works through a round of tiles in
-// (tile area) x K x 2 / (4.63 MFLOP/us x the shape's relative rate) (measured at K = 4096: larger
-// tiles move fewer bytes per product) and 3 us to start and end.  A last round of a one-a-CU shape
+// (tile area) x K x 2 / (4.63 MFLOP/us x the shape's relative rate) (measured at K = 4096, with a loop
+// that issued a block's loads in a row: larger tiles move fewer bytes per product) and 3 us to start
+// and end.  On the loop that runs now, weights cold, four products of six model sizes at 96 to 4,001
+// rows, the shape picked is within 8 % of the best of all shapes in 174 of 212 cases (that loop: 177)
+// and 2.2 % from it in the mean; rates fitted to these very cases bring that to 1.7 % and make some
+// 8 % slower, and so the rates stand.  A last round of a one-a-CU shape
 // that is cut along K takes its share of that, plus the time to write and read its float32
 // partial tiles (about 4 TB/s) and to start two more kernels.  A small tile cut along K as a
 // whole pays for its partial sums likewise, unless the caller takes them as they are
@@ -845,8 +849,7 @@ static int pick_tile(int M, int N, int K, bool partials_wanted = false) {
         // 64 x 64, 31.2 as tiles of 128 x 128 cut along K four ways; 576 x 1024 x 3072 18.7 against 22.3)
         // (up to 256 rows only for a w of up to 32 MB: 128 x 4096 x 4096 with its norm 19.2 us against 21.1 in
         // tiles of 64 x 128; on a large w every tile of 64 rows of w reads all of x again: 128 x 24576 x 4096
-        // 61.8 against 50.8 in tiles of 192 x 128.  Measured over the four products of six model sizes at 96 to
-        // 4,096 rows, the shape picked is within 8 % of the best of all shapes in 208 of 216 cases.)
+        // 61.8 against 50.8 in tiles of 192 x 128)
         if (t == TILE_64x64 && M <= 256 && (long long)N * K > (1ll << 24)) continue;
         const long long tiles = tile_count(t, M, N);
         const double area = (double)tile_bm(t) * tile_bn(t);

@@ -76,7 +76,7 @@ __device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
 // bytes that L2 holds): the 16 loads of a wave of the 256 x 256 tile, four waves at once, are a
 // thousand clocks in which a wave that issues them in a row issues no product.  In a row, behind
 // the barrier or in the first k-step (us; the same sums): 2,048 x 24576 x 4096 with SwiGLU 367,
-// 2,048 x 4096 x 12288 193, 2,048 x 2048 x 2048 26.3; spread: 328, 171 and 22.9 (the matrix cores
+// 2,048 x 4096 x 12288 193, 2,048 x 2048 x 2048 26.3; spread over the first half: 328, 171 and 22.9 (the matrix cores
 // busy 69 % of the clocks instead of 56, at a clock that the power limit takes from 1.84 to
 // 1.64 GHz; 2.4 without load).
 constexpr int TL_K = 64;
@@ -121,13 +121,16 @@ struct TileLoop {
                 (lds_ptr_t)(lds + S * A_STAGE + stage * B_STAGE + ((idx - LPA) * NW + wave) * 1024), 16, 0, 0);
     };
     // Where the loads of a block sit among the products: position 0 is the first product behind the barrier that frees their
-    // stage.  With two stages they have to be back at the next barrier and are issued in the first half; with more they are spread
-    // over the whole block but its end (from a third to the whole of it: within 2 %; two stages and three quarters: 345 us
-    // where 328 stand above).
+    // stage.  With more than two stages they are spread over the whole block but its end (from a third to the whole of it: within
+    // 2 %).  With two they have to be back at the next barrier and are issued in its first quarter: in a row, over the first half,
+    // over the first quarter, over an eighth (geometric means of four shapes of tile, 212 products of 96 to 4,001 rows on cold data):
+    // 1, 1.007, 0.973, 0.989; 192 x 256 of up to 333 rows 1, 1.08, 1.04, 1.04.  Few rows wait for w and want its loads early; many are
+    // bound by the matrix cores and want them late (us, in a row, half, quarter: 4,001 x 4096 x 4096 121, 110, 115; 1,024 x 4096 x
+    // 4096 49, 43, 45; 2,048 x 4096 x 12288 198, 173, 171; 576 x 19456 x 2560 61, 67, 65).
     constexpr int BAR = NM / 4;                                // the product after which a block's last k-step syncs
     constexpr int WIN = KS * NM;                               // products between two barriers
     constexpr int NA = NM - 1 - BAR;                           // of them in the block that frees the stage
-    constexpr int SPAN = S == 2 ? WIN / 2 : WIN * 7 / 8;
+    constexpr int SPAN = S == 2 ? WIN / 4 : WIN * 7 / 8;
     static_assert(SPAN >= 1 && SPAN < WIN, "all loads of a block are issued before the next barrier");
     struct At { static constexpr int of(int l) { return l * SPAN / LP; } };      // load l's position
     // Tiles of two stages with few products a block are several to a CU and bound by how much is on its way, and issue a whole
