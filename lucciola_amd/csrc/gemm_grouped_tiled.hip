@@ -463,11 +463,17 @@ bool grouped_tiled_takes(const GroupedArgs& a, int tile_rows) {
 // faster at every size tried; below it depends on how many workgroups there are (us, gemm_grouped.hip and these):
 //   stream   one round of two workgroups a CU gains (16 heads, 512 columns of 128 k, 64 rows 4.2 and 3.8), more lose: the same
 //            at 32 heads 5.1 and 5.4, 400 rows over 32 experts of 2,048 x 128 6.0 and 7.5.  Products per head from 256 k on gain too.
-//   128 rows likewise one round gains (8,192 rows, 32 experts of 512 x 256 19.0 and 16.2), more lose (8 of 2,048 x 256 24.8 and 27.1)
+//   128 rows (the even tiles) likewise one round gains (8 experts of 256 rows, 2,048 x 256 16.8 and 10.8, of 400 rows, 512 x 128
+//            11.8 and 9.0); less than 192 k has to be one round of one even workgroup a CU, as a round is then mostly what it starts
+//            and ends with: 96 experts of 200 rows, 128 columns of 128 k, 13.0 and 11.0, 128 of them (328 workgroups) 13.5 and 14.4,
+//            256 20.8 and 26.6.  More rounds than that mostly gain too (8 x 1,024 rows, 2,048 x 256 34.2 and 24.9; 64 x 256 rows,
+//            4,096 x 256 102.0 and 111.5) and are not taken.  With the activation in it a
+//            product saves a kernel, and the line below 192 k is not drawn (128 x 200 rows, 2 x 64 columns of 128 k 19.7 and 15.5;
+//            256 x 200 rows 30.3 and 30.2).
 //   64 rows  experts: 384 k and a workgroup for every CU (18.0 and 18.3 at the worst, 116 and 84 at the best); 256 k lose 10 % at
 //            few workgroups.  Per head: the shorter K, the more full tiles it takes: of 128 k 160 rows, 16 heads, 512 columns 5.8 and
 //            6.6, 2,048 rows 22.7 and 21.6; of 192 k 6.5 and 7.0, and 8.0 and 7.3 at 512 rows; of 64 k it mostly loses (10.1 and 12.4).
-bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows) {
+static bool rounds_pay(const GroupedArgs& a, int max_tiles, int tile_rows) {
     const double columns = (a.N + (tile_rows == 16 ? STREAM_N : 128) - 1) / (tile_rows == 16 ? STREAM_N : 128);
     const double workgroups =
         columns * (a.row_start ? (max_tiles < a.M ? max_tiles : a.M) : (double)((a.M + tile_rows - 1) / tile_rows) * a.G);
@@ -480,6 +486,11 @@ bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows) {
     return a.K >= 128 && full * full / workgroups >= 32 * short_by * short_by * short_by;
 }
 
+bool grouped_tiled_pays(const GroupedArgs& a, int max_tiles, int tile_rows) {
+    if (tile_rows == 128 && a.K < 192 && (double)(a.M / 128 + a.G) * ((a.N + EVEN_N - 1) / EVEN_N) > device_cus()) return false;
+    return rounds_pay(a, max_tiles, tile_rows);
+}
+
 int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, bool out_bf16, bool forced, hipStream_t stream) {
     return out_bf16 ? grouped_tiled<bf16>(a, max_tiles, tile_rows, forced, stream)
                     : grouped_tiled<float>(a, max_tiles, tile_rows, forced, stream);
@@ -488,7 +499,7 @@ int launch_grouped_tiled(const GroupedArgs& a, int max_tiles, int tile_rows, boo
 // a.N: gate and up columns together
 bool grouped_gates(const GroupedArgs& a, int tile_rows, bool forced) {
     if (tile_rows == 16 || a.N % 16 || !even_takes(a)) return false;
-    return forced || (even_pays(a, tile_rows, true) && grouped_tiled_pays(a, a.M / tile_rows + a.G, tile_rows));
+    return forced || (even_pays(a, tile_rows, true) && rounds_pay(a, a.M / tile_rows + a.G, tile_rows));
 }
 
 bool grouped_evens(const GroupedArgs& a, int max_tiles, int tile_rows) {

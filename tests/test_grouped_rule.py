@@ -26,6 +26,14 @@ def test_experts(tile, tokens, top, experts, columns, K, tiled):
     assert bool(ops.library().lc_gemm_grouped_picks_tiled(tile, rows, columns, K, experts, rows // tile + experts)) == tiled
 
 
+@pytest.mark.parametrize("experts,columns,K,tiled", [
+    (96, 128, 128, True), (128, 128, 128, False), (128, 128, 160, False), (128, 128, 192, True), (128, 129, 192, False), (8, 2048, 128, True),
+    (48, 512, 128, True), (64, 512, 128, False)])
+def test_experts_of_a_short_k(experts, columns, K, tiled):
+    rows = experts * 200 // 4 * 4
+    assert bool(ops.library().lc_gemm_grouped_picks_tiled(128, rows, columns, K, experts, rows // 128 + experts)) == tiled
+
+
 # lists for tiles of 64 rows: one workgroup of 64 x 128 a CU and fewer, more of them, w so large that memory counts, a short K
 @pytest.mark.parametrize("rows,experts,columns,K,even", [
     (400, 4, 1024, 2048, False), (1520, 8, 1024, 4096, False), (1600, 16, 1024, 2048, False), (800, 4, 512, 1024, False), (2240, 16, 768, 2048, True),
