@@ -271,6 +271,17 @@ def test_attention_general_kernel_same_bits_alone_and_in_a_prompt(dtype, nh, nkv
     assert torch.equal(odd, got[1:])
 
 
+# float32 that the general kernel serves: heads above 128, and pages of which the cache's rows of values are not whole 16-byte pieces
+@pytest.mark.parametrize("nh,nkv,d,page,window", [(4, 2, 144, 16, 0), (6, 2, 200, 16, 700), (4, 4, 256, 16, 1100), (16, 2, 256, 32, 0),
+                                                   (8, 8, 160, 8, 33), (6, 2, 48, 6, 0), (4, 4, 128, 2, 700), (5, 1, 64, 30, 40)])
+def test_attention_general_kernel_float32(nh, nkv, d, page, window):
+    """The same bits alone, in a prompt and with the spans shared out, and a mixed batch, at float32 sizes of the general kernel."""
+    q = torch.empty((nh + 2 * nkv) * d, device=DEV)
+    assert not ops.library().lc_attention_f32_takes(ops._ptr(q), q.numel(), ops._ptr(q), ops._ptr(q), nh, nkv, d, page)
+    test_attention_general_kernel_same_bits_alone_and_in_a_prompt(torch.float32, nh, nkv, d, page, window)
+    test_attention_mixed_batch(torch.float32, nh, nkv, d, page, window)
+
+
 @pytest.mark.parametrize("dtype", DTYPES)
 def test_attention_far_key_stands_out(dtype):
     """One key among many hundreds gets a large score: the output must be its value row, so a
