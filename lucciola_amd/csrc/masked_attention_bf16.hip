@@ -345,10 +345,11 @@ __device__ __forceinline__ void finish_column(const ColumnState<DVB, MAPS>& st, 
 }
 
 // The order in which workgroups start.  Grid (kv heads; tiles; a layer for every 65,535 tiles): a tile's kv heads are neighbours and the longest
-// tiles of all heads come first.  Where all workgroups are on the card at once there is nothing to gain by that, and a tile's kv heads, whose
-// keys are neighbours in memory, are better read by one XCD (workgroup number % 8) than by several at once: grid (tiles; kv heads; zsplits).
-// Lone tokens, 16 heads over 4, keys of 64 and values of 128: 64 at 2,048, 256 workgroups, 51 and 37 us, 8 at 2,048 20.3 and 15.6; keys and values
-// of 128, heads over 16, 64 tokens at 128 to 2,047, 1,024 workgroups, 98 and 147.
+// tiles of all heads come first, so that of the two workgroups of a CU one is long and one short.  Lone tokens, up to one workgroup a CU,
+// have nothing of that, and a tile's kv heads, whose keys are neighbours in memory, are read by one XCD (workgroup number % 8):
+// grid (tiles; kv heads; zsplits).  us, by heads and by tiles, 16 heads over 4, keys of 64 and values of 128: 64 tokens at 2,048, 256
+// workgroups, 51 and 37, 8 at 2,048 20.3 and 15.6 (8 at 191 to 2,047, two maps, 25.5 and 30.6: shares of a long token on one XCD); keys and
+// values of 128, 64 tokens at 511 to 8,000: heads over 8, 512 workgroups, 180 and 292, over 16 288 and 507.
 constexpr int MB_GRID = 65535;
 
 template <int DSTEPS, int DVB, int MAPS>
@@ -772,7 +773,7 @@ LC_API int lc_masked_attention_bf16(const void* q, const void* k_cache, const vo
     if (staged_lds < meet_lds) staged_lds = meet_lds;
     a.lone_only = staged ? 1 : 0;
     const bool main_kernel = !staged || any_lone;
-    a.at_once = zsplits > 1 || (long long)num_tiles * kv_heads <= 2 * device_cus() ? 1 : 0;
+    a.at_once = zsplits > 1 || (long long)num_tiles * kv_heads <= device_cus() ? 1 : 0;
     const dim3 portions_grid(kv_heads, num_tiles < MB_GRID ? num_tiles : MB_GRID, (num_tiles + MB_GRID - 1) / MB_GRID);
     const dim3 grid = a.at_once ? dim3(num_tiles, kv_heads, zsplits) : portions_grid;
     const dim3 join_grid(num_tiles, kv_heads);         // on the XCDs that left the shares

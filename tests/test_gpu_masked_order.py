@@ -52,7 +52,7 @@ def test_heads_a_kv_head(heads, kv, maps, d, dv):
     near(*both([0, 70, 300, 9], [100, 33, 17, 1], heads, kv, maps, d, dv))
 
 
-@pytest.mark.parametrize("requests,kv", [(1, 3), (7, 4), (9, 4), (128, 4), (129, 4), (200, 16), (1030, 1)])
+@pytest.mark.parametrize("requests,kv", [(1, 3), (7, 4), (9, 4), (64, 4), (65, 4), (128, 4), (129, 4), (200, 16), (1030, 1)])
 @pytest.mark.parametrize("window", [0, 100])
 def test_lone_tokens(requests, kv, window):
     history = [1 + (37 * r) % 700 for r in range(requests)]
