@@ -21,7 +21,8 @@
 // bytes in a row of the transposed page), so the weights never leave the registers.
 // The workgroups go tile by tile, a tile's kv heads beside each other, and the list has the longest tiles first: with all tiles of
 // one kv head before the next head's, the last head's longest tile began when half of the card had run dry (2,048 tokens, four kv
-// heads, a workgroup a CU: 202 -> 136 us for two maps of 64, 207 -> 143 for one of 128 with the bias; 1,523 tokens 102 -> 78).
+// heads, a workgroup a CU: 202 -> 136 us for two maps of 64, 207 -> 143 for one of 128 with the bias; 1,523 tokens 102 -> 78; with two
+// blocks of keys a step, below, 123 for two maps, 100 for one of 128 without the bias, 69).
 #include "common.h"
 
 namespace lc {
