@@ -549,6 +549,10 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
     const size_t k_row = (size_t)a.kv_heads * d_all;
     constexpr int PIECES = 2;                                   // a thread's pieces of each kind at most
     constexpr int SETS = (MAPS == 2 && DVB == 8) || (MAPS == 1 && !PAIRS) ? 1 : 2;    // stages on their way in registers: two if there is room
+    // Where operands and sums leave next to no registers, what a pass over a group's heads needs at its start and at its end is worked out there and
+    // not kept through the stages: two maps of 64, values of 128 had 20 to 72 bytes of scratch a lane (2,048 tokens, 16 heads over 4, with the bias 110 us, 103
+    // so; without 96.7 and 97.4).  Elsewhere it is kept: one map of 128, 128 68.7 us, and 70 worked out anew.
+    constexpr bool FULL = PAIRS && MAPS == 2 && DVB == 8;
     typedef int int4v __attribute__((ext_vector_type(4)));
     struct Pieces { int4v k[PIECES], v[PIECES]; };
     // A thread's places in a stage are counted in units that the build knows (KP pieces a key row, DVB * 32 pieces a
@@ -567,8 +571,8 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
     const int k_to = key * K_PITCH + piece * 16, v_to = K_BYTES + row * MB_VALUE_PITCH + v_block * 32 + half * 16;
     // The pages' numbers: a lane holds the one of the walk's block 64 c + lane, 64 blocks at a time, the next 64 asked for while these
     // are walked.  (Read as scalars when they are needed they would be waited for at the next operand from LDS: both count there.)
-    auto pages_of = [&](int first) {
-        const int block = blocks.block(min(first + lane, blocks.count - 1));
+    auto pages_of = [&](int first, int of_lane) {
+        const int block = blocks.block(min(first + of_lane, blocks.count - 1));
         return table[a.page_size == 16 ? block : block * 16 / a.page_size];
     };
     int pages_now = 0, pages_next = 0;
@@ -577,7 +581,7 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
         const int first = stage * stage_blocks;
         if (first > 0 && first % kWave == 0 && first < blocks.count) {
             pages_now = pages_next;
-            pages_next = pages_of(first + kWave);
+            pages_next = pages_of(first + kWave, lane);
         }
         auto one = [&](int blk, int& page, int& within) {
             const int at = first + blk;
@@ -612,21 +616,24 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
     };
     ColumnState<DVB, MAPS> st;
     for (int h0 = 0; h0 < group; h0 += places) {
+        int lane_now = lane;
+        if constexpr (FULL) asm volatile("" : "+v"(lane_now));
+        const int col_now = lane_now & 15;
         const int hh = h0 + place;
         const bool wave_on = hh < group && split < splits;
-        const bool on = wave_on && col < n;
+        const bool on = wave_on && col_now < n;
         const int head = g * group + (hh < group ? hh : 0);
-        const int tok = t0 + (col < n ? col : 0);
-        const int pos = on ? p0 + col : -1;
-        const int lo = on ? first_key(pos) : 0;
+        const int tok = t0 + (col_now < n ? col_now : 0);
+        const int pos = on ? p0 + col_now : -1;
+        const int lo = (FULL ? pos >= 0 : on) ? first_key(pos) : 0;
         bf16x8 bq[MAPS][DSTEPS];
-        load_queries<DSTEPS, MAPS>(bq, a, tok, head, pos, lane);
+        load_queries<DSTEPS, MAPS>(bq, a, tok, head, pos, lane_now);
         const float bias1 = (a.r1 && pos >= 0) ? a.r1[head] : 0.f, bias2 = (a.r1 && pos >= 0) ? a.r2[head] : 0.f;
         clear_state<DVB, MAPS>(st);
         Places ahead;
         Pieces first, second;
-        pages_now = pages_of(0);
-        pages_next = pages_of(kWave);
+        pages_now = pages_of(0, lane_now);
+        pages_next = pages_of(kWave, lane_now);
         look_up(0, ahead);
         fetch(ahead, first);
         look_up(1, ahead);
@@ -709,12 +716,15 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
         } else {
             for (int stage = 0; stage < stages; ++stage) work(stage, first, first);
         }
+        int lane_then = lane;
+        if constexpr (FULL) asm volatile("" : "+v"(lane_then));
+        const int col_then = lane_then & 15;
         if (splits > 1) {
 #pragma unroll
             for (int m = 0; m < MAPS; ++m) {
                 __syncthreads();
                 if (split == 1 && wave_on) {
-                    float* mine = meet[place][lane];
+                    float* mine = meet[place][lane_then];
                     mine[0] = st.m[m];
                     mine[1] = st.l[m];
 #pragma unroll
@@ -724,7 +734,7 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
                 }
                 __syncthreads();
                 if (split == 0 && wave_on) {
-                    const float* its = meet[place][lane];
+                    const float* its = meet[place][lane_then];
                     const float m_new = fmaxf(st.m[m], its[0]);
                     const float base = m_new == -INFINITY ? 0.f : m_new;
                     const float mine_by = exp2f(st.m[m] - base), its_by = exp2f(its[0] - base);
@@ -737,7 +747,12 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_staged_kerne
                 }
             }
         }
-        if (split == 0 && wave_on) finish_column<DVB, MAPS>(st, a, tok, head, pos, lane);
+        if (split == 0 && wave_on) {
+            if constexpr (FULL)
+                finish_column<DVB, MAPS>(st, a, t0 + (col_then < n ? col_then : 0), head, col_then < n ? p0 + col_then : -1, lane_then);
+            else
+                finish_column<DVB, MAPS>(st, a, tok, head, pos, lane_then);
+        }
     }
 }
 
@@ -902,4 +917,39 @@ LC_API int lc_masked_attention_bf16(const void* q, const void* k_cache, const vo
 #undef LC_MB_STAGED
     LC_LAUNCH_CHECK("masked_attention_bf16");
     return 0;
+}
+
+template <int DSTEPS, int DVB, int MAPS>
+static int staged_scratch() {
+    constexpr bool room = MB_ROOM<DSTEPS, DVB, MAPS>, always = room && MB_VALUES<DSTEPS, DVB, MAPS>, often = room && MAPS * DSTEPS < 8;
+    const void* kernels[] = {
+        (const void*)masked_attention_bf16_staged_kernel<FORM_PLAIN, DSTEPS, DVB, MAPS, always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_BIAS, DSTEPS, DVB, MAPS, always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_CAP, DSTEPS, DVB, MAPS, always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_ANY, DSTEPS, DVB, MAPS, always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_PLAIN, DSTEPS, DVB, MAPS, often || always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_BIAS, DSTEPS, DVB, MAPS, often || always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_CAP, DSTEPS, DVB, MAPS, often || always>,
+        (const void*)masked_attention_bf16_staged_kernel<FORM_ANY, DSTEPS, DVB, MAPS, often || always>,
+    };
+    int most = 0;
+    for (const void* kernel : kernels) {
+        hipFuncAttributes attr;
+        if (hipFuncGetAttributes(&attr, kernel) != hipSuccess) {
+            (void)hipGetLastError();
+            return -1;
+        }
+        if ((int)attr.localSizeBytes > most) most = (int)attr.localSizeBytes;
+    }
+    return most;
+}
+
+// Bytes of scratch memory a lane of the staged kernels for d (one map's entries), dv and maps that the library was built with; -1: the runtime could not
+// be asked.
+LC_API int lc_masked_attention_bf16_scratch(int maps, int d, int dv) {
+    const int dsteps = (d + 31) / 32, dvb = dv / 16;
+#define LC_MB_SCRATCH(DS, VB) (maps == 1 ? staged_scratch<DS, VB, 1>() : staged_scratch<DS, VB, 2>())
+    if (dsteps <= 2) return dvb <= 2 ? LC_MB_SCRATCH(2, 2) : dvb <= 4 ? LC_MB_SCRATCH(2, 4) : LC_MB_SCRATCH(2, 8);
+    return dvb <= 2 ? LC_MB_SCRATCH(4, 2) : dvb <= 4 ? LC_MB_SCRATCH(4, 4) : LC_MB_SCRATCH(4, 8);
+#undef LC_MB_SCRATCH
 }

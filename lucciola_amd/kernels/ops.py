@@ -131,6 +131,7 @@ _SIGNATURES = {
     "lc_masked_attention_bf16_supported": "iiii",
     "lc_masked_attention_bf16": "ppp" + "pi" + "pii" + "iiiii" + "f" + "iiif" + "ppp" + "f" + "i" + "ff" + "pii" + "ppiiip",
     "lc_masked_attention_bf16_staged": "i",
+    "lc_masked_attention_bf16_scratch": "iii",
     "lc_masked_attention_bf16_workspace": "iiiiii",
     "lc_state_space_prepare": "piiiiii" + "ppi" + "ppp" + "ppp" + "pp" + "p",
     "lc_state_space_readout": "pppiipiipifipip",

@@ -40,3 +40,12 @@ def test_against_the_general_kernel(heads, kv, maps, d, dv, window, keep, page):
         near(fast, call(), float(vc.abs().max()))
     finally:
         ops.masked_attention_matrix_cores(before)
+
+
+@pytest.mark.parametrize("maps", [1, 2])
+@pytest.mark.parametrize("d", [64, 128])
+@pytest.mark.parametrize("dv", [32, 64, 128])
+def test_the_stages_kernels_have_no_scratch(maps, d, dv):
+    """Every build of the kernel, whatever becomes of the scores, keeps its operands and sums in registers (two maps of 64 with values of 128
+    need 254 of the 256)."""
+    assert ops.library().lc_masked_attention_bf16_scratch(maps, d, dv) == 0
