@@ -47,20 +47,6 @@ __device__ __forceinline__ float gelu_erf(float z) {
     }
 }
 
-// tanh, for results of type T.  Those that are rounded to bfloat16 take (1 - t) / (1 + t) with t = e^(-2 |x|), and the series up to x^9 below 0.4,
-// where the difference would cancel: 1e-6 of the result at most, half a unit of bfloat16 is 2e-3.
-template <typename T>
-__device__ __forceinline__ float tanh_for(float x) {
-    if constexpr (sizeof(T) == 2) {
-        const float t = __builtin_amdgcn_exp2f(-2.88539008f * fabsf(x)), y = x * x;
-        const float far = (1.f - t) * __builtin_amdgcn_rcpf(1.f + t);
-        const float near = x * fmaf(y, fmaf(y, fmaf(y, fmaf(y, 62.f / 2835.f, -17.f / 315.f), 2.f / 15.f), -1.f / 3.f), 1.f);
-        return fabsf(x) < 0.4f ? near : copysignf(far, x);
-    } else {
-        return tanhf(x);
-    }
-}
-
 // T: the type of the result
 template <typename T>
 __device__ __forceinline__ float activate(float z, int kind) {

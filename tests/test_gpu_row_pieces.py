@@ -47,3 +47,14 @@ def test_dynamic_tanh(T, n, offset, dtype):
     assert bool(((h.double() - want_h).abs() <= 2.0 ** -24 * want_h.abs()).all())
     want = torch.tanh(0.5 * want_h) * w.double()
     assert bool(((got.double() - want).abs() <= want.abs() * (2.0 ** -8 + 2e-6 if dtype == torch.bfloat16 else 1e-6) + 1e-30).all())
+
+
+@pytest.mark.parametrize("T", [3, 300])
+def test_dynamic_tanh_of_bfloat16_rounds_what_float32_gives(T):
+    """The tanh of bfloat16 results is the one of float32 results: nothing of it is less exact."""
+    gen = torch.Generator(device="cuda").manual_seed(T)
+    n = 2048
+    h = torch.randn(T, n, device="cuda", generator=gen) * 2
+    w, b = torch.ones(n, device="cuda"), torch.zeros(n, device="cuda")
+    exact = ops.dynamic_tanh(h.clone(), None, w, b, 0.5, torch.float32)
+    assert torch.equal(ops.dynamic_tanh(h.clone(), None, w, b, 0.5, torch.bfloat16), exact.to(torch.bfloat16))
