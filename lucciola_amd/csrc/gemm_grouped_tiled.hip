@@ -263,10 +263,7 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGat
             switch (a.epilogue) {
                 case ACT_NONE: unrolled([](float z, float) { return z; }); break;
                 case ACT_RELU_SQUARED: unrolled([](float z, float) { return activate<TO>(z, ACT_RELU_SQUARED); }); break;
-                case ACT_GELU_ERF:
-                    if constexpr (sizeof(TO) == 2) unrolled([](float z, float) { return gelu_erf<TO>(z); });
-                    else rolled([](float z, float) { return gelu_erf<TO>(z); });
-                    break;
+                case ACT_GELU_ERF: rolled([](float z, float) { return gelu_erf<TO>(z); }); break;
                 default:
                     if constexpr (sizeof(TO) == 2) unrolled([](float z, float) { return gelu_tanh<TO>(z); });
                     else rolled([](float z, float) { return gelu_tanh<TO>(z); });
