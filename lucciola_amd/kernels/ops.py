@@ -793,6 +793,7 @@ class AttentionBatch:
     max_ctx: int = 0                               # longest cached length in the batch
     all_decode: bool = False
     even_lengths: bool = False                     # the longest decoding request is within a tenth of the mean length
+    decode_items_launched: int = 0                 # how many of the list's items the kernel is started for (0: all)
     decode_longest: int = 0                        # tokens of the longest decoding request, and of all of them
     decode_total: int = 0
 
@@ -867,39 +868,64 @@ def plan_attention(layout, nkv: int = 8):
     longest, total = (int(lengths.max()), int(lengths.sum())) if lengths.size else (0, 0)
     # what a captured step must share with the batches it is replayed for: the classes of lengths
     # between which the decode kernel's launch changes (even; up to a quarter above the mean;
-    # up to three times the mean; beyond: the thresholds of lc_attn_decode_by_items)
+    # up to three times the mean; beyond: the thresholds of lc_attn_decode_by_items; how many items, if not all)
     spread = longest * int(lengths.size)
+    launched = decode_items_launched(items, nkv)
     hint = (even, 0 if spread * 4 <= total * 5 else 1 if spread < total * 3 else 2)
+    if hint[1] and launched < items.shape[0]:
+        hint += (launched,)
     return ({"decode_rows": decode, "decode_items": items, "prefill_tiles": tiles},
             {"num_decode": int(singles.size), "all_decode": int(singles.size) == R, "even_lengths": even,
-             "decode_longest": longest, "decode_total": total, "graph_hint": hint})
+             "decode_items_launched": launched, "decode_longest": longest, "decode_total": total, "graph_hint": hint})
 
 
 ITEM_PAGES_MIN = 8       # kernel pages of the smallest work item that a request is cut into
-DECODE_WORKGROUPS = 256  # of few decoding requests: one a CU
 ITEM_SHARES_MOST = 32    # items of one request at most (the join kernel takes up to 64)
 
 
-def decode_item_count(num_decode: int, nkv: int = 8) -> int:
-    """Work items that the planner makes for a step with ``num_decode`` single tokens: a number
-    that follows from the count and the kv heads alone, so that steps of one make-up have lists of one size (a
-    captured step is replayed with the next step's list in the same buffer).  For few tokens as many as give every CU
-    one workgroup, an item and kv head each: a second one shares the CU's way from memory and makes the items smaller, not the step
-    faster (8 kv heads, a layer of a decode step with 64, 48, 32 and 24 items, us: 12 requests of up to 900 tokens 55.0, 55.5, 52.5, 53.4;
-    8 of up to 8,000 70.8, 69.7, 66.3, 66.7; 16 of up to 8,000 85.7, 91.0, 87.0, 93.5)."""
-    return max(num_decode + num_decode // 2, min(max(16, min(64, DECODE_WORKGROUPS // nkv)), 8 * num_decode)) if num_decode else 0
+def decode_item_count(num_decode: int) -> int:
+    """Work items that the planner has room for in a step with ``num_decode`` single tokens: a number
+    that follows from the count alone, so that steps of one make-up have lists of one size (a
+    captured step is replayed with the next step's list in the same buffer)."""
+    return max(num_decode + num_decode // 2, min(64, 8 * num_decode)) if num_decode else 0
+
+
+@functools.lru_cache(maxsize=None)
+def _compute_units() -> int:
+    return torch.cuda.get_device_properties(torch.cuda.current_device()).multi_processor_count if torch.cuda.is_available() else 256
+
+
+def decode_items_launched(items: np.ndarray, nkv: int) -> int:
+    """How many of the list's items the kernel is started for: those that have shares, up to a whole number of workgroups a CU (an item
+    and kv head each).  The workgroups go kv head by kv head, so empty ones push others into a round more: 13 items and 16 kv
+    heads 9.8 us where the kernel is started for 16 and 13.1 for 24."""
+    rounds = -(-int(np.count_nonzero(items[:, 6])) * nkv // _compute_units())
+    return min(items.shape[0], rounds * _compute_units() // nkv)
+
+
+def _pages_enough(rounds: int) -> int:
+    """Pages of the largest item that need not be cut further where every CU has ``rounds`` workgroups."""
+    return max(192 // (rounds + 1), 40)
 
 
 def _decode_items(decode: np.ndarray, lengths: np.ndarray, nkv: int = 8) -> np.ndarray:
-    """The decode rows' pages (of ATTENTION_PAGE_GRANULE tokens) cut into ``decode_item_count``
-    work items so that the largest item is as small as may be: every row one item, the spare ones
+    """The decode rows' pages (of ATTENTION_PAGE_GRANULE tokens) cut into work items so that the largest item is as small as
+    may be: every row one item, the spare ones
     to whichever row has the largest items then (at most ITEM_SHARES_MOST a row, none smaller than
-    ITEM_PAGES_MIN pages).  Eight numbers an item: token row, request, position, row, first page,
+    ITEM_PAGES_MIN pages), until there are ``decode_item_count`` items, or every CU has the same number of workgroups, an item and
+    kv head each, and no item more than ``_pages_enough``: another workgroup shares its CU's way from memory and
+    makes the items smaller, not the step faster, until the largest item is what the step waits for.
+    A layer's decode attention, heads of 128, caches from memory, us, with ``decode_item_count`` items and so (how many): 8 kv heads, 12
+    requests of up to 2,000 tokens 18.7 and 16.8 (32), 12 of up to 8,000 40.2 and 40.2 (64; 32 take up to 49), 16 of up to 8,000 52.2 (64; 32 54.2),
+    24 of which one has 8,192 22.4 and 21.9 (32); 16 kv heads, 8 of up to 2,000 24.6 and 19.0 (16), 16 of which one has 8,192 34.7 and 31.5 (32);
+    32, 8 of which one has 8,192 51 and 43 (16); with 4, 48 of which one has 8,192 21.3 and 18.4 (64).  Over 410 makings of 2 to 48 rows
+    and 2 to 40 kv heads 0.95 in the mean, none slower beyond the runs' spread.
+    Eight numbers an item: token row, request, position, row, first page,
     end page, the row's number of items, 0; a row's items are neighbours; items that are left over
     have no shares and do nothing.  Writes each row's first item and number of items into
     ``decode[:, 3]``.  ``lengths`` in the order of ``decode``."""
     nd = int(decode.shape[0])
-    total = decode_item_count(nd, nkv)
+    total = decode_item_count(nd)
     items = np.zeros((total, 8), dtype=np.int32)
     if nd == 0:
         return items
@@ -908,15 +934,18 @@ def _decode_items(decode: np.ndarray, lengths: np.ndarray, nkv: int = 8) -> np.n
     shares = np.ones(nd, dtype=np.int64)
     # lengths so even that no launcher would take the list: every row its one item, no search
     uneven = int(lengths.max()) * nd * 4 > int(lengths.sum()) * 5
-    spare = total - nd
-    if uneven and spare > 0:
+    if uneven and total > nd:
         most = np.minimum(ITEM_SHARES_MOST, np.maximum(1, pages // ITEM_PAGES_MIN))
         heap = [(-int(pages[r]), r) for r in np.nonzero(most > 1)[0].tolist()]
         heapq.heapify(heap)
-        while spare > 0 and heap:
+        cus, used = _compute_units(), nd
+        while used < total and heap:
+            rounds = -(-used * nkv // cus)
+            if (used + 1) * nkv > rounds * cus and -heap[0][0] <= _pages_enough(rounds):
+                break
             _, r = heapq.heappop(heap)
             shares[r] += 1
-            spare -= 1
+            used += 1
             if shares[r] < most[r]:
                 heapq.heappush(heap, (-int((pages[r] + shares[r] - 1) // shares[r]), r))
     first = np.cumsum(shares) - shares
@@ -958,6 +987,7 @@ def attention_batch(batch, pages, plan=None, key=ATTENTION_PLAN) -> AttentionBat
         if plan is not None:
             done = replace(done, decode_rows=plan.arrays["decode_rows"],
                            decode_items=plan.arrays.get("decode_items"),
+                           decode_items_launched=plan.info.get("decode_items_launched", 0),
                            decode_longest=plan.info.get("decode_longest", 0),
                            decode_total=plan.info.get("decode_total", 0),
                            prefill_tiles=plan.arrays["prefill_tiles"],
@@ -1059,13 +1089,14 @@ def attention(qkv, batch: AttentionBatch, k_cache: torch.Tensor,
                 items = batch.decode_items
             splits = 1 if items is not None else lib.lc_attn_decode_splits(nd, nkv, batch.max_ctx)
             part_o = part_ml = None
-            parts = items.shape[0] if items is not None else (nd * splits if splits > 1 else 0)
+            num_items = (batch.decode_items_launched or items.shape[0]) if items is not None else 0
+            parts = num_items if items is not None else (nd * splits if splits > 1 else 0)
             if parts:
                 part_o = torch.empty((parts * nh * d,), dtype=torch.float32, device=qkv.device)
                 part_ml = torch.empty((parts * nh * 2,), dtype=torch.float32, device=qkv.device)
             _call("lc_attn_decode_bf16", _ptr(qkv if shares is None else None), qkv.shape[1], _ptr(k_cache), _ptr(v_cache),
                   _ptr(out), _ptr(part_o), _ptr(part_ml), _ptr(batch.decode_rows),
-                  _ptr(items), items.shape[0] if items is not None else 0,
+                  _ptr(items), num_items,
                   _ptr(batch.block_table), mb, nd, nh,
                   nkv, d, page_size, scale, window, splits, 1 if batch.even_lengths else 0,
                   1 if in_kernel else 0,

@@ -1,6 +1,7 @@
 """The attention kernels' work lists of a step (``ops.plan_attention``): made on the host from the
 batch's layout alone, so checked here without a GPU."""
 import numpy as np
+import pytest
 
 from lucciola_amd.engine.batch import HostLayout
 from lucciola_amd.kernels import ops
@@ -100,3 +101,44 @@ def test_decode_items_cover_every_row_once():
     # few requests of uneven lengths: the spare items go where the pages are
     rows, items = check_items([1] * 4, [3999, 299, 199, 99], single=True)
     assert (rows[:, 3] >> 20).tolist() == [28, 2, 1, 1]       # 32 items for four rows
+
+
+@pytest.mark.parametrize("nkv", [1, 2, 4, 8, 16, 32, 40, 300])
+def test_items_for_any_number_of_kv_heads(nkv):
+    """The list covers every row once however many kv heads share the CUs, the items that the kernel is started for hold all shares, and
+    they are whole rounds of workgroups unless the list ends first; the largest is small enough where the list does not go on."""
+    import random
+    rng = random.Random(nkv)
+    cus = ops._compute_units()
+    for trial in range(60):
+        n = rng.choice([1, 2, 3, 7, 8, 12, 16, 17, 24, 33, 48, 70])
+        cached = [rng.choice([0, 5, 127, 128, 500, 2000, 9000]) if trial % 2 else rng.randint(10, 700) for _ in range(n)]
+        if trial % 5 == 0:
+            cached[0] = 8191
+        arrays, info = ops.plan_attention(layout([1] * n, cached, single=True), nkv=nkv)
+        rows, items, launched = arrays["decode_rows"], arrays["decode_items"], info["decode_items_launched"]
+        assert items.shape == (ops.decode_item_count(n), 8)
+        used = 0
+        for r, (t, req, p, packed) in enumerate(rows.tolist()):
+            first, count = packed & 0xFFFFF, packed >> 20
+            assert first == used and 1 <= count <= ops.ITEM_SHARES_MOST
+            mine = items[first:first + count].tolist()
+            assert all(i[:4] == [t, req, p, r] and i[6:] == [count, 0] for i in mine)
+            assert [i[4] for i in mine] == [0] + [i[5] for i in mine[:-1]] and mine[-1][5] == p // 16 + 1
+            used += count
+        assert not items[used:].any() and used <= launched <= len(items)
+        rounds = -(-used * nkv // cus)
+        assert launched == min(len(items), rounds * cus // nkv)
+        sizes = items[:used, 5] - items[:used, 4]
+        even = info["graph_hint"][1] == 0
+        cut = [s for s, i in zip(sizes, items[:used]) if i[6] < min(ops.ITEM_SHARES_MOST, (i[2] // 16 + 1) // ops.ITEM_PAGES_MIN)]
+        assert even or used == len(items) or not cut or max(cut) <= ops._pages_enough(rounds)
+        # a captured step starts the same number: all, or what the class says (lengths so even that every row has one item make one class)
+        assert info["graph_hint"][2:] == (() if even or launched == len(items) else (launched,)) and (not even or used == n)
+
+
+def test_one_workgroup_a_cu_where_no_item_is_long():
+    """8 kv heads: 12 requests of up to 900 tokens in 32 items; of up to 8,000, whose largest of 32 items would have some 100 pages, in 64."""
+    assert ops._compute_units() != 256 or [
+        ops.plan_attention(layout([1] * 12, [longest * (i + 1) // 12 for i in range(12)], single=True))[1]["decode_items_launched"]
+        for longest in (900, 8000)] == [32, 64]
