@@ -535,6 +535,22 @@ __global__ __launch_bounds__(64 * WM * WN, 2) void gemm_planes_kernel(const unsi
 
 bool gemm_split_takes(int K) { return K % 32 == 0; }
 
+// gemm_planes_kernel reads LDS by inline assembly into registers that the compiler takes to hold values before its wait for them: were
+// one spilled to scratch memory in between, the spill would store what the register held before.  So the compiled kernel is asked, once:
+// if it uses scratch memory (or cannot be asked), products go by tiles.
+static int planes_state() {          // 1: in registers, 0: spilled, -1: could not ask
+    static const int state = [] {
+        hipFuncAttributes attr;
+        if (hipFuncGetAttributes(&attr, (const void*)gemm_planes_kernel<GP_M, GP_N, 2, 4, 4>) != hipSuccess) {
+            (void)hipGetLastError();
+            return -1;
+        }
+        return attr.localSizeBytes != 0 ? 0 : 1;
+    }();
+    return state;
+}
+LC_API int lc_gemm_planes_ok() { return planes_state(); }
+
 // Whether a product goes by planes.  A round of 256 tiles of 128 x 256 takes 1.53 times as long as one of 512 tiles of 64 x 128, which is
 // half as many places (K of 4,096: 182 and 119 us where several rounds follow each other); fewer whole rounds than that pay for the
 // cut.  us, tiles of 64 x 128 and planes: 300 rows, 24,576 x 4,096 (2 rounds each) 244 and 314, 566 rows (4 and 2) 424 and 357, 100 rows (1 and 1)
@@ -545,7 +561,7 @@ static bool planes_pay(int M, int N, int K) {
         return ((m + bm - 1) / bm * ((n + bn - 1) / bn) + places - 1) / places;
     };
     return 1.53 * rounds(M, N, GP_M, GP_N, device_cus()) < rounds(M, N, 64, 128, 2 * device_cus()) &&
-           (long long)((M + GP_M - 1) / GP_M) * ((N + GP_N - 1) / GP_N) < 1ll << 30;
+           (long long)((M + GP_M - 1) / GP_M) * ((N + GP_N - 1) / GP_N) < 1ll << 30 && planes_state() == 1;
 }
 
 long long gemm_split_words(int M, int N, int K) { return planes_pay(M, N, K) ? (3ll * M * K + 1) / 2 : 0; }

@@ -31,6 +31,7 @@ _SIGNATURES = {
     "lc_rmsnorm_act": "pqpfpiiip",
     "lc_gemm_generic": "pipipiiiipp",
     "lc_gemm_generic_parts": "iii",
+    "lc_gemm_planes_ok": "",
     "lc_gemm_generic_in_parts": "pppiiip",
     "lc_gemm_bf16": "pppiiiiipp",
     "lc_gemm_bf16_gated": "pppiiiifffpp",

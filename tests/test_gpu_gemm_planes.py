@@ -47,3 +47,8 @@ def test_eight_waves(M, N, K):
         assert torch.equal(got[first:first + 11], ops.gemm(x[first:first + 11].clone(), w, torch.float32))
     want, sizes = x.double() @ w.double().T, x.double().abs() @ w.double().abs().T
     assert bool(((got.double() - want).abs() <= sizes * K * 2.0 ** -24).all())
+
+
+def test_planes_stay_in_registers():
+    """The kernel's operands land in registers behind the compiler's back: with scratch memory the products go by tiles."""
+    assert ops.library().lc_gemm_planes_ok() == 1
