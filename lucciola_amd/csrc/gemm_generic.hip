@@ -325,10 +325,17 @@ static int launch_generic(const void* x, const void* w, void* out, int M, int N,
 
 using namespace lc;
 
-// float32 words of workspace that lc_gemm_generic needs for these sizes (0: none)
+// float32 words of workspace that lc_gemm_generic needs for these sizes (0: none), of whatever types the operands are
 LC_API long long lc_gemm_generic_workspace(int M, int N, int K) {
     if (M <= 0 || N <= 0 || K <= 0) return 0;
     return chunks_per_workgroup(M, N, K) > 0 ? (long long)((K + GB_CHUNK - 1) / GB_CHUNK) * M * N : gemm_split_words(M, N, K);
+}
+
+// ... and of these types: x's parts are laid out for float32 x, bfloat16 w and a float32 result alone
+LC_API long long lc_gemm_generic_workspace_of(int M, int x_dt, int N, int w_dt, int K, int out_dt) {
+    if (M <= 0 || N <= 0 || K <= 0) return 0;
+    const bool splits = x_dt == DT_F32 && w_dt == DT_BF16 && out_dt == DT_F32;
+    return splits || chunks_per_workgroup(M, N, K) > 0 ? lc_gemm_generic_workspace(M, N, K) : 0;
 }
 
 // The chunks' float32 sums of a product of float32 x and bfloat16 w that is shared out, for a norm kernel that sums them itself: their

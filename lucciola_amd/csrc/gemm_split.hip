@@ -564,7 +564,13 @@ static bool planes_pay(int M, int N, int K) {
            (long long)((M + GP_M - 1) / GP_M) * ((N + GP_N - 1) / GP_N) < 1ll << 30 && planes_state() == 1;
 }
 
-long long gemm_split_words(int M, int N, int K) { return planes_pay(M, N, K) ? (3ll * M * K + 1) / 2 : 0; }
+// Rows whose parts are in the workspace at once: no more than 64 M words (256 MiB) of them, in whole tiles.
+static int rows_at_once(int M, int K) {
+    const long long most = (128ll << 20) / 3 / K / GP_M * GP_M;
+    return M <= most ? M : most < GP_M ? GP_M : (int)most;
+}
+
+long long gemm_split_words(int M, int N, int K) { return planes_pay(M, N, K) ? (3ll * rows_at_once(M, K) * K + 1) / 2 : 0; }
 
 template <bool WHOLE, bool SHARED>
 static void launch_split(const float* x, const bf16* w, float* out, int M, int N, int K, float* part, int per, int shares, hipStream_t stream) {
@@ -582,12 +588,17 @@ void launch_gemm_split(const float* x, const bf16* w, float* out, int M, int N, 
                        hipStream_t stream) {
     if (!part && workspace && (uintptr_t)w % 16 == 0 && (uintptr_t)workspace % 16 == 0 && planes_pay(M, N, K)) {
         unsigned short* planes = reinterpret_cast<unsigned short*>(workspace);
-        const size_t pieces = (size_t)M * K / 8;
-        const int blocks = (int)((pieces + 255) / 256 < 2048 ? (pieces + 255) / 256 : 2048);
-        if ((uintptr_t)x % 16 == 0) cut_planes_kernel<true><<<blocks, 256, 0, stream>>>(x, planes, pieces);
-        else cut_planes_kernel<false><<<blocks, 256, 0, stream>>>(x, planes, pieces);
-        const int tiles_m = (M + GP_M - 1) / GP_M, tiles_n = (N + GP_N - 1) / GP_N;
-        gemm_planes_kernel<GP_M, GP_N, 2, 4, 4><<<tiles_m * tiles_n, 512, 0, stream>>>(planes, w, x, out, M, N, K, tiles_m);
+        const int at_once = rows_at_once(M, K);
+        for (int first = 0; first < M; first += at_once) {          // one after the other in the workspace
+            const int rows = M - first < at_once ? M - first : at_once;
+            const float* from = x + (size_t)first * K;
+            const size_t pieces = (size_t)rows * K / 8;
+            const int blocks = (int)((pieces + 255) / 256 < 2048 ? (pieces + 255) / 256 : 2048);
+            if ((uintptr_t)x % 16 == 0) cut_planes_kernel<true><<<blocks, 256, 0, stream>>>(from, planes, pieces);
+            else cut_planes_kernel<false><<<blocks, 256, 0, stream>>>(from, planes, pieces);
+            const int tiles_m = (rows + GP_M - 1) / GP_M, tiles_n = (N + GP_N - 1) / GP_N;
+            gemm_planes_kernel<GP_M, GP_N, 2, 4, 4><<<tiles_m * tiles_n, 512, 0, stream>>>(planes, w, from, out + (size_t)first * N, rows, N, K, tiles_m);
+        }
         return;
     }
     const bool whole = ((uintptr_t)x | (uintptr_t)w) % 16 == 0;

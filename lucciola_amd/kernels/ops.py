@@ -199,6 +199,8 @@ def library():
         lib.lc_gemm_bf16_workspace.argtypes = [ctypes.c_int] * 3
         lib.lc_gemm_generic_workspace.restype = ctypes.c_longlong
         lib.lc_gemm_generic_workspace.argtypes = [ctypes.c_int] * 3
+        lib.lc_gemm_generic_workspace_of.restype = ctypes.c_longlong
+        lib.lc_gemm_generic_workspace_of.argtypes = [ctypes.c_int] * 6
         lib.lc_attention_f32_workspace.restype = ctypes.c_longlong
         lib.lc_attention_f32_workspace.argtypes = [ctypes.c_void_p, ctypes.c_int, ctypes.c_void_p, ctypes.c_void_p] + [ctypes.c_int] * 8
         lib.lc_attention_generic_workspace.restype = ctypes.c_longlong
@@ -635,7 +637,7 @@ def gemm(x, w: torch.Tensor, out_dtype: Optional[torch.dtype] = None, defer: boo
             _say_once(("gemm", N, K),
                       f"a bfloat16 product with w [{N}, {K}] has no matrix-core kernel (K must be a multiple "
                       f"of {library().lc_gemm_bf16_kblock()}): the general kernel runs, correct and many times slower")
-        words = library().lc_gemm_generic_workspace(M, N, K)
+        words = library().lc_gemm_generic_workspace_of(M, _dt(x), N, _dt(w), K, _dt(out))
         workspace = torch.empty((words,), dtype=torch.float32, device=x.device) if words else None
         _call("lc_gemm_generic", _ptr(x), _c_int(_dt(x)), _ptr(w), _c_int(_dt(w)), _ptr(out),
               _c_int(_dt(out)), _c_int(M), _c_int(N), _c_int(K), _ptr(workspace), _stream())

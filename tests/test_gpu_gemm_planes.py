@@ -52,3 +52,19 @@ def test_eight_waves(M, N, K):
 def test_planes_stay_in_registers():
     """The kernel's operands land in registers behind the compiler's back: with scratch memory the products go by tiles."""
     assert ops.library().lc_gemm_planes_ok() == 1
+
+
+def test_room_for_planes():
+    """Only the types that are multiplied by planes ask for room, and never for more than 256 MiB: more rows go one portion after the other, with
+    the same bits."""
+    lib, f32, bf16 = ops.library(), ops.DT_F32, ops.DT_BF16
+    M, N, K = 512, 65000, 1024
+    assert lib.lc_gemm_generic_workspace_of(M, f32, N, bf16, K, f32) == (3 * M * K + 1) // 2
+    for types in ((f32, f32, f32), (bf16, f32, f32), (bf16, f32, bf16), (bf16, bf16, f32), (bf16, bf16, bf16)):
+        assert lib.lc_gemm_generic_workspace_of(M, types[0], N, types[1], K, types[2]) == 0
+    M, N, K = 1500, 5000, 32768
+    assert (3 * M * K + 1) // 2 > 1 << 26 >= lib.lc_gemm_generic_workspace_of(M, f32, N, bf16, K, f32) > 0
+    x, w = _operands(M, N, K)
+    got = ops.gemm(x, w, torch.float32)
+    for first in (0, 1270, 1355, 1365, M - 9):
+        assert torch.equal(got[first:first + 9], ops.gemm(x[first:first + 9].clone(), w, torch.float32))
