@@ -827,7 +827,9 @@ static int shares_for(int t, int M, int N, int K, bool partials_wanted = false) 
 // tiles of 128 x 128 and 128 x 64 in one round (0.70 to 1.09), and is within 8 % of the best of all in 342.  A last round of a one-a-CU shape
 // that is cut along K takes its share of that, plus the time to write and read its float32
 // partial tiles (about 4 TB/s) and to start two more kernels.  A small tile cut along K as a
-// whole pays for its partial sums likewise, unless the caller takes them as they are
+// whole pays for its partial sums likewise, and 3 us for the kernel that adds them, which reads what lies in the caches: of 1,647 products
+// of 65 to 4,001 rows the pick is another one than with 10 us in 136, which take 0.91 of that one's time in the mean (0.66 to 1.16; us,
+// 10 and 3: 128 x 3840 x 2560 24.4 and 16.1, 128 x 5120 x 5120 42.4 and 29.2, 300 x 2560 x 2560 17.1 and 19.8).  Not where the caller takes the sums as they are
 // (partials_wanted).
 static int pick_tile(int M, int N, int K, bool partials_wanted = false) {
     if (g_force_tile != TILE_AUTO) return g_force_tile;

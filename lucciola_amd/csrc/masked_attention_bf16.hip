@@ -22,7 +22,7 @@
 // The workgroups go tile by tile, a tile's kv heads beside each other, and the list has the longest tiles first: with all tiles of
 // one kv head before the next head's, the last head's longest tile began when half of the card had run dry (2,048 tokens, four kv
 // heads, a workgroup a CU: 202 -> 136 us for two maps of 64, 207 -> 143 for one of 128 with the bias; 1,523 tokens 102 -> 78; with two
-// blocks of keys a step and the scores' forms known to the build 118, 114 and 67; with two stages in LDS, below, 106, 82 and 46).
+// blocks of keys a step and the scores' forms known to the build 118, 114 and 67; with two stages in LDS, below, 99, 78 and 50).
 #include "common.h"
 
 namespace lc {
@@ -493,8 +493,10 @@ __global__ __launch_bounds__(MB_THREADS) void masked_attention_bf16_kernel(Maske
 //
 // One workgroup is what a CU has room for, so nothing hides what its eight waves wait for together: with one stage in LDS, its pages
 // looked up as scalars in the chain of the stage's loads, and addresses and places worked out by every thread for every stage, a stage
-// took 3.5 us, a sixth of it products.  us, 16 heads over 4, then and now: 2,048 tokens, 128, 128 102 and 72, with the bias 119 and 82, with
-// the cap 124 and 83, two maps of 64 126 and 106, 64, 64 76 and 52; 16 over 16, 64, 64 147 and 108; 576 tokens after 2,048, 128, 128 112 and 73.
+// took 3.5 us, a sixth of it products.  us, 16 heads over 4, then and now: 2,048 tokens, 128, 128 105 and 75, with the bias 119 and 78, with
+// the cap 124 and 84, with both 139 and 95, two maps of 64 120 and 99, with the bias 133 and 105, 64, 64 78 and 53; 16 over 16, 64, 64 147 and 110;
+// 576 tokens after 2,048, 128, 128 117 and 78.  (Scores of a standard deviation of one.  In a whole step between products, whose scores spread
+// more and whose power the matrix cores have used up, two maps 110 and one with the bias 97.)
 // What is left is the operands' way from LDS (16 KB a wave and stage for 16 columns), the scores and the barrier one after the other.
 constexpr int MB_STAGE_BLOCKS = 2;
 
