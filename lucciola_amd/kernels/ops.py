@@ -942,10 +942,14 @@ def _decode_items(decode: np.ndarray, lengths: np.ndarray, nkv: int = 8) -> np.n
         heap = [(-int(pages[r]), r) for r in np.nonzero(most > 1)[0].tolist()]
         heapq.heapify(heap)
         cus, used = _compute_units(), nd
+        rounds = -(-used * nkv // cus)
+        whole = rounds * cus // nkv             # items that so many rounds of workgroups hold
         while used < total and heap:
-            rounds = -(-used * nkv // cus)
-            if (used + 1) * nkv > rounds * cus and -heap[0][0] <= _pages_enough(rounds):
-                break
+            if used == whole:
+                if -heap[0][0] <= _pages_enough(rounds):
+                    break
+                rounds = -(-(used + 1) * nkv // cus)
+                whole = rounds * cus // nkv
             _, r = heapq.heappop(heap)
             shares[r] += 1
             used += 1
