@@ -570,7 +570,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
                                                          int M, int N, int K, int tiles_m, int strip, int tile_base,
                                                          int tile_count, int compact, int skew_step,
                                                          GateForm form) {
-    typedef TileLoop<BM, BN, TL_STAGES, WM, WN, BM == 256> Loop;
+    typedef TileLoop<BM, BN, TL_STAGES, WM, WN, BM == 256, (BM / WM) * (BN / WN) >= 64 * 128> Loop;
     constexpr int TM = Loop::TM, TN = Loop::TN, LPA = Loop::LPA, LPB = Loop::LPB;
     __shared__ __attribute__((aligned(1024))) char lds[Loop::LDS];
 
@@ -592,7 +592,6 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
-    const int lr = lane & 31;
 
     const int nk_all = K / TL_K;
     const int kb0 = SPLIT ? (int)((long long)blockIdx.y * nk_all / gridDim.y) : 0;
@@ -614,16 +613,63 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
     // (tile number times skew_step, modulo the number of k-blocks) and wraps around: 37.2 us.  (With several rows of tiles the workgroups that share a tile of w
     // should read it at the same time, and do.)
     const int skew = (!SPLIT && tiles_m == 1 && skew_step) ? (int)(((unsigned)id * (unsigned)skew_step) % (unsigned)nk) : 0;
-    floatx16 acc[TM][TN];
+    typename Loop::Sum acc[TM][TN];
     Loop::run(lds, xg, wg, nk, skew, wave, lane, acc);
 
-    // acc[i][j][v]: row m = (v/4)*8 + (lane/32)*4 + v%4, column n = lane%32 of the 32x32 tile.
-    const int mrow = m0 + wm + (lane >> 5) * 4;     // + i * 32 + (v / 4) * 8 + v % 4
-    const int ncol = n0 + wn + lr;                  // + j * 32
+    // acc[i][j][v]: row m = (v/4)*8 + (lane/32)*4 + v%4, column n = lane%32 of the 32x32 product, row (lane/16)*4 + v, column lane%16 of the
+    // 16x16 one
+    constexpr int MF = Loop::MF;
+    const int mrow = m0 + wm + (lane / MF) * 4;             // + i * MF + (v / 4) * 8 + v % 4
+    const int ncol = n0 + wn + (lane & (MF - 1));           // + j * MF
+    if constexpr (!SPLIT) {
+        // Whole pieces of 16 bytes: 32 rows at a time pass through the wave's part of the ring, so that a lane gets neighbouring columns and a
+        // row's are stored in whole lines (pairs of lanes stored 64 bytes of a row at a time; us, so and through LDS, both with products of
+        // 32 x 32: 2,048 x 4096 x 1024 20.8 and 20.0, x 6144 x 1024 with SwiGLU 29.3 and 28.0, 1,523 x 2048 x 2048 17.3 and 16.7, x 2048 x 2048
+        // 20.0 and 19.7).  float32 results of large products were stored 256 bytes at a time and are no faster for it; products of 16 x 16
+        // would halve that.
+        constexpr int WC = BN / WN, STRIDE = WC + 4, E = PIECE<TO>, PIECES = (EPI == 1 ? WC / 2 : WC) / E;
+        static_assert(WM * WN * 32 * STRIDE * 4 <= Loop::LDS, "a strip of every wave");
+        const int ldo = EPI == 1 ? N / 2 : N;
+        if ((sizeof(TO) == 2 || MF == 16) && ldo % E == 0 && (uintptr_t)out % 16 == 0) {
+            float* strip = reinterpret_cast<float*>(lds) + wave * 32 * STRIDE;
+            __syncthreads();                                // the ring is no longer read
+#pragma unroll
+            for (int i0 = 0; i0 < TM; i0 += 32 / MF) {
+#pragma unroll
+                for (int i = 0; i < 32 / MF; ++i)
+#pragma unroll
+                    for (int j = 0; j < TN; ++j)
+#pragma unroll
+                        for (int v = 0; v < Loop::SV; ++v)
+                            strip[(i * MF + (v >> 2) * 8 + (lane / MF) * 4 + (v & 3)) * STRIDE + j * MF + (lane & (MF - 1))] = acc[i0 + i][j][v];
+                __builtin_amdgcn_wave_barrier();
+#pragma unroll
+                for (int p0 = 0; p0 < 32 * PIECES; p0 += 64) {
+                    const int p = p0 + lane, row = p / PIECES, c = (p - row * PIECES) * E;
+                    const int m = m0 + wm + i0 * MF + row, n = (EPI == 1 ? (n0 + wn) / 2 : n0 + wn) + c;
+                    // (gated: columns come in blocks of 16, 8 gate, then their 8 up)
+                    const float* from = strip + row * STRIDE + (EPI == 1 ? c / 8 * 16 + c % 8 : c);
+                    float r[E];
+#pragma unroll
+                    for (int x = 0; x < E; x += 4) *reinterpret_cast<float4*>(r + x) = *reinterpret_cast<const float4*>(from + x);
+                    if (EPI == 1) {
+                        float u[E];
+#pragma unroll
+                        for (int x = 0; x < E; x += 4) *reinterpret_cast<float4*>(u + x) = *reinterpret_cast<const float4*>(from + 8 + x);
+#pragma unroll
+                        for (int x = 0; x < E; ++x) r[x] = gated_f(r[x], u[x], form);
+                    }
+                    if (m < M && n < ldo) store_piece<TO>(out + (size_t)m * ldo + n, r);
+                }
+                __builtin_amdgcn_wave_barrier();
+            }
+            return;
+        }
+    }
     if (EPI == 1 && !SPLIT) {
         // columns come in blocks of 16: 8 gate, then their 8 up (8 lanes further on).  Of two
         // consecutive rows the gate lane finishes the first and the up lane the second.
-        const bool up = lr & 8;
+        const bool up = lane & 8;
         const int ng = up ? ncol - 8 : ncol;
         TO* dst = out + (size_t)(mrow + (up ? 1 : 0)) * (N / 2) + (size_t)(ng >> 4) * 8 + (ng & 7);
 #pragma unroll
@@ -631,14 +677,14 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
 #pragma unroll
             for (int j = 0; j < TN; ++j)
 #pragma unroll
-                for (int v = 0; v < 16; v += 2) {
+                for (int v = 0; v < Loop::SV; v += 2) {
                     float first = acc[i][j][v], second = acc[i][j][v + 1];
                     asm volatile("" : "+v"(first), "+v"(second));   // two values, not one indexed by `up`
                     const float got = lane_swap<0x128>(up ? first : second);   // lane ^ 8
                     const float r = gated_f(up ? got : first, up ? second : got, form);
-                    const int dm = i * 32 + (v >> 2) * 8 + (v & 3);
-                    if (mrow + (up ? 1 : 0) + dm < M && ng + j * 32 < N)
-                        store_out<TO>(dst + (size_t)dm * (N / 2) + j * 16, r);
+                    const int dm = i * MF + (v >> 2) * 8 + (v & 3);
+                    if (mrow + (up ? 1 : 0) + dm < M && ng + j * MF < N)
+                        store_out<TO>(dst + (size_t)dm * (N / 2) + j * (MF / 2), r);
                 }
     } else {
         using TS = typename std::conditional<SPLIT, float, TO>::type;
@@ -658,13 +704,13 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; v += 2) {
+                    for (int v = 0; v < Loop::SV; v += 2) {
                         float first = acc[i][j][v], second = acc[i][j][v + 1];
                         asm volatile("" : "+v"(first), "+v"(second));   // two values, not one indexed by `odd`
                         const float got = lane_swap<0xB1>(odd ? first : second);   // lane ^ 1
-                        const int dm = i * 32 + (v >> 2) * 8 + (v & 3);
-                        if (mrow + (odd ? 1 : 0) + dm < M && (ncol & ~1) + j * 32 < N)
-                            store_pair<TS>(dst + (size_t)dm * ld + j * 32, odd ? got : first, odd ? second : got);
+                        const int dm = i * MF + (v >> 2) * 8 + (v & 3);
+                        if (mrow + (odd ? 1 : 0) + dm < M && (ncol & ~1) + j * MF < N)
+                            store_pair<TS>(dst + (size_t)dm * ld + j * MF, odd ? got : first, odd ? second : got);
                     }
         } else {
             TS* dst = base + (size_t)(mrow - r0) * ld + (ncol - c0);
@@ -673,10 +719,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
 #pragma unroll
                 for (int j = 0; j < TN; ++j)
 #pragma unroll
-                    for (int v = 0; v < 16; ++v) {
-                        const int dm = i * 32 + (v >> 2) * 8 + (v & 3);
-                        if (mrow + dm < M && ncol + j * 32 < N)
-                            store_out<TS>(dst + (size_t)dm * ld + j * 32, acc[i][j][v]);
+                    for (int v = 0; v < Loop::SV; ++v) {
+                        const int dm = i * MF + (v >> 2) * 8 + (v & 3);
+                        if (mrow + dm < M && ncol + j * MF < N)
+                            store_out<TS>(dst + (size_t)dm * ld + j * MF, acc[i][j][v]);
                     }
         }
     }

@@ -56,6 +56,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_grouped_tiled_kernel(Groupe
 #pragma unroll
     for (int i = 0; i < Loop::LPB; ++i)
         wg[i] = w + (size_t)min(n0 + Loop::row_of(i, wave, lane), N - 1) * K + Loop::chunk_of(i, wave, lane) * 8;
+    static_assert(Loop::MF == 32, "the epilogue's layout");
     floatx16 acc[TM][TN];
     Loop::run(lds, xg, wg, K / TL_K, 0, wave, lane, acc);
 
@@ -205,46 +206,38 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGat
         const int n = GATED ? min(n0 / 2 + (r >> 6) * 32 + (r & 31), N / 2 - 1) + ((r >> 5) & 1) * (N / 2) : min(n0 + r, N - 1);
         wg[i] = w + (size_t)n * K + Loop::chunk_of(i, wave, lane) * 8;
     }
-    floatx16 acc[TM][TN];
+    typename Loop::Sum acc[TM][TN];
     // Rows of w lie 2 K bytes apart, so workgroups that walk k in step ask the same few memory channels at every moment: each group
     // starts at a block of its own and wraps around.  Its tiles and columns start together, because they share rows in L2.
     Loop::run(lds, xg, wg, blocks, (int)((unsigned)tile.group * 13u % (unsigned)blocks), wave, lane, acc);
 
-    // 32 rows at a time pass through the wave's part of the ring, so that a lane gets 8 neighbouring columns
-    // (acc[i][j][v]: row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32 of the 32 x 32 tile)
-    constexpr int WIDTH = 32 * TN, STRIDE = WIDTH + 4;
+    // 32 rows at a time pass through the wave's part of the ring, so that a lane gets neighbouring columns, 16 bytes of them
+    // (acc[i][j][v]: row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32 of the 32 x 32 product, row (lane / 16) * 4 + v, column
+    // lane % 16 of the 16 x 16 one)
+    constexpr int MF = Loop::MF, WIDTH = MF * TN, STRIDE = WIDTH + 4;
     static_assert(4 * 32 * STRIDE * 4 <= EVEN_LDS, "a strip of every wave");
     float* strip = reinterpret_cast<float*>(lds) + wave * 32 * STRIDE;
-    constexpr int OUT = GATED ? WIDTH / 2 : WIDTH, LANES = OUT / 8, ROWS = 64 / LANES;      // stored columns, lanes a row, rows a pass
+    constexpr int E = PIECE<TO>, OUT = GATED ? WIDTH / 2 : WIDTH, LANES = OUT / E, ROWS = 64 / LANES;      // stored columns, lanes a row, rows a pass
+    static_assert(64 % LANES == 0 && 32 % ROWS == 0, "whole passes");
     TO* out = reinterpret_cast<TO*>(a.out);
     const int top_row = (wave / WN) * (BM / WM), columns = GATED ? N / 2 : N;
-    const int r0 = lane / LANES, c = lane % LANES * 8, n = (GATED ? n0 / 2 : n0) + (wave % WN) * OUT + c;
+    const int r0 = lane / LANES, c = lane % LANES * E, n = (GATED ? n0 / 2 : n0) + (wave % WN) * OUT + c;
     const int place = GATED ? c / 32 * 64 + c % 32 : c;         // in the strip; GATED: the up entries stand 32 behind
     // finish: a sum (GATED: a gate's and an up column's) to the stored entry
     auto store = [&](int i, int r, auto finish) {
         const int m = tile.first + top_row + i * 32 + r;
         const float* from = strip + r * STRIDE + place;
-        float v[8], u[8];
-        *reinterpret_cast<float4*>(v) = *reinterpret_cast<const float4*>(from);
-        *reinterpret_cast<float4*>(v + 4) = *reinterpret_cast<const float4*>(from + 4);
-        if (GATED) {
-            *reinterpret_cast<float4*>(u) = *reinterpret_cast<const float4*>(from + 32);
-            *reinterpret_cast<float4*>(u + 4) = *reinterpret_cast<const float4*>(from + 36);
+        float v[E], u[E];
+#pragma unroll
+        for (int e = 0; e < E; e += 4) {
+            *reinterpret_cast<float4*>(v + e) = *reinterpret_cast<const float4*>(from + e);
+            if (GATED) *reinterpret_cast<float4*>(u + e) = *reinterpret_cast<const float4*>(from + 32 + e);
         }
         if (m >= tile.end || n >= columns) return;              // columns % 8 == 0
         const float weight = GATED && gate.weights ? row_weight[top_row + i * 32 + r] : 1.f;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) v[e] = GATED ? finish(weight * v[e], weight * u[e]) : finish(v[e], 0.f);
-        TO* to = out + (size_t)m * a.ldo + n;
-        if constexpr (sizeof(TO) == 2) {
-            bf16x8 packed;
-#pragma unroll
-            for (int e = 0; e < 8; ++e) packed[e] = static_cast<bf16>(v[e]);
-            *reinterpret_cast<bf16x8*>(to) = packed;
-        } else {
-            *reinterpret_cast<float4*>(to) = make_float4(v[0], v[1], v[2], v[3]);
-            *reinterpret_cast<float4*>(to + 4) = make_float4(v[4], v[5], v[6], v[7]);
-        }
+        for (int e = 0; e < E; ++e) v[e] = GATED ? finish(weight * v[e], weight * u[e]) : finish(v[e], 0.f);
+        store_piece<TO>(out + (size_t)m * a.ldo + n, v);
     };
     // one test of the epilogue for 32 rows (one an entry cost 10 to 30 us of a product of 8,192 rows); the long forms stay rolled
     auto finish = [&](int i) {
@@ -272,14 +265,16 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGat
     };
     __syncthreads();
 #pragma unroll
-    for (int i = 0; i < TM; ++i) {
+    for (int i0 = 0; i0 < TM; i0 += 32 / MF) {
 #pragma unroll
-        for (int j = 0; j < TN; ++j)
+        for (int i = 0; i < 32 / MF; ++i)
 #pragma unroll
-            for (int v = 0; v < 16; ++v)
-                strip[((v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)) * STRIDE + j * 32 + (lane & 31)] = acc[i][j][v];
+            for (int j = 0; j < TN; ++j)
+#pragma unroll
+                for (int v = 0; v < Loop::SV; ++v)
+                    strip[(i * MF + (v >> 2) * 8 + (lane / MF) * 4 + (v & 3)) * STRIDE + j * MF + (lane & (MF - 1))] = acc[i0 + i][j][v];
         __builtin_amdgcn_wave_barrier();
-        finish(i);
+        finish(i0 * MF / 32);
         __builtin_amdgcn_wave_barrier();
     }
 }

@@ -4,6 +4,8 @@
 
 #include "common.h"
 
+#include <type_traits>
+
 namespace lc {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
@@ -28,6 +30,19 @@ template <> __device__ __forceinline__ void store_pair<bf16>(bf16* p, float a, f
     v[0] = static_cast<bf16>(a);
     v[1] = static_cast<bf16>(b);
     *reinterpret_cast<bf16x2*>(p) = v;
+}
+
+// 16 bytes of adjacent elements in one store; p is aligned to 16 bytes
+template <typename TO> constexpr int PIECE = 16 / sizeof(TO);
+template <typename TO> __device__ __forceinline__ void store_piece(TO* p, const float (&v)[PIECE<TO>]) {
+    if constexpr (sizeof(TO) == 2) {
+        bf16x8 packed;
+#pragma unroll
+        for (int e = 0; e < 8; ++e) packed[e] = static_cast<bf16>(v[e]);
+        *reinterpret_cast<bf16x8*>(p) = packed;
+    } else {
+        *reinterpret_cast<float4*>(p) = make_float4(v[0], v[1], v[2], v[3]);
+    }
 }
 
 // the value of another lane of the same row of 16 lanes, by a DPP move: CTRL 0xB1 swaps
@@ -82,15 +97,23 @@ __device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
 constexpr int TL_K = 64;
 
 // BM x BN rows of x and of w, TL_STAGES stages, WM x WN waves, each owning (BM / WM) x (BN / WN) of the tile as TM x TN products
-// of 32 x 32.  LATE: of two stages whose loads go out over the first half of a block.
-template <int BM, int BN, int TL_STAGES, int WM, int WN, bool LATE = false>
+// of 32 x 32.  LATE: of two stages whose loads go out later in a block (below).  FINE: products of 16 x 16 x 32 instead of 32 x 32 x 16, the
+// same sums to the bit wherever tried.  Both take the matrix cores' time for as many operations, but the small ones read and write each sum half as often,
+// and a product of large tiles is held back by the power limit: us, large and small, with the epilogue in whole lines (gemm_bf16.hip) 326 and 311 for
+// 2,048 x 24576 x 4096 with SwiGLU, 87.0 and 81.3 for x 6144 x 4096, 171.7 and 166.0 for x 4096 x 12288, 57.2 and 54.0 for x 8192 x 2048.  Not for
+// tiles whose waves own less than 64 x 128 (bound by the way from L2: no change), nor for the experts' (up to 1.07 of the time: bound by memory).
+template <int BM, int BN, int TL_STAGES, int WM, int WN, bool LATE = false, bool FINE = false>
 struct TileLoop {
+    static constexpr int MF = FINE ? 16 : 32;                 // rows and columns of a product
+    typedef typename std::conditional<FINE, floatx4, floatx16>::type Sum;
+    static constexpr int SV = MF * MF / 64;                   // sums of a product a lane
     static constexpr int S = TL_STAGES;
     static constexpr int NW = WM * WN;
-    static constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN);
-    static constexpr int KS = TL_K / 16;                      // k-steps per block
+    static constexpr int TM = BM / (MF * WM), TN = BN / (MF * WN);
+    static constexpr int KP = FINE ? 32 : 16;                 // k of a product
+    static constexpr int KS = TL_K / KP;                      // k-steps per block
     static constexpr int LPA = BM * 8 / (64 * NW), LPB = BN * 8 / (64 * NW), LP = LPA + LPB;   // load instructions per thread and stage
-    static_assert(BM % (32 * WM) == 0 && BN % (32 * WN) == 0, "whole products per wave");
+    static_assert(BM % (MF * WM) == 0 && BN % (MF * WN) == 0, "whole products per wave");
     static_assert((BM * 8) % (64 * NW) == 0 && (BN * 8) % (64 * NW) == 0, "whole load instructions per wave");
     static constexpr int NM = TM * TN, NR = TM + TN;          // products and operand reads per k-step
     static constexpr int A_STAGE = BM * TL_K * 2, B_STAGE = BN * TL_K * 2;   // bytes
@@ -106,9 +129,9 @@ struct TileLoop {
 
     // xg, wg: where load instruction i of this lane reads block 0; nk blocks, the first of them block `skew` (wrapping around)
     __device__ static __forceinline__ void run(char* lds, const bf16* const (&xg)[LPA], const bf16* const (&wg)[LPB], int nk,
-                                               int skew, int wave, int lane, floatx16 (&acc)[TM][TN]) {
+                                               int skew, int wave, int lane, Sum (&acc)[TM][TN]) {
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
-    const int lr = lane & 31, kg = lane >> 5;
+    const int lr = lane & (MF - 1), kg = lane / MF;
     // load instruction idx (x first, then w) of block kb into a stage
     auto issue_one = [&](int idx, int kb, int stage) {
         kb += skew;
@@ -128,17 +151,20 @@ struct TileLoop {
     // bound by the matrix cores and want them late (us, in a row, half, quarter: 4,001 x 4096 x 4096 121, 110, 115; 1,024 x 4096 x
     // 4096 49, 43, 45; 2,048 x 4096 x 12288 198, 173, 171; 576 x 19456 x 2560 61, 67, 65).  So the dense tiles of 256 rows, which
     // are taken for many, are LATE: over 50 products of 700 to 4,001 rows for which they are among the best, 256 x 256 0.98 of the
-    // time of a quarter (0.94 to 0.99), 256 x 192 0.99 (0.985 to 1.02).
-    constexpr int BAR = NM / 4;                                // the product after which a block's last k-step syncs
+    // time of a quarter (0.94 to 0.99), 256 x 192 0.99 (0.985 to 1.02).  FINE (us, the whole of those two shapes and 256 x 128; 24576 x 4096, 6144 x
+    // 4096, 1,523 x 24576 x 4096): barrier after a quarter, loads over 6/16, reads over half of the products 318, 82.9, 252; an eighth and 6/16
+    // 308, 82.6, 248; 3/16 and 5/16 313, 81.6, 247; a sixteenth and 5/16 307, 80.9, 248; an eighth, 5/16 and reads over three quarters 310,
+    // 81.5, 249; over a quarter 314, 83.6, 252; loads over 12/16 352, 99.6 and 103 for the 94 of 2,039 x 10240 x 2048.
+    constexpr int BAR = FINE ? NM / 8 : NM / 4;                // the product after which a block's last k-step syncs
     constexpr int WIN = KS * NM;                               // products between two barriers
     constexpr int NA = NM - 1 - BAR;                           // of them in the block that frees the stage
-    constexpr int SPAN = S == 2 ? (LATE ? WIN / 2 : WIN / 4) : WIN * 7 / 8;
+    constexpr int SPAN = S == 2 ? (LATE ? (FINE ? WIN * 5 / 16 : WIN / 2) : WIN / 4) : WIN * 7 / 8;
     static_assert(SPAN >= 1 && SPAN < WIN, "all loads of a block are issued before the next barrier");
     struct At { static constexpr int of(int l) { return l * SPAN / LP; } };      // load l's position
     // Tiles of two stages with few products a block are several to a CU and bound by how much is on its way, and issue a whole
     // block's loads behind a barrier of their own before they wait for the block before it (8,192 rows over 32 matrices of
     // 2,048 x 2,048 in tiles of 128 x 128: 127 us, 141 spread).
-    constexpr bool EARLY = S == 2 && NM <= 4;
+    constexpr bool EARLY = S == 2 && NM * MF * MF <= 4096;
     constexpr int PA = EARLY ? LP : [] { int n = 0; for (int l = 0; l < LP; ++l) n += l * SPAN / LP < NA; return n; }();   // loads in that block
     static_assert((S - 1) * LP + PA <= 63, "the load counter holds 63");
 #pragma unroll
@@ -154,7 +180,7 @@ struct TileLoop {
 #pragma unroll
         for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.f;
+            for (int v = 0; v < SV; ++v) acc[i][j][v] = 0.f;
 
     // LDS address of this lane's operand rows in stage 0, with the lane's part of the swizzle;
     // k-step ks flips chunk bits: ((2 ks + kg) ^ swz) * 16 = ((kg ^ swz) * 16) ^ (ks * 32)
@@ -162,22 +188,22 @@ struct TileLoop {
     unsigned pa[TM], pb[TN];
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
-        const int row = wm + i * 32 + lr;
+        const int row = wm + i * MF + lr;
         pa[i] = lds0 + row * 128 + ((kg ^ swz(row)) * 16);
     }
 #pragma unroll
     for (int j = 0; j < TN; ++j) {
-        const int row = wn + j * 32 + lr;
+        const int row = wn + j * MF + lr;
         pb[j] = lds0 + S * A_STAGE + row * 128 + ((kg ^ swz(row)) * 16);
     }
 
     bf16x8 a[2][TM], b[2][TN];
     auto read_one = [&](int r, int stage, int ks, int buf) {
         if (r < TM) {
-            const unsigned addr = (pa[r] ^ (ks * 32)) + stage * A_STAGE;
+            const unsigned addr = (pa[r] ^ (ks * KP * 2)) + stage * A_STAGE;
             asm volatile("ds_read_b128 %0, %1" : "=v"(a[buf][r]) : "v"(addr));
         } else {
-            const unsigned addr = (pb[r - TM] ^ (ks * 32)) + stage * B_STAGE;
+            const unsigned addr = (pb[r - TM] ^ (ks * KP * 2)) + stage * B_STAGE;
             asm volatile("ds_read_b128 %0, %1" : "=v"(b[buf][r - TM]) : "v"(addr));
         }
     };
@@ -188,14 +214,34 @@ struct TileLoop {
 #pragma unroll
         for (int j = 0; j < TN; ++j) asm volatile("" : "+v"(b[buf][j]));
     };
+    // sums of small products stay in registers of their own, or the compiler moves them about all through the loop
+    auto hold = [&](Sum& sum) {
+        if constexpr (FINE) asm volatile("" : "+a"(sum));
+    };
+    auto hold_all = [&]() {
+#pragma unroll
+        for (int i = 0; i < TM; ++i)
+#pragma unroll
+            for (int j = 0; j < TN; ++j) hold(acc[i][j]);
+    };
+    hold_all();
     auto product = [&](int k, int buf) {
         const int i = k / TN, j = k % TN;
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0);
+        if constexpr (FINE) {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0);
+            hold(acc[i][j]);
+        } else {
+            acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(a[buf][i], b[buf][j], acc[i][j], 0, 0, 0);
+        }
     };
 
     // where the reads sit among the NM products of a k-step
     constexpr int QR = (2 * NR + NM - 1) / NM;                 // reads after each product, from the first on
     constexpr int QT = NM - BAR - 1 > 0 ? (NR + (NM - BAR - 1) - 1) / (NM - BAR - 1) : NR;
+    struct Read {       // the product after which read r goes out, and so behind a block's barrier; FINE: spread over half of the products
+        static constexpr int of(int r) { return FINE ? r * (NM / 2) / NR : r / QR; }
+        static constexpr int behind(int r) { return FINE ? r * ((NM - BAR - 1) / 2) / NR : r / QT; }
+    };
 
     if (nk >= S) wait_vmcnt<(S - 2) * LP + PA>(); else wait_vmcnt<0>();
     __builtin_amdgcn_s_barrier();
@@ -220,8 +266,8 @@ struct TileLoop {
                 __builtin_amdgcn_sched_barrier(0);
                 if (ks < KS - 1) {
 #pragma unroll
-                    for (int r = k * QR; r < (k + 1) * QR; ++r)
-                        if (r < NR) read_one(r, stage, ks + 1, nxt);
+                    for (int r = 0; r < NR; ++r)
+                        if (Read::of(r) == k) read_one(r, stage, ks + 1, nxt);
                 }
                 if (REST && (ks < KS - 1 || k <= BAR)) {
 #pragma unroll
@@ -246,8 +292,8 @@ struct TileLoop {
                     }
                     if (k > BAR && (REST || it + 1 < nk)) {
 #pragma unroll
-                        for (int r = (k - BAR - 1) * QT; r < (k - BAR) * QT; ++r)
-                            if (r < NR) read_one(r, nstage, 0, nxt);
+                        for (int r = 0; r < NR; ++r)
+                            if (Read::behind(r) == k - BAR - 1) read_one(r, nstage, 0, nxt);
                     }
                     if (FREE && !EARLY && k > BAR) {
 #pragma unroll
@@ -265,6 +311,7 @@ struct TileLoop {
     for (; it + S < nk; ++it) block(it, std::true_type{}, std::true_type{});
     if (it + S - 1 < nk) { block(it, std::false_type{}, std::true_type{}); ++it; }
     for (; it < nk; ++it) block(it, std::false_type{}, std::false_type{});
+    hold_all();
 
     }
 };

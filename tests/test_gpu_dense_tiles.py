@@ -53,3 +53,18 @@ def test_taken_by_size():
     for M, N, K in ((2048, 2048, 2048), (1523, 2048, 4096), (1903, 1024, 3072)):
         assert ops.library().lc_gemm_bf16_tile(M, N, K, 0) in (13, 14)
         _check(*_operands(M, N, K), -1)
+
+
+@pytest.mark.parametrize("tile", [2, 3, 4, 6, 9, 11, 13])
+@pytest.mark.parametrize("M,N", [(31, 8), (193, 392), (257, 264), (300, 1000)])
+def test_stored_through_lds(tile, M, N):
+    """Columns that are stored in pieces of 16 bytes are, to the bit, those of a product with one or four more, which is stored in pairs or one
+    by one."""
+    x, w = _operands(M, N + 16, 512)
+    ops.force_gemm_tile(tile)
+    try:
+        for dtype, more in ((torch.bfloat16, 4), (torch.bfloat16, 1), (torch.float32, 1), (torch.float32, 2)):
+            whole, other = ops.gemm(x, w[:N], dtype), ops.gemm(x, w[:N + more], dtype)
+            assert torch.equal(whole, other[:, :N])
+    finally:
+        ops.force_gemm_tile(-1)
