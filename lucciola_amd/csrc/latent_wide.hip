@@ -66,13 +66,20 @@ struct WideArgs {
     bf16* out; long long ldo;
 };
 
-// Four operands of LDS and the wait for them in one piece: the compiler would wait for every load to LDS in flight before
-// an LDS read of its own.
-__device__ __forceinline__ void lds_four(bf16x8 (&r)[4], unsigned a, unsigned b, unsigned c, unsigned d) {
-    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %5\n\tds_read_b128 %2, %6\n\tds_read_b128 %3, %7\n\ts_waitcnt lgkmcnt(0)"
+// Four operands of LDS, asked for: two places and the same OFFSET bytes further on; lds_have waits until at most LEFT of the reads asked for
+// are still on their way and ties the operands to that point.  (The compiler would wait for every load to LDS in flight before an LDS read of
+// its own.)
+template <int OFFSET>
+__device__ __forceinline__ void lds_ask(bf16x8 (&r)[4], unsigned one, unsigned two) {
+    asm volatile("ds_read_b128 %0, %4\n\tds_read_b128 %1, %4 offset:%6\n\tds_read_b128 %2, %5\n\tds_read_b128 %3, %5 offset:%6"
                  : "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3])
-                 : "v"(a), "v"(b), "v"(c), "v"(d)
+                 : "v"(one), "v"(two), "n"(OFFSET)
                  : "memory");
+}
+template <int LEFT> __device__ __forceinline__ void lds_have(bf16x8 (&r)[4]) {
+    wait_lgkmcnt<LEFT>();
+    asm volatile("" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]));
+    __builtin_amdgcn_sched_barrier(0);
 }
 
 // grid (heads, tiles of 128 tokens, the last first: it sees the most keys).  Head h runs on XCD h % 8, whose L2 keeps its keys and
@@ -85,8 +92,8 @@ __device__ __forceinline__ void lds_four(bf16x8 (&r)[4], unsigned a, unsigned b,
 // HALVES 2: eight waves, of which four take every other stage of the same queries, with a ring of their own; their sums are joined at the
 // end.  A stage keeps a wave busy for 2.2 us where it is alone on its SIMD (its loads, products and weights wait for each other) and
 // two waves for little more, so where there are no more workgroups than two a CU the halves are the second wave, and they halve the
-// longest chain (us, one and two halves: 2,048 tokens of 16 heads 67 and 52, behind 2,048 others 129 and 98, 512 behind 4,000 129 and
-// 97; 4,000 tokens, 512 workgroups, 133 and 107).  With more workgroups a CU has its second wave anyway, and the halves only wait for
+// longest chain (us, one and two halves, both before the halves worked a turn apart: 2,048 tokens of 16 heads 67 and 52, behind 2,048 others
+// 129 and 98, 512 behind 4,000 129 and 97; 4,000 tokens, 512 workgroups, 133 and 107).  With more workgroups a CU has its second wave anyway, and the halves only wait for
 // each other (768 workgroups 93 and 124, 1,024 354 and 380).
 template <int HALVES>
 __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a) {
@@ -111,6 +118,7 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
     const int tile_lo = a.window > 0 ? max(0, a.position - a.lo + tile * LW_TOKENS - a.window + 1) : 0;
     const int s_begin = tile_lo / LW_KEYS, s_end = (a.position - a.lo + tile_last) / LW_KEYS + 1;
 
+    const float scale = a.scale_log2 == 0.f ? 1.f : fabsf(a.scale_log2);
     bf16x8 qf[KS];
     {
         const bf16* plain = a.q + (size_t)token * a.ldq + (size_t)head * (LW_DIM + LW_ROT) + 8 * half;
@@ -118,43 +126,37 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
 #pragma unroll
         for (int k = 0; k < KS; ++k)
             qf[k] = *reinterpret_cast<const bf16x8*>(k < LW_DIM / 16 ? plain + 16 * k : turned + 16 * k - LW_DIM);
+        if (!(a.scale_log2 > 0.f)) {    // below, the scale of the scores is positive: the largest score times it is the largest
+#pragma unroll
+            for (int k = 0; k < KS; ++k)
+#pragma unroll
+                for (int e = 0; e < 8; ++e) qf[k][e] = static_cast<bf16>(static_cast<float>(qf[k][e]) * (a.scale_log2 < 0.f ? -1.f : 0.f));
+        }
     }
-    // load instructions: four rows of 256 bytes of the keys, eight of 128 of their rotated parts and of the values
+    // load instructions: four rows of 256 bytes of the keys, eight of 128 of their rotated parts and of the values; a lane's bytes from the
+    // first row on, of the first instruction (instruction i of the keys: place xor 4 i) and, the values', of the second
     const int r4 = lane >> 4, r8 = lane >> 3;
-    const bf16 *k_from[4], *t_from[2], *v_from[4];
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-        const int key = 16 * wave + 4 * i + r4;
-        k_from[i] = a.keys + (size_t)key * a.H * LW_DIM + (size_t)head * LW_DIM + (((lane & 15) ^ (key & 15)) * 8);
-        const int entry = 32 * wave + 8 * i + r8;
-        v_from[i] = a.values + ((size_t)head * LW_VDIM + entry) * a.ldv + (((lane & 7) ^ ((entry >> 1) & 7)) * 8);
-    }
-#pragma unroll
-    for (int i = 0; i < 2; ++i) {
-        const int key = 16 * wave + 8 * i + r8;
-        t_from[i] = a.turned + (size_t)key * LW_ROT + (((lane & 7) ^ ((key >> 1) & 7)) * 8);
-    }
-    auto issue = [&](int s, int turn) {
+    const unsigned k_off = (unsigned)r4 * a.H * (LW_DIM * 2) + (((lane & 15) ^ r4) * 16), t_off = r8 * (LW_ROT * 2) + (((lane & 7) ^ (r8 >> 1)) * 16);
+    const unsigned v_off[2] = {(unsigned)(r8 * a.ldv * 2) + (((lane & 7) ^ (r8 >> 1)) * 16), (unsigned)(r8 * a.ldv * 2) + (((lane & 7) ^ 4 ^ (r8 >> 1)) * 16)};
+    // Load n of a wave, of stage s into that turn's place: 0 to 3 the keys', 4 and 5 their rotated parts', 6 to 9 the values'.
+    constexpr int LOADS = 10, KEY_LOADS = 6;
+    auto load = [&](int n, int s, int turn) {
         char* stage = lds + (turn & 1) * STAGE;
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds((glb_ptr_t)(k_from[i] + (size_t)s * LW_KEYS * a.H * LW_DIM),
-                                             (lds_ptr_t)(stage + (4 * wave + i) * 1024), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 2; ++i)
-            __builtin_amdgcn_global_load_lds((glb_ptr_t)(t_from[i] + (size_t)s * LW_KEYS * LW_ROT),
-                                             (lds_ptr_t)(stage + KB + (2 * wave + i) * 1024), 16, 0, 0);
-#pragma unroll
-        for (int i = 0; i < 4; ++i)
-            __builtin_amdgcn_global_load_lds((glb_ptr_t)(v_from[i] + (size_t)s * LW_KEYS),
-                                             (lds_ptr_t)(stage + KB + TB + (4 * wave + i) * 1024), 16, 0, 0);
+        const char* from;
+        if (n < 4) from = reinterpret_cast<const char*>(a.keys + ((size_t)(s * LW_KEYS + 16 * wave + 4 * n) * a.H + head) * LW_DIM) + (k_off ^ (n * 64));
+        else if (n < 6) from = reinterpret_cast<const char*>(a.turned + (size_t)(s * LW_KEYS + 16 * wave + 8 * (n - 4)) * LW_ROT) + (t_off ^ ((n - 4) * 64));
+        else from = reinterpret_cast<const char*>(a.values + ((size_t)head * LW_VDIM + 32 * wave + 8 * (n - 6)) * a.ldv + (size_t)s * LW_KEYS) + v_off[n & 1];
+        const int at = n < 4 ? (4 * wave + n) * 1024 : n < 6 ? KB + (2 * wave + n - 4) * 1024 : KB + TB + (4 * wave + n - 6) * 1024;
+        __builtin_amdgcn_global_load_lds((glb_ptr_t)from, (lds_ptr_t)(stage + at), 16, 0, 0);
     };
     // row r of a tile of S^T is key 16 (r / 16) + 8 ((r / 4) % 2) + 4 ((r / 8) % 2) + r % 4 of its 32: the lane's 16 values, rows
     // 8 (v / 4) + 4 half + v % 4, are then the keys 16 (v / 8) + 8 half + v % 8
     const int key = 16 * (col >> 4) + 8 * ((col >> 2) & 1) + 4 * ((col >> 3) & 1) + (col & 3);
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)lds;
-    const unsigned k_row = lds0 + key * 256, t_row = lds0 + KB + key * 128, v_row = lds0 + KB + TB + col * 128;
-    const unsigned k_swz = key & 15, t_swz = (key >> 1) & 7, v_swz = (col >> 1) & 7;     // the same for the rows 32 further on
+    // place p of a row of K is chunk p ^ (key % 16): chunk 2 x + half of the lane's row is 32 x further on or back, in these bits alone
+    static_assert(STAGE % 1024 == 0 && KB % 1024 == 0 && TB % 1024 == 0, "rows do not reach into the places' bits");
+    const unsigned k_row = lds0 + key * 256 + (half ^ (key & 15)) * 16, t_row = lds0 + KB + key * 128 + (half ^ ((key >> 1) & 7)) * 16;
+    const unsigned v_row = lds0 + KB + TB + col * 128 + (half ^ ((col >> 1) & 7)) * 16;         // the same for the rows 32 further on
 
     floatx16 o[VT];
 #pragma unroll
@@ -162,53 +164,60 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
 #pragma unroll
         for (int v = 0; v < 16; ++v) o[i][v] = 0.f;
     float m_ref = -INFINITY, l = 0.f;
-    if (s_begin + part < s_end) issue(s_begin + part, 0);
-    const int turns = (s_end - s_begin + HALVES - 1) / HALVES;
-    for (int turn = 0; turn < turns; ++turn) {
-        const int s = s_begin + part + turn * HALVES;
-        wait_vmcnt<0>();                                    // this wave's loads of the stage have landed
-        __builtin_amdgcn_s_barrier();                       // everybody's have; nobody reads the other stage any more
-        asm volatile("" ::: "memory");
-        if (s + HALVES < s_end) issue(s + HALVES, turn + 1);
-        const int c0 = s * LW_KEYS;
-        if (!wave_live || s >= s_end || c0 > wave_hi || c0 + LW_KEYS <= wave_lo) continue;
-        const unsigned stage = (turn & 1) * STAGE;
-        floatx16 sc[2];
+    floatx16 sc[2];
+    // S^T of the stage in this turn's place; the next four operands are on their way while four are multiplied
+    auto scores = [&](unsigned stage) {
+        // entries 16 x .. 16 x + 31 of both tiles of 32 keys; the tiles' sums take turns, so that no product waits for the one before it
+        constexpr int GROUPS = KS / 2;
+        bf16x8 ka[2][4];
+        const unsigned k_at = k_row + stage, t_at = t_row + stage;
+        auto ask = [&](int g) {
+            const int x = 2 * g;
+            if (x < LW_DIM / 16) lds_ask<32 * 256>(ka[g & 1], k_at ^ (x * 32), k_at ^ ((x + 1) * 32));
+            else lds_ask<32 * 128>(ka[g & 1], t_at ^ ((x - LW_DIM / 16) * 32), t_at ^ ((x + 1 - LW_DIM / 16) * 32));
+        };
 #pragma unroll
-        for (int t = 0; t < 2; ++t) {
+        for (int t = 0; t < 2; ++t)
 #pragma unroll
             for (int v = 0; v < 16; ++v) sc[t][v] = 0.f;
+        ask(0);
 #pragma unroll
-            for (int k = 0; k < KS; k += 4) {
-                bf16x8 ka[4];
-                unsigned where[4];
+        for (int g = 0; g < GROUPS; ++g) {
+            if (g + 1 < GROUPS) { ask(g + 1); lds_have<4>(ka[g & 1]); }
+            else lds_have<0>(ka[g & 1]);
 #pragma unroll
-                for (int i = 0; i < 4; ++i) {
-                    const int x = k + i;
-                    where[i] = x < LW_DIM / 16 ? k_row + stage + t * 32 * 256 + (((2 * x + half) ^ k_swz) * 16)
-                                               : t_row + stage + t * 32 * 128 + (((2 * (x - LW_DIM / 16) + half) ^ t_swz) * 16);
-                }
-                lds_four(ka, where[0], where[1], where[2], where[3]);
-#pragma unroll
-                for (int i = 0; i < 4; ++i) sc[t] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[i], qf[k + i], sc[t], 0, 0, 0);
-            }
+            for (int i = 0; i < 4; ++i)
+                sc[i & 1] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(ka[g & 1][i], qf[2 * g + (i >> 1)], sc[i & 1], 0, 0, 0);
         }
+    };
+    // the weights of stage s, whose scores are in sc, and their products with its values
+    auto weigh = [&](int s, unsigned stage) {
+        const int c0 = s * LW_KEYS;
+        // keys 16 b .. 16 b + 31 of two tiles of 32 entries
+        bf16x8 va[2][4];
+        const unsigned v_at = v_row + stage;
+        auto ask = [&](int g) {
+            const int b = g % 2 * 2;
+            const unsigned from = v_at + g / 2 * 64 * 128;
+            lds_ask<32 * 128>(va[g & 1], from ^ (b * 32), from ^ ((b + 1) * 32));
+        };
         // scores in units of log 2; what the query does not see is -infinity
         const bool all = c0 + LW_KEYS - 1 <= wave_hi - 31 && c0 >= wave_lo + 31;       // every query of the wave sees every key
+        if (!all) {
+#pragma unroll
+            for (int t = 0; t < 2; ++t)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) {
+                    const int j = c0 + 32 * t + 16 * (v >> 3) + 8 * half + (v & 7);
+                    sc[t][v] = j <= at && j >= from ? sc[t][v] : -INFINITY;
+                }
+        }
         float mx = -INFINITY;
 #pragma unroll
         for (int t = 0; t < 2; ++t)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                float x = sc[t][v] * a.scale_log2;
-                if (!all) {
-                    const int j = c0 + 32 * t + 16 * (v >> 3) + 8 * half + (v & 7);
-                    x = j <= at && j >= from ? x : -INFINITY;
-                }
-                sc[t][v] = x;
-                mx = fmaxf(mx, x);
-            }
-        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave));
+            for (int v = 0; v < 16; ++v) mx = fmaxf(mx, sc[t][v]);
+        mx = fmaxf(mx, __shfl_xor(mx, 32, kWave)) * scale;
         if (__builtin_amdgcn_ballot_w64(mx > m_ref + 8.f) != 0) {      // also at a query's first visible key
             const float m_new = mx > m_ref + 8.f ? mx : m_ref;
             const float keep = m_ref == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(m_ref - m_new);
@@ -222,24 +231,62 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
         const float ref = m_ref == -INFINITY ? 0.f : m_ref;
         bf16x8 p[4];
 #pragma unroll
-        for (int t = 0; t < 2; ++t)
+        for (int b = 0; b < 4; ++b) {
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const float w = __builtin_amdgcn_exp2f(sc[t][v] - ref);
+            for (int v = 0; v < 8; ++v) {
+                const float w = __builtin_amdgcn_exp2f(fmaf(sc[b >> 1][(b & 1) * 8 + v], scale, -ref));
                 l += w;
-                p[2 * t + (v >> 3)][v & 7] = static_cast<bf16>(w);
+                p[b][v] = static_cast<bf16>(w);
             }
-#pragma unroll
-        for (int i = 0; i < VT; ++i) {
-            bf16x8 va[4];
-            unsigned where[4];
-#pragma unroll
-            for (int b = 0; b < 4; ++b) where[b] = v_row + stage + i * 32 * 128 + (((2 * b + half) ^ v_swz) * 16);
-            lds_four(va, where[0], where[1], where[2], where[3]);
-#pragma unroll
-            for (int b = 0; b < 4; ++b) o[i] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[b], p[b], o[i], 0, 0, 0);
         }
+        ask(0);
+#pragma unroll
+        for (int g = 0; g < VT; ++g) {
+            if (g + 1 < VT) { ask(g + 1); lds_have<4>(va[g & 1]); }
+            else lds_have<0>(va[g & 1]);
+#pragma unroll
+            for (int i = 0; i < 4; ++i) {
+                floatx16& sum = o[g / 2 * 2 + (i & 1)];
+                sum = __builtin_amdgcn_mfma_f32_32x32x16_bf16(va[g & 1][i], p[g % 2 * 2 + (i >> 1)], sum, 0, 0, 0);
+            }
+        }
+    };
+    // The second half is a turn behind with its weights and values: while one half's waves multiply for their scores the other's, on the same
+    // SIMDs, work out weights.  A CU takes loads at 64 bytes a clock at most, 1,300 clocks for a turn's 80 KB, and a wave that issues its own in
+    // a row does nothing else until they are taken (clock stamps: 700 to 2,000 of a turn's 6,000 clocks): so each half issues them at a moment of
+    // its own, the first behind its scores, the second its values at the turn's start and its keys behind its weights.  us, as it was before there was any of
+    // this, a turn behind, so, and with the priority below: 1,953 tokens of 16 heads behind 2,048 others 95.4, 89.3, 83.1 and 82; 2,048 tokens
+    // 56.6, 54.3, 48.5 and 48; 512 behind 4,000 99.1, 91.0, 78.1 and 77; 1,500 of 32 heads behind 600 (a single half) 79.3, 76.1, 71.5 and 71.
+    const bool behind = HALVES == 2 && part == 1;
+    const int turns = (s_end - s_begin + HALVES - 1) / HALVES;
+    auto seen = [&](int s) { return wave_live && s < s_end && s * LW_KEYS <= wave_hi && s * LW_KEYS + LW_KEYS > wave_lo; };
+#pragma unroll
+    for (int n = 0; n < LOADS; ++n)
+        if (n < KEY_LOADS || !behind) load(n, min(s_begin + part, s_end - 1), 0);
+    for (int turn = 0; turn < turns + HALVES - 1; ++turn) {
+        const int s = s_begin + part + turn * HALVES;
+        wait_vmcnt<0>();                                    // this wave's loads of the stage have landed
+        __builtin_amdgcn_s_barrier();                       // everybody's have; nobody reads the other stage any more
+        asm volatile("" ::: "memory");
+        // behind the last stage it is loaded again, and not read
+        auto ahead = [&](int from, int to) {
+            const int s_keys = min(s + HALVES, s_end - 1), s_values = behind ? min(s, s_end - 1) : s_keys;
+#pragma unroll
+            for (int n = 0; n < LOADS; ++n)
+                if (n >= from && n < to) load(n, n < KEY_LOADS ? s_keys : s_values, n >= KEY_LOADS && behind ? turn : turn + 1);
+        };
+        // (conditions of their own: in one block for each half the compiler makes two loops of the turns, and spills)
+        if (behind) ahead(KEY_LOADS, LOADS);
+        if (behind && turn > 0 && seen(s - HALVES)) weigh(s - HALVES, ((turn - 1) & 1) * STAGE);
+        if (behind) ahead(0, KEY_LOADS);
+        const bool see = seen(s);
+        __builtin_amdgcn_s_setprio(1);                      // products leave most of the issue slots to the other wave
+        if (see) scores((turn & 1) * STAGE);
+        __builtin_amdgcn_s_setprio(0);
+        if (!behind) ahead(0, LOADS);
+        if (!behind && see) weigh(s, (turn & 1) * STAGE);
     }
+    wait_vmcnt<0>();
     if constexpr (HALVES == 2) {
         static_assert((VT * 16 + 2) * 256 * 4 <= HALVES * 2 * STAGE, "the second half's sums");
         float* its = reinterpret_cast<float*>(all_lds) + (threadIdx.x & 255);       // [m, l, the sums][thread]
@@ -334,6 +381,7 @@ LC_API int lc_latent_wide(const void* q, long long ldq, const void* q_turned, lo
     LC_CHECK(window == 0 ? lo == 0 : lo <= (position - window + 1 > 0 ? position - window + 1 : 0), "latent_wide: rows are missing");
     LC_CHECK(((uintptr_t)q | (uintptr_t)q_turned | (uintptr_t)keys | (uintptr_t)turned | (uintptr_t)values) % 16 == 0 &&
                  (ldq | q_row | q_head | ldv) % 8 == 0, "latent_wide: not aligned to 16 bytes");
+    LC_CHECK(ldv < 1ll << 28 && H < 1 << 20, "latent_wide: rows too long");
     LC_CHECK(ldv >= (position + tokens - lo + LW_KEYS - 1) / LW_KEYS * LW_KEYS, "latent_wide: the values' rows are too short");
     LC_CHECK((uintptr_t)out % 8 == 0 && ldo % 4 == 0, "latent_wide: the output is not aligned to 8 bytes");
     LC_CHECK(!gate || gate_head == 1 || (gate_head == LW_VDIM && (uintptr_t)gate % 8 == 0 && ldg % 4 == 0), "latent_wide: bad gates");

@@ -257,3 +257,31 @@ def test_a_model_whose_portions_attend_head_by_head(monkeypatch, model):
     assert len(got) == sum(len(ids) for ids in prompts.values())
     assert calls.count("lc_latent_wide") == 2 * 5, "two layers, five portions of 100 tokens and more"
     print(f"{cfg['architecture']}: worst relative error {compare(got, cfg, weights, prompts, 4e-2, refs):.3e}")
+
+
+@pytest.mark.parametrize("halves", [1, 2])
+@pytest.mark.parametrize("scale", [-0.3, 0.0])
+def test_scales_that_are_not_positive(halves, scale):
+    """A score's sign goes with the query, and a scale of zero weighs every visible key alike: against float64, whose values are exact here,
+    with weights rounded to bfloat16 (2^-9 each) and a bfloat16 result."""
+    H, T, position, window = 3, 200, 70, 90
+    lo = max(0, position - window + 1)
+    rows = -(-(position + T - lo) // 64) * 64
+    g = torch.Generator().manual_seed(5)
+    q, turned_q, keys, turned, values = ((torch.randn(*shape, generator=g) * 0.5).bfloat16().to(DEV) for shape in (
+        (T, H * 192), (T, H * 64), (rows, H * 128), (rows, 64), (H * 128, rows)))
+    out = torch.empty(T, H * 128, dtype=torch.bfloat16, device=DEV)
+    before = ops.library().lc_latent_wide_halves(halves)
+    try:
+        ops._call("lc_latent_wide", ops._ptr(q), H * 192, ops._ptr(turned_q), H * 64, 64, ops._ptr(keys), ops._ptr(turned), ops._ptr(values),
+                  rows, H, 0, T, position, lo, scale, window, None, None, 0, 0, ops._ptr(out), H * 128, ops._stream())
+    finally:
+        ops.library().lc_latent_wide_halves(before)
+    i, j = torch.arange(T, device=DEV)[:, None] + position, torch.arange(rows, device=DEV)[None] + lo
+    seen = (j <= i) & (j > i - window)
+    for h in range(H):
+        a = torch.cat([q[:, h * 192:h * 192 + 128], turned_q[:, h * 64:h * 64 + 64]], 1).double()
+        s = a @ torch.cat([keys[:, h * 128:h * 128 + 128], turned], 1).double().T * scale
+        want = s.masked_fill(~seen, float("-inf")).softmax(1) @ values[h * 128:h * 128 + 128].double().T
+        got = out[:, h * 128:h * 128 + 128].double()
+        assert float((got - want).norm() / want.norm()) <= 2.0 ** -8
