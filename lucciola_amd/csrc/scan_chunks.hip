@@ -2,7 +2,7 @@
 //     S <- diag(decay) S - removal (probe^T S) + write v^T,    o = S^T read,
 // for portions of prompts, a chunk of SC = 32 tokens at a time on the float32 matrix instruction.  Token by token a step
 // is a chain of dependent vector instructions, 0.21 us a token without and 0.29 us with the removal term, on a wave that
-// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 107 and 185).
+// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 89 and 162).
 //
 // Inside a chunk, from the state S that the chunk before left, with a_i the product of the decays of tokens 0..i (key
 // channel by key channel), r_ij that of the tokens j+1..i, and y_i = probe_i^T S_(i-1) what token i takes out:
@@ -27,6 +27,8 @@
 // finite meets no row of W - R T M above its own: such a token reaches what comes behind it and nothing before.
 #include "common.h"
 
+#include <type_traits>
+
 namespace lc {
 
 constexpr int SC = 32;                  // tokens of a chunk: two blocks of 16
@@ -42,7 +44,7 @@ __device__ __forceinline__ f32x4 mfma4(float a, float b, f32x4 c) { return __bui
 // W^ [SC][SC], and with a removal term T probe~ [SC][DK] and -removal~^T [DK][SC].  The matrices lie as the operands that the
 // second kernel loads, 1 KB a [16 x 16] tile: lane (row, quad) has entries 4 quad .. + 3 of a row (in rows
 // the walk, whose loads then touch sixteen half lines each, took 109 us where it took 95 and, removing, 199 us where 145, in its form with
-// four waves; 80 and 122 now).
+// four waves; 63 and 98 now).
 template <int DK, bool REMOVE>
 struct ChunkRecord {
     static constexpr int READ = 0, Z = SC * DK, DECAY = 2 * SC * DK, MIX = DECAY + 2 * DK, PROBE = MIX + SC * SC,
@@ -397,9 +399,11 @@ __device__ __forceinline__ void walk_tokens(const float* __restrict__ coef, cons
 // (KT tiles of 16), which are B operands of the next products as they are, and take it from chunk to chunk; four others make
 // the chunks' read-outs from copies of S that the first leave in LDS, a chunk behind.  So a SIMD has two waves, and one's loads,
 // LDS trips and address arithmetic pass beside the other's products (with the read-outs made by the waves that keep S, one wave a
-// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 80 and 122).  What the
-// waves make of their key rows meets in LDS, two buffers in turn, one barrier a chunk.  A chunk's record is asked for two chunks
-// ahead.  Workgroups are numbered so that the blocks of one head, which read the same records, run on one XCD (workgroup
+// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 76 and 115, and with the loads
+// placed by hand, fewer of them and whole lines stored 63 and 98).  What the waves make of their key rows meets in LDS, two buffers in turn,
+// one barrier a chunk.  A chunk's record is asked for two chunks ahead, its values, of which each wave brings an eighth for all, four.  A chunk
+// takes 1.0 us and, removing, 1.5, of which the matrix cores 0.5 and 0.9; the rest is the chain: a trip through LDS to the readers
+// and back, the barrier, and what the loads' 40 or 70 KB keep the CU's way to L2 busy.  Workgroups are numbered so that the blocks of one head, which read the same records, run on one XCD (workgroup
 // i on XCD i % 8) where the heads are a multiple of 8.
 template <int DK, bool REMOVE>
 __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __restrict__ records, const uint2* __restrict__ alone,
@@ -410,9 +414,10 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     typedef ChunkRecord<DK, REMOVE> Rec;
     constexpr int KT = DK / 64, TT = SC / 16, KEYS = DK / 16;
     __shared__ f32x4 states[2][4][KT][kWave], reads[2][4][TT][kWave], taken[REMOVE ? 2 : 1][4][TT][kWave];
+    __shared__ __attribute__((aligned(16))) float shared_value[3][TT * 4][kWave], shared_decay[3][4][2 * 16 * KT];
     const int lane = threadIdx.x % kWave, row = lane & 15, quad = lane >> 4;
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) & 3;
-    const bool keeps = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave) < 4;
+    const int all = __builtin_amdgcn_readfirstlane(threadIdx.x / kWave), wave = all & 3;
+    const bool keeps = all < 4;
     const int head = blockIdx.x % heads, block = blockIdx.x / heads, req = blockIdx.y;
     const int first = q_offsets[req], last = q_offsets[req + 1];
     if (last - first < least) return;
@@ -432,14 +437,22 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     const unsigned line = heads * dv;                       // floats from a token's values to the next one's, below 2^23
     const float* values = v + (size_t)first * line + (size_t)head * dv;
     const float* record = records + ((size_t)first_record(q_offsets, req, least) * heads + head) * Rec::SIZE;
-    // a chunk's record and values; behind the last chunk the last one's once more.  Entries that lie behind the request's
-    // end are zero in the records, so such a token's value (the last token's) only has to be a number.
-    auto record_of = [&](int c) { return record + (size_t)min(c, chunks - 1) * heads * Rec::SIZE; };
-    auto tile = [&](const float* rec, int matrix, int n) { return *reinterpret_cast<const f32x4*>(rec + (matrix + n * 256) + lane * 4); };
-    auto value_of = [&](int c, int t, int i) {
-        const int base = min(c, chunks - 1) * SC;
-        const unsigned token = min(16 * t + 4 * quad + i, last - first - 1 - base);
-        return (values + (size_t)base * line)[__umul24(token, line) + column];
+    const size_t record_line = (size_t)heads * Rec::SIZE;
+    // A chunk's record, and the value that this wave brings for all of them; behind the last chunk the last one's once more.  Entries that
+    // lie behind the request's end are zero in the records, so such a token's value (the last token's) only has to be a number.
+    auto record_of = [&](int c) {
+        const float* rec = record + (size_t)min(c, chunks - 1) * record_line;
+        asm volatile("" : "+s"(rec));
+        return rec;
+    };
+    auto tile = [&](const float* rec, int matrix, int n) { return *reinterpret_cast<const f32x4*>(rec + (matrix + n * 256) + (unsigned)lane * 4); };
+    static_assert(TT == 2, "eight waves, a value each");
+    const int token = 16 * (all >> 2) + 4 * quad + (all & 3), over = last - first - 1 - (chunks - 1) * SC;
+    const unsigned place = __umul24(token, line) + column, place_last = __umul24(min(token, over), line) + column;
+    auto fetch_value = [&](int c) {
+        const float* at = values + (size_t)(min(c, chunks - 1) * SC) * line;
+        asm volatile("" : "+s"(at));
+        return at[c >= chunks - 1 ? place_last : place];
     };
     // only LDS has to be in order between the waves: loads from memory stay in flight
     auto meet = []() {
@@ -448,45 +461,85 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
         __builtin_amdgcn_s_barrier();
         asm volatile("" ::: "memory");
     };
+    // Loads stay where they stand among the products.  Left alone, the compiler put three chunks' loads side by side, so that every third
+    // chunk waited for memory twice.  And a CU takes one of these loads in 16 clocks: eight waves that ask for all of a chunk's at once wait a
+    // thousand clocks and more for that.  With a removal term they go out between the products (walk of 2,048 tokens, 16 heads of 128 x 128, all
+    // at once 122 us, spread 98); without it there are too few products to hide them, and a chunk's go out at its start, where the reading
+    // waves have nothing else to do (63 us, spread 71, at other places 66 to 82).
+    constexpr bool SPREAD = REMOVE;
+    auto pin = []() { __builtin_amdgcn_sched_barrier(6); };
+    float raw[3];
+#pragma unroll
+    for (int n = 0; n < 3; ++n) raw[n] = fetch_value(n);
+    shared_value[0][all][lane] = raw[0];
+    shared_value[1][all][lane] = raw[1];
+    raw[0] = fetch_value(3);
     if (keeps) {
         float* home = state + (((size_t)slot_ids[req] * heads + head) * dv + column) * DK + wave * 16 * KT + 4 * quad;
         f32x4 S[KT];
 #pragma unroll
         for (int k = 0; k < KT; ++k) S[k] = *reinterpret_cast<const f32x4*>(home + 16 * k);
         struct Loaded {
-            f32x4 z[KT][TT], probe[REMOVE ? TT : 1][KT], removal[KT][REMOVE ? TT : 1], decay[KT], rest[KT];
-            float value[TT][4];
+            f32x4 z[KT][TT], probe[REMOVE ? TT : 1][KT], removal[KT][REMOVE ? TT : 1];
+            float decay;
+        };
+        const unsigned decay_place = lane / (16 * KT) * DK + wave * 16 * KT + lane % (16 * KT);
+        // load number n of a chunk's
+        constexpr int TILES = TT * KT, LOADS = 1 + (REMOVE ? 3 : 1) * TILES;
+        auto fetch_one = [&](Loaded& l, const float* rec, int n) {
+            if (n == 0) l.decay = rec[Rec::DECAY + (16 * KT * 2 == kWave || lane < 32 * KT ? decay_place : 0u)];
+            else if (n <= TILES) l.z[(n - 1) % KT][(n - 1) / KT] = tile(rec, Rec::Z, (wave * KT + (n - 1) % KT) * TT + (n - 1) / KT);
+            else if constexpr (REMOVE) {
+                const int m = n - 1 - TILES;
+                if (m < TILES) l.probe[m / KT][m % KT] = tile(rec, Rec::PROBE, m / KT * KEYS + wave * KT + m % KT);
+                else l.removal[m % KT][m / KT - TT] = tile(rec, Rec::REMOVAL, (wave * KT + m % KT) * TT + m / KT - TT);
+            }
         };
         auto fetch = [&](Loaded& l, int c) {
             const float* rec = record_of(c);
-            if constexpr (REMOVE) {
 #pragma unroll
-                for (int t = 0; t < TT; ++t)
-#pragma unroll
-                    for (int k = 0; k < KT; ++k) l.probe[t][k] = tile(rec, Rec::PROBE, t * KEYS + wave * KT + k);
-            }
+            for (int n = 0; n < LOADS; ++n) fetch_one(l, rec, n);
+        };
+        float value[TT][4];
+        f32x4 decay[KT], rest[KT];
+        // what the wave works with in the chunk, out of LDS
+        auto take = [&](int n) {
 #pragma unroll
             for (int k = 0; k < KT; ++k) {
-                const float* decay = rec + (Rec::DECAY + 16 * (wave * KT + k)) + 4 * quad;
-                l.decay[k] = *reinterpret_cast<const f32x4*>(decay);
-                l.rest[k] = *reinterpret_cast<const f32x4*>(decay + DK);
+                decay[k] = *reinterpret_cast<const f32x4*>(&shared_decay[n][wave][16 * k + 4 * quad]);
+                rest[k] = *reinterpret_cast<const f32x4*>(&shared_decay[n][wave][16 * KT + 16 * k + 4 * quad]);
             }
 #pragma unroll
-            for (int t = 0; t < TT; ++t) {
+            for (int t = 0; t < TT; ++t)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) l.value[t][i] = value_of(c, t, i);
-#pragma unroll
-                for (int k = 0; k < KT; ++k) l.z[k][t] = tile(rec, Rec::Z, (wave * KT + k) * TT + t);
-            }
-            if constexpr (REMOVE) {
-#pragma unroll
-                for (int t = 0; t < TT; ++t)
-#pragma unroll
-                    for (int k = 0; k < KT; ++k) l.removal[k][t] = tile(rec, Rec::REMOVAL, (wave * KT + k) * TT + t);
-            }
+                for (int i = 0; i < 4; ++i) value[t][i] = shared_value[n][4 * t + i][lane];
         };
-        auto work = [&](const Loaded& l, int c) {
+        auto leave_decay = [&](int n, float d) {
+            if (16 * KT * 2 == kWave || lane < 32 * KT) shared_decay[n][wave][lane] = d;
+        };
+        auto work = [&](const Loaded& l, const Loaded& next, Loaded& coming, int c, auto turn3) {
+            constexpr int n = decltype(turn3)::value;       // c % 3
             const int turn = c & 1;
+            const float* rec = record_of(c + 2);
+            constexpr int EVERY = 2;
+            static_assert(!SPREAD || EVERY * LOADS < 12 * TILES, "a product for every load");
+            auto ask_all = [&]() {
+                pin();
+#pragma unroll
+                for (int l = 0; l < LOADS; ++l) fetch_one(coming, rec, l);
+                raw[(n + 1) % 3] = fetch_value(c + 4);
+                pin();
+            };
+            auto between = [&](int product) {
+                if constexpr (!SPREAD) return;
+                pin();
+                if (product % EVERY == 0 && product / EVERY <= LOADS) {
+                    if (product == 0) raw[(n + 1) % 3] = fetch_value(c + 4);
+                    else fetch_one(coming, rec, product / EVERY - 1);
+                    pin();
+                }
+            };
+            if constexpr (!SPREAD) ask_all();
 #pragma unroll
             for (int k = 0; k < KT; ++k) states[turn][wave][k][lane] = S[k];
             if constexpr (REMOVE) {
@@ -498,20 +551,29 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
 #pragma unroll
-                        for (int t = 0; t < TT; ++t) y[t] = mfma4(l.probe[t][k][i], S[k][i], y[t]);
+                        for (int t = 0; t < TT; ++t) {
+                            y[t] = mfma4(l.probe[t][k][i], S[k][i], y[t]);
+                            between((k * 4 + i) * TT + t);
+                        }
 #pragma unroll
                 for (int t = 0; t < TT; ++t) taken[turn][wave][t][lane] = y[t];
             }
+            shared_value[(n + 2) % 3][all][lane] = raw[(n + 2) % 3];
+            leave_decay((n + 1) % 3, next.decay);
 #pragma unroll
             for (int k = 0; k < KT; ++k)
 #pragma unroll
-                for (int i = 0; i < 4; ++i) S[k][i] = fmaf(S[k][i], l.rest[k][i], S[k][i] * l.decay[k][i]);
+                for (int i = 0; i < 4; ++i) S[k][i] = fmaf(S[k][i], rest[k][i], S[k][i] * decay[k][i]);
 #pragma unroll
             for (int t = 0; t < TT; ++t)
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
 #pragma unroll
-                    for (int k = 0; k < KT; ++k) S[k] = mfma4(l.z[k][t][i], l.value[t][i], S[k]);
+                    for (int k = 0; k < KT; ++k) {
+                        S[k] = mfma4(l.z[k][t][i], value[t][i], S[k]);
+                        between((REMOVE ? 4 * TILES : 0) + (t * 4 + i) * KT + k);
+                    }
+            take((n + 1) % 3);
             meet();
             if constexpr (REMOVE) {
 #pragma unroll
@@ -521,22 +583,29 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
 #pragma unroll
                     for (int i = 0; i < 4; ++i)
 #pragma unroll
-                        for (int k = 0; k < KT; ++k) S[k] = mfma4(l.removal[k][t][i], y[i], S[k]);
+                        for (int k = 0; k < KT; ++k) {
+                            S[k] = mfma4(l.removal[k][t][i], y[i], S[k]);
+                            between(8 * TILES + (t * 4 + i) * KT + k);
+                        }
                 }
             }
         };
         Loaded sets[3];
         fetch(sets[0], 0);
         fetch(sets[1], 1);
+        leave_decay(0, sets[0].decay);
+        meet();                                             // the first two chunks' values are there
+        take(0);
+        auto turn = [&](int c, auto turn3) {
+            constexpr int n = decltype(turn3)::value;
+            work(sets[n], sets[(n + 1) % 3], sets[(n + 2) % 3], c, turn3);
+        };
         for (int c = 0;;) {
-            fetch(sets[2], c + 2);
-            work(sets[0], c);
+            turn(c, std::integral_constant<int, 0>{});
             if (++c == chunks) break;
-            fetch(sets[0], c + 2);
-            work(sets[1], c);
+            turn(c, std::integral_constant<int, 1>{});
             if (++c == chunks) break;
-            fetch(sets[1], c + 2);
-            work(sets[2], c);
+            turn(c, std::integral_constant<int, 2>{});
             if (++c == chunks) break;
         }
         meet();                                             // the last chunk's read-outs
@@ -547,85 +616,128 @@ __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __res
     } else {
         struct Loaded {
             f32x4 read[TT][KT], mix;
-            float value[4];
+        };
+        constexpr int LOADS = 1 + TT * KT;
+        auto fetch_one = [&](Loaded& l, const float* rec, int n) {
+            if (n == 0) l.mix = tile(rec, Rec::MIX, wave);
+            else l.read[(n - 1) / KT][(n - 1) % KT] = tile(rec, Rec::READ, (n - 1) / KT * KEYS + wave * KT + (n - 1) % KT);
         };
         auto fetch = [&](Loaded& l, int c) {
             const float* rec = record_of(c);
 #pragma unroll
-            for (int t = 0; t < TT; ++t)
-#pragma unroll
-                for (int k = 0; k < KT; ++k) l.read[t][k] = tile(rec, Rec::READ, t * KEYS + wave * KT + k);
-            l.mix = tile(rec, Rec::MIX, wave);
-#pragma unroll
-            for (int i = 0; i < 4; ++i) l.value[i] = value_of(c, wave & 1, i);
+            for (int n = 0; n < LOADS; ++n) fetch_one(l, rec, n);
         };
-        auto work = [&](const Loaded& l, int c) {
-            const int turn = c & 1;
-            meet();                                         // the state before chunk c is there
-            f32x4 o[TT], mixed = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-            for (int t = 0; t < TT; ++t) o[t] = mixed;
-            // a wave takes one of the four blocks of W^ (the one above the diagonal is zero)
-#pragma unroll
-            for (int i = 0; i < 4; ++i) mixed = mfma4(l.mix[i], l.value[i], mixed);
-#pragma unroll
-            for (int k = 0; k < KT; ++k) {
-                const f32x4 S = states[turn][wave][k][lane];
+        // chunk c's read-outs, a tile of tokens by each of two waves, four channels of a token a lane, once every wave has left its part
+        float* to = out + (size_t)first * line + (size_t)head * dv;
+        const int channel = block * 16 + 4 * quad;
+        const bool whole = dv % 4 == 0 && ((uintptr_t)out & 15) == 0;
+        const unsigned store_place = __umul24(16 * (wave & 1) + row, line) + channel;
+        auto write = [&](int c) {
+            if (wave >= TT) return;
+            const f32x4* part = &reads[c & 1][0][wave][lane];
+            constexpr int NEXT = TT * kWave;                // from a wave's part to the next one's
+            const f32x4 o = (part[0] + part[NEXT]) + (part[2 * NEXT] + part[3 * NEXT]);
+            float* at = to + (size_t)(c * SC) * line;
+            if (16 * wave + row >= last - first - c * SC) return;
+            if (whole) {
+                if (channel < dv) *reinterpret_cast<f32x4*>(at + store_place) = o;
+            } else {
 #pragma unroll
                 for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int t = 0; t < TT; ++t) o[t] = mfma4(l.read[t][k][i], S[i], o[t]);
+                    if (channel + i < dv) at[store_place + i] = o[i];
             }
+        };
+        // a wave takes one of the four blocks of W^ (the one above the diagonal is zero)
+        auto mix = [&](const f32x4& w, int n) {
+            float value[4];
+            f32x4 mixed = {0.f, 0.f, 0.f, 0.f};
             unsigned most = 0;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) most = max(most, __float_as_uint(l.value[i]) & 0x7FFFFFFFu);
-            if (__builtin_amdgcn_ballot_w64(most >= 0x7F800000u) != 0) {        // token by token, each for its own row and those behind it
+            for (int i = 0; i < 4; ++i) {
+                value[i] = shared_value[n][4 * (wave & 1) + i][lane];
+                most = max(most, __float_as_uint(value[i]) & 0x7FFFFFFFu);
+            }
+#pragma unroll
+            for (int i = 0; i < 4; ++i) mixed = mfma4(value[i], w[i], mixed);
+            if (__builtin_expect(__builtin_amdgcn_ballot_w64(most >= 0x7F800000u) != 0, 0)) {       // token by token, each for its own row and those behind it
                 mixed = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int s = 0; s < 16; ++s) {
-                    const float value = __shfl(l.value[s & 3], (s >> 2) * 16 + row, kWave);
+                    const float by = __shfl(w[s & 3], (s >> 2) * 16 + row, kWave);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
-                        const int to = 4 * quad + i;
-                        const float w = __shfl(l.mix[s & 3], (s >> 2) * 16 + to, kWave);
-                        if (s <= to + 16 * ((wave >> 1) - (wave & 1))) mixed[i] = fmaf(w, value, mixed[i]);
+                        const float of = __shfl(value[s & 3], (s >> 2) * 16 + 4 * quad + i, kWave);
+                        if (s <= row + 16 * ((wave >> 1) - (wave & 1))) mixed[i] = fmaf(by, of, mixed[i]);
                     }
                 }
             }
+            return mixed;
+        };
+        f32x4 mixed;
+        auto work = [&](const Loaded& l, const Loaded& next, Loaded& coming, int c, auto turn3) {
+            constexpr int n = decltype(turn3)::value;       // c % 3
+            const int turn = c & 1;
+            const float* rec = record_of(c + 2);
+            constexpr int EVERY = 4 * TT * KT / (LOADS + 1);
+            static_assert(EVERY >= 1, "a product for every load");
+            auto ask_all = [&]() {
+                pin();
+#pragma unroll
+                for (int l = 0; l < LOADS; ++l) fetch_one(coming, rec, l);
+                raw[(n + 1) % 3] = fetch_value(c + 4);
+                pin();
+            };
+            auto between = [&](int product) {
+                if constexpr (!SPREAD) return;
+                pin();
+                if (product % EVERY == 0 && product / EVERY <= LOADS) {
+                    if (product == 0) raw[(n + 1) % 3] = fetch_value(c + 4);
+                    else fetch_one(coming, rec, product / EVERY - 1);
+                    pin();
+                }
+            };
+            if constexpr (!SPREAD) ask_all();
+            shared_value[(n + 2) % 3][all][lane] = raw[(n + 2) % 3];
+            meet();                                         // the state before chunk c is there, and chunk c - 1's parts
+            f32x4 S[KT], o[TT];
+#pragma unroll
+            for (int k = 0; k < KT; ++k) S[k] = states[turn][wave][k][lane];
+#pragma unroll
+            for (int t = 0; t < TT; ++t) o[t] = f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+            for (int k = 0; k < KT; ++k)
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int t = 0; t < TT; ++t) {
+                        o[t] = mfma4(S[k][i], l.read[t][k][i], o[t]);
+                        between((k * 4 + i) * TT + t);
+                    }
+            const f32x4 mixed_next = mix(next.mix, (n + 1) % 3);
+            if (c > 0) write(c - 1);
 #pragma unroll
             for (int t = 0; t < TT; ++t) {
 #pragma unroll
                 for (int i = 0; i < 4; ++i) o[t][i] += wave >> 1 == t ? mixed[i] : 0.f;
                 reads[turn][wave][t][lane] = o[t];
             }
-        };
-        // chunk c's read-outs, two of a tile's rows a wave, once every wave has left its part
-        float* to = out + (size_t)first * line + (size_t)head * dv;
-        const int t = wave & 1, half = wave >> 1;
-        auto write = [&](int c) {
-            const float2* part = reinterpret_cast<const float2*>(&reads[c & 1][0][t][lane]) + half;
-            constexpr int NEXT = TT * kWave * 2;            // float2s from a wave's part to the next one's
-            const float2 p = part[0], q = part[NEXT], r = part[2 * NEXT], s = part[3 * NEXT];
-            const int token = 16 * t + 4 * quad + 2 * half, count = last - first - c * SC;
-            float* at = to + (size_t)(c * SC) * line;
-            if (mine && token < count) at[__umul24(token, line) + j] = (p.x + q.x) + (r.x + s.x);
-            if (mine && token + 1 < count) at[__umul24(token + 1, line) + j] = (p.y + q.y) + (r.y + s.y);
+            mixed = mixed_next;
         };
         Loaded sets[3];
         fetch(sets[0], 0);
         fetch(sets[1], 1);
+        meet();
+        mixed = mix(sets[0].mix, 0);
+        auto turn = [&](int c, auto turn3) {
+            constexpr int n = decltype(turn3)::value;
+            work(sets[n], sets[(n + 1) % 3], sets[(n + 2) % 3], c, turn3);
+        };
         for (int c = 0;;) {
-            fetch(sets[2], c + 2);
-            work(sets[0], c);
-            if (c > 0) write(c - 1);
+            turn(c, std::integral_constant<int, 0>{});
             if (++c == chunks) break;
-            fetch(sets[0], c + 2);
-            work(sets[1], c);
-            write(c - 1);
+            turn(c, std::integral_constant<int, 1>{});
             if (++c == chunks) break;
-            fetch(sets[1], c + 2);
-            work(sets[2], c);
-            write(c - 1);
+            turn(c, std::integral_constant<int, 2>{});
             if (++c == chunks) break;
         }
         meet();

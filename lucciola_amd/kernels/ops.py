@@ -2232,7 +2232,8 @@ class ScanPortions:
 # (planes, key channels) -> us: token by token (before the first token, a token of the longest request, a token and 16 value channels
 # of a head, a million entries of state); in chunks (before the first chunk, a token of the longest request, a token and head, a token and
 # 16 value channels of a head).  Fitted to 1,876 steps of 64 to 2,600 tokens in portions of 64 to 640 beside none to 200 lone or short
-# requests, 2 to 32 heads of 16 to 257 value channels; eight of ten are within 13 % of their time.
+# requests, 2 to 32 heads of 16 to 257 value channels; eight of ten are within 13 % of their time (the walk over chunks has got up to
+# a sixth faster since: the line errs towards token by token).
 _SCAN_TIMES = {
     (3, 64): ((4.4, 0.162, 2.25e-4, 1.69), (12.0, 0.0235, 4.24e-4, 1.00e-4)),
     (3, 128): ((0.8, 0.249, 4.44e-4, 1.48), (14.2, 0.0392, 4.70e-4, 2.06e-4)),
@@ -2246,7 +2247,7 @@ def scan_chunks_pay(portions: ScanPortions, planes: int, heads: int, key_dim: in
     CUs.  Token by token a step is its longest request's chain (half as long again a token where the requests bring fewer than 16 tokens
     each: the shallower kernel), or the states' and tokens' trips where these are longer; the chunks' kernels take that one's place
     for the portions, but the other requests then follow in a launch of their own.  16 heads of 128 x 128, five planes, us token by
-    token and in chunks: one portion of 64 tokens 19 and 21, of 96 31 and 24, of 2,048 590 and 185; beside 64 lone tokens 64 46 and 62, 128
+    token and in chunks: one portion of 64 tokens 19 and 21, of 96 31 and 24, of 2,048 590 and 162; beside 64 lone tokens 64 46 and 62, 128
     68 and 63, 256 119 and 72; beside 200 lone tokens 192 120 and 142, 384 204 and 161; 16 portions of 64 120 and 100.  The chunks have
     to gain an eighth: where decays leave their range (known to the kernel alone) their first pass takes up to twice its time."""
     (start, token, work, state), (c_start, c_token, c_head, c_work) = _SCAN_TIMES[planes, key_dim]

@@ -205,3 +205,11 @@ def test_decays_around_the_range(planes, dk, where, exponent):
     for t in range(T):
         error, beside = (float((x[t] - want[t]).norm()) for x in (got, plain))
         assert error <= max(4 * beside, 2 * UNIT * float(reach[t].norm())), t
+
+
+# every number of chunks modulo the walk's three turns, and value channels stored four at a time or, where a row is no whole 16 bytes, one
+# by one, with the last block of 16 channels partly filled either way
+@pytest.mark.parametrize("planes", [5, 3])
+@pytest.mark.parametrize("dk,dv", [(128, 20), (128, 50), (64, 36), (64, 130)])
+def test_turns_and_columns(planes, dk, dv):
+    test_chunks(planes, "by channel", 2, dk, dv, [64, 65, 97, 129, 161, 193, 225])
