@@ -2,7 +2,7 @@
 //     S <- diag(decay) S - removal (probe^T S) + write v^T,    o = S^T read,
 // for portions of prompts, a chunk of SC = 32 tokens at a time on the float32 matrix instruction.  Token by token a step
 // is a chain of dependent vector instructions, 0.21 us a token without and 0.29 us with the removal term, on a wave that
-// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 89 and 162).
+// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 84 and 162).
 //
 // Inside a chunk, from the state S that the chunk before left, with a_i the product of the decays of tokens 0..i (key
 // channel by key channel), r_ij that of the tokens j+1..i, and y_i = probe_i^T S_(i-1) what token i takes out:
@@ -81,15 +81,22 @@ __device__ __forceinline__ f32x4 tile_product(A a, B b) {
     return c[0];
 }
 
-// grid (records, heads).  coef [5 or 3][T, heads DK] as delta_rule.hip has it.  alone [records][heads][8]: not all zero where the
-// chunk holds what has to go token by token, and its record is not to be used.  2,048 tokens, 16 heads of 128: 26 us, and with
-// a removal term, where a workgroup fills its CU's LDS and its steps follow each other, 63 us.
+// A record of a head is an item; a workgroup takes every gridDim.x-th.  coef [5 or 3][T, heads DK] as delta_rule.hip has it.  alone
+// [records][heads][8]: not all zero where the chunk holds what has to go token by token, and its record is not to be used.
+// An item asks for the next one's vectors before it makes its pairs, so that loads, products and stores of a CU pass beside each other (with
+// a workgroup an item they follow each other; 2,048 tokens, 16 heads of 128 28 -> 21 us, 32 heads 53 -> 40, which is 4.4 TB/s; two workgroups a
+// CU, four for heads of 64 without removal, are what its LDS and registers hold and measured best of one to four).  With heads of 128 and
+// a removal term a workgroup fills its CU's LDS, has no registers for another item's vectors (29 of them spilled: 66 us against 63) and
+// its steps follow each other: 63 us for 2,048 tokens and 16 heads, 16 us an item, of which the trips to memory are half.
+template <int DK, bool REMOVE> constexpr bool prepare_turns = !(REMOVE && DK == 128);
+
 template <int DK, bool REMOVE, int THREADS>
 __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float* __restrict__ coef,
                                                                      const int* __restrict__ q_offsets, int R, int T,
-                                                                     int heads, int least, float* __restrict__ records,
+                                                                     int heads, int least, int items, float* __restrict__ records,
                                                                      unsigned char* __restrict__ alone) {
     typedef ChunkRecord<DK, REMOVE> Rec;
+    constexpr bool TURNS = prepare_turns<DK, REMOVE>;
     constexpr int DKP = DK + 4, WAVES = THREADS / kWave, NP = REMOVE ? 5 : 3;
     constexpr int DECAY = 0, PROBE = 1, REMOVAL = 2, WRITE = REMOVE ? 3 : 1, READ = REMOVE ? 4 : 2;
     constexpr int MATS = REMOVE ? 4 : 1;                    // W = read x write, R = read x removal, M = probe x write, L = probe x removal
@@ -98,33 +105,78 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     __shared__ __attribute__((aligned(16))) float inverse[REMOVE ? SC : 1][SCP], scratch[REMOVE ? 16 : 1][20];
     __shared__ __attribute__((aligned(16))) float total[2][DK];     // a block's decay
     __shared__ double whole[2][DK];
-    const int tid = threadIdx.x, wave = tid / kWave, lane = tid % kWave, row = lane & 15, quad = lane >> 4;
-    const int record = blockIdx.x, head = blockIdx.y;
-    int low = 0, high = R - 1;                              // the request whose records hold this one
-    while (low < high) {
-        const int mid = (low + high + 1) / 2;
-        if (first_record(q_offsets, mid, least) <= record) low = mid;
-        else high = mid - 1;
-    }
-    const int last = q_offsets[low + 1], t0 = q_offsets[low] + (record - first_record(q_offsets, low, least)) * SC;
-    if (t0 >= last || last - q_offsets[low] < least) return;
-    const int count = min(SC, last - t0);
-    float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
-
+    __shared__ int far_waves[WAVES];
+    // only LDS has to be in order between the waves: loads and stores of memory stay in flight
+    auto meet = []() {
+        asm volatile("" ::: "memory");
+        wait_lgkmcnt<0>();
+        __builtin_amdgcn_s_barrier();
+        asm volatile("" ::: "memory");
+    };
+    // where an item's chunk begins and its tokens; 0: the record is nobody's
+    struct Chunk { int record, head, t0, count; };
+    auto chunk_of = [&](int item) {
+        Chunk c{item / heads, item % heads, 0, 0};
+        int low = 0, high = R - 1;                          // the request whose records hold this one
+        while (low < high) {
+            const int mid = (low + high + 1) / 2;
+            if (first_record(q_offsets, mid, least) <= c.record) low = mid;
+            else high = mid - 1;
+        }
+        const int last = q_offsets[low + 1];
+        c.t0 = q_offsets[low] + (c.record - first_record(q_offsets, low, least)) * SC;
+        if (c.t0 < last && last - q_offsets[low] >= least) c.count = min(SC, last - c.t0);
+        return c;
+    };
     // the chunk's vectors; a place behind the request's end keeps the state and adds nothing
-    unsigned most = 0;                                      // the largest entry's bits: NaN and infinity lie above all numbers
-    for (int idx = tid; idx < NP * SC * (DK / 4); idx += THREADS) {
-        const int i = idx % (DK / 4), t = idx / (DK / 4) % SC, p = idx / (DK / 4 * SC);
-        const float pad = p == DECAY ? 1.f : 0.f;
-        f32x4 x = {pad, pad, pad, pad};
-        if (t < count) x = *reinterpret_cast<const f32x4*>(coef + ((size_t)p * T + t0 + t) * heads * DK + (size_t)head * DK + 4 * i);
+    constexpr int PIECES = NP * SC * (DK / 4) / THREADS, TOKENS = THREADS / (DK / 4);        // 16 bytes each; tokens a pass of all threads
+    static_assert(SC % TOKENS == 0 && PIECES * TOKENS == NP * SC, "whole passes, each within a plane");
+    f32x4 held[PIECES];
+    auto ask = [&](const Chunk& c) {
+        const int tid = threadIdx.x;
+        const float* from = coef + ((size_t)c.t0 * heads + c.head) * DK;
+        asm volatile("" : "+s"(from));
+        const int t = tid / (DK / 4);
 #pragma unroll
-        for (int e = 0; e < 4; ++e) most = max(most, __float_as_uint(x[e]) & 0x7FFFFFFFu);
-        *reinterpret_cast<f32x4*>(&plane[p][t][4 * i]) = x;
+        for (int n = 0; n < PIECES; ++n) {
+            const int p = n * TOKENS / SC, first = n * TOKENS % SC;
+            const float pad = p == DECAY ? 1.f : 0.f;
+            held[n] = f32x4{pad, pad, pad, pad};
+            const float* row = from + ((size_t)p * T + first) * heads * DK;
+            if (first + t < c.count) held[n] = *reinterpret_cast<const f32x4*>(row + (unsigned)(t * heads * DK + tid % (DK / 4) * 4));
+        }
+        asm volatile("" ::: "memory");
+        __builtin_amdgcn_sched_barrier(0);
+    };
+    Chunk chunk = chunk_of(blockIdx.x);
+    ask(chunk);
+    for (int item = blockIdx.x; item < items; item += gridDim.x) {
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));                           // places in LDS are worked out when they are wanted: kept for all turns they spill
+    const int wave = tid / kWave, lane = tid % kWave, row = lane & 15, quad = lane >> 4;
+    const int record = chunk.record, head = chunk.head, count = chunk.count;
+    auto ask_next = [&]() {
+        if (TURNS && item + (int)gridDim.x < items) {
+            chunk = chunk_of(item + gridDim.x);
+            ask(chunk);
+        }
+    };
+    if (count == 0) {
+        ask_next();
+        continue;
+    }
+    float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
+    meet();                                                 // nobody reads the chunk before any more
+    unsigned most = 0;                                      // the largest entry's bits: NaN and infinity lie above all numbers
+#pragma unroll
+    for (int n = 0; n < PIECES; ++n) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) most = max(most, __float_as_uint(held[n][e]) & 0x7FFFFFFFu);
+        *reinterpret_cast<f32x4*>(&plane[n * TOKENS / SC][n * TOKENS % SC + tid / (DK / 4)][tid % (DK / 4) * 4]) = held[n];
     }
     const bool odd = __builtin_amdgcn_ballot_w64(most > __float_as_uint(SC_MOST)) != 0;
     if (lane < 8 / WAVES) alone[((size_t)record * heads + head) * 8 + wave * (8 / WAVES) + lane] = odd;
-    __syncthreads();
+    meet();
 
     // every vector at its block's border.  A thread is a key channel of a block, and of the reading (read, probe) or the
     // writing side (write, removal); the products of the decays are made in 64 bits and rounded once.
@@ -149,7 +201,13 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     // products of the vectors times and over the decays from the block's first token on, on the matrix instruction: a division
     // by what is far from the smallest number loses nothing.  Else the pairs are made one by one, by vector instructions,
     // several times as long.
-    const bool far = __syncthreads_or(!(least_through >= 0x1p-60 && most_through <= 0x1p60 && through == through));
+    const bool far_here = __builtin_amdgcn_ballot_w64(!(least_through >= 0x1p-60 && most_through <= 0x1p60 && through == through)) != 0;
+    if (lane == 0) far_waves[wave] = far_here;
+    meet();
+    bool far = false;
+#pragma unroll
+    for (int n = 0; n < WAVES; ++n) far |= far_waves[n] != 0;
+    far = __builtin_amdgcn_readfirstlane(far);
     const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
     auto put = [&](float (*to)[SCP], int r0, int c0, f32x4 v) {
 #pragma unroll
@@ -209,7 +267,7 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
                 }
             }
         }
-        __syncthreads();
+        meet();
     }
     // far: read and probe from the block's first token on, write and removal to its last; else those over the decays
     auto scale_reading = [&]() {
@@ -232,7 +290,7 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     };
     if (side == 0) scale_reading();
     if (side == SIDES - 1) scale_writing();
-    __syncthreads();
+    meet();
 
     // pairs between the two blocks (nothing of the second reaches the first), and, unless they are there, inside them
     auto rows_of = [&](int p, int first) { return [&, p, first](int t) { return along(&plane[p][0][0], DKP, first, 16 * t); }; };
@@ -259,8 +317,9 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
             put(mat[m], base, base, v);
         }
     }
-    __syncthreads();
+    meet();
 
+    ask_next();
     // from the chunk's first token on, and to its last
     for (int idx = tid; idx < 16 * DK; idx += THREADS) {
         const int i = idx / DK, k = idx % DK;
@@ -281,7 +340,7 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
         out[Rec::DECAY + DK + k] = (float)(d - (double)near);
     }
 
-    __syncthreads();
+    meet();
     constexpr int KEYS = DK / 16, TILES = 2 * KEYS;
     if constexpr (REMOVE) {
         const float *W = mat[0][0], *Rm = mat[1][0], *M = mat[2][0], *L = mat[3][0];
@@ -303,18 +362,18 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
                 if (base) inverse[i][16 + c] = 0.f;
             }
         }
-        __syncthreads();
+        meet();
         // T10 = -T11 L10 T00
         if (wave == 0) {
             const f32x4 lt = tile_product<1>([&](int) { return along(L, SCP, 16, 0); }, [&](int) { return down(inv, SCP, 0, 0); });
 #pragma unroll
             for (int i = 0; i < 4; ++i) scratch[4 * quad + i][row] = -lt[i];
         }
-        __syncthreads();
+        meet();
         if (wave == 0)
             put(inverse, 16, 0, tile_product<1>([&](int) { return along(inv, SCP, 16, 16); },
                                                 [&](int) { return down(scratch[0], 20, 0, 0); }));
-        __syncthreads();
+        meet();
         // T M over M's place (kept in registers until everybody has read M); T probe~, transposed, over the decays
         f32x4 tm = zero;
         if (wave < 4)
@@ -327,9 +386,9 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
             *reinterpret_cast<f32x4*>(&plane[DECAY][t0 + row][k0 + 4 * quad]) = v;
             keep_tile(Rec::PROBE, tile, v);
         }
-        __syncthreads();
+        meet();
         if (wave < 4) put(mat[2], 16 * (wave >> 1), 16 * (wave & 1), tm);
-        __syncthreads();
+        meet();
         // read^ = read~ - R (T probe~);  Z = write~^T - removal~^T (T M);  W^ = W - R (T M): each transposed, as a lane's entries lie
         for (int tile = wave; tile < TILES; tile += WAVES) {
             const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
@@ -356,7 +415,7 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
             keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, 16 * (tile % 2), 16 * (tile / 2)));
         }
         for (int tile = wave; tile < 4; tile += WAVES) keep_tile(Rec::MIX, tile, along(mat[0][0], SCP, 16 * (tile >> 1), 16 * (tile & 1)));
-    }
+    }    }
 }
 
 // The recurrence as it stands, for 16 value channels: 32 lanes a channel, DK / 32 key rows a lane.
@@ -754,8 +813,9 @@ static void scan_chunks(const float* coef, const float* v, float* state, float* 
     constexpr int THREADS = REMOVE ? 4 * DK : 2 * DK;
     const int places = record_places(T, R, least);
     float* alone = records + (size_t)places * heads * ChunkRecord<DK, REMOVE>::SIZE;
-    scan_chunk_prepare_kernel<DK, REMOVE, THREADS>
-        <<<dim3(places, heads), THREADS, 0, stream>>>(coef, q_offsets, R, T, heads, least, records, reinterpret_cast<unsigned char*>(alone));
+    const int items = places * heads, at_once = prepare_turns<DK, REMOVE> ? device_cus() * (DK == 64 && !REMOVE ? 4 : 2) : items;
+    scan_chunk_prepare_kernel<DK, REMOVE, THREADS><<<min(items, at_once), THREADS, 0, stream>>>(coef, q_offsets, R, T, heads, least, items, records,
+                                                                                                reinterpret_cast<unsigned char*>(alone));
     scan_chunk_walk_kernel<DK, REMOVE><<<dim3(heads * ((dv + 15) / 16), R), 512, 0, stream>>>(
         records, reinterpret_cast<const uint2*>(alone), coef, v, state, out, q_offsets, slot_ids, T, heads, dv, least);
 }

@@ -213,3 +213,23 @@ def test_decays_around_the_range(planes, dk, where, exponent):
 @pytest.mark.parametrize("dk,dv", [(128, 20), (128, 50), (64, 36), (64, 130)])
 def test_turns_and_columns(planes, dk, dv):
     test_chunks(planes, "by channel", 2, dk, dv, [64, 65, 97, 129, 161, 193, 225])
+
+
+# more records than workgroups at once, so that these take several, ones that nobody owns among them: a head's results are those of a step that
+# has this head alone, to the bit
+@pytest.mark.parametrize("planes,dk", [(3, 128), (3, 64), (5, 64), (5, 128)])
+def test_records_in_turns(planes, dk):
+    heads, dv, lengths = 30, 16, [900, 2, 70, 500, 1, 65]
+    g = torch.Generator().manual_seed(planes + dk)
+    T, R = sum(lengths), len(lengths)
+    coef = vectors("by channel", T, heads, dk, g)[0 if planes == 5 else 1].to(DEV)
+    v, state = torch.randn(T, heads * dv, generator=g).to(DEV), torch.randn(R, heads, dv, dk, generator=g).to(DEV)
+    lists = torch.tensor([0] + torch.tensor(lengths).cumsum(0).tolist(), dtype=torch.int32, device=DEV), torch.arange(R, dtype=torch.int32, device=DEV)
+    whole = state.clone()
+    out = ops.delta_scan_chunks(coef, v, whole, *lists, R, heads, dk, dv, some_short=True)
+    for head in (0, 17, heads - 1):
+        one = state[:, head:head + 1].contiguous()
+        got = ops.delta_scan_chunks(coef[..., head * dk:(head + 1) * dk].contiguous(), v[:, head * dv:(head + 1) * dv].contiguous(), one, *lists,
+                                    R, 1, dk, dv, some_short=True)
+        assert torch.equal(got, out[:, head * dv:(head + 1) * dv]), "read-outs"
+        assert torch.equal(one[:, 0], whole[:, head]), "states"
