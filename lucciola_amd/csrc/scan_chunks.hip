@@ -87,7 +87,8 @@ __device__ __forceinline__ f32x4 tile_product(A a, B b) {
 // a workgroup an item they follow each other; 2,048 tokens, 16 heads of 128 28 -> 21 us, 32 heads 53 -> 40, which is 4.4 TB/s; two workgroups a
 // CU, four for heads of 64 without removal, are what its LDS and registers hold and measured best of one to four).  With heads of 128 and
 // a removal term a workgroup fills its CU's LDS, has no registers for another item's vectors (29 of them spilled: 66 us against 63) and
-// its steps follow each other: 63 us for 2,048 tokens and 16 heads, 16 us an item, of which the trips to memory are half.
+// its steps follow each other: 63 us for 2,048 tokens and 16 heads, 16 us an item, whose 155 KB
+// in and out take half of that at the rate of a copy.
 template <int DK, bool REMOVE> constexpr bool prepare_turns = !(REMOVE && DK == 128);
 
 template <int DK, bool REMOVE, int THREADS>
@@ -151,271 +152,272 @@ __global__ __launch_bounds__(THREADS) void scan_chunk_prepare_kernel(const float
     Chunk chunk = chunk_of(blockIdx.x);
     ask(chunk);
     for (int item = blockIdx.x; item < items; item += gridDim.x) {
-    int tid = threadIdx.x;
-    asm volatile("" : "+v"(tid));                           // places in LDS are worked out when they are wanted: kept for all turns they spill
-    const int wave = tid / kWave, lane = tid % kWave, row = lane & 15, quad = lane >> 4;
-    const int record = chunk.record, head = chunk.head, count = chunk.count;
-    auto ask_next = [&]() {
-        if (TURNS && item + (int)gridDim.x < items) {
-            chunk = chunk_of(item + gridDim.x);
-            ask(chunk);
-        }
-    };
-    if (count == 0) {
-        ask_next();
-        continue;
-    }
-    float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
-    meet();                                                 // nobody reads the chunk before any more
-    unsigned most = 0;                                      // the largest entry's bits: NaN and infinity lie above all numbers
-#pragma unroll
-    for (int n = 0; n < PIECES; ++n) {
-#pragma unroll
-        for (int e = 0; e < 4; ++e) most = max(most, __float_as_uint(held[n][e]) & 0x7FFFFFFFu);
-        *reinterpret_cast<f32x4*>(&plane[n * TOKENS / SC][n * TOKENS % SC + tid / (DK / 4)][tid % (DK / 4) * 4]) = held[n];
-    }
-    const bool odd = __builtin_amdgcn_ballot_w64(most > __float_as_uint(SC_MOST)) != 0;
-    if (lane < 8 / WAVES) alone[((size_t)record * heads + head) * 8 + wave * (8 / WAVES) + lane] = odd;
-    meet();
-
-    // every vector at its block's border.  A thread is a key channel of a block, and of the reading (read, probe) or the
-    // writing side (write, removal); the products of the decays are made in 64 bits and rounded once.
-    constexpr int SIDES = THREADS / (2 * DK);
-    static_assert(SIDES >= 1, "a thread a channel of a block");
-    const int block = tid / DK % 2, channel = tid % DK, side = tid / (2 * DK);
-    float decay[16];
-#pragma unroll
-    for (int i = 0; i < 16; ++i) decay[i] = plane[DECAY][16 * block + i][channel];
-    double through = 1.0, least_through = 1.0, most_through = 1.0;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) {
-        through *= (double)decay[i];
-        least_through = fmin(least_through, through);
-        most_through = fmax(most_through, through);
-    }
-    if (side == 0) {
-        whole[block][channel] = through;
-        total[block][channel] = (float)through;
-    }
-    // Where no channel's decays multiply to less than 2^-60 or more than 2^60 anywhere in the 16 tokens, the pairs of a block are
-    // products of the vectors times and over the decays from the block's first token on, on the matrix instruction: a division
-    // by what is far from the smallest number loses nothing.  Else the pairs are made one by one, by vector instructions,
-    // several times as long.
-    const bool far_here = __builtin_amdgcn_ballot_w64(!(least_through >= 0x1p-60 && most_through <= 0x1p60 && through == through)) != 0;
-    if (lane == 0) far_waves[wave] = far_here;
-    meet();
-    bool far = false;
-#pragma unroll
-    for (int n = 0; n < WAVES; ++n) far |= far_waves[n] != 0;
-    far = __builtin_amdgcn_readfirstlane(far);
-    const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
-    auto put = [&](float (*to)[SCP], int r0, int c0, f32x4 v) {
-#pragma unroll
-        for (int i = 0; i < 4; ++i) to[r0 + 4 * quad + i][c0 + row] = v[i];
-    };
-    auto keep_tile = [&](int matrix, int tile, f32x4 v) { *reinterpret_cast<f32x4*>(out + matrix + tile * 256 + lane * 4) = v; };
-    // four neighbouring entries of the lane's row of a matrix or plane, and of its column
-    auto along = [&](const float* m, int pitch, int r0, int c0) { return *reinterpret_cast<const f32x4*>(m + (r0 + row) * pitch + c0 + 4 * quad); };
-    auto down = [&](const float* m, int pitch, int r0, int c0) {
-        f32x4 v;
-#pragma unroll
-        for (int i = 0; i < 4; ++i) v[i] = m[(r0 + 4 * quad + i) * pitch + c0 + row];
-        return v;
-    };
-    if (far) {
-        // lane (j, quad) carries write_j and removal_j through the decays of the tokens behind j, for every fourth group of
-        // four key channels, and meets read_i or probe_i (which does not see token i's decay) on the way
-        constexpr int ROLES = REMOVE ? 4 : 2;               // (block, read or probe)
-        constexpr int G = DK / 16;
-        static_assert(WAVES >= ROLES, "a wave a role");
-        if (wave < ROLES) {
-            const int base = 16 * (wave & 1);
-            const bool by_probe = wave >= 2;
-            f32x4 w[G], x[REMOVE ? G : 1];
-#pragma unroll
-            for (int m = 0; m < G; ++m) {
-                w[m] = *reinterpret_cast<const f32x4*>(&plane[WRITE][base + row][16 * m + 4 * quad]);
-                if constexpr (REMOVE) x[m] = *reinterpret_cast<const f32x4*>(&plane[REMOVAL][base + row][16 * m + 4 * quad]);
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));                           // places in LDS are worked out when they are wanted: kept for all turns they spill
+        const int wave = tid / kWave, lane = tid % kWave, row = lane & 15, quad = lane >> 4;
+        const int record = chunk.record, head = chunk.head, count = chunk.count;
+        auto ask_next = [&]() {
+            if (TURNS && item + (int)gridDim.x < items) {
+                chunk = chunk_of(item + gridDim.x);
+                ask(chunk);
             }
-            for (int i = 0; i < 16; ++i) {
-                const int from = by_probe ? i - 1 : i;      // the last decay that the reader sees
-                float with_w = 0.f, with_x = 0.f;
-                const float* by = &plane[REMOVE && by_probe ? PROBE : READ][base + i][4 * quad];
-                const float* keep = &plane[DECAY][base + max(from, 0)][4 * quad];
-#pragma unroll
-                for (int m = 0; m < G; ++m) {
-                    const f32x4 d = *reinterpret_cast<const f32x4*>(keep + 16 * m), q = *reinterpret_cast<const f32x4*>(by + 16 * m);
-#pragma unroll
-                    for (int e = 0; e < 4; ++e) {
-                        const float f = from > row ? d[e] : 1.f;
-                        w[m][e] *= f;
-                        with_w = fmaf(q[e], w[m][e], with_w);
-                        if constexpr (REMOVE) {
-                            x[m][e] *= f;
-                            with_x = fmaf(q[e], x[m][e], with_x);
-                        }
-                    }
-                }
-                with_w += __shfl_xor(with_w, 16, kWave);
-                with_w += __shfl_xor(with_w, 32, kWave);
-                const bool seen = by_probe ? row < i : row <= i;
-                if (quad == 0) mat[REMOVE && by_probe ? 2 : 0][base + i][base + row] = seen ? with_w : 0.f;
-                if constexpr (REMOVE) {
-                    with_x += __shfl_xor(with_x, 16, kWave);
-                    with_x += __shfl_xor(with_x, 32, kWave);
-                    if (quad == 0) mat[by_probe ? 3 : 1][base + i][base + row] = seen ? with_x : 0.f;
-                }
-            }
+        };
+        if (count == 0) {
+            ask_next();
+            continue;
         }
+        float* out = records + ((size_t)record * heads + head) * Rec::SIZE;
+        meet();                                                 // nobody reads the chunk before any more
+        unsigned most = 0;                                      // the largest entry's bits: NaN and infinity lie above all numbers
+#pragma unroll
+        for (int n = 0; n < PIECES; ++n) {
+#pragma unroll
+            for (int e = 0; e < 4; ++e) most = max(most, __float_as_uint(held[n][e]) & 0x7FFFFFFFu);
+            *reinterpret_cast<f32x4*>(&plane[n * TOKENS / SC][n * TOKENS % SC + tid / (DK / 4)][tid % (DK / 4) * 4]) = held[n];
+        }
+        const bool odd = __builtin_amdgcn_ballot_w64(most > __float_as_uint(SC_MOST)) != 0;
+        if (lane < 8 / WAVES) alone[((size_t)record * heads + head) * 8 + wave * (8 / WAVES) + lane] = odd;
         meet();
-    }
-    // far: read and probe from the block's first token on, write and removal to its last; else those over the decays
-    auto scale_reading = [&]() {
-        double a = 1.0;
+
+        // every vector at its block's border.  A thread is a key channel of a block, and of the reading (read, probe) or the
+        // writing side (write, removal); the products of the decays are made in 64 bits and rounded once.
+        constexpr int SIDES = THREADS / (2 * DK);
+        static_assert(SIDES >= 1, "a thread a channel of a block");
+        const int block = tid / DK % 2, channel = tid % DK, side = tid / (2 * DK);
+        float decay[16];
+#pragma unroll
+        for (int i = 0; i < 16; ++i) decay[i] = plane[DECAY][16 * block + i][channel];
+        double through = 1.0, least_through = 1.0, most_through = 1.0;
 #pragma unroll
         for (int i = 0; i < 16; ++i) {
-            if constexpr (REMOVE) plane[PROBE][16 * block + i][channel] *= (float)a;
-            a *= (double)decay[i];
-            plane[READ][16 * block + i][channel] *= (float)a;
+            through *= (double)decay[i];
+            least_through = fmin(least_through, through);
+            most_through = fmax(most_through, through);
         }
-    };
-    auto scale_writing = [&]() {
-        double a = far ? 1.0 : 1.0 / through;
-#pragma unroll
-        for (int i = 15; i >= 0; --i) {
-            plane[WRITE][16 * block + i][channel] *= (float)a;
-            if constexpr (REMOVE) plane[REMOVAL][16 * block + i][channel] *= (float)a;
-            a *= (double)decay[i];
+        if (side == 0) {
+            whole[block][channel] = through;
+            total[block][channel] = (float)through;
         }
-    };
-    if (side == 0) scale_reading();
-    if (side == SIDES - 1) scale_writing();
-    meet();
-
-    // pairs between the two blocks (nothing of the second reaches the first), and, unless they are there, inside them
-    auto rows_of = [&](int p, int first) { return [&, p, first](int t) { return along(&plane[p][0][0], DKP, first, 16 * t); }; };
-    for (int role = wave; role < MATS * 3; role += WAVES) {
-        const int m = role % MATS, tile = role / MATS;      // tile 0: between; 1, 2: inside
-        const bool probes = REMOVE && m >= 2;
-        const int by = probes ? PROBE : READ, with = REMOVE && (m & 1) ? REMOVAL : WRITE;
-        if (tile == 0) {
-            auto lasting = [&](int t) {
-                f32x4 v = rows_of(with, 0)(t);
-                if (!far) v *= *reinterpret_cast<const f32x4*>(&total[0][16 * t + 4 * quad]);
-                return v;
-            };
-            put(mat[m], 16, 0, tile_product<DK / 16>(rows_of(by, 16), lasting));
-            put(mat[m], 0, 16, zero);
-        } else if (!far) {
-            const int base = 16 * (tile - 1);
-            f32x4 v = tile_product<DK / 16>(rows_of(by, base), rows_of(with, base));
+        // Where no channel's decays multiply to less than 2^-60 or more than 2^60 anywhere in the 16 tokens, the pairs of a block are
+        // products of the vectors times and over the decays from the block's first token on, on the matrix instruction: a division
+        // by what is far from the smallest number loses nothing.  Else the pairs are made one by one, by vector instructions,
+        // several times as long.
+        const bool far_here = __builtin_amdgcn_ballot_w64(!(least_through >= 0x1p-60 && most_through <= 0x1p60 && through == through)) != 0;
+        if (lane == 0) far_waves[wave] = far_here;
+        meet();
+        bool far = false;
 #pragma unroll
-            for (int i = 0; i < 4; ++i) {
-                const int reader = 4 * quad + i;
-                v[i] = (probes ? row < reader : row <= reader) ? v[i] : 0.f;
+        for (int n = 0; n < WAVES; ++n) far |= far_waves[n] != 0;
+        far = __builtin_amdgcn_readfirstlane(far);
+        const f32x4 zero = {0.f, 0.f, 0.f, 0.f};
+        auto put = [&](float (*to)[SCP], int r0, int c0, f32x4 v) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) to[r0 + 4 * quad + i][c0 + row] = v[i];
+        };
+        auto keep_tile = [&](int matrix, int tile, f32x4 v) { *reinterpret_cast<f32x4*>(out + matrix + tile * 256 + lane * 4) = v; };
+        // four neighbouring entries of the lane's row of a matrix or plane, and of its column
+        auto along = [&](const float* m, int pitch, int r0, int c0) { return *reinterpret_cast<const f32x4*>(m + (r0 + row) * pitch + c0 + 4 * quad); };
+        auto down = [&](const float* m, int pitch, int r0, int c0) {
+            f32x4 v;
+#pragma unroll
+            for (int i = 0; i < 4; ++i) v[i] = m[(r0 + 4 * quad + i) * pitch + c0 + row];
+            return v;
+        };
+        if (far) {
+            // lane (j, quad) carries write_j and removal_j through the decays of the tokens behind j, for every fourth group of
+            // four key channels, and meets read_i or probe_i (which does not see token i's decay) on the way
+            constexpr int ROLES = REMOVE ? 4 : 2;               // (block, read or probe)
+            constexpr int G = DK / 16;
+            static_assert(WAVES >= ROLES, "a wave a role");
+            if (wave < ROLES) {
+                const int base = 16 * (wave & 1);
+                const bool by_probe = wave >= 2;
+                f32x4 w[G], x[REMOVE ? G : 1];
+#pragma unroll
+                for (int m = 0; m < G; ++m) {
+                    w[m] = *reinterpret_cast<const f32x4*>(&plane[WRITE][base + row][16 * m + 4 * quad]);
+                    if constexpr (REMOVE) x[m] = *reinterpret_cast<const f32x4*>(&plane[REMOVAL][base + row][16 * m + 4 * quad]);
+                }
+                for (int i = 0; i < 16; ++i) {
+                    const int from = by_probe ? i - 1 : i;      // the last decay that the reader sees
+                    float with_w = 0.f, with_x = 0.f;
+                    const float* by = &plane[REMOVE && by_probe ? PROBE : READ][base + i][4 * quad];
+                    const float* keep = &plane[DECAY][base + max(from, 0)][4 * quad];
+#pragma unroll
+                    for (int m = 0; m < G; ++m) {
+                        const f32x4 d = *reinterpret_cast<const f32x4*>(keep + 16 * m), q = *reinterpret_cast<const f32x4*>(by + 16 * m);
+#pragma unroll
+                        for (int e = 0; e < 4; ++e) {
+                            const float f = from > row ? d[e] : 1.f;
+                            w[m][e] *= f;
+                            with_w = fmaf(q[e], w[m][e], with_w);
+                            if constexpr (REMOVE) {
+                                x[m][e] *= f;
+                                with_x = fmaf(q[e], x[m][e], with_x);
+                            }
+                        }
+                    }
+                    with_w += __shfl_xor(with_w, 16, kWave);
+                    with_w += __shfl_xor(with_w, 32, kWave);
+                    const bool seen = by_probe ? row < i : row <= i;
+                    if (quad == 0) mat[REMOVE && by_probe ? 2 : 0][base + i][base + row] = seen ? with_w : 0.f;
+                    if constexpr (REMOVE) {
+                        with_x += __shfl_xor(with_x, 16, kWave);
+                        with_x += __shfl_xor(with_x, 32, kWave);
+                        if (quad == 0) mat[by_probe ? 3 : 1][base + i][base + row] = seen ? with_x : 0.f;
+                    }
+                }
             }
-            put(mat[m], base, base, v);
+            meet();
         }
-    }
-    meet();
+        // far: read and probe from the block's first token on, write and removal to its last; else those over the decays
+        auto scale_reading = [&]() {
+            double a = 1.0;
+#pragma unroll
+            for (int i = 0; i < 16; ++i) {
+                if constexpr (REMOVE) plane[PROBE][16 * block + i][channel] *= (float)a;
+                a *= (double)decay[i];
+                plane[READ][16 * block + i][channel] *= (float)a;
+            }
+        };
+        auto scale_writing = [&]() {
+            double a = far ? 1.0 : 1.0 / through;
+#pragma unroll
+            for (int i = 15; i >= 0; --i) {
+                plane[WRITE][16 * block + i][channel] *= (float)a;
+                if constexpr (REMOVE) plane[REMOVAL][16 * block + i][channel] *= (float)a;
+                a *= (double)decay[i];
+            }
+        };
+        if (side == 0) scale_reading();
+        if (side == SIDES - 1) scale_writing();
+        meet();
 
-    ask_next();
-    // from the chunk's first token on, and to its last
-    for (int idx = tid; idx < 16 * DK; idx += THREADS) {
-        const int i = idx / DK, k = idx % DK;
-        const float to_border = far ? 1.f : total[0][k], rest = far ? 1.f : total[1][k];
-        plane[READ][16 + i][k] *= total[0][k];
-        plane[WRITE][i][k] *= to_border * total[1][k];
-        plane[WRITE][16 + i][k] *= rest;
+        // pairs between the two blocks (nothing of the second reaches the first), and, unless they are there, inside them
+        auto rows_of = [&](int p, int first) { return [&, p, first](int t) { return along(&plane[p][0][0], DKP, first, 16 * t); }; };
+        for (int role = wave; role < MATS * 3; role += WAVES) {
+            const int m = role % MATS, tile = role / MATS;      // tile 0: between; 1, 2: inside
+            const bool probes = REMOVE && m >= 2;
+            const int by = probes ? PROBE : READ, with = REMOVE && (m & 1) ? REMOVAL : WRITE;
+            if (tile == 0) {
+                auto lasting = [&](int t) {
+                    f32x4 v = rows_of(with, 0)(t);
+                    if (!far) v *= *reinterpret_cast<const f32x4*>(&total[0][16 * t + 4 * quad]);
+                    return v;
+                };
+                put(mat[m], 16, 0, tile_product<DK / 16>(rows_of(by, 16), lasting));
+                put(mat[m], 0, 16, zero);
+            } else if (!far) {
+                const int base = 16 * (tile - 1);
+                f32x4 v = tile_product<DK / 16>(rows_of(by, base), rows_of(with, base));
+#pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    const int reader = 4 * quad + i;
+                    v[i] = (probes ? row < reader : row <= reader) ? v[i] : 0.f;
+                }
+                put(mat[m], base, base, v);
+            }
+        }
+        meet();
+
+        ask_next();
+        // from the chunk's first token on, and to its last
+        for (int idx = tid; idx < 16 * DK; idx += THREADS) {
+            const int i = idx / DK, k = idx % DK;
+            const float to_border = far ? 1.f : total[0][k], rest = far ? 1.f : total[1][k];
+            plane[READ][16 + i][k] *= total[0][k];
+            plane[WRITE][i][k] *= to_border * total[1][k];
+            plane[WRITE][16 + i][k] *= rest;
+            if constexpr (REMOVE) {
+                plane[PROBE][16 + i][k] *= total[0][k];
+                plane[REMOVAL][i][k] *= to_border * total[1][k];
+                plane[REMOVAL][16 + i][k] *= rest;
+            }
+        }
+        for (int k = tid; k < DK; k += THREADS) {
+            const double d = whole[0][k] * whole[1][k];
+            const float near = (float)d;
+            out[Rec::DECAY + k] = near;
+            out[Rec::DECAY + DK + k] = (float)(d - (double)near);
+        }
+
+        meet();
+        constexpr int KEYS = DK / 16, TILES = 2 * KEYS;
         if constexpr (REMOVE) {
-            plane[PROBE][16 + i][k] *= total[0][k];
-            plane[REMOVAL][i][k] *= to_border * total[1][k];
-            plane[REMOVAL][16 + i][k] *= rest;
+            const float *W = mat[0][0], *Rm = mat[1][0], *M = mat[2][0], *L = mat[3][0];
+            float* inv = inverse[0];
+            // T's diagonal blocks: lane (column, block) by forward substitution
+            if (wave == 0 && lane < 32) {
+                const int base = lane & 16, c = lane & 15;
+                float x[16];
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    float s = i == c ? 1.f : 0.f;
+#pragma unroll
+                    for (int j = 0; j < i; ++j) s = fmaf(-L[(base + i) * SCP + base + j], x[j], s);
+                    x[i] = s;
+                }
+#pragma unroll
+                for (int i = 0; i < 16; ++i) {
+                    inverse[base + i][base + c] = x[i];
+                    if (base) inverse[i][16 + c] = 0.f;
+                }
+            }
+            meet();
+            // T10 = -T11 L10 T00
+            if (wave == 0) {
+                const f32x4 lt = tile_product<1>([&](int) { return along(L, SCP, 16, 0); }, [&](int) { return down(inv, SCP, 0, 0); });
+#pragma unroll
+                for (int i = 0; i < 4; ++i) scratch[4 * quad + i][row] = -lt[i];
+            }
+            meet();
+            if (wave == 0)
+                put(inverse, 16, 0, tile_product<1>([&](int) { return along(inv, SCP, 16, 16); },
+                                                    [&](int) { return down(scratch[0], 20, 0, 0); }));
+            meet();
+            // T M over M's place (kept in registers until everybody has read M); T probe~, transposed, over the decays
+            f32x4 tm = zero;
+            if (wave < 4)
+                tm = tile_product<2>([&](int t) { return along(inv, SCP, 16 * (wave >> 1), 16 * t); },
+                                     [&](int t) { return down(M, SCP, 16 * t, 16 * (wave & 1)); });
+            for (int tile = wave; tile < TILES; tile += WAVES) {
+                const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
+                const f32x4 v = tile_product<2>([&](int t) { return down(plane[PROBE][0], DKP, 16 * t, k0); },
+                                                [&](int t) { return along(inv, SCP, t0, 16 * t); });
+                *reinterpret_cast<f32x4*>(&plane[DECAY][t0 + row][k0 + 4 * quad]) = v;
+                keep_tile(Rec::PROBE, tile, v);
+            }
+            meet();
+            if (wave < 4) put(mat[2], 16 * (wave >> 1), 16 * (wave & 1), tm);
+            meet();
+            // read^ = read~ - R (T probe~);  Z = write~^T - removal~^T (T M);  W^ = W - R (T M): each transposed, as a lane's entries lie
+            for (int tile = wave; tile < TILES; tile += WAVES) {
+                const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
+                const f32x4 v = tile_product<2>([&](int t) { return down(plane[DECAY][0], DKP, 16 * t, k0); },
+                                                [&](int t) { return along(Rm, SCP, t0, 16 * t); });
+                keep_tile(Rec::READ, tile, along(plane[READ][0], DKP, t0, k0) - v);
+            }
+            for (int tile = wave; tile < TILES; tile += WAVES) {
+                const int k0 = 16 * (tile / 2), t0 = 16 * (tile % 2);
+                const f32x4 z = tile_product<2>([&](int t) { return down(M, SCP, 16 * t, t0); },
+                                                [&](int t) { return down(plane[REMOVAL][0], DKP, 16 * t, k0); });
+                keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, t0, k0) - z);
+                keep_tile(Rec::REMOVAL, tile, -down(plane[REMOVAL][0], DKP, t0, k0));
+            }
+            if (wave < 4) {
+                const int r0 = 16 * (wave >> 1), c0 = 16 * (wave & 1);
+                const f32x4 v = tile_product<2>([&](int t) { return down(M, SCP, 16 * t, c0); },
+                                                [&](int t) { return along(Rm, SCP, r0, 16 * t); });
+                keep_tile(Rec::MIX, wave, along(W, SCP, r0, c0) - v);
+            }
+        } else {
+            for (int tile = wave; tile < TILES; tile += WAVES) {
+                keep_tile(Rec::READ, tile, along(plane[READ][0], DKP, 16 * (tile / KEYS), 16 * (tile % KEYS)));
+                keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, 16 * (tile % 2), 16 * (tile / 2)));
+            }
+            for (int tile = wave; tile < 4; tile += WAVES) keep_tile(Rec::MIX, tile, along(mat[0][0], SCP, 16 * (tile >> 1), 16 * (tile & 1)));
         }
     }
-    for (int k = tid; k < DK; k += THREADS) {
-        const double d = whole[0][k] * whole[1][k];
-        const float near = (float)d;
-        out[Rec::DECAY + k] = near;
-        out[Rec::DECAY + DK + k] = (float)(d - (double)near);
-    }
-
-    meet();
-    constexpr int KEYS = DK / 16, TILES = 2 * KEYS;
-    if constexpr (REMOVE) {
-        const float *W = mat[0][0], *Rm = mat[1][0], *M = mat[2][0], *L = mat[3][0];
-        float* inv = inverse[0];
-        // T's diagonal blocks: lane (column, block) by forward substitution
-        if (wave == 0 && lane < 32) {
-            const int base = lane & 16, c = lane & 15;
-            float x[16];
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                float s = i == c ? 1.f : 0.f;
-#pragma unroll
-                for (int j = 0; j < i; ++j) s = fmaf(-L[(base + i) * SCP + base + j], x[j], s);
-                x[i] = s;
-            }
-#pragma unroll
-            for (int i = 0; i < 16; ++i) {
-                inverse[base + i][base + c] = x[i];
-                if (base) inverse[i][16 + c] = 0.f;
-            }
-        }
-        meet();
-        // T10 = -T11 L10 T00
-        if (wave == 0) {
-            const f32x4 lt = tile_product<1>([&](int) { return along(L, SCP, 16, 0); }, [&](int) { return down(inv, SCP, 0, 0); });
-#pragma unroll
-            for (int i = 0; i < 4; ++i) scratch[4 * quad + i][row] = -lt[i];
-        }
-        meet();
-        if (wave == 0)
-            put(inverse, 16, 0, tile_product<1>([&](int) { return along(inv, SCP, 16, 16); },
-                                                [&](int) { return down(scratch[0], 20, 0, 0); }));
-        meet();
-        // T M over M's place (kept in registers until everybody has read M); T probe~, transposed, over the decays
-        f32x4 tm = zero;
-        if (wave < 4)
-            tm = tile_product<2>([&](int t) { return along(inv, SCP, 16 * (wave >> 1), 16 * t); },
-                                 [&](int t) { return down(M, SCP, 16 * t, 16 * (wave & 1)); });
-        for (int tile = wave; tile < TILES; tile += WAVES) {
-            const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
-            const f32x4 v = tile_product<2>([&](int t) { return down(plane[PROBE][0], DKP, 16 * t, k0); },
-                                            [&](int t) { return along(inv, SCP, t0, 16 * t); });
-            *reinterpret_cast<f32x4*>(&plane[DECAY][t0 + row][k0 + 4 * quad]) = v;
-            keep_tile(Rec::PROBE, tile, v);
-        }
-        meet();
-        if (wave < 4) put(mat[2], 16 * (wave >> 1), 16 * (wave & 1), tm);
-        meet();
-        // read^ = read~ - R (T probe~);  Z = write~^T - removal~^T (T M);  W^ = W - R (T M): each transposed, as a lane's entries lie
-        for (int tile = wave; tile < TILES; tile += WAVES) {
-            const int t0 = 16 * (tile / KEYS), k0 = 16 * (tile % KEYS);
-            const f32x4 v = tile_product<2>([&](int t) { return down(plane[DECAY][0], DKP, 16 * t, k0); },
-                                            [&](int t) { return along(Rm, SCP, t0, 16 * t); });
-            keep_tile(Rec::READ, tile, along(plane[READ][0], DKP, t0, k0) - v);
-        }
-        for (int tile = wave; tile < TILES; tile += WAVES) {
-            const int k0 = 16 * (tile / 2), t0 = 16 * (tile % 2);
-            const f32x4 z = tile_product<2>([&](int t) { return down(M, SCP, 16 * t, t0); },
-                                            [&](int t) { return down(plane[REMOVAL][0], DKP, 16 * t, k0); });
-            keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, t0, k0) - z);
-            keep_tile(Rec::REMOVAL, tile, -down(plane[REMOVAL][0], DKP, t0, k0));
-        }
-        if (wave < 4) {
-            const int r0 = 16 * (wave >> 1), c0 = 16 * (wave & 1);
-            const f32x4 v = tile_product<2>([&](int t) { return down(M, SCP, 16 * t, c0); },
-                                            [&](int t) { return along(Rm, SCP, r0, 16 * t); });
-            keep_tile(Rec::MIX, wave, along(W, SCP, r0, c0) - v);
-        }
-    } else {
-        for (int tile = wave; tile < TILES; tile += WAVES) {
-            keep_tile(Rec::READ, tile, along(plane[READ][0], DKP, 16 * (tile / KEYS), 16 * (tile % KEYS)));
-            keep_tile(Rec::Z, tile, down(plane[WRITE][0], DKP, 16 * (tile % 2), 16 * (tile / 2)));
-        }
-        for (int tile = wave; tile < 4; tile += WAVES) keep_tile(Rec::MIX, tile, along(mat[0][0], SCP, 16 * (tile >> 1), 16 * (tile & 1)));
-    }    }
 }
 
 // The recurrence as it stands, for 16 value channels: 32 lanes a channel, DK / 32 key rows a lane.
@@ -458,12 +460,13 @@ __device__ __forceinline__ void walk_tokens(const float* __restrict__ coef, cons
 // (KT tiles of 16), which are B operands of the next products as they are, and take it from chunk to chunk; four others make
 // the chunks' read-outs from copies of S that the first leave in LDS, a chunk behind.  So a SIMD has two waves, and one's loads,
 // LDS trips and address arithmetic pass beside the other's products (with the read-outs made by the waves that keep S, one wave a
-// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 76 and 115, and with the loads
-// placed by hand, fewer of them and whole lines stored 63 and 98).  What the waves make of their key rows meets in LDS, two buffers in turn,
-// one barrier a chunk.  A chunk's record is asked for two chunks ahead, its values, of which each wave brings an eighth for all, four.  A chunk
-// takes 1.0 us and, removing, 1.5, of which the matrix cores 0.5 and 0.9; the rest is the chain: a trip through LDS to the readers
-// and back, the barrier, and what the loads' 40 or 70 KB keep the CU's way to L2 busy.  Workgroups are numbered so that the blocks of one head, which read the same records, run on one XCD (workgroup
-// i on XCD i % 8) where the heads are a multiple of 8.
+// SIMD: 87 us for the 64 chunks of 2,048 tokens, 16 heads of 128 x 128, and 137 us with a removal term; so 76 and 115, and with the
+// loads placed by hand, fewer of them and whole lines stored 63 and 98).  What the waves make of their key rows meets in LDS, two
+// buffers in turn, one barrier a chunk.  A chunk's record is asked for two chunks ahead, its values, of which each wave brings an
+// eighth for all, four.  A chunk takes 1.0 us and, removing, 1.5, of which the matrix cores 0.5 and 0.9; the rest is the chain: a trip
+// through LDS to the readers and back, the barrier, and what the loads' 40 or 70 KB keep the CU's way to L2 busy.  Workgroups are
+// numbered so that the blocks of one head, which read the same records, run on one XCD (workgroup i on XCD i % 8) where the heads
+// are a multiple of 8.
 template <int DK, bool REMOVE>
 __global__ __launch_bounds__(512) void scan_chunk_walk_kernel(const float* __restrict__ records, const uint2* __restrict__ alone,
                                                               const float* __restrict__ coef, const float* __restrict__ v,
