@@ -234,7 +234,9 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
         for (int b = 0; b < 4; ++b) {
 #pragma unroll
             for (int v = 0; v < 8; ++v) {
-                const float w = __builtin_amdgcn_exp2f(fmaf(sc[b >> 1][(b & 1) * 8 + v], scale, -ref));
+                float x = sc[b >> 1][(b & 1) * 8 + v] * scale;      // rounded before the reference is taken off, not in one multiply-add:
+                asm("" : "+v"(x));                                  // the same bits as ever (2 to 4 % of the kernel's time)
+                const float w = __builtin_amdgcn_exp2f(x - ref);
                 l += w;
                 p[b][v] = static_cast<bf16>(w);
             }
@@ -257,6 +259,8 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
     // its own, the first behind its scores, the second its values at the turn's start and its keys behind its weights.  us, as it was before there was any of
     // this, a turn behind, so, and with the priority below: 1,953 tokens of 16 heads behind 2,048 others 95.4, 89.3, 83.1 and 82; 2,048 tokens
     // 56.6, 54.3, 48.5 and 48; 512 behind 4,000 99.1, 91.0, 78.1 and 77; 1,500 of 32 heads behind 600 (a single half) 79.3, 76.1, 71.5 and 71.
+    // All of it beside the kernel before, warm, side by side on another card, a score rounded by itself as there: 88.4 and 76.5, 50.2 and 43.1,
+    // 97.0 and 75.2, 70.6 and 63.1.
     const bool behind = HALVES == 2 && part == 1;
     const int turns = (s_end - s_begin + HALVES - 1) / HALVES;
     auto seen = [&](int s) { return wave_live && s < s_end && s * LW_KEYS <= wave_hi && s * LW_KEYS + LW_KEYS > wave_lo; };

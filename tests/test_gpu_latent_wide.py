@@ -285,3 +285,32 @@ def test_scales_that_are_not_positive(halves, scale):
         want = s.masked_fill(~seen, float("-inf")).softmax(1) @ values[h * 128:h * 128 + 128].double().T
         got = out[:, h * 128:h * 128 + 128].double()
         assert float((got - want).norm() / want.norm()) <= 2.0 ** -8
+
+
+@pytest.mark.parametrize("halves", [1, 2])
+@pytest.mark.parametrize("scale", [0.7, -0.7])
+def test_scores_are_rounded_before_the_weights(halves, scale):
+    """A weight is 2 to the power of a score times the scale, rounded to float32, less the largest such.  Scores of 2^17 and a few, exact in
+    float32, of one stage of keys: the product's rounding is up to 2^-8 there, so that one rounding more or less changes three results of ten
+    in bfloat16.  An exponential off by a unit of 2^-24 and the sum's rounding turn one in 2^14 to its neighbour; one in 200 may."""
+    T, sign = 64, 1.0 if scale > 0 else -1.0
+    g = torch.Generator().manual_seed(11)
+    q, keys, turned, values = torch.zeros(T, 192), torch.zeros(64, 128), torch.zeros(64, 64), torch.zeros(128, 64)
+    q[:, 0], q[:, 1], keys[:, 0], keys[:, 1] = 512.0 * sign, sign, 256.0, torch.randint(0, 256, (64,), generator=g) / 32.0
+    values[:64] = torch.eye(64)
+    q, keys, turned, values = (x.bfloat16().to(DEV) for x in (q, keys, turned, values))
+    turned_q, out = torch.zeros(T, 64, dtype=torch.bfloat16, device=DEV), torch.empty(T, 128, dtype=torch.bfloat16, device=DEV)
+    before = ops.library().lc_latent_wide_halves(halves)
+    try:
+        ops._call("lc_latent_wide", ops._ptr(q), 192, ops._ptr(turned_q), 64, 64, ops._ptr(keys), ops._ptr(turned), ops._ptr(values),
+                  64, 1, 0, T, 0, 0, scale, 0, None, None, 0, 0, ops._ptr(out), 128, ops._stream())
+    finally:
+        ops.library().lc_latent_wide_halves(before)
+    by = torch.tensor(scale, dtype=torch.float32) * torch.tensor(1.4426950408889634, dtype=torch.float32)
+    x = (q.float().cpu() @ torch.cat([keys, turned], 1).float().cpu().T) * by
+    x = x.masked_fill(torch.ones(T, 64, dtype=torch.bool).triu(1), float("-inf")).double()
+    w = torch.exp2(x - x.max(1, keepdim=True).values)
+    want = (w.bfloat16().double() / w.sum(1, keepdim=True)).bfloat16()
+    got = out[:, :64].cpu()
+    assert float((got != want).float().mean()) <= 1 / 200
+    assert bool(((got.double() - want.double()).abs() <= want.double().abs() * 2.0 ** -7).all())
