@@ -18,6 +18,9 @@
 
 #include "gemm_tile.h"
 
+#include <algorithm>
+#include <initializer_list>
+
 namespace lc {
 
 
@@ -589,7 +592,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
     place_tile(id, tiles_m, (N + BN - 1) / BN, strip, tm, tn);
     const int m0 = tm * BM, n0 = tn * BN;
 
-    const int tid = threadIdx.x, lane = tid & 63;
+    const int tid = threadIdx.x;
+    int lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
     const int wm = (wave / WN) * (BM / WM), wn = (wave % WN) * (BN / WN);
 
@@ -615,6 +619,10 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
     const int skew = (!SPLIT && tiles_m == 1 && skew_step) ? (int)(((unsigned)id * (unsigned)skew_step) % (unsigned)nk) : 0;
     typename Loop::Sum acc[TM][TN];
     Loop::run(lds, xg, wg, nk, skew, wave, lane, acc);
+    // The lane's number anew, out of no register: kept through the loop it was spilled where that needs them all (tiles of 256 x 256), and a
+    // loop whose operands come by inline assembly has to have none spilled.
+    lane = __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, 0));
+    asm volatile("" : "+v"(lane));
 
     // acc[i][j][v]: row m = (v/4)*8 + (lane/32)*4 + v%4, column n = lane%32 of the 32x32 product, row (lane/16)*4 + v, column lane%16 of the
     // 16x16 one
@@ -823,6 +831,60 @@ static TailPlan tail_plan(int t, int M, int N, int K) {
     return plan;
 }
 
+// The tiles' loop reads LDS by inline assembly into registers that the compiler takes to hold values before its wait for them: were one
+// spilled to scratch memory in between, the spill would store what the register held before.  So the compiled kernels are asked, once: bytes of scratch
+// memory that a lane of a shape's kernels uses, at most (-1: could not ask).  A shape that uses any is not taken.
+static int kernels_scratch(std::initializer_list<const void*> kernels) {
+    int most = 0;
+    for (const void* kernel : kernels) {
+        hipFuncAttributes attr;
+        if (hipFuncGetAttributes(&attr, kernel) != hipSuccess) {
+            (void)hipGetLastError();
+            return -1;
+        }
+        most = std::max(most, (int)attr.localSizeBytes);
+    }
+    return most;
+}
+template <int BM, int BN, int STAGES, int WM = 2, int WN = 2> static int shape_scratch() {
+    const int whole = kernels_scratch({(const void*)gemm_tiled_kernel<BM, BN, STAGES, 0, false, bf16, WM, WN>,
+                                       (const void*)gemm_tiled_kernel<BM, BN, STAGES, 0, false, float, WM, WN>,
+                                       (const void*)gemm_tiled_kernel<BM, BN, STAGES, 1, false, bf16, WM, WN>,
+                                       (const void*)gemm_tiled_kernel<BM, BN, STAGES, 1, false, float, WM, WN>});
+    if constexpr (WM != 2 || WN != 2 || (BM == 128 && STAGES > 2)) {        // not cut along K
+        return whole;
+    } else {
+        const int cut = kernels_scratch({(const void*)gemm_tiled_kernel<BM, BN, STAGES, 0, true, bf16>,
+                                         (const void*)gemm_tiled_kernel<BM, BN, STAGES, 0, true, float>});
+        return whole < 0 ? whole : cut < 0 ? cut : std::max(whole, cut);
+    }
+}
+static int tile_scratch(int t) {
+    struct All { int of[TILE_COUNT]; };
+    static const All all = [] {
+        All a;
+        a.of[TILE_64x128] = shape_scratch<64, 128, 3>();
+        a.of[TILE_128x128] = shape_scratch<128, 128, 2>();
+        a.of[TILE_256x128] = shape_scratch<256, 128, 3>();
+        a.of[TILE_256x192] = shape_scratch<256, 192, 2>();
+        a.of[TILE_256x256] = shape_scratch<256, 256, 2>();
+        a.of[TILE_192x128] = shape_scratch<192, 128, 3>();
+        a.of[TILE_192x256] = shape_scratch<192, 256, 2>();
+        a.of[TILE_64x64] = shape_scratch<64, 64, 3>();
+        const int deep = kernels_scratch({(const void*)gemm_tiled_kernel<64, 64, 5, 0, true, float>});
+        a.of[TILE_64x64] = std::min(a.of[TILE_64x64], deep) < 0 ? -1 : std::max(a.of[TILE_64x64], deep);
+        a.of[TILE_64x96] = shape_scratch<64, 96, 6, 2, 1>();
+        a.of[TILE_192x320] = shape_scratch<192, 320, 2>();
+        a.of[TILE_64x224] = shape_scratch<64, 224, 4, 2, 1>();
+        a.of[TILE_64x128_ONE] = shape_scratch<64, 128, 5, 2, 1>();
+        a.of[TILE_64x160] = shape_scratch<64, 160, 4, 2, 1>();
+        a.of[TILE_128x128_ONE] = shape_scratch<128, 128, 4>();
+        a.of[TILE_128x64] = shape_scratch<128, 64, 6, 4, 1>();
+        return a;
+    }();
+    return all.of[t];
+}
+
 // Into how many shares of K a product with this tile is cut as a whole (1: not at all): as many
 // as it takes to give every CU about two workgroups when whole-K tiles would be too few.  Only
 // the small tiles are cut as a whole; the shares are summed by splitk_reduce_kernel, or by
@@ -910,6 +972,7 @@ static int pick_tile(int M, int N, int K, bool partials_wanted = false) {
     const int candidates[] = {TILE_64x128, TILE_128x128, TILE_256x128, TILE_256x192, TILE_256x256, TILE_192x128,
                               TILE_192x256, TILE_192x320, TILE_64x64, TILE_128x128_ONE, TILE_128x64};
     for (const int t : candidates) {
+        if (tile_scratch(t) > 0) continue;
         if (t == TILE_64x128 && M > 128) continue;
         // 64 x 64 above 256 rows: for the narrow products of a portion of a prompt, which have few
         // larger tiles (2,048 x 1024 x 2048 with the norm that follows: 24.6 us in 512 whole tiles of
@@ -1197,6 +1260,7 @@ static int launch_bf16(const bf16* x, const bf16* w, TO* out, float* workspace, 
     const int shares = splitk_shares(M, N, K);
     const int tile = pick_tile(M, N, K);
     const TailPlan tail = tail_plan(tile, M, N, K);
+    LC_CHECK(tile_scratch(tile) <= 0, "gemm_bf16: the kernels of the tile %dx%d use scratch memory", tile_bm(tile), tile_bn(tile));
     switch (tile) {
     case TILE_64x128:  return launch_tiled<64, 128, 3, EPI, TO>(x, w, out, workspace, M, N, K, shares, tail, form, s);
     case TILE_128x128: return launch_tiled<128, 128, 2, EPI, TO>(x, w, out, workspace, M, N, K, shares, tail, form, s);
@@ -1246,6 +1310,11 @@ LC_API int lc_gemm_bf16_force_tile(int tile) {
     LC_CHECK(tile >= TILE_AUTO && tile < TILE_COUNT, "gemm_bf16: no tile shape %d", tile);
     g_force_tile = tile;
     return 0;
+}
+
+// Bytes of scratch memory a lane of a tile shape's kernels, as the library was built (-1: the runtime could not be asked).
+LC_API int lc_gemm_bf16_tile_scratch(int tile) {
+    return tile < 0 || tile >= TILE_COUNT ? -1 : tile_scratch(tile);
 }
 
 // The tile shape that a product of these sizes goes through (the numbers of lc_gemm_bf16_force_tile;
@@ -1440,7 +1509,9 @@ LC_API int lc_gemm_bf16_partials(const void* x, const void* w, float* partials, 
              "gemm_bf16_partials: operands must be 16-byte aligned");
     const bf16* xb = (const bf16*)x;
     const bf16* wb = (const bf16*)w;
-    if (pick_tile(M, N, K, true) == TILE_64x64) {
+    const int tile = pick_tile(M, N, K, true);
+    LC_CHECK(tile_scratch(tile) <= 0, "gemm_bf16_partials: the kernels of the tile %dx%d use scratch memory", tile_bm(tile), tile_bn(tile));
+    if (tile == TILE_64x64) {
         const int tiles_m = (M + 63) / 64, tiles = tiles_m * ((N + 63) / 64);
         if (M <= 64 && tiles * shares <= kCUs && K / TL_K / shares >= ONE_ROUND_BLOCKS)
             gemm_tiled_kernel<64, 64, 5, 0, true, float><<<dim3(tiles, shares), 256, 0, stream>>>(
@@ -1448,7 +1519,7 @@ LC_API int lc_gemm_bf16_partials(const void* x, const void* w, float* partials, 
         else
             gemm_tiled_kernel<64, 64, 3, 0, true, float><<<dim3(tiles, shares), 256, 0, stream>>>(
                 xb, wb, nullptr, partials, M, N, K, tiles_m, tiles_m, 0, tiles, 0, g_skew, kSilu);
-    } else if (pick_tile(M, N, K, true) == TILE_64x128) {
+    } else if (tile == TILE_64x128) {
         const int tiles_m = (M + 63) / 64, tiles = tiles_m * ((N + 127) / 128);
         gemm_tiled_kernel<64, 128, 3, 0, true, float><<<dim3(tiles, shares), 256, 0, stream>>>(
             xb, wb, nullptr, partials, M, N, K, tiles_m, tiles_m, 0, tiles, 0, g_skew, kSilu);

@@ -60,6 +60,7 @@ _SIGNATURES = {
     "lc_attn_bf16_supported": "iiii",
     "lc_attn_page_granule": "",
     "lc_gemm_bf16_runs_ring_ok": "",
+    "lc_gemm_bf16_tile_scratch": "i",
     "lc_attn_decode_splits": "iii",
     "lc_attn_decode_waves": "i",
     "lc_attn_decode_deep": "i",

@@ -68,3 +68,9 @@ def test_stored_through_lds(tile, M, N):
             assert torch.equal(whole, other[:, :N])
     finally:
         ops.force_gemm_tile(-1)
+
+
+@pytest.mark.parametrize("tile", range(15))
+def test_tiles_keep_their_operands_in_registers(tile):
+    """A loop whose operands come by inline assembly may have none of them spilled: such a shape would not be taken."""
+    assert ops.library().lc_gemm_bf16_tile_scratch(tile) == 0
