@@ -95,7 +95,10 @@ template <int LEFT> __device__ __forceinline__ void lds_have(bf16x8 (&r)[4]) {
 // longest chain (us, one and two halves, both before the halves worked a turn apart: 2,048 tokens of 16 heads 67 and 52, behind 2,048 others
 // 129 and 98, 512 behind 4,000 129 and 97; 4,000 tokens, 512 workgroups, 133 and 107).  With more workgroups a CU has its second wave anyway, and the halves only wait for
 // each other (768 workgroups 93 and 124, 1,024 354 and 380).
-template <int HALVES>
+//
+// Offset: a lane's place within the rows of a load, in bytes: 32 bits where three rows of the keys and seven of the values fit, so that a load's address
+// is one register beside a scalar base; 64 bits for rows longer than that.
+template <int HALVES, typename Offset>
 __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a) {
     constexpr int KB = LW_KEYS * LW_DIM * 2, TB = LW_KEYS * LW_ROT * 2, VB = LW_VDIM * LW_KEYS * 2, STAGE = KB + TB + VB;
     constexpr int KS = (LW_DIM + LW_ROT) / 16, VT = LW_VDIM / 32;
@@ -136,8 +139,9 @@ __global__ __launch_bounds__(256 * HALVES, 2) void latent_wide_kernel(WideArgs a
     // load instructions: four rows of 256 bytes of the keys, eight of 128 of their rotated parts and of the values; a lane's bytes from the
     // first row on, of the first instruction (instruction i of the keys: place xor 4 i) and, the values', of the second
     const int r4 = lane >> 4, r8 = lane >> 3;
-    const unsigned k_off = (unsigned)r4 * a.H * (LW_DIM * 2) + (((lane & 15) ^ r4) * 16), t_off = r8 * (LW_ROT * 2) + (((lane & 7) ^ (r8 >> 1)) * 16);
-    const unsigned v_off[2] = {(unsigned)(r8 * a.ldv * 2) + (((lane & 7) ^ (r8 >> 1)) * 16), (unsigned)(r8 * a.ldv * 2) + (((lane & 7) ^ 4 ^ (r8 >> 1)) * 16)};
+    const Offset k_off = (Offset)r4 * a.H * (LW_DIM * 2) + (((lane & 15) ^ r4) * 16), v_row_off = (Offset)(r8 * a.ldv * 2);
+    const unsigned t_off = r8 * (LW_ROT * 2) + (((lane & 7) ^ (r8 >> 1)) * 16);
+    const Offset v_off[2] = {v_row_off + (((lane & 7) ^ (r8 >> 1)) * 16), v_row_off + (((lane & 7) ^ 4 ^ (r8 >> 1)) * 16)};
     // Load n of a wave, of stage s into that turn's place: 0 to 3 the keys', 4 and 5 their rotated parts', 6 to 9 the values'.
     constexpr int LOADS = 10, KEY_LOADS = 6;
     auto load = [&](int n, int s, int turn) {
@@ -385,7 +389,6 @@ LC_API int lc_latent_wide(const void* q, long long ldq, const void* q_turned, lo
     LC_CHECK(window == 0 ? lo == 0 : lo <= (position - window + 1 > 0 ? position - window + 1 : 0), "latent_wide: rows are missing");
     LC_CHECK(((uintptr_t)q | (uintptr_t)q_turned | (uintptr_t)keys | (uintptr_t)turned | (uintptr_t)values) % 16 == 0 &&
                  (ldq | q_row | q_head | ldv) % 8 == 0, "latent_wide: not aligned to 16 bytes");
-    LC_CHECK(ldv < 1ll << 28 && H < 1 << 20, "latent_wide: rows too long");
     LC_CHECK(ldv >= (position + tokens - lo + LW_KEYS - 1) / LW_KEYS * LW_KEYS, "latent_wide: the values' rows are too short");
     LC_CHECK((uintptr_t)out % 8 == 0 && ldo % 4 == 0, "latent_wide: the output is not aligned to 8 bytes");
     LC_CHECK(!gate || gate_head == 1 || (gate_head == LW_VDIM && (uintptr_t)gate % 8 == 0 && ldg % 4 == 0), "latent_wide: bad gates");
@@ -395,8 +398,14 @@ LC_API int lc_latent_wide(const void* q, long long ldq, const void* q_turned, lo
                H, first, tokens, position, lo, scale * 1.4426950408889634f, window, sink, (const bf16*)gate, ldg, gate_head,
                (bf16*)out, ldo};
     const int halves = g_wide_halves ? g_wide_halves : (long long)H * tiles <= 2 * device_cus() ? 2 : 1;
-    if (halves == 2) latent_wide_kernel<2><<<dim3(H, tiles), 512, 0, stream>>>(a);
-    else latent_wide_kernel<1><<<dim3(H, tiles), 256, 0, stream>>>(a);
+    const bool near = ldv < 1ll << 28 && H < 1 << 22;       // 3 rows of 256 H bytes and 7 of 2 ldv are below 2^32
+    if (halves == 2) {
+        if (near) latent_wide_kernel<2, unsigned><<<dim3(H, tiles), 512, 0, stream>>>(a);
+        else latent_wide_kernel<2, unsigned long long><<<dim3(H, tiles), 512, 0, stream>>>(a);
+    } else {
+        if (near) latent_wide_kernel<1, unsigned><<<dim3(H, tiles), 256, 0, stream>>>(a);
+        else latent_wide_kernel<1, unsigned long long><<<dim3(H, tiles), 256, 0, stream>>>(a);
+    }
     LC_LAUNCH_CHECK("latent_wide");
     return 0;
 }

@@ -314,3 +314,28 @@ def test_scores_are_rounded_before_the_weights(halves, scale):
     got = out[:, :64].cpu()
     assert float((got != want).float().mean()) <= 1 / 200
     assert bool(((got.double() - want.double()).abs() <= want.double().abs() * 2.0 ** -7).all())
+
+
+@pytest.mark.parametrize("halves", [1, 2])
+def test_rows_of_values_beyond_32_bits(halves):
+    """Values whose rows lie so far apart that a lane's place within eight of them needs more than 32 bits: the same bits as side by side."""
+    T, rows, far = 130, 192, (1 << 28) + (1 << 26)
+    if torch.cuda.mem_get_info()[0] < 128 * far * 2 + (4 << 30):
+        pytest.skip("needs 90 GB of the card")
+    g = torch.Generator().manual_seed(3)
+    q, turned_q, keys, turned, values = ((torch.randn(*shape, generator=g) * 0.5).bfloat16().to(DEV) for shape in (
+        (T, 192), (T, 64), (rows, 128), (rows, 64), (128, rows)))
+    apart = torch.empty(128, far, dtype=torch.bfloat16, device=DEV)
+    apart[:, :rows] = values
+    outs = []
+    before = ops.library().lc_latent_wide_halves(halves)
+    try:
+        for v in (values, apart):
+            outs.append(torch.empty(T, 128, dtype=torch.bfloat16, device=DEV))
+            ops._call("lc_latent_wide", ops._ptr(q), 192, ops._ptr(turned_q), 64, 64, ops._ptr(keys), ops._ptr(turned), ops._ptr(v),
+                      v.shape[1], 1, 0, T, 60, 0, 0.1, 0, None, None, 0, 0, ops._ptr(outs[-1]), 128, ops._stream())
+        assert torch.equal(*outs)
+    finally:
+        ops.library().lc_latent_wide_halves(before)
+        del v, apart
+        torch.cuda.empty_cache()
