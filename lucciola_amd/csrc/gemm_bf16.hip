@@ -637,6 +637,7 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
         // would halve that.
         constexpr int WC = BN / WN, STRIDE = WC + 4, E = PIECE<TO>, PIECES = (EPI == 1 ? WC / 2 : WC) / E;
         static_assert(WM * WN * 32 * STRIDE * 4 <= Loop::LDS, "a strip of every wave");
+        static_assert(32 * PIECES % 64 == 0 && WC % (2 * E) == 0, "whole passes of the wave, within its strip's columns");
         const int ldo = EPI == 1 ? N / 2 : N;
         if ((sizeof(TO) == 2 || MF == 16) && ldo % E == 0 && (uintptr_t)out % 16 == 0) {
             float* strip = reinterpret_cast<float*>(lds) + wave * 32 * STRIDE;

@@ -55,7 +55,10 @@ def test_taken_by_size():
         _check(*_operands(M, N, K), -1)
 
 
-@pytest.mark.parametrize("tile", [2, 3, 4, 6, 9, 11, 13])
+FINE = (2, 3, 4, 6, 9)      # tiles of products of 16 x 16, whose float32 results pass through LDS too
+
+
+@pytest.mark.parametrize("tile", [*FINE, 11, 13])
 @pytest.mark.parametrize("M,N", [(31, 8), (193, 392), (257, 264), (300, 1000)])
 def test_stored_through_lds(tile, M, N):
     """Columns that are stored in pieces of 16 bytes are, to the bit, those of a product with one or four more, which is stored in pairs or one
@@ -63,11 +66,42 @@ def test_stored_through_lds(tile, M, N):
     x, w = _operands(M, N + 16, 512)
     ops.force_gemm_tile(tile)
     try:
-        for dtype, more in ((torch.bfloat16, 4), (torch.bfloat16, 1), (torch.float32, 1), (torch.float32, 2)):
+        for dtype, more in ((torch.bfloat16, 4), (torch.bfloat16, 1)) + ((torch.float32, 1), (torch.float32, 2)) * (tile in FINE):
             whole, other = ops.gemm(x, w[:N], dtype), ops.gemm(x, w[:N + more], dtype)
             assert torch.equal(whole, other[:, :N])
     finally:
         ops.force_gemm_tile(-1)
+
+
+@pytest.mark.parametrize("tile", [*FINE, 0, 5, 7, 8, 10, 11, 12, 13, 14])
+@pytest.mark.parametrize("M,N", [(31, 16), (193, 400), (300, 1008)])
+@pytest.mark.parametrize("gated", [False, True])
+def test_results_that_begin_anywhere(tile, M, N, gated):
+    """Results that begin at a whole 16 bytes (through LDS, where the tile does that) and 8 bytes further on (from the registers): the same
+    bits, plain and gated, and nothing stored beside them."""
+    x, w = _operands(M, N, 256)
+    width, got = N // 2 if gated else N, {}
+    ops.force_gemm_tile(tile)
+    ops.library().lc_gemm_bf16_force_shares(1)
+    try:
+        for dtype in (torch.bfloat16, torch.float32):
+            for shift in (0, 8 // dtype.itemsize):
+                room = torch.full((16 + M * width + 16,), 7.0, dtype=dtype, device="cuda")
+                out = room[16 + shift:16 + shift + M * width]
+                ops._call("lc_gemm_bf16", ops._ptr(x), ops._ptr(w), ops._ptr(out), ops._dt(out), M, N, 256, int(gated), None, ops._stream())
+                assert bool((room[:16 + shift] == 7.0).all()) and bool((room[16 + shift + M * width:] == 7.0).all())
+                got[dtype, shift > 0] = out.clone()
+    finally:
+        ops.force_gemm_tile(-1)
+        ops.library().lc_gemm_bf16_force_shares(0)
+    for dtype in (torch.bfloat16, torch.float32):
+        assert torch.equal(got[dtype, False], got[dtype, True])
+    want = x.double() @ w.double().T
+    if gated:
+        blocks = want.view(M, -1, 2, 8)
+        g, u = blocks[:, :, 0].reshape(M, -1), blocks[:, :, 1].reshape(M, -1)
+        want = g * torch.sigmoid(g) * u
+    assert float((got[torch.bfloat16, False].double().view(M, width) - want).norm() / want.norm()) <= 2.0 ** -8
 
 
 @pytest.mark.parametrize("tile", range(15))
