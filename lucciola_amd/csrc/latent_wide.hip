@@ -360,9 +360,30 @@ LC_API int lc_latent_wide_halves(int halves) {
     return before;
 }
 
+// The kernels' operands are asked for and waited for in two pieces of inline assembly (lds_ask, lds_have), and in between the compiler takes
+// their registers to hold values already: were one spilled to scratch memory there, the spill would store what it held before.  So the compiled
+// kernels are asked, once: 1 all in registers, 0 one uses scratch memory, -1 could not ask.  Unless it is 1, portions stay in the latent's space.
+static int wide_state() {
+    static const int state = [] {
+        const void* kernels[] = {(const void*)latent_wide_kernel<1, unsigned>, (const void*)latent_wide_kernel<2, unsigned>,
+                                 (const void*)latent_wide_kernel<1, unsigned long long>, (const void*)latent_wide_kernel<2, unsigned long long>};
+        for (const void* kernel : kernels) {
+            hipFuncAttributes attr;
+            if (hipFuncGetAttributes(&attr, kernel) != hipSuccess) {
+                (void)hipGetLastError();
+                return -1;
+            }
+            if (attr.localSizeBytes != 0) return 0;
+        }
+        return 1;
+    }();
+    return state;
+}
+LC_API int lc_latent_wide_ok() { return wide_state(); }
+
 // Whether these heads have a kernel.
 LC_API int lc_latent_wide_supported(int R, int dim, int rot, int vdim) {
-    return dim == LW_DIM && rot == LW_ROT && vdim == LW_VDIM && R > 0 && R % 64 == 0 ? 1 : 0;
+    return dim == LW_DIM && rot == LW_ROT && vdim == LW_VDIM && R > 0 && R % 64 == 0 && wide_state() == 1 ? 1 : 0;
 }
 
 LC_API int lc_latent_rows(const void* cache, const int* table, int page_size, int R, int rot, int lo, int count, int rows, void* c,
@@ -392,6 +413,7 @@ LC_API int lc_latent_wide(const void* q, long long ldq, const void* q_turned, lo
     LC_CHECK(ldv >= (position + tokens - lo + LW_KEYS - 1) / LW_KEYS * LW_KEYS, "latent_wide: the values' rows are too short");
     LC_CHECK((uintptr_t)out % 8 == 0 && ldo % 4 == 0, "latent_wide: the output is not aligned to 8 bytes");
     LC_CHECK(!gate || gate_head == 1 || (gate_head == LW_VDIM && (uintptr_t)gate % 8 == 0 && ldg % 4 == 0), "latent_wide: bad gates");
+    LC_CHECK(wide_state() != 0, "latent_wide: a kernel uses scratch memory");
     const int tiles = (tokens + LW_TOKENS - 1) / LW_TOKENS;
     LC_CHECK(tiles <= 65535, "latent_wide: too many tokens");
     WideArgs a{(const bf16*)q, ldq, (const bf16*)q_turned, q_row, q_head, (const bf16*)keys, (const bf16*)turned, (const bf16*)values, ldv,

@@ -100,6 +100,7 @@ _SIGNATURES = {
     "lc_latent_lone_picks": "iiiii",
     "lc_latent_lone_splits": "ii",
     "lc_latent_wide_supported": "iiii",
+    "lc_latent_wide_ok": "",
     "lc_latent_wide_halves": "i",
     "lc_latent_rows": "ppiiiiiippp",
     "lc_latent_wide": "pqpqqpppqiiiiifippqqpqp",

@@ -339,3 +339,10 @@ def test_rows_of_values_beyond_32_bits(halves):
         ops.library().lc_latent_wide_halves(before)
         del v, apart
         torch.cuda.empty_cache()
+
+
+def test_the_operands_stay_in_registers():
+    """Asked for in one piece of inline assembly and waited for in another: none may be spilled in between, or portions would stay in the
+    latent's space."""
+    assert ops.library().lc_latent_wide_ok() == 1
+    assert ops.latent_wide_takes(512, DIM, ROT, VDIM, torch.bfloat16, torch.device(DEV))
