@@ -206,15 +206,15 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGat
         const int n = GATED ? min(n0 / 2 + (r >> 6) * 32 + (r & 31), N / 2 - 1) + ((r >> 5) & 1) * (N / 2) : min(n0 + r, N - 1);
         wg[i] = w + (size_t)n * K + Loop::chunk_of(i, wave, lane) * 8;
     }
-    typename Loop::Sum acc[TM][TN];
+    static_assert(Loop::MF == 32, "the epilogue's layout");
+    floatx16 acc[TM][TN];
     // Rows of w lie 2 K bytes apart, so workgroups that walk k in step ask the same few memory channels at every moment: each group
     // starts at a block of its own and wraps around.  Its tiles and columns start together, because they share rows in L2.
     Loop::run(lds, xg, wg, blocks, (int)((unsigned)tile.group * 13u % (unsigned)blocks), wave, lane, acc);
 
     // 32 rows at a time pass through the wave's part of the ring, so that a lane gets neighbouring columns, 16 bytes of them
-    // (acc[i][j][v]: row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32 of the 32 x 32 product, row (lane / 16) * 4 + v, column
-    // lane % 16 of the 16 x 16 one)
-    constexpr int MF = Loop::MF, WIDTH = MF * TN, STRIDE = WIDTH + 4;
+    // (acc[i][j][v]: row (v / 4) * 8 + (lane / 32) * 4 + v % 4, column lane % 32 of the 32 x 32 product)
+    constexpr int WIDTH = 32 * TN, STRIDE = WIDTH + 4;
     static_assert(4 * 32 * STRIDE * 4 <= EVEN_LDS, "a strip of every wave");
     float* strip = reinterpret_cast<float*>(lds) + wave * 32 * STRIDE;
     constexpr int E = PIECE<TO>, OUT = GATED ? WIDTH / 2 : WIDTH, LANES = OUT / E, ROWS = 64 / LANES;      // stored columns, lanes a row, rows a pass
@@ -265,16 +265,14 @@ __device__ __forceinline__ void even_tile(const GroupedArgs& a, const GroupedGat
     };
     __syncthreads();
 #pragma unroll
-    for (int i0 = 0; i0 < TM; i0 += 32 / MF) {
+    for (int i = 0; i < TM; ++i) {
 #pragma unroll
-        for (int i = 0; i < 32 / MF; ++i)
+        for (int j = 0; j < TN; ++j)
 #pragma unroll
-            for (int j = 0; j < TN; ++j)
-#pragma unroll
-                for (int v = 0; v < Loop::SV; ++v)
-                    strip[(i * MF + (v >> 2) * 8 + (lane / MF) * 4 + (v & 3)) * STRIDE + j * MF + (lane & (MF - 1))] = acc[i0 + i][j][v];
+            for (int v = 0; v < 16; ++v)
+                strip[((v >> 2) * 8 + (lane >> 5) * 4 + (v & 3)) * STRIDE + j * 32 + (lane & 31)] = acc[i][j][v];
         __builtin_amdgcn_wave_barrier();
-        finish(i0 * MF / 32);
+        finish(i);
         __builtin_amdgcn_wave_barrier();
     }
 }
