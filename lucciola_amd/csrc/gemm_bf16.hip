@@ -633,7 +633,8 @@ __global__ __launch_bounds__(64 * WM * WN) void gemm_tiled_kernel(const bf16* __
         // Whole pieces of 16 bytes: 32 rows at a time pass through the wave's part of the ring, so that a lane gets neighbouring columns and a
         // row's are stored in whole lines (pairs of lanes stored 64 bytes of a row at a time; us, so and through LDS, both with products of
         // 32 x 32: 2,048 x 4096 x 1024 20.8 and 20.0, x 6144 x 1024 with SwiGLU 29.3 and 28.0, 1,523 x 2048 x 2048 17.3 and 16.7, x 2048 x 2048
-        // 20.0 and 19.7).  float32 results of large products were stored 256 bytes at a time and are no faster for it; products of 16 x 16
+        // 20.0 and 19.7; 104 products of 17 to 64 rows 1.00 of the time in the mean, 0.93 to 1.02, and one of 8 us, whose
+        // runs differ by as much, 1.09).  float32 results of large products were stored 256 bytes at a time and are no faster for it; products of 16 x 16
         // would halve that.
         constexpr int WC = BN / WN, STRIDE = WC + 4, E = PIECE<TO>, PIECES = (EPI == 1 ? WC / 2 : WC) / E;
         static_assert(WM * WN * 32 * STRIDE * 4 <= Loop::LDS, "a strip of every wave");
@@ -931,9 +932,10 @@ static int shares_for(int t, int M, int N, int K, bool partials_wanted = false) 
 // the least estimated time in microseconds.  A CU works through a round of tiles in
 // (tile area) x K x 2 / (4.63 MFLOP/us x the shape's relative rate) (measured at K = 4096, with a loop
 // that issued a block's loads in a row: larger tiles move fewer bytes per product) and 3 us to start
-// and end.  On the loop that runs now, weights cold, 364 products of 96 to 4,001 rows of the layers' sizes at widths of
+// and end.  On the loop as it was with products of 32 x 32 alone, weights cold, 364 products of 96 to 4,001 rows of the layers' sizes at widths of
 // 1,024 to 4,096: the shape picked takes 0.97 of the time of the one picked before there were
-// tiles of 128 x 128 and 128 x 64 in one round (0.70 to 1.09), and is within 8 % of the best of all in 342.  A last round of a one-a-CU shape
+// tiles of 128 x 128 and 128 x 64 in one round (0.70 to 1.09), and is within 8 % of the best of all in 342; the tiles
+// whose waves own 64 x 128 and more have become 0 to 13 % faster since, which the rates do not know.  A last round of a one-a-CU shape
 // that is cut along K takes its share of that, plus the time to write and read its float32
 // partial tiles (about 4 TB/s) and to start two more kernels.  A small tile cut along K as a
 // whole pays for its partial sums likewise, and 3 us for the kernel that adds them, which reads what lies in the caches: of 1,647 products

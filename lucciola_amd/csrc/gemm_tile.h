@@ -77,8 +77,8 @@ __device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
 // (16 consecutive rows, one chunk) then cover all 64 banks.
 //
 // The loop is scheduled by hand, because a SIMD holds a single wave of this kernel and nothing
-// else hides a stall.  Per k-step of 16 the wave issues its (BM/64)*(BN/64) products; between
-// them, one at a time, go the LDS reads of the NEXT k-step's operands (ds_read_b128 in inline
+// else hides a stall.  Per k-step, which is one product deep (16 or 32 k), the wave issues its
+// TM * TN products; between them, one at a time, go the LDS reads of the NEXT k-step's operands (ds_read_b128 in inline
 // assembly with explicit waits: the compiler cannot tell the stages apart and would make every
 // load in flight land before any read) and the global loads.  In a block's last k-step the wave
 // waits for its own loads of the next block and meets the others at a bare barrier, the only one
@@ -86,6 +86,7 @@ __device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
 // last operands of this block in registers, so that its stage is free.  From there on the wave
 // reads the next block's first operands and issues, a few products apart, the loads of the block
 // TL_STAGES ahead into the freed stage, on into the next block.  sched_barrier pins that order.
+// (Figures below that name no product's size are of the loop with products of 32 x 32 x 16.)
 //
 // The loads are spread because a CU takes them at 64 bytes a clock (58 measured for rows of 128
 // bytes that L2 holds): the 16 loads of a wave of the 256 x 256 tile, four waves at once, are a
@@ -97,11 +98,14 @@ __device__ __forceinline__ float gated_f(float g, float u, GateForm form) {
 constexpr int TL_K = 64;
 
 // BM x BN rows of x and of w, TL_STAGES stages, WM x WN waves, each owning (BM / WM) x (BN / WN) of the tile as TM x TN products
-// of 32 x 32.  LATE: of two stages whose loads go out later in a block (below).  FINE: products of 16 x 16 x 32 instead of 32 x 32 x 16, the
-// same sums to the bit wherever tried.  Both take the matrix cores' time for as many operations, but the small ones read and write each sum half as often,
-// and a product of large tiles is held back by the power limit: us, large and small, with the epilogue in whole lines (gemm_bf16.hip) 326 and 311 for
-// 2,048 x 24576 x 4096 with SwiGLU, 87.0 and 81.3 for x 6144 x 4096, 171.7 and 166.0 for x 4096 x 12288, 57.2 and 54.0 for x 8192 x 2048.  Not for
-// tiles whose waves own less than 64 x 128 (bound by the way from L2: no change), nor for the experts' (up to 1.07 of the time: bound by memory).
+// of MF x MF and KP deep.  LATE: of two stages whose loads go out later in a block (below).  FINE: products of 16 x 16 x 32 instead of
+// 32 x 32 x 16, the same sums to the bit wherever tried.  Both take the matrix cores' time for as many operations, but the small ones read and
+// write each sum half as often, and a product of large tiles is held back by the power limit: at 2,048 rows, held for three seconds, us and the
+// clock meanwhile, large (stored in pairs) and small (in whole lines, gemm_bf16.hip): 24576 x 4096 with SwiGLU 325.5 at 1.78 GHz and 315 at 2.00, 6144 x
+// 4096 82.4 at 1.82 and 80.3 at 2.08, 4096 x 12288 173 at 1.755 and 169.5 at 1.95, 4096 x 4096 60.4 at 1.86 and 59 at 2.07.  (The first twenty
+// after a rest take up to a quarter longer, either way.)  23 products of 233 to 3,868 rows that take
+// such tiles: 0.97 of the time in the mean, 0.87 to 1.01.
+// Not for tiles whose waves own less than 64 x 128 (bound by the way from L2: no change), nor for the experts' (up to 1.07 of the time: bound by memory).
 template <int BM, int BN, int TL_STAGES, int WM, int WN, bool LATE = false, bool FINE = false>
 struct TileLoop {
     static constexpr int MF = FINE ? 16 : 32;                 // rows and columns of a product
@@ -183,7 +187,7 @@ struct TileLoop {
             for (int v = 0; v < SV; ++v) acc[i][j][v] = 0.f;
 
     // LDS address of this lane's operand rows in stage 0, with the lane's part of the swizzle;
-    // k-step ks flips chunk bits: ((2 ks + kg) ^ swz) * 16 = ((kg ^ swz) * 16) ^ (ks * 32)
+    // k-step ks flips chunk bits: ((KP / 8 * ks + kg) ^ swz) * 16 = ((kg ^ swz) * 16) ^ (ks * KP * 2)
     const unsigned lds0 = (unsigned)(uintptr_t)(lds_ptr_t)lds;
     unsigned pa[TM], pb[TN];
 #pragma unroll

@@ -90,11 +90,12 @@ template <int LEFT> __device__ __forceinline__ void lds_have(bf16x8 (&r)[4]) {
 // rows meet a bank twice.  Two workgroups a CU, whose waves fill each other's waits.
 //
 // HALVES 2: eight waves, of which four take every other stage of the same queries, with a ring of their own; their sums are joined at the
-// end.  A stage keeps a wave busy for 2.2 us where it is alone on its SIMD (its loads, products and weights wait for each other) and
+// end.  A stage keeps a wave that is alone on its SIMD busy for about 1.7 us (its loads, products and weights wait for each other) and
 // two waves for little more, so where there are no more workgroups than two a CU the halves are the second wave, and they halve the
-// longest chain (us, one and two halves, both before the halves worked a turn apart: 2,048 tokens of 16 heads 67 and 52, behind 2,048 others
-// 129 and 98, 512 behind 4,000 129 and 97; 4,000 tokens, 512 workgroups, 133 and 107).  With more workgroups a CU has its second wave anyway, and the halves only wait for
-// each other (768 workgroups 93 and 124, 1,024 354 and 380).
+// longest chain (us, one and two halves: 2,048 tokens of 16 heads 57 and 43, 1,953 behind 2,048 others 101 and 77, 512 behind 4,000 109 and 75; 4,000
+// tokens, 512 workgroups, 119 and 95; not everywhere: 64 heads, 700 tokens, 384 workgroups, 24 and 29, 1,024 behind 4,000, 512 workgroups, 192 and
+// 194).  With more workgroups a CU has its second wave anyway, and the halves gain little or only wait for each other (528 workgroups 128 and 111,
+// 768 213 and 212 and, 48 heads, 84 and 92, 1,024 337 and 348 and, 64 heads, 99 and 113).
 //
 // Offset: a lane's place within the rows of a load, in bytes: 32 bits where three rows of the keys and seven of the values fit, so that a load's address
 // is one register beside a scalar base; 64 bits for rows longer than that.

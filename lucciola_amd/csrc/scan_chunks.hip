@@ -2,7 +2,7 @@
 //     S <- diag(decay) S - removal (probe^T S) + write v^T,    o = S^T read,
 // for portions of prompts, a chunk of SC = 32 tokens at a time on the float32 matrix instruction.  Token by token a step
 // is a chain of dependent vector instructions, 0.21 us a token without and 0.29 us with the removal term, on a wave that
-// is alone on its SIMD (16 heads of 128 x 128: 439 and 590 us for 2,048 tokens whatever the number of heads; here 84 and 162).
+// is alone on its SIMD (16 heads of 128 x 128: 437 and 580 us for 2,048 tokens whatever the number of heads; here 88 and 168).
 //
 // Inside a chunk, from the state S that the chunk before left, with a_i the product of the decays of tokens 0..i (key
 // channel by key channel), r_ij that of the tokens j+1..i, and y_i = probe_i^T S_(i-1) what token i takes out:
@@ -85,7 +85,10 @@ __device__ __forceinline__ f32x4 tile_product(A a, B b) {
 // [records][heads][8]: not all zero where the chunk holds what has to go token by token, and its record is not to be used.
 // An item asks for the next one's vectors before it makes its pairs, so that loads, products and stores of a CU pass beside each other (with
 // a workgroup an item they follow each other; 2,048 tokens, 16 heads of 128 28 -> 21 us, 32 heads 53 -> 40, which is 4.4 TB/s; two workgroups a
-// CU, four for heads of 64 without removal, are what its LDS and registers hold and measured best of one to four).  With heads of 128 and
+// CU, four for heads of 64 without removal, are what its LDS and registers hold and measured best of one to four.  With the walk, before this and the
+// walk's loads placed by hand and now: heads of 64, values of 128, 2,048 tokens 73 -> 69 us and, removing, 111 -> 102; 16 portions of 64 tokens 38 -> 35
+// and 69 -> 66, 60 of them 107 -> 102 and 204 -> 208, 100 portions of 70 and 4 heads, whose every item looks for its request, 41 -> 36 and 76 -> 68; heads of
+// 128, 2,048 tokens 105 -> 88 and 183 -> 168, 60 portions of 64 179 -> 157 and 358 -> 356).  With heads of 128 and
 // a removal term a workgroup fills its CU's LDS, has no registers for another item's vectors (29 of them spilled: 66 us against 63) and
 // its steps follow each other: 63 us for 2,048 tokens and 16 heads, 16 us an item, whose 155 KB
 // in and out take half of that at the rate of a copy.

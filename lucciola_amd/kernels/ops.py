@@ -1443,15 +1443,17 @@ def plan_latent_attention(layout):
 def latent_wide_time(tokens: int, position: int, heads: int, window: int) -> float:
     """us that a portion of ``tokens`` tokens behind ``position`` others takes head by head (``latent_wide``) on 256 CUs: a workgroup
     of 128 tokens of a head takes 1.15 us for 64 rows, two a CU, whoever is alone walks all of them, the keys and values cost 0.52
-    ns a row and head, and there are four launches more."""
+    ns a row and head, and there are four launches more.  (Fitted to a kernel that took 10 to 25 % longer where its halves share a portion; measured
+    now and the estimate, us: 16 heads, 700 tokens 36 and 39, 2,048 71 and 74, 256 behind 4,000 others 108 and 133, 1,953 behind 2,048 109 and 126; 64
+    heads, 1,024 behind 4,000, 313 and 278.  So portions near the line stay in the latent's space.)"""
     span = position + tokens if not window else min(position + tokens, window + tokens - 1)
     return 20.0 + -(-span // 64) * 1.15 * -(-(-(-tokens // 128) * heads) // 512) + span * heads * 5.2e-4
 
 
 def latent_wide_pays(tokens: int, position: int, heads: int, window: int) -> bool:
     """Whether a portion alone is faster head by head than in the latent's space, where a workgroup of 16 tokens and four heads
-    takes 3 us for 32 rows, a CU holds one, and few tiles share out their rows.  (A layer with 16 heads: 2,048 tokens 430 us and
-    85; behind 2,048 others 830 and 175; 256 tokens behind 4,000 others 100 and 125; below some 700 tokens of a fresh prompt the
+    takes 3 us for 32 rows, a CU holds one, and few tiles share out their rows.  (A layer with 16 heads, in the latent's space and head by
+    head: 2,048 tokens 430 us and 71; behind 2,048 others 830 and 115; 256 tokens behind 4,000 others 100 and 108; below some 700 tokens of a fresh prompt the
     launches weigh more than either.)"""
     span = position + tokens if not window else min(position + tokens, window + tokens - 1)
     return latent_wide_time(tokens, position, heads, window) < -(-tokens // 16) * -(-heads // 4) * -(-span // 32) * 3.0 / 256
@@ -2234,8 +2236,10 @@ class ScanPortions:
 # (planes, key channels) -> us: token by token (before the first token, a token of the longest request, a token and 16 value channels
 # of a head, a million entries of state); in chunks (before the first chunk, a token of the longest request, a token and head, a token and
 # 16 value channels of a head).  Fitted to 1,876 steps of 64 to 2,600 tokens in portions of 64 to 640 beside none to 200 lone or short
-# requests, 2 to 32 heads of 16 to 257 value channels; eight of ten are within 13 % of their time (the walk over chunks has got up to
-# a sixth faster since: the line errs towards token by token).
+# requests, 2 to 32 heads of 16 to 257 value channels; eight of ten were within 13 % of their time.  The chunks' kernels have become faster since, the
+# walk by up to a sixth and the preparation without removal by a quarter, and the columns in chunks are up to 20 % too long for 2,048 tokens
+# of 16 heads (us, estimated and measured: (3, 64) 74 and 69, (3, 128) 110 and 89, (5, 64) 111 and 102, (5, 128) 192 and 169): the line errs
+# towards token by token.
 _SCAN_TIMES = {
     (3, 64): ((4.4, 0.162, 2.25e-4, 1.69), (12.0, 0.0235, 4.24e-4, 1.00e-4)),
     (3, 128): ((0.8, 0.249, 4.44e-4, 1.48), (14.2, 0.0392, 4.70e-4, 2.06e-4)),
@@ -2249,8 +2253,8 @@ def scan_chunks_pay(portions: ScanPortions, planes: int, heads: int, key_dim: in
     CUs.  Token by token a step is its longest request's chain (half as long again a token where the requests bring fewer than 16 tokens
     each: the shallower kernel), or the states' and tokens' trips where these are longer; the chunks' kernels take that one's place
     for the portions, but the other requests then follow in a launch of their own.  16 heads of 128 x 128, five planes, us token by
-    token and in chunks: one portion of 64 tokens 19 and 21, of 96 31 and 24, of 2,048 590 and 162; beside 64 lone tokens 64 46 and 62, 128
-    68 and 63, 256 119 and 72; beside 200 lone tokens 192 120 and 142, 384 204 and 161; 16 portions of 64 120 and 100.  The chunks have
+    token and in chunks: one portion of 64 tokens 22 and 21, of 96 33 and 23, of 2,048 580 and 169; beside 64 lone tokens 64 46 and 60, 128
+    71 and 63, 256 123 and 70; beside 200 lone tokens 192 123 and 137, 384 196 and 149; 16 portions of 64 121 and 94.  The chunks have
     to gain an eighth: where decays leave their range (known to the kernel alone) their first pass takes up to twice its time."""
     (start, token, work, state), (c_start, c_token, c_head, c_work) = _SCAN_TIMES[planes, key_dim]
     blocks, entries = heads * -(-value_dim // 16), heads * value_dim * key_dim * 1e-6
